@@ -56,10 +56,16 @@ struct MovingShape {
     int64_t n_splits, nodes_per_split;
     int ez_rows;                      // kz rows of one column tile (LDS buffer rows)
     size_t part_bytes;                // (n_splits, M, L, KV) float2 partial tiles
+    bool pairs;                       // L, K count real rows (PairAxis)
 };
 MovingShape moving_shape(const CartesianTables &c, int64_t N, int V);
 void launch_cart_moving_bf16(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,
                              const float *modes, int R, const double *mcoef, float2 *part, hipStream_t st);
+// The same with lines and kz planes as real rows (cart_moving_pairs_bf16.hip);
+// `pairs` is false where the general form is taken.
+MovingShape moving_pairs_shape(const CartesianTables &c, int64_t N, int V);
+void launch_cart_moving_pairs_bf16(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,
+                                   const float *modes, int R, const double *mcoef, float2 *part, hipStream_t st);
 // FP64 form (cart_moving_f64.hip): row and column blocks of 16, double2 partials.
 MovingShape moving_shape_f64(const CartesianTables &c, int64_t N, int V);
 void launch_cart_moving_f64(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,

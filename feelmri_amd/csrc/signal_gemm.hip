@@ -25,7 +25,9 @@
 // FP64 in a fixed order by a second kernel.  Workgroups that share a node
 // split (and so the same E tiles) are mapped onto the same XCD so the tiles
 // are fetched from HBM once per split and served from that XCD's L2.
+#include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "cart_gemm.h"
@@ -36,6 +38,103 @@ namespace fm {
 // ---------------------------------------------------------------------------
 // Sampling analysis (host)
 // ---------------------------------------------------------------------------
+// Real rows of the n offsets of one axis (PairAxis) about the centre c: the
+// offsets sorted, partners found from both ends.  Partners lie within 4e-15
+// of the largest |offset| of c +- D, a few roundings, so the phases differ
+// from the given ones by no more than their own rounding.
+static PairAxis pair_axis_about(const std::vector<double> &g, int64_t n, const double (&c)[3])
+{
+    PairAxis a;
+    double gmax = 0.0;
+    for (double v : g) gmax = std::max(gmax, std::fabs(v));
+    const double tol = 4e-15 * gmax;
+    std::vector<int32_t> order((size_t)n);
+    for (int64_t j = 0; j < n; ++j) order[(size_t)j] = (int32_t)j;
+    std::sort(order.begin(), order.end(), [&](int32_t p, int32_t q) {
+        for (int d = 0; d < 3; ++d) {
+            const double vp = g[(size_t)(3 * p + d)], vq = g[(size_t)(3 * q + d)];
+            if (vp != vq) return vp < vq;
+        }
+        return p < q;
+    });
+    for (int d = 0; d < 3; ++d) a.c[d] = c[d];
+    std::vector<double> D;                 // per entity
+    std::vector<char> centred;
+    auto add = [&](int32_t p, int32_t q) {  // q = -1: no partner
+        bool zero = q < 0;
+        for (int d = 0; d < 3; ++d) {
+            const double gp = g[(size_t)(3 * p + d)];
+            const double v = q < 0 ? gp - c[d] : 0.5 * (gp - g[(size_t)(3 * q + d)]);
+            zero = zero && std::fabs(v) <= tol;
+            D.push_back(v);
+        }
+        if (zero) D[D.size() - 3] = D[D.size() - 2] = D[D.size() - 1] = 0.0;
+        centred.push_back(zero);
+        a.ent.insert(a.ent.end(), {p, q, 0, 0});
+    };
+    int64_t lo = 0, hi = n - 1;
+    while (lo <= hi) {
+        const int32_t p = order[(size_t)lo], q = order[(size_t)hi];
+        if (lo == hi) {
+            add(p, -1);
+            break;
+        }
+        bool match = true;
+        int side = 0;                      // sign of the first component off the centre
+        for (int d = 0; d < 3; ++d) {
+            const double s = g[(size_t)(3 * p + d)] + g[(size_t)(3 * q + d)] - 2.0 * c[d];
+            match = match && std::fabs(s) <= tol;
+            if (side == 0 && std::fabs(s) > tol) side = s > 0.0 ? 1 : -1;
+        }
+        if (match) {
+            add(p, q);
+            ++lo;
+            --hi;
+        } else if (side < 0) {             // p lies further out than q
+            add(p, -1);
+            ++lo;
+        } else {
+            add(q, -1);
+            --hi;
+        }
+    }
+    // cosine rows first, then the sine rows
+    a.n_ent = (int64_t)centred.size();
+    for (int64_t e = 0; e < a.n_ent; ++e) {
+        a.ent[(size_t)(4 * e + 2)] = (int32_t)e;
+        a.rows.insert(a.rows.end(), {D[(size_t)(3 * e)], D[(size_t)(3 * e + 1)], D[(size_t)(3 * e + 2)], 0.25});
+    }
+    a.n_rows = a.n_ent;
+    for (int64_t e = 0; e < a.n_ent; ++e) {
+        if (centred[(size_t)e]) {
+            a.ent[(size_t)(4 * e + 3)] = -1;
+            continue;
+        }
+        a.ent[(size_t)(4 * e + 3)] = (int32_t)a.n_rows++;
+        a.rows.insert(a.rows.end(), {D[(size_t)(3 * e)], D[(size_t)(3 * e + 1)], D[(size_t)(3 * e + 2)], 0.0});
+    }
+    return a;
+}
+
+// The centre that leaves the fewest rows: the middle of the offsets (an even
+// count -n/2 .. n/2 - 1 pairs up completely about its half step), or 0 (where
+// single-precision offsets are symmetric to the last bit).
+static PairAxis pair_axis(const std::vector<double> &g, int64_t n)
+{
+    double mid[3] = {0.0, 0.0, 0.0};
+    const double zero[3] = {0.0, 0.0, 0.0};
+    for (int d = 0; d < 3; ++d) {
+        double lo = g[(size_t)d], hi = lo;
+        for (int64_t j = 1; j < n; ++j) {
+            lo = std::min(lo, g[(size_t)(3 * j + d)]);
+            hi = std::max(hi, g[(size_t)(3 * j + d)]);
+        }
+        mid[d] = 0.5 * (lo + hi);
+    }
+    PairAxis a = pair_axis_about(g, n, mid), b = pair_axis_about(g, n, zero);
+    return b.n_rows < a.n_rows ? b : a;
+}
+
 bool cartesian_analyse(fm_signal_plan *p, const double *kx, const double *ky, const double *kz,
                        const double *t)
 {
@@ -97,6 +196,11 @@ bool cartesian_analyse(fm_signal_plan *p, const double *kx, const double *ky, co
     c.axis_aligned = true;
     for (int64_t j = 0; j < L; ++j) c.axis_aligned &= c.G[(size_t)(3 * j)] == 0.0 && c.G[(size_t)(3 * j + 2)] == 0.0;
     for (int64_t k = 0; k < K; ++k) c.axis_aligned &= c.H[(size_t)(3 * k)] == 0.0 && c.H[(size_t)(3 * k + 1)] == 0.0;
+    c.lines = pair_axis(c.G, L);
+    c.kzs = pair_axis(c.H, K);
+    c.F_pairs = c.F;
+    for (int64_t i = 0; i < R; ++i)
+        for (int d = 0; d < 3; ++d) c.F_pairs[(size_t)(3 * i + d)] += c.lines.c[d] + c.kzs.c[d];
     c.ok = true;
     return true;
 }
@@ -112,6 +216,25 @@ int cartesian_upload(fm_signal_plan *p)
     FM_HIP(hipMemcpy(c.d_G, c.G.data(), sizeof(double) * c.G.size(), hipMemcpyHostToDevice));
     FM_HIP(hipMemcpy(c.d_H, c.H.data(), sizeof(double) * c.H.size(), hipMemcpyHostToDevice));
     FM_HIP(hipMemcpy(c.d_t, c.t.data(), sizeof(double) * c.t.size(), hipMemcpyHostToDevice));
+    {   // the pair tables in one allocation: rows (32 B each), entities (16 B), F
+        size_t off[6] = {0, 0, 0, 0, 0, 0};
+        const void *src[5] = {c.lines.rows.data(), c.kzs.rows.data(), c.lines.ent.data(), c.kzs.ent.data(),
+                              c.F_pairs.data()};
+        const size_t len[5] = {sizeof(double) * c.lines.rows.size(), sizeof(double) * c.kzs.rows.size(),
+                               sizeof(int32_t) * c.lines.ent.size(), sizeof(int32_t) * c.kzs.ent.size(),
+                               sizeof(double) * c.F_pairs.size()};
+        for (int q = 0; q < 5; ++q) off[q + 1] = off[q] + len[q];
+        std::vector<char> host(off[5]);
+        for (int q = 0; q < 5; ++q) std::memcpy(host.data() + off[q], src[q], len[q]);
+        FM_HIP(hipMalloc(&c.d_pairs, off[5]));
+        FM_HIP(hipMemcpy(c.d_pairs, host.data(), off[5], hipMemcpyHostToDevice));
+        char *d = reinterpret_cast<char *>(c.d_pairs);
+        c.lines.d_rows = reinterpret_cast<double4 *>(d + off[0]);
+        c.kzs.d_rows = reinterpret_cast<double4 *>(d + off[1]);
+        c.lines.d_ent = reinterpret_cast<int4 *>(d + off[2]);
+        c.kzs.d_ent = reinterpret_cast<int4 *>(d + off[3]);
+        c.d_F_pairs = reinterpret_cast<double *>(d + off[4]);
+    }
     FM_HIP(hipMalloc(&c.d_ro_group, sizeof(int32_t) * c.ro_group.size()));
     FM_HIP(hipMemcpy(c.d_ro_group, c.ro_group.data(), sizeof(int32_t) * c.ro_group.size(), hipMemcpyHostToDevice));
     return FM_OK;
@@ -125,6 +248,8 @@ void cartesian_free(fm_signal_plan *p)
     (void)hipFree(c.d_H);
     (void)hipFree(c.d_t);
     (void)hipFree(c.d_ro_group);
+    (void)hipFree(c.d_pairs);
+    c.d_pairs = nullptr;
     c.d_F = c.d_G = c.d_H = c.d_t = nullptr;
     c.d_ro_group = nullptr;
 }
@@ -402,6 +527,85 @@ __global__ void k_cart_reduce(const P *__restrict__ part, int64_t n_splits, int6
     out[i] = make_double2(re, im);
 }
 
+// Samples from the partial sums over real rows: part is (n_splits, M, Lr,
+// Kr V) with Lr cosine and sine rows of the lines and, KPAIR, Kr rows of the
+// kz planes (else Kr = K planes with their own complex columns).  One thread
+// group of G sums the splits of one (readout, line entity, kz entity,
+// encoding) in FP64, each thread a contiguous share of them, the shares added
+// in order, and writes the entity's up to four samples:
+//   (C_a -+ i S_a) (C_b -+ i S_b) = CC - s_a s_b SS - i (s_b CS + s_a SC).
+template <typename P, int G, bool KPAIR>
+__global__ __launch_bounds__(256) void k_cart_reduce_pairs(
+    const P *__restrict__ part, int64_t n_splits, int64_t M, int64_t Lr, int64_t KVr, int64_t V,
+    const int4 *__restrict__ lent, int64_t n_lent, const int4 *__restrict__ kent, int64_t n_kent, int64_t L, int64_t K,
+    double2 *__restrict__ out)
+{
+    constexpr int kOut = 256 / G;
+    __shared__ double2 sum[4][G][kOut];
+    const int o = threadIdx.x % kOut, g = threadIdx.x / kOut;
+    const int64_t t = (int64_t)blockIdx.x * kOut + o;
+    const bool live = t < M * n_lent * n_kent * V;
+    const int64_t tc = live ? t : 0;
+    const int64_t v = tc % V, e = (tc / V) % n_kent, f = (tc / (V * n_kent)) % n_lent, i = tc / (V * n_kent * n_lent);
+    const int4 le = lent[f];
+    const int4 ke = KPAIR ? kent[e] : make_int4((int)e, -1, (int)e, -1);
+    const int rows[2] = {le.z, le.w}, cols[2] = {ke.z, ke.w};
+    const int64_t s0 = n_splits * g / G, s1 = n_splits * (g + 1) / G;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int r = rows[c / 2], q = cols[c % 2];
+        double re = 0.0, im = 0.0;
+        if (live && r >= 0 && q >= 0) {
+            const P *src = part + (i * Lr + r) * KVr + q * V + v;
+#pragma unroll 4
+            for (int64_t s = s0; s < s1; ++s) {
+                const P x = src[s * M * Lr * KVr];
+                re += (double)x.x;
+                im += (double)x.y;
+            }
+        }
+        sum[c][g][o] = make_double2(re, im);
+    }
+    __syncthreads();
+    if (g != 0 || !live) return;
+    double2 w[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        w[c] = sum[c][0][o];
+#pragma unroll
+        for (int q = 1; q < G; ++q) {
+            w[c].x += sum[c][q][o].x;
+            w[c].y += sum[c][q][o].y;
+        }
+    }
+    // w: CC, CS (kz sine), SC (line sine), SS
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int j = c / 2 ? le.y : le.x, k = c % 2 ? ke.y : ke.x;
+        if (j < 0 || k < 0) continue;
+        const double sa = c / 2 ? -1.0 : 1.0, sb = c % 2 ? -1.0 : 1.0;
+        const double ar = w[0].x - sa * sb * w[3].x, ai = w[0].y - sa * sb * w[3].y;
+        const double br = sb * w[1].x + sa * w[2].x, bi = sb * w[1].y + sa * w[2].y;
+        out[((i * L + j) * K + k) * V + v] = make_double2(ar + bi, ai - br);
+    }
+}
+
+// Threads per sample group: 16 where the samples alone would leave most of
+// the device idle in a long chain of loads, else 4.
+template <typename P, bool KPAIR>
+static void launch_reduce_pairs(const P *part, int64_t n_splits, int64_t M, int64_t Lr, int64_t KVr, int64_t V,
+                                const CartesianTables &c, double2 *out, hipStream_t st)
+{
+    const int64_t n_kent = KPAIR ? c.kzs.n_ent : c.n_kz;
+    const int64_t n = M * c.lines.n_ent * n_kent * V;
+    if (n < 64 * 1024)
+        k_cart_reduce_pairs<P, 16, KPAIR><<<(unsigned)cdiv(n, 16), 256, 0, st>>>(
+            part, n_splits, M, Lr, KVr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
+    else
+        k_cart_reduce_pairs<P, 4, KPAIR><<<(unsigned)cdiv(n, 64), 256, 0, st>>>(
+            part, n_splits, M, Lr, KVr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
+}
+
 int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, const double *packed, void *wsv,
                       size_t ws_bytes, double *out, hipStream_t st)
 {
@@ -457,10 +661,18 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
     return FM_OK;
 }
 
+// The moving form a shape takes: real rows where the plan has them.
+static MovingShape moving_form(const CartesianTables &c, bool f64, int64_t N, int V)
+{
+    if (f64) return moving_shape_f64(c, N, V);
+    const MovingShape s = moving_pairs_shape(c, N, V);
+    return s.pairs ? s : moving_shape(c, N, V);
+}
+
 size_t cartesian_moving_workspace(const fm_signal_plan *p, int precision, int64_t N, int V)
 {
     if (p->n_samples == 0 || N == 0 || V > kMovMaxV) return 0;
-    return (precision == FM_PREC_F64 ? moving_shape_f64(p->cart, N, V) : moving_shape(p->cart, N, V)).part_bytes;
+    return moving_form(p->cart, precision == FM_PREC_F64, N, V).part_bytes;
 }
 
 int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, int V, const double *packed,
@@ -478,7 +690,7 @@ int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, 
         return FM_ERR_UNSUPPORTED;
     }
     const bool f64 = precision == FM_PREC_F64;
-    const MovingShape s = f64 ? moving_shape_f64(c, N, V) : moving_shape(c, N, V);
+    const MovingShape s = moving_form(c, f64, N, V);
     if (s.part_bytes > ws_bytes) {
         set_error("signal workspace too small: need %zu bytes, got %zu", s.part_bytes, ws_bytes);
         return FM_ERR_WORKSPACE;
@@ -499,10 +711,14 @@ int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, 
                                                                           reinterpret_cast<double2 *>(out));
     } else {
         float2 *part = reinterpret_cast<float2 *>(ws);
-        launch_cart_moving_bf16(s, c, packed, N, modes, R, mcoef, part, st);
+        if (s.pairs) launch_cart_moving_pairs_bf16(s, c, packed, N, modes, R, mcoef, part, st);
+        else launch_cart_moving_bf16(s, c, packed, N, modes, R, mcoef, part, st);
         plan_timing_stop(p, st);
         FM_LAUNCH_CHECK("k_cart_moving_bf16");
-        k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
+        if (s.pairs)
+            launch_reduce_pairs<float2, true>(part, s.n_splits, s.M, s.L, s.KV, s.V, c, reinterpret_cast<double2 *>(out),
+                                              st);
+        else k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
                                                                          reinterpret_cast<double2 *>(out));
     }
     FM_LAUNCH_CHECK("k_cart_reduce");

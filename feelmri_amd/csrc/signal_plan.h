@@ -46,6 +46,24 @@ struct SignalTile {
     int32_t pad;
 };
 
+// One axis of a Cartesian stack (its lines or its kz planes) as real rows.
+// Offsets that lie symmetrically about a centre c pair up as c + D and c - D,
+// and
+//   exp(-2 pi i (c +- D).x) = exp(-2 pi i c.x) (cos 2 pi D.x -+ i sin 2 pi D.x):
+// the pair's two sums over the nodes are P -+ i Q with P and Q the sums over
+// one cosine and one sine row.  A contraction with real rows takes half the
+// multiplications of one with the complex factors; the centre's phase joins
+// another factor.  An offset without a partner takes both rows for itself, an
+// offset at the centre the cosine row only.
+struct PairAxis {
+    double c[3] = {0.0, 0.0, 0.0};
+    int64_t n_rows = 0, n_ent = 0;
+    std::vector<double> rows;    // (n_rows, 4): D, then the quarter turn added to D.x: 1/4 cosine, 0 sine
+    std::vector<int32_t> ent;    // (n_ent, 4): index of c + D, of c - D or -1, cosine row, sine row or -1
+    double4 *d_rows = nullptr;
+    int4 *d_ent = nullptr;
+};
+
 struct CartesianTables {
     bool ok = false;
     int64_t n_ro = 0, n_ln = 0, n_kz = 0;
@@ -59,6 +77,12 @@ struct CartesianTables {
     bool axis_aligned = false;
     double *d_F = nullptr, *d_G = nullptr, *d_H = nullptr, *d_t = nullptr;
     int32_t *d_ro_group = nullptr;
+    // lines and kz planes as real rows, and F with the centres' offset added:
+    // of both axes
+    PairAxis lines, kzs;
+    std::vector<double> F_pairs;
+    double *d_F_pairs = nullptr;
+    void *d_pairs = nullptr;     // one allocation behind the pair tables
 };
 
 }  // namespace fm
