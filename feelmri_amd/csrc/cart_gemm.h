@@ -21,6 +21,9 @@ struct GemmShape {
     int64_t n_rt, n_ct;    // row tiles, column tiles (per workgroup)
     int64_t ksteps;        // K steps in total
     int64_t n_splits, steps_per_split;
+    // real rows (PairAxis): rows are the lines' cosine and sine rows, columns
+    // (readout index, kz, encoding), and the Ey table holds the readout factors
+    bool pairs;
     // workspace offsets (bytes)
     size_t off_E, off_Ey, off_Ez, off_part, total;
 };

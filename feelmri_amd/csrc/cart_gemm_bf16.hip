@@ -13,7 +13,11 @@
 // global -> LDS DMA (global_load_lds_dwordx4), one step ahead.  One barrier
 // per step.
 //
-// Two kernels differ in where the A operand (Ey * Ezb per column, split into
+// Lines that pair up about a centre (PairAxis) are taken as real rows instead
+// (k_cart_gemm_pairs_bf16 below, and k_cart_gemm_bf16<RB, true>): 6 MFMAs per
+// row block and step.
+//
+// The kernels differ in where the A operand (Ey * Ezb per column, split into
 // bf16 hi and lo) comes from:
 //   * k_cart_gemm_bf16_lds: 8 waves (256 columns) per workgroup when RB is
 //     even, else 4; the distinct Ey and Ezb rows of the workgroup's
@@ -24,9 +28,10 @@
 //   * k_cart_gemm_bf16: every lane loads its column's Ey/Ezb values from
 //     global memory one step ahead and builds the A operand after the
 //     step's MFMAs; any shape.
-#include "cart_gemm.h"
-
+#include <algorithm>
 #include <type_traits>
+
+#include "cart_gemm.h"
 
 namespace fm {
 
@@ -92,27 +97,31 @@ __device__ inline bf16x8 neg_bf16x8(bf16x8 v)
     return __builtin_bit_cast(bf16x8, u);
 }
 
-// Copy one E stage (RB tiles of 4 KB) into LDS: each wave moves RB KB,
-// 1 KB (64 lanes x 16 B) per instruction.
-template <int RB>
+// Copy one E stage (CHUNKS pieces of 1 KB, 64 lanes x 16 B per instruction)
+// into LDS: wave w of 4 moves pieces w, w + 4, ...
+template <int CHUNKS>
 __device__ inline void stage_E_to_lds(const uint4 *__restrict__ src, uint4 *dst, int wave, int lane)
 {
 #pragma unroll
-    for (int e = 0; e < RB; ++e) {
-        const int chunk = wave * RB + e;  // 1 KB chunks, RB*4 per stage
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void *)(src + chunk * 64 + lane),
-            (__attribute__((address_space(3))) void *)(dst + chunk * 64), 16, 0, 0);
+    for (int e = 0; e < (CHUNKS + 3) / 4; ++e) {
+        const int chunk = wave + 4 * e;
+        if (CHUNKS % 4 == 0 || chunk < CHUNKS)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)(src + chunk * 64 + lane),
+                (__attribute__((address_space(3))) void *)(dst + chunk * 64), 16, 0, 0);
     }
 }
 
-template <int RB>
+// REAL: real rows (PairAxis), an E tile holds 2 planes (hi, lo) and a row
+// block takes 6 MFMAs a step.
+template <int RB, bool REAL>
 __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_bf16(
     const uint4 *__restrict__ E, const float2 *__restrict__ Ey, const float2 *__restrict__ Ez, int64_t Np,
     int64_t Mp, int64_t M, int64_t NC, int64_t n_kzV, int64_t n_rt, int64_t n_ct, int64_t n_splits,
     int64_t steps_per_split, int64_t ksteps, float2 *__restrict__ part)
 {
-    constexpr int kStage = RB * 4 * 64;  // uint4 per stage
+    constexpr int kPl = REAL ? 2 : 4;    // planes of an E tile
+    constexpr int kStage = RB * kPl * 64;  // uint4 per stage
     __shared__ uint4 sE[2][kStage];
     int64_t split, rt, ct;
     gemm_tile_ids(n_rt, n_ct, n_splits, split, rt, ct);
@@ -137,7 +146,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_bf16(
 
     BFrag cur;
     if (k0 < k1) {
-        stage_E_to_lds<RB>(E + (k0 * nrb + rt * RB) * 4 * 64, sE[0], wave, lane);
+        stage_E_to_lds<RB * kPl>(E + (k0 * nrb + rt * RB) * kPl * 64, sE[0], wave, lane);
         float4 y[4], z[4];
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
@@ -154,7 +163,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_bf16(
         // buffer): unconditional, so the loaded registers are used in place
         // and nothing waits on them before the MFMAs below.
         const int64_t kn = (ks + 1 < k1) ? ks + 1 : ks;
-        stage_E_to_lds<RB>(E + (kn * nrb + rt * RB) * 4 * 64, sE[buf ^ 1], wave, lane);
+        stage_E_to_lds<RB * kPl>(E + (kn * nrb + rt * RB) * kPl * 64, sE[buf ^ 1], wave, lane);
         float4 ny[4], nz[4];
 #pragma unroll
         for (int h = 0; h < 4; ++h) {
@@ -167,11 +176,13 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_bf16(
         bf16x8 erh[RB], erl[RB], eih[RB], eil[RB];
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
-            const uint4 *t = &sE[buf][r * 4 * 64];
+            const uint4 *t = &sE[buf][r * kPl * 64];
             erh[r] = __builtin_bit_cast(bf16x8, t[0 * 64 + lane]);
             erl[r] = __builtin_bit_cast(bf16x8, t[1 * 64 + lane]);
-            eih[r] = __builtin_bit_cast(bf16x8, t[2 * 64 + lane]);
-            eil[r] = __builtin_bit_cast(bf16x8, t[3 * 64 + lane]);
+            if constexpr (!REAL) {
+                eih[r] = __builtin_bit_cast(bf16x8, t[2 * 64 + lane]);
+                eil[r] = __builtin_bit_cast(bf16x8, t[3 * 64 + lane]);
+            }
         }
 #define FM_MFMA(ACC, A, B)                                                                   \
     _Pragma("unroll") for (int r = 0; r < RB; ++r) ACC[r] =                                  \
@@ -182,12 +193,14 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_bf16(
         FM_MFMA(acc_im, erh, cur.il)
         FM_MFMA(acc_re, erl, cur.rh)
         FM_MFMA(acc_im, erl, cur.ih)
-        FM_MFMA(acc_re, eih, nih)
-        FM_MFMA(acc_im, eih, cur.rh)
-        FM_MFMA(acc_re, eih, nil)
-        FM_MFMA(acc_im, eih, cur.rl)
-        FM_MFMA(acc_re, eil, nih)
-        FM_MFMA(acc_im, eil, cur.rh)
+        if constexpr (!REAL) {
+            FM_MFMA(acc_re, eih, nih)
+            FM_MFMA(acc_im, eih, cur.rh)
+            FM_MFMA(acc_re, eih, nil)
+            FM_MFMA(acc_im, eih, cur.rl)
+            FM_MFMA(acc_re, eil, nih)
+            FM_MFMA(acc_im, eil, cur.rh)
+        }
 #undef FM_MFMA
         // keep the next step's operand build after the MFMA issue, so the
         // wait for its global loads does not stall the MFMAs
@@ -456,6 +469,216 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_cart_gemm_bf16_lds(
     }
 }
 
+// Workgroup barrier behind which all but this wave's latest N copies have
+// landed (copies complete in order; LDS reads before it are done).
+template <int N>
+__device__ inline void barrier_but_vmcnt()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));  // vmcnt(N) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Real rows (PairAxis): S = sum_n A[r,n] (Ex[i,n] Ezb[kv,n]) with A the cosine
+// and sine rows of the lines, bf16 hi and lo planes (2 KB per 32-row tile and
+// 16-node step), and columns (readout index i, kz, encoding).
+//
+// WAVES waves of 32 columns share the E tiles.  As in k_cart_gemm_bf16_lds the
+// distinct Ex and Ezb rows of the columns are staged and the column operand of
+// step ks + 1 is built while the matrix cores run step ks; with 6 MFMAs a row
+// block and step instead of 12 a step is short against the memory latency, so
+// the copies run two steps ahead (rows: three) and a wave waits only for those
+// of earlier steps: every wave issues the same number of copies a step (NP of
+// the rows; waves past the last repeat one), so that one vmcnt tells this
+// step's from the others.  Per step ks, ring slot ks % 3:
+//   E(ks + 2) goes to slot (ks + 2) % 3, last read in step ks - 1;
+//   rows(ks + 3) go to slot ks % 3, last read in step ks - 1 (operand of ks);
+//   the wait and barrier at the end of step ks make E(ks + 1) and rows(ks + 2)
+//   visible, which were issued in step ks - 1.
+// Bound by the MFMAs (24 of 32 x 32 x 16 a wave-step at RB = 4) plus the
+// operand build's VALU issue.  512 000 nodes, 128 x 128 x 32, whole call:
+// 2.64 ms against 4.67 ms with complex rows (813 against 460 TFLOP/s of 8 flops
+// per node * sample), error against 64 bits 2.6e-6 against 3.8e-6; 10 007
+// nodes, 64 x 64: 42 against 52 us.
+template <int RB, int WAVES, int NP>
+__global__ __launch_bounds__(64 * WAVES, 2) void k_cart_gemm_pairs_bf16(
+    const uint4 *__restrict__ E, const float2 *__restrict__ Ex, const float2 *__restrict__ Ez, int64_t Np,
+    int64_t Mp, int64_t M, int64_t NC, int64_t n_kzV, int64_t n_rt, int64_t n_ct, int64_t n_splits,
+    int64_t steps_per_split, int64_t ksteps, float2 *__restrict__ part)
+{
+    constexpr int kThreads = 64 * WAVES;
+    constexpr int kCols = 32 * WAVES;
+    constexpr int kChunks = RB * 2;                       // 1 KB pieces of an E stage
+    constexpr int kEPer = (kChunks + WAVES - 1) / WAVES;  // copied by one wave
+    // each ring slot a variable of its own: an LDS read then names no variable
+    // that a copy in flight writes
+    __shared__ uint4 sE0[kChunks * 64], sE1[kChunks * 64], sE2[kChunks * 64];
+    __shared__ uint4 sY0[NP * kThreads], sY1[NP * kThreads], sY2[NP * kThreads];
+    int64_t split, rt, ct;
+    gemm_tile_ids(n_rt, n_ct, n_splits, split, rt, ct);
+    const int tid = threadIdx.x, lane = tid % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int64_t nrb = Mp / 32;
+    const int64_t k0 = split * steps_per_split;
+    const int64_t k1 = (k0 + steps_per_split < ksteps) ? k0 + steps_per_split : ksteps;
+
+    const int64_t c0 = ct * kCols;
+    const int64_t clast = (c0 + kCols - 1 < NC) ? c0 + kCols - 1 : NC - 1;
+    const int64_t jf = c0 / n_kzV;
+    const int nJ = (int)(clast / n_kzV - jf) + 1;
+    const int nK = (int)(n_kzV < kCols ? n_kzV : kCols);
+    // kYZStride (nJ + nK) <= NP kThreads
+
+    // staging: LDS slot s = tid + kThreads p holds piece s%9 of row s/9 (the
+    // pad slot 8 repeats piece 7); rows are 144 B apart, so lanes reading the
+    // same piece of consecutive rows hit distinct banks.  Slots past the last
+    // row repeat the first.
+    const float2 *stg[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int s = tid + kThreads * p;
+        const int row = s / kYZStride;
+        const int prt = (s % kYZStride) < 8 ? s % kYZStride : 7;
+        const float2 *base = Ex + jf * Np;
+        if (row < nJ + nK) base = row < nJ ? Ex + (jf + row) * Np : Ez + ((c0 + row - nJ) % n_kzV) * Np;
+        stg[p] = base + 2 * prt;
+    }
+
+    // this lane's output column (clamped for padding lanes; results discarded)
+    const int64_t col = c0 + wave * 32 + (lane % 32);
+    const int64_t colc = col < NC ? col : NC - 1;
+    const int ys = (int)(colc / n_kzV - jf);
+    const int zs = nJ + (int)((colc - c0) % nK);
+    const int hb = lane / 32;
+    const int yoff = ys * kYZStride + 4 * hb, zoff = zs * kYZStride + 4 * hb;
+    const uint4 *const E_rt = E + rt * RB * 2 * 64;
+
+    f32x16 acc_re[RB], acc_im[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc_re[r][q] = acc_im[r][q] = 0.0f;
+
+    auto stage_e = [&](int64_t ks, uint4 *dst) {
+        const uint4 *src = E_rt + ks * nrb * 2 * 64;
+#pragma unroll
+        for (int e = 0; e < kEPer; ++e) {
+            const int chunk = (wave + WAVES * e) % kChunks;
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)(src + chunk * 64 + lane),
+                (__attribute__((address_space(3))) void *)(dst + chunk * 64), 16, 0, 0);
+        }
+    };
+    auto stage_yz = [&](int64_t ks, uint4 *dst) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void *)(stg[p] + ks * 16),
+                (__attribute__((address_space(3))) void *)(dst + wave * 64 + kThreads * p), 16, 0, 0);
+    };
+    auto ybuf = [&](auto b) -> uint4 * {
+        if constexpr (decltype(b)::value == 0) return sY0;
+        else if constexpr (decltype(b)::value == 1) return sY1;
+        else return sY2;
+    };
+    auto ebuf = [&](auto b) -> uint4 * {
+        if constexpr (decltype(b)::value == 0) return sE0;
+        else if constexpr (decltype(b)::value == 1) return sE1;
+        else return sE2;
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+
+    BFrag cur;
+    if (k0 < k1) {
+        const int64_t a1 = std::min(k0 + 1, k1 - 1), a2 = std::min(k0 + 2, k1 - 1);
+        stage_e(k0, sE0);
+        stage_yz(k0, sY0);
+        stage_yz(a1, sY1);
+        stage_e(a1, sE1);
+        stage_yz(a2, sY2);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        float4 y[4], z[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            y[h] = __builtin_bit_cast(float4, sY0[yoff + h]);
+            z[h] = __builtin_bit_cast(float4, sY0[zoff + h]);
+        }
+        cur = make_bfrag(y, z);
+        __syncthreads();  // step k0 copies into slot 0 of the rows
+    }
+
+    auto step = [&](int64_t ks, auto B) {
+        constexpr int b = decltype(B)::value;
+        using N1 = std::integral_constant<int, (b + 1) % 3>;
+        using N2 = std::integral_constant<int, (b + 2) % 3>;
+        stage_e(std::min(ks + 2, k1 - 1), ebuf(N2{}));
+        stage_yz(std::min(ks + 3, k1 - 1), ybuf(B));
+        __builtin_amdgcn_sched_barrier(0);
+
+        const uint4 *tE = ebuf(B) + lane;
+        const uint4 *tY = ybuf(N1{});
+        BFrag nxt;
+        bf16x8 eh[RB], el[RB];
+        float4 y[4], z[4];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) eh[r] = __builtin_bit_cast(bf16x8, tE[(r * 2 + 0) * 64]);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            y[h] = __builtin_bit_cast(float4, tY[yoff + h]);
+            z[h] = __builtin_bit_cast(float4, tY[zoff + h]);
+        }
+#pragma unroll
+        for (int r = 0; r < RB; ++r) el[r] = __builtin_bit_cast(bf16x8, tE[(r * 2 + 1) * 64]);
+#define FM_MFMA(ACC, A, Bv)                                                                  \
+    _Pragma("unroll") for (int r = 0; r < RB; ++r) ACC[r] =                                  \
+        __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[r], Bv, ACC[r], 0, 0, 0);
+        FM_MFMA(acc_re, eh, cur.rh)
+        FM_MFMA(acc_im, eh, cur.ih)
+        FM_MFMA(acc_re, eh, cur.rl)
+        FM_MFMA(acc_im, eh, cur.il)
+        FM_MFMA(acc_re, el, cur.rh)
+        FM_MFMA(acc_im, el, cur.ih)
+#undef FM_MFMA
+#pragma unroll
+        for (int h = 0; h < 4; ++h) build_chunk(nxt, h, y[h], z[h]);
+        // the build's VALU between the MFMAs, spread over all of them
+#pragma unroll
+        for (int i = 0; i < 6 * RB; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x002, (96 + 6 * RB - 1) / (6 * RB), 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        cur = nxt;
+        barrier_but_vmcnt<kEPer + NP>();
+    };
+
+    int64_t ks = k0;
+    for (; ks + 3 <= k1; ks += 3) {
+        step(ks, I0{});
+        step(ks + 1, I1{});
+        step(ks + 2, I2{});
+    }
+    if (ks < k1) step(ks, I0{});
+    if (ks + 1 < k1) step(ks + 1, I1{});
+    __builtin_amdgcn_s_waitcnt(0);  // no copy in flight past the end
+
+    if (col < NC) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int64_t row = (rt * RB + r) * 32 + 8 * (q / 4) + 4 * (lane / 32) + (q % 4);
+                if (row < M) part[(split * M + row) * NC + col] = make_float2(acc_re[r][q], acc_im[r][q]);
+            }
+        }
+    }
+}
+
 // Largest number of distinct Ey + Ezb rows any workgroup's `cols` columns use.
 static int max_yz_rows(int64_t NC, int64_t n_kzV, int64_t cols)
 {
@@ -483,15 +706,49 @@ static bool launch_bf16_lds(const GemmShape &s, char *ws, int64_t n_kzV, hipStre
     return true;
 }
 
+// Staged kernel over real rows with WAVES waves and NP row pieces a thread,
+// where the column tiles' rows fit them.
+template <int RB, int WAVES, int NP>
+static bool launch_pairs_lds(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t st)
+{
+    constexpr int kCols = 32 * WAVES;
+    if (max_yz_rows(s.NC, n_kzV, kCols) * kYZStride > NP * 64 * WAVES) return false;
+    const int64_t n_ct = cdiv(s.NC, kCols);
+    const unsigned grid = (unsigned)(s.n_rt * n_ct * s.n_splits);
+    k_cart_gemm_pairs_bf16<RB, WAVES, NP><<<grid, 64 * WAVES, 0, st>>>(
+        reinterpret_cast<const uint4 *>(ws + s.off_E), reinterpret_cast<const float2 *>(ws + s.off_Ey),
+        reinterpret_cast<const float2 *>(ws + s.off_Ez), s.Np, s.Mp, s.M, s.NC, n_kzV, s.n_rt, n_ct, s.n_splits,
+        s.steps_per_split, s.ksteps, reinterpret_cast<float2 *>(ws + s.off_part));
+    return true;
+}
+
+// 2, 4 or 8 waves by the columns there are (a tile has 32 a wave), and the
+// fewest pieces that hold the tile's rows.
+template <int RB>
+static bool launch_pairs(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t st)
+{
+    if (s.NC <= 64) return launch_pairs_lds<RB, 2, 5>(s, ws, n_kzV, st);
+    if (s.NC > 128 && (launch_pairs_lds<RB, 8, 1>(s, ws, n_kzV, st) || launch_pairs_lds<RB, 8, 2>(s, ws, n_kzV, st)))
+        return true;
+    return launch_pairs_lds<RB, 4, 1>(s, ws, n_kzV, st) || launch_pairs_lds<RB, 4, 3>(s, ws, n_kzV, st);
+}
+
 template <int RB>
 static void launch_bf16(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t st)
 {
     const unsigned grid = (unsigned)(s.n_rt * s.n_ct * s.n_splits);
+#define FM_GEMM_ARGS                                                                                              \
+    reinterpret_cast<const uint4 *>(ws + s.off_E), reinterpret_cast<const float2 *>(ws + s.off_Ey),              \
+        reinterpret_cast<const float2 *>(ws + s.off_Ez), s.Np, s.Mp, s.M, s.NC, n_kzV, s.n_rt, s.n_ct, s.n_splits, \
+        s.steps_per_split, s.ksteps, reinterpret_cast<float2 *>(ws + s.off_part)
+    if (s.pairs) {
+        if (launch_pairs<RB>(s, ws, n_kzV, st)) return;
+        k_cart_gemm_bf16<RB, true><<<grid, kGemmThreads, 0, st>>>(FM_GEMM_ARGS);
+        return;
+    }
     if (launch_bf16_lds<RB, lds_waves<RB>()>(s, ws, n_kzV, st)) return;
-    k_cart_gemm_bf16<RB><<<grid, kGemmThreads, 0, st>>>(
-        reinterpret_cast<const uint4 *>(ws + s.off_E), reinterpret_cast<const float2 *>(ws + s.off_Ey),
-        reinterpret_cast<const float2 *>(ws + s.off_Ez), s.Np, s.Mp, s.M, s.NC, n_kzV, s.n_rt, s.n_ct, s.n_splits,
-        s.steps_per_split, s.ksteps, reinterpret_cast<float2 *>(ws + s.off_part));
+    k_cart_gemm_bf16<RB, false><<<grid, kGemmThreads, 0, st>>>(FM_GEMM_ARGS);
+#undef FM_GEMM_ARGS
 }
 
 void launch_cart_gemm_bf16(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t st)

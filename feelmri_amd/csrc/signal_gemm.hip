@@ -17,6 +17,11 @@
 // operand in registers from Ey and Ezb, so the (N x lines*kz*V) matrix A is
 // never stored.
 //
+// Lines that pair up about a centre are taken as real rows (PairAxis,
+// signal_plan.h): the roles turn, S[r, (i,k,v)] = sum_n A[r,n] (Ex[i,n]
+// Ezb[(k,v),n]) with A the lines' cosine and sine rows and Ex the readout
+// factors, half the products, and the reduction forms each pair's samples.
+//
 // Mixed form: E and A are split into bf16 hi + lo parts and each real product
 // x*y is formed as xh*yh + xh*yl + xl*yh on v_mfma_f32_32x32x16_bf16 with
 // FP32 accumulation (12 MFMAs per 16 nodes per 32x32 complex tile).  FP64
@@ -198,9 +203,13 @@ bool cartesian_analyse(fm_signal_plan *p, const double *kx, const double *ky, co
     for (int64_t k = 0; k < K; ++k) c.axis_aligned &= c.H[(size_t)(3 * k)] == 0.0 && c.H[(size_t)(3 * k + 1)] == 0.0;
     c.lines = pair_axis(c.G, L);
     c.kzs = pair_axis(c.H, K);
-    c.F_pairs = c.F;
+    c.F_pairs.assign((size_t)R * 6, 0.0);
     for (int64_t i = 0; i < R; ++i)
-        for (int d = 0; d < 3; ++d) c.F_pairs[(size_t)(3 * i + d)] += c.lines.c[d] + c.kzs.c[d];
+        for (int d = 0; d < 3; ++d) {
+            const double f = c.F[(size_t)(3 * i + d)] + c.lines.c[d];
+            c.F_pairs[(size_t)(3 * i + d)] = f;
+            c.F_pairs[(size_t)(3 * (R + i) + d)] = f + c.kzs.c[d];
+        }
     c.ok = true;
     return true;
 }
@@ -233,7 +242,8 @@ int cartesian_upload(fm_signal_plan *p)
         c.kzs.d_rows = reinterpret_cast<double4 *>(d + off[1]);
         c.lines.d_ent = reinterpret_cast<int4 *>(d + off[2]);
         c.kzs.d_ent = reinterpret_cast<int4 *>(d + off[3]);
-        c.d_F_pairs = reinterpret_cast<double *>(d + off[4]);
+        c.d_F_lines = reinterpret_cast<double *>(d + off[4]);
+        c.d_F_pairs = c.d_F_lines + 3 * c.n_ro;
     }
     FM_HIP(hipMalloc(&c.d_ro_group, sizeof(int32_t) * c.ro_group.size()));
     FM_HIP(hipMemcpy(c.d_ro_group, c.ro_group.data(), sizeof(int32_t) * c.ro_group.size(), hipMemcpyHostToDevice));
@@ -257,22 +267,26 @@ void cartesian_free(fm_signal_plan *p)
 
 // mixed: row block 32, K stage 16 nodes, column block 32 per wave (4 per WG)
 // f64:   row block 16, K stage 16 nodes (4 MFMA k-steps), column block 16 per wave
-static GemmShape gemm_shape(const fm_signal_plan *p, int precision, int64_t N, int V)
+// Complex rows (pairs = false): rows are the readout indices, columns (line,
+// kz, encoding).  Real rows: the lines' cosine and sine rows, columns
+// (readout index, kz, encoding).
+static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, int V, bool pairs)
 {
     GemmShape s{};
-    const CartesianTables &c = p->cart;
-    s.mixed = precision != FM_PREC_F64;
+    s.mixed = mixed;
+    s.pairs = pairs;
     const int rowblk = s.mixed ? 32 : 16;
     const int colblk = s.mixed ? 32 : 16;
-    const int max_rb = s.mixed ? 4 : 4;
+    const int max_rb = 4;
+    const int64_t outer = pairs ? c.n_ro : c.n_ln;  // the columns' outer index
     s.N = N;
     s.Np = cdiv(std::max<int64_t>(N, 1), 16) * 16;
-    s.M = c.n_ro;
+    s.M = pairs ? c.lines.n_rows : c.n_ro;
     const int64_t nrb = cdiv(s.M, rowblk);
     s.rb_per_wave = (int)std::min<int64_t>(max_rb, nrb);
     s.n_rt = cdiv(nrb, s.rb_per_wave);
     s.Mp = s.n_rt * s.rb_per_wave * rowblk;
-    s.NC = c.n_ln * c.n_kz * V;
+    s.NC = outer * c.n_kz * V;
     s.n_ct = cdiv(s.NC, 4 * colblk);
     s.NCp = s.n_ct * 4 * colblk;
     s.ksteps = s.Np / 16;
@@ -294,19 +308,33 @@ static GemmShape gemm_shape(const fm_signal_plan *p, int precision, int64_t N, i
         off += (bytes + 255) & ~size_t(255);
         return o;
     };
+    const size_t planes = pairs ? 1 : 2;                                     // Re (and Im)
     if (s.mixed) {
-        s.off_E = take((size_t)s.Mp * s.Np * 4 * sizeof(uint16_t));          // 4 bf16 planes
-        s.off_Ey = take((size_t)c.n_ln * s.Np * sizeof(float2));
+        s.off_E = take((size_t)s.Mp * s.Np * planes * 2 * sizeof(uint16_t));  // each as bf16 hi, lo
+        s.off_Ey = take((size_t)outer * s.Np * sizeof(float2));
         s.off_Ez = take((size_t)c.n_kz * V * s.Np * sizeof(float2));
         s.off_part = take((size_t)s.n_splits * s.M * s.NC * sizeof(float2));
     } else {
-        s.off_E = take((size_t)s.Mp * s.Np * 2 * sizeof(double));            // Re, Im planes
-        s.off_Ey = take((size_t)c.n_ln * s.Np * sizeof(double2));
+        s.off_E = take((size_t)s.Mp * s.Np * planes * sizeof(double));
+        s.off_Ey = take((size_t)outer * s.Np * sizeof(double2));
         s.off_Ez = take((size_t)c.n_kz * V * s.Np * sizeof(double2));
         s.off_part = take((size_t)s.n_splits * s.M * s.NC * sizeof(double2));
     }
     s.total = off;
     return s;
+}
+
+// Real rows where they take fewer MFMAs (half as many per row and column
+// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32) and no more
+// workspace than complex rows do.
+static GemmShape gemm_shape(const fm_signal_plan *p, int precision, int64_t N, int V)
+{
+    const CartesianTables &c = p->cart;
+    const bool mixed = precision != FM_PREC_F64;
+    const GemmShape g = gemm_shape_of(c, mixed, N, V, false);
+    if (!mixed) return g;
+    const GemmShape s = gemm_shape_of(c, mixed, N, V, true);
+    return s.Mp * s.NCp < 2 * g.Mp * g.NCp && s.total <= g.total ? s : g;
 }
 
 size_t cartesian_workspace(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc)
@@ -444,35 +472,104 @@ __device__ __forceinline__ void cart_E_bf16(int64_t t, const double *__restrict_
     }
 }
 
-// Ey rows exp(-2 pi i (G_j . x_n)) and Ezb rows exp(-2 pi i (H_k . x_n)) b_v[n]
-// (the encoding's weighted magnetisation folded into the kz factor).  One
-// thread per node keeps its position in registers and walks a block of
-// kYZRowsPerBlock rows (Ey rows first, then Ezb).
+// Real rows, mixed: tiles of (32 rows x 16 nodes) per 2 planes (hi, lo) in the
+// lane order of cart_E_bf16; row r holds sin 2 pi (D_r . x + quarter turn of a
+// cosine row).
+__device__ __forceinline__ void cart_rows_bf16(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
+                                               int64_t M, int64_t Mp, const double4 *__restrict__ rows,
+                                               uint4 *__restrict__ E)
+{
+    // t over (Np / 16) * 64
+    if (t >= (Np / 16) * 64) return;
+    const int lane = (int)(t % 64);
+    const int64_t kb = t / 64;
+    const int64_t nrb = Mp / 32;
+    const int64_t n0 = kb * 16 + 8 * (lane / 32);
+    double x[8], y[8], z[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int64_t n = n0 + q;
+        const bool ok = n < N;
+        x[q] = ok ? packed[n] : 0.0;
+        y[q] = ok ? packed[N + n] : 0.0;
+        z[q] = ok ? packed[2 * N + n] : 0.0;
+    }
+    const int nvalid = (int)(N - n0 < 8 ? (N - n0 > 0 ? N - n0 : 0) : 8);
+    for (int64_t rb = 0; rb < nrb; ++rb) {
+        const int64_t i = rb * 32 + (lane % 32);
+        const bool row_ok = i < M;
+        const double4 d = rows[row_ok ? i : 0];
+        unsigned short h[2][8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            float e = 0.0f;
+            if (row_ok && q < nvalid)
+                e = __builtin_amdgcn_sinf(turns_f32(fma(d.x, x[q], fma(d.y, y[q], fma(d.z, z[q], d.w)))));
+            const __bf16 eh = (__bf16)e;
+            const __bf16 el = (__bf16)(e - (float)eh);
+            h[0][q] = __builtin_bit_cast(unsigned short, eh);
+            h[1][q] = __builtin_bit_cast(unsigned short, el);
+        }
+        const int64_t tile = kb * nrb + rb;
+#pragma unroll
+        for (int pl = 0; pl < 2; ++pl) {
+            uint4 v;
+            v.x = (unsigned)h[pl][0] | ((unsigned)h[pl][1] << 16);
+            v.y = (unsigned)h[pl][2] | ((unsigned)h[pl][3] << 16);
+            v.z = (unsigned)h[pl][4] | ((unsigned)h[pl][5] << 16);
+            v.w = (unsigned)h[pl][6] | ((unsigned)h[pl][7] << 16);
+            E[(tile * 2 + pl) * 64 + lane] = v;
+        }
+    }
+}
+
+// The columns' outer rows -- complex rows: Ey, exp(-2 pi i (G_j . x_n)) of the
+// lines; real rows: Ex, exp(-t_i/T2) exp(i phi t_i) exp(-2 pi i F_i . x) of the
+// readout indices -- and Ezb rows exp(-2 pi i (H_k . x_n)) b_v[n] (the
+// encoding's weighted magnetisation folded into the kz factor).  One thread
+// per node keeps its position in registers and walks a block of
+// kYZRowsPerBlock rows (outer rows first, then Ezb).
 constexpr int kYZRowsPerBlock = 16;
 
-template <bool MIXED>
+template <bool MIXED, bool PAIRS>
 __device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, const double *__restrict__ packed, int64_t N,
-                                        int64_t Np, int V, int64_t n_ln, int64_t n_kz,
-                                        const double *__restrict__ G, const double *__restrict__ H,
-                                        void *__restrict__ Ey, void *__restrict__ Ez)
+                                        int64_t Np, int V, int64_t n_out, int64_t n_kz,
+                                        const double *__restrict__ G, const double *__restrict__ tr,
+                                        const double *__restrict__ H, void *__restrict__ Ey, void *__restrict__ Ez)
 {
     if (n >= Np) return;
     const int64_t r0 = rblk * kYZRowsPerBlock;
-    const int64_t r1 = (r0 + kYZRowsPerBlock < n_ln + n_kz) ? r0 + kYZRowsPerBlock : n_ln + n_kz;
+    const int64_t r1 = (r0 + kYZRowsPerBlock < n_out + n_kz) ? r0 + kYZRowsPerBlock : n_out + n_kz;
     const bool ok = n < N;
     const double x = ok ? packed[n] : 0.0, y = ok ? packed[N + n] : 0.0, z = ok ? packed[2 * N + n] : 0.0;
+    double phi = 0.0, r2 = 0.0;
+    if (PAIRS && ok) {
+        phi = packed[3 * N + n];
+        r2 = packed[4 * N + n];
+    }
     for (int64_t row = r0; row < r1; ++row) {
-        const bool is_y = row < n_ln;
-        const double *kv = is_y ? &G[3 * row] : &H[3 * (row - n_ln)];
+        const bool outer = row < n_out;
+        const double *kv = outer ? &G[3 * row] : &H[3 * (row - n_out)];
         double c = 0.0, s = 0.0;
-        if (ok) cis_neg_cycles<MIXED>(fma(kv[0], x, fma(kv[1], y, kv[2] * z)), c, s);
-        if (is_y) {
+        if (ok) {
+            double u = fma(kv[0], x, fma(kv[1], y, kv[2] * z));
+            const double ti = PAIRS && outer ? tr[row] : 0.0;
+            if (PAIRS && outer) u -= phi * ti * (1.0 / kTwoPi);
+            cis_neg_cycles<MIXED>(u, c, s);
+            if (PAIRS && outer) {
+                const double d = MIXED ? (double)__builtin_amdgcn_exp2f((float)(-ti * r2 * 1.4426950408889634))
+                                       : exp(-ti * r2);
+                c *= d;
+                s *= d;
+            }
+        }
+        if (outer) {
             if (MIXED)
                 reinterpret_cast<float2 *>(Ey)[row * Np + n] = make_float2((float)c, (float)s);
             else
                 reinterpret_cast<double2 *>(Ey)[row * Np + n] = make_double2(c, s);
         } else {
-            const int64_t k = row - n_ln;
+            const int64_t k = row - n_out;
             for (int v = 0; v < V; ++v) {
                 double br = 0.0, bi = 0.0;
                 if (ok) {
@@ -490,27 +587,31 @@ __device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, const double *_
 }
 
 // Both operand tables in one launch: blocks [0, nb_E) build the E table,
-// the rest the Ey/Ezb rows (nb_n node blocks x row blocks), so the two
+// the rest the outer and Ezb rows (nb_n node blocks x row blocks), so the two
 // memory-bound jobs overlap instead of running back to back.
-template <bool MIXED>
+template <bool MIXED, bool PAIRS>
 __global__ __launch_bounds__(256) void k_cart_tables(const double *__restrict__ packed, int64_t N, int64_t Np,
                                                      int64_t M, int64_t Mp, const double *__restrict__ F,
+                                                     const double4 *__restrict__ lrows,
                                                      const double *__restrict__ tr, void *__restrict__ E,
-                                                     int64_t nb_E, int V, int64_t n_ln, int64_t n_kz,
+                                                     int64_t nb_E, int V, int64_t n_out, int64_t n_kz,
                                                      const double *__restrict__ G, const double *__restrict__ H,
                                                      void *__restrict__ Ey, void *__restrict__ Ez, int64_t nb_n)
 {
     const int64_t b = blockIdx.x;
     if (b < nb_E) {
         const int64_t t = b * 256 + threadIdx.x;
-        if (MIXED)
+        if (MIXED && PAIRS)
+            cart_rows_bf16(t, packed, N, Np, M, Mp, lrows, reinterpret_cast<uint4 *>(E));
+        else if (MIXED)
             cart_E_bf16(t, packed, N, Np, M, Mp, F, tr, reinterpret_cast<uint4 *>(E));
         else
             cart_E_f64(t, packed, N, Np, M, Mp, F, tr, reinterpret_cast<double *>(E));
         return;
     }
     const int64_t c = b - nb_E;
-    cart_yz<MIXED>((c % nb_n) * 256 + threadIdx.x, c / nb_n, packed, N, Np, V, n_ln, n_kz, G, H, Ey, Ez);
+    cart_yz<MIXED, PAIRS>((c % nb_n) * 256 + threadIdx.x, c / nb_n, packed, N, Np, V, n_out, n_kz, PAIRS ? F : G, tr,
+                          H, Ey, Ez);
 }
 
 template <typename P>
@@ -527,16 +628,17 @@ __global__ void k_cart_reduce(const P *__restrict__ part, int64_t n_splits, int6
     out[i] = make_double2(re, im);
 }
 
-// Samples from the partial sums over real rows: part is (n_splits, M, Lr,
-// Kr V) with Lr cosine and sine rows of the lines and, KPAIR, Kr rows of the
-// kz planes (else Kr = K planes with their own complex columns).  One thread
+// Samples from the partial sums over real rows: Lr cosine and sine rows of the
+// lines and, KPAIR, Kr rows of the kz planes (else Kr = K planes with their own
+// complex columns); readout index i, line row r, column q V + v of one split
+// at i si + r sr + q V + v, M Lr Kr V to a split.  One thread
 // group of G sums the splits of one (readout, line entity, kz entity,
 // encoding) in FP64, each thread a contiguous share of them, the shares added
 // in order, and writes the entity's up to four samples:
 //   (C_a -+ i S_a) (C_b -+ i S_b) = CC - s_a s_b SS - i (s_b CS + s_a SC).
 template <typename P, int G, bool KPAIR>
 __global__ __launch_bounds__(256) void k_cart_reduce_pairs(
-    const P *__restrict__ part, int64_t n_splits, int64_t M, int64_t Lr, int64_t KVr, int64_t V,
+    const P *__restrict__ part, int64_t n_splits, int64_t M, int64_t per_split, int64_t si, int64_t sr, int64_t V,
     const int4 *__restrict__ lent, int64_t n_lent, const int4 *__restrict__ kent, int64_t n_kent, int64_t L, int64_t K,
     double2 *__restrict__ out)
 {
@@ -556,10 +658,10 @@ __global__ __launch_bounds__(256) void k_cart_reduce_pairs(
         const int r = rows[c / 2], q = cols[c % 2];
         double re = 0.0, im = 0.0;
         if (live && r >= 0 && q >= 0) {
-            const P *src = part + (i * Lr + r) * KVr + q * V + v;
+            const P *src = part + i * si + r * sr + q * V + v;
 #pragma unroll 4
             for (int64_t s = s0; s < s1; ++s) {
-                const P x = src[s * M * Lr * KVr];
+                const P x = src[s * per_split];
                 re += (double)x.x;
                 im += (double)x.y;
             }
@@ -593,17 +695,19 @@ __global__ __launch_bounds__(256) void k_cart_reduce_pairs(
 // Threads per sample group: 16 where the samples alone would leave most of
 // the device idle in a long chain of loads, else 4.
 template <typename P, bool KPAIR>
-static void launch_reduce_pairs(const P *part, int64_t n_splits, int64_t M, int64_t Lr, int64_t KVr, int64_t V,
+static void launch_reduce_pairs(const P *part, int64_t n_splits, int64_t si, int64_t sr, int64_t V,
                                 const CartesianTables &c, double2 *out, hipStream_t st)
 {
+    const int64_t M = c.n_ro;
+    const int64_t per_split = M * c.lines.n_rows * (KPAIR ? c.kzs.n_rows : c.n_kz) * V;
     const int64_t n_kent = KPAIR ? c.kzs.n_ent : c.n_kz;
     const int64_t n = M * c.lines.n_ent * n_kent * V;
     if (n < 64 * 1024)
         k_cart_reduce_pairs<P, 16, KPAIR><<<(unsigned)cdiv(n, 16), 256, 0, st>>>(
-            part, n_splits, M, Lr, KVr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
+            part, n_splits, M, per_split, si, sr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
     else
         k_cart_reduce_pairs<P, 4, KPAIR><<<(unsigned)cdiv(n, 64), 256, 0, st>>>(
-            part, n_splits, M, Lr, KVr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
+            part, n_splits, M, per_split, si, sr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
 }
 
 int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, const double *packed, void *wsv,
@@ -625,19 +729,20 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
     {
         const int64_t nb_E = s.mixed ? cdiv(s.Np / 16 * 64, 256) : cdiv(s.Np / 16 * 256, 256);
         const int64_t nb_n = cdiv(s.Np, 256);
-        const int64_t nb = nb_E + nb_n * cdiv(c.n_ln + c.n_kz, kYZRowsPerBlock);
+        const int64_t n_out = s.pairs ? c.n_ro : c.n_ln;
+        const int64_t nb = nb_E + nb_n * cdiv(n_out + c.n_kz, kYZRowsPerBlock);
         if (nb > (int64_t)0x7fffffff) {
             set_error("Cartesian operand tables exceed the launch grid (%lld blocks)", (long long)nb);
             return FM_ERR_UNSUPPORTED;
         }
-        if (s.mixed)
-            k_cart_tables<true><<<(unsigned)nb, 256, 0, st>>>(packed, N, s.Np, s.M, s.Mp, c.d_F, c.d_t,
-                                                             ws + s.off_E, nb_E, V, c.n_ln, c.n_kz, c.d_G, c.d_H,
-                                                             ws + s.off_Ey, ws + s.off_Ez, nb_n);
-        else
-            k_cart_tables<false><<<(unsigned)nb, 256, 0, st>>>(packed, N, s.Np, s.M, s.Mp, c.d_F, c.d_t,
-                                                              ws + s.off_E, nb_E, V, c.n_ln, c.n_kz, c.d_G, c.d_H,
-                                                              ws + s.off_Ey, ws + s.off_Ez, nb_n);
+#define FM_TABLES(MX, PR)                                                                                            \
+    k_cart_tables<MX, PR><<<(unsigned)nb, 256, 0, st>>>(packed, N, s.Np, s.M, s.Mp, PR ? c.d_F_lines : c.d_F,       \
+                                                        c.lines.d_rows, c.d_t, ws + s.off_E, nb_E, V, n_out, c.n_kz, \
+                                                        c.d_G, c.d_H, ws + s.off_Ey, ws + s.off_Ez, nb_n)
+        if (s.mixed && s.pairs) FM_TABLES(true, true);
+        else if (s.mixed) FM_TABLES(true, false);
+        else FM_TABLES(false, false);
+#undef FM_TABLES
         FM_LAUNCH_CHECK("k_cart_tables");
     }
     if (s.mixed) {
@@ -646,7 +751,10 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
         plan_timing_stop(p, st);
         FM_LAUNCH_CHECK("k_cart_gemm_bf16");
         const int64_t MNC = s.M * s.NC;
-        k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(
+        if (s.pairs)
+            launch_reduce_pairs<float2, false>(reinterpret_cast<const float2 *>(ws + s.off_part), s.n_splits, n_kzV,
+                                               s.NC, V, c, reinterpret_cast<double2 *>(out), st);
+        else k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(
             reinterpret_cast<const float2 *>(ws + s.off_part), s.n_splits, MNC, reinterpret_cast<double2 *>(out));
     } else {
         plan_timing_start(p, st);
@@ -716,8 +824,8 @@ int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, 
         plan_timing_stop(p, st);
         FM_LAUNCH_CHECK("k_cart_moving_bf16");
         if (s.pairs)
-            launch_reduce_pairs<float2, true>(part, s.n_splits, s.M, s.L, s.KV, s.V, c, reinterpret_cast<double2 *>(out),
-                                              st);
+            launch_reduce_pairs<float2, true>(part, s.n_splits, s.L * s.KV, s.KV, s.V, c,
+                                              reinterpret_cast<double2 *>(out), st);
         else k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
                                                                          reinterpret_cast<double2 *>(out));
     }

@@ -77,11 +77,11 @@ struct CartesianTables {
     bool axis_aligned = false;
     double *d_F = nullptr, *d_G = nullptr, *d_H = nullptr, *d_t = nullptr;
     int32_t *d_ro_group = nullptr;
-    // lines and kz planes as real rows, and F with the centres' offset added:
-    // of both axes
+    // lines and kz planes as real rows, and F plus the lines' centre (R
+    // entries), then F plus both centres
     PairAxis lines, kzs;
     std::vector<double> F_pairs;
-    double *d_F_pairs = nullptr;
+    double *d_F_lines = nullptr, *d_F_pairs = nullptr;
     void *d_pairs = nullptr;     // one allocation behind the pair tables
 };
 
