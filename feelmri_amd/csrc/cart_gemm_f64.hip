@@ -16,26 +16,37 @@ namespace fm {
 // (double-buffered), copied by direct global -> LDS DMA a stage ahead, so
 // the workgroup synchronises once per 32 nodes and stages through no
 // registers; the B operands (Ey * Ez) come from global memory one step ahead.
-template <int RB>
+//
+// REAL: real rows (PairAxis; rows are the lines' cosine and sine rows, columns
+// (readout index, kz, encoding)): one E plane and 2 MFMAs per row block and
+// k-step instead of 4.  Up to 8 row blocks then share a column operand (RB = 8:
+// 128 accumulator registers, as RB = 4 needs for E's two planes and their
+// products).  150 001 nodes, 125 x 127 x 31, whole call:
+// 5.94 ms against 11.69 ms with complex rows (99 against 50 TFLOP/s of 8 flops
+// per node * sample), error against 64 bits 6.4e-15 against 4.7e-15 (both at
+// the rounding of the phases).  Bound by the FP64 MFMAs.
+template <int CHUNKS>
 __device__ inline void stage_E64_to_lds(const double *__restrict__ src, double *dst, int wave, int lane)
 {
-    // RB row-block tiles of 4 KB: RB * 4 chunks of 1 KB (64 lanes x 16 B)
+    // chunks of 1 KB (64 lanes x 16 B), wave w of 4 moves w, w + 4, ...
 #pragma unroll
-    for (int e = 0; e < RB; ++e) {
-        const int chunk = wave * RB + e;
+    for (int e = 0; e < (CHUNKS + 3) / 4; ++e) {
+        const int chunk = wave + 4 * e;
+        if (CHUNKS % 4 != 0 && chunk >= CHUNKS) break;
         __builtin_amdgcn_global_load_lds(
             (const __attribute__((address_space(1))) void *)(reinterpret_cast<const uint4 *>(src) + chunk * 64 + lane),
             (__attribute__((address_space(3))) void *)(reinterpret_cast<uint4 *>(dst) + chunk * 64), 16, 0, 0);
     }
 }
 
-template <int RB>
-__global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_f64(
+template <int RB, bool REAL>
+__global__ __launch_bounds__(kGemmThreads, 2) void k_cart_gemm_f64(
     const double *__restrict__ E, const double2 *__restrict__ Ey, const double2 *__restrict__ Ez, int64_t Np,
     int64_t Mp, int64_t M, int64_t NC, int64_t n_kzV, int64_t n_rt, int64_t n_ct, int64_t n_splits,
     int64_t steps_per_split, int64_t ksteps, double2 *__restrict__ part)
 {
-    constexpr int kStep = RB * 2 * 4 * 64;             // doubles of one step's E tiles
+    constexpr int kPl = REAL ? 1 : 2;                  // planes of an E tile
+    constexpr int kStep = RB * kPl * 4 * 64;           // doubles of one step's E tiles
     __shared__ double sE[2][2 * kStep];
     int64_t split, rt, ct;
     gemm_tile_ids(n_rt, n_ct, n_splits, split, rt, ct);
@@ -62,7 +73,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_f64(
 #pragma unroll
         for (int h = 0; h < 2; ++h)
             if (ks + h < k1)
-                stage_E64_to_lds<RB>(E + ((ks + h) * nrb + rt * RB) * 2 * 4 * 64, sE[b] + h * kStep, wave, lane);
+                stage_E64_to_lds<RB * kPl * 2>(E + ((ks + h) * nrb + rt * RB) * kPl * 4 * 64, sE[b] + h * kStep, wave, lane);
     };
 
     double2 cy[4], cz[4], ny[4], nz[4];
@@ -99,20 +110,22 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_f64(
             const double *se = sE[buf] + h * kStep;
 #pragma unroll
             for (int st = 0; st < 4; ++st) {
-                double er[RB], ei[RB];
+                double er[RB], ei[REAL ? 1 : RB];
 #pragma unroll
                 for (int r = 0; r < RB; ++r) {
-                    er[r] = se[(r * 2 * 4 + 0 * 4 + st) * 64 + lane];
-                    ei[r] = se[(r * 2 * 4 + 1 * 4 + st) * 64 + lane];
+                    er[r] = se[(r * kPl * 4 + 0 * 4 + st) * 64 + lane];
+                    if constexpr (!REAL) ei[r] = se[(r * kPl * 4 + 1 * 4 + st) * 64 + lane];
                 }
 #pragma unroll
                 for (int r = 0; r < RB; ++r) acc_re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[r], br[st], acc_re[r], 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < RB; ++r) acc_im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[r], bi[st], acc_im[r], 0, 0, 0);
+                if constexpr (!REAL) {
 #pragma unroll
-                for (int r = 0; r < RB; ++r) acc_re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ei[r], bi[st], acc_re[r], 0, 0, 0);
+                    for (int r = 0; r < RB; ++r) acc_re[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ei[r], bi[st], acc_re[r], 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < RB; ++r) acc_im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[r], br[st], acc_im[r], 0, 0, 0);
+                    for (int r = 0; r < RB; ++r) acc_im[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[r], br[st], acc_im[r], 0, 0, 0);
+                }
             }
             if (ks + 1 < k1) {
 #pragma unroll
@@ -139,11 +152,11 @@ __global__ __launch_bounds__(kGemmThreads) void k_cart_gemm_f64(
     }
 }
 
-template <int RB>
+template <int RB, bool REAL>
 static void launch_f64(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t st)
 {
     const unsigned grid = (unsigned)(s.n_rt * s.n_ct * s.n_splits);
-    k_cart_gemm_f64<RB><<<grid, kGemmThreads, 0, st>>>(
+    k_cart_gemm_f64<RB, REAL><<<grid, kGemmThreads, 0, st>>>(
         reinterpret_cast<const double *>(ws + s.off_E), reinterpret_cast<const double2 *>(ws + s.off_Ey),
         reinterpret_cast<const double2 *>(ws + s.off_Ez), s.Np, s.Mp, s.M, s.NC, n_kzV, s.n_rt, s.n_ct, s.n_splits,
         s.steps_per_split, s.ksteps, reinterpret_cast<double2 *>(ws + s.off_part));
@@ -151,15 +164,24 @@ static void launch_f64(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t 
 
 void launch_cart_gemm_f64(const GemmShape &s, char *ws, int64_t n_kzV, hipStream_t st)
 {
+    if (s.pairs) {
+        switch (s.rb_per_wave) {
+        case 1: launch_f64<1, true>(s, ws, n_kzV, st); break;
+        case 2: launch_f64<2, true>(s, ws, n_kzV, st); break;
+        case 3: launch_f64<3, true>(s, ws, n_kzV, st); break;
+        case 4: launch_f64<4, true>(s, ws, n_kzV, st); break;
+        case 5: launch_f64<5, true>(s, ws, n_kzV, st); break;
+        case 6: launch_f64<6, true>(s, ws, n_kzV, st); break;
+        case 7: launch_f64<7, true>(s, ws, n_kzV, st); break;
+        default: launch_f64<8, true>(s, ws, n_kzV, st); break;
+        }
+        return;
+    }
     switch (s.rb_per_wave) {
-    case 1: launch_f64<1>(s, ws, n_kzV, st); break;
-    case 2: launch_f64<2>(s, ws, n_kzV, st); break;
-    case 3: launch_f64<3>(s, ws, n_kzV, st); break;
-    case 4: launch_f64<4>(s, ws, n_kzV, st); break;
-    case 5: launch_f64<5>(s, ws, n_kzV, st); break;
-    case 6: launch_f64<6>(s, ws, n_kzV, st); break;
-    case 7: launch_f64<7>(s, ws, n_kzV, st); break;
-    default: launch_f64<8>(s, ws, n_kzV, st); break;
+    case 1: launch_f64<1, false>(s, ws, n_kzV, st); break;
+    case 2: launch_f64<2, false>(s, ws, n_kzV, st); break;
+    case 3: launch_f64<3, false>(s, ws, n_kzV, st); break;
+    default: launch_f64<4, false>(s, ws, n_kzV, st); break;
     }
 }
 

@@ -21,6 +21,15 @@
 //     are formed between the step's barrier and its MFMAs;
 //   * per k-step and column block, 4 MFMAs: Re += Ar Br - Ai Bi,
 //     Im += Ar Bi + Ai Br.
+// REAL: lines along y and kz planes along z that pair up about a centre are
+// taken as real rows (PairAxis; the decomposition is described in
+// cart_moving_pairs_bf16.hip): A is one sine per row and node, B the kz row
+// times c_i (two products per entry), and a k-step takes 2 MFMAs per column
+// block: Re += A Re B, Im += A Im B.  150 001 nodes, 63 x 65 x 17, 3
+// encodings, 6 modes: 6.25 ms against 13.1 ms with complex rows, error against
+// 64 bits 1.7e-15 against 1.6e-15.  Real rows need few enough registers for 3
+// waves per SIMD up to 4 column blocks: 6.25 ms against 7.28 ms with 2 (MFMA 41 %
+// busy, the waves waiting at the step barriers).
 // FP64 accumulators need no bound on the split length; node splits exist for
 // parallelism only and are summed in FP64 by k_cart_reduce.
 #include <algorithm>
@@ -43,8 +52,9 @@ __device__ inline void cis_neg_f64(double u, double &c, double &s)
 // kz rows of the kz-factor buffer: 16 nodes + 1 entry of pad
 constexpr int kEz64Stride = 17;
 
-template <int W, int CB>
-__global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
+// G and H: line and kz offsets (3 a row), REAL: real rows (4 a row).
+template <int W, int CB, bool REAL>
+__global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving_f64(
     const double *__restrict__ packed, int64_t N, int V, const float *__restrict__ modes, int R,
     const double *__restrict__ mcoef, const int32_t *__restrict__ ro_group, const double *__restrict__ F,
     const double *__restrict__ G, const double *__restrict__ H, const double *__restrict__ tr, int64_t M,
@@ -63,6 +73,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
     __shared__ double sH[3 * (kCols + 1)];
     __shared__ double scoef[kMaxModes + 3];
     extern __shared__ double2 sEz64[];           // ez_rows rows of kEz64Stride
+    double *const sKz64 = reinterpret_cast<double *>(sEz64);
 
     // workgroup -> (split, readout index, row tile, column tile); the ids of
     // one split are contiguous and dealt onto one XCD
@@ -90,15 +101,20 @@ __global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
     // this lane's A row
     const int64_t row = (rt * W + wave) * 16 + (lane % 16);
     const bool row_ok = row < L;
-    const double Gx = row_ok ? G[3 * row] : 0.0, Gy = row_ok ? G[3 * row + 1] : 0.0,
-                 Gz = row_ok ? G[3 * row + 2] : 0.0;
+    constexpr int kG = REAL ? 4 : 3;
+    const double Gx = row_ok ? G[kG * row] : 0.0, Gy = row_ok ? G[kG * row + 1] : 0.0,
+                 Gz = row_ok ? G[kG * row + (REAL ? 3 : 2)] : 0.0;  // REAL: the quarter turn
 
     // the column tile's kz rows
     const int64_t c0 = ct * kCols;
     const int64_t kmin = c0 / V;
     const int64_t kmax = std::min<int64_t>(K - 1, (c0 + kCols - 1) / V);
     const int nk = (int)(kmax - kmin + 1);  // <= ez_rows
-    for (int q = tid; q < 3 * nk; q += kThreads) sH[q] = H[3 * kmin + q];
+    if constexpr (REAL) {
+        for (int q = tid; q < 2 * nk; q += kThreads) sH[q] = H[4 * kmin + 4 * (q / 2) + 2 + q % 2];
+    } else {
+        for (int q = tid; q < 3 * nk; q += kThreads) sH[q] = H[3 * kmin + q];
+    }
 
     // this thread's B fragments: fragment f = (tid + r kThreads) / 64 is
     // (column block f / 4, k-step f % 4) and feeds lane tid % 64 (= lane)
@@ -124,10 +140,14 @@ __global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
         double2 *dst = sEz64;
         for (int e = tid; e < nk * 16; e += kThreads) {
             const int kk = e / 16, m = s * 16 + e % 16;
-            const double u = fma(sH[3 * kk], sx[m], fma(sH[3 * kk + 1], sy[m], sH[3 * kk + 2] * sz[m]));
-            double c, sn;
-            cis_neg_f64(u, c, sn);
-            dst[kk * kEz64Stride + e % 16] = make_double2(c, sn);
+            if constexpr (REAL) {
+                sKz64[kk * kEz64Stride + e % 16] = sin_cycles_f64(fma(sH[2 * kk], sz[m], sH[2 * kk + 1]));
+            } else {
+                const double u = fma(sH[3 * kk], sx[m], fma(sH[3 * kk + 1], sy[m], sH[3 * kk + 2] * sz[m]));
+                double c, sn;
+                cis_neg_f64(u, c, sn);
+                dst[kk * kEz64Stride + e % 16] = make_double2(c, sn);
+            }
         }
     };
 
@@ -186,10 +206,17 @@ __global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
                     if (f < kFrag) {
                         const int st = f % 4;
                         const int m = 4 * st + lane / 16;
-                        const double2 a = ez[bkk[r] * kEz64Stride + m];
                         const double2 b = sc[bv[r]][s * 16 + m];
-                        const double br = bok[r] ? a.x * b.x - a.y * b.y : 0.0;
-                        const double bi = bok[r] ? a.x * b.y + a.y * b.x : 0.0;
+                        double br, bi;
+                        if constexpr (REAL) {  // columns past the last: finite, not written
+                            const double a = sKz64[bkk[r] * kEz64Stride + m];
+                            br = a * b.x;
+                            bi = a * b.y;
+                        } else {
+                            const double2 a = ez[bkk[r] * kEz64Stride + m];
+                            br = bok[r] ? a.x * b.x - a.y * b.y : 0.0;
+                            bi = bok[r] ? a.x * b.y + a.y * b.x : 0.0;
+                        }
                         sB[(f * 2 + 0) * 64 + lane] = br;
                         sB[(f * 2 + 1) * 64 + lane] = bi;
                     }
@@ -200,8 +227,12 @@ __global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
 #pragma unroll
             for (int st = 0; st < 4; ++st) {
                 const int m = s * 16 + 4 * st + lane / 16;
-                const double u = fma(Gx, sx[m], fma(Gy, sy[m], Gz * sz[m]));
-                cis_neg_f64(u, ar[st], ai[st]);
+                if constexpr (REAL) {
+                    ar[st] = sin_cycles_f64(fma(Gy, sy[m], Gz));
+                } else {
+                    const double u = fma(Gx, sx[m], fma(Gy, sy[m], Gz * sz[m]));
+                    cis_neg_f64(u, ar[st], ai[st]);
+                }
             }
             __syncthreads();  // B planes written, kz factors of step s read
             if (s + 1 < nsteps) ez_gen(s + 1);
@@ -214,6 +245,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_cart_moving_f64(
                     acc_re[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[st], br, acc_re[cb], 0, 0, 0);
                     acc_im[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[st], bi, acc_im[cb], 0, 0, 0);
                 }
+                if constexpr (!REAL)
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb) {
                     const int f = cb * 4 + st;
@@ -258,38 +290,47 @@ static size_t lds_bytes_f64(int W, int CB, int ez_rows)
            3 * (16 * (size_t)CB + 1) * 8 + (kMaxModes + 3) * 8 + (size_t)ez_rows * kEz64Stride * 16;
 }
 
-template <int W>
+template <int W, bool REAL>
 static int mf64_blocks_w(int CB, size_t dyn)
 {
     switch (CB) {
-    case 1: return blocks_per_cu(k_cart_moving_f64<W, 1>, 64 * W, dyn);
-    case 2: return blocks_per_cu(k_cart_moving_f64<W, 2>, 64 * W, dyn);
-    case 3: if constexpr (W >= 2) return blocks_per_cu(k_cart_moving_f64<W, 3>, 64 * W, dyn); break;
-    case 4: if constexpr (W >= 2) return blocks_per_cu(k_cart_moving_f64<W, 4>, 64 * W, dyn); break;
-    case 6: if constexpr (W >= 3) return blocks_per_cu(k_cart_moving_f64<W, 6>, 64 * W, dyn); break;
+    case 1: return blocks_per_cu(k_cart_moving_f64<W, 1, REAL>, 64 * W, dyn);
+    case 2: return blocks_per_cu(k_cart_moving_f64<W, 2, REAL>, 64 * W, dyn);
+    case 3: if constexpr (W >= 2) return blocks_per_cu(k_cart_moving_f64<W, 3, REAL>, 64 * W, dyn); break;
+    case 4: if constexpr (W >= 2) return blocks_per_cu(k_cart_moving_f64<W, 4, REAL>, 64 * W, dyn); break;
+    case 6: if constexpr (W >= 3) return blocks_per_cu(k_cart_moving_f64<W, 6, REAL>, 64 * W, dyn); break;
     default: break;
     }
     return 1;
 }
 
+static size_t mf64_dyn(int ez_rows, bool real)
+{
+    return (size_t)ez_rows * kEz64Stride * (real ? sizeof(double) : sizeof(double2));
+}
+
 // Workgroups of the shape's instantiation that one CU holds at once.
+template <bool REAL>
 static int mf64_blocks_per_cu(int W, int CB, int ez_rows)
 {
-    const size_t dyn = (size_t)ez_rows * kEz64Stride * sizeof(double2);
+    const size_t dyn = mf64_dyn(ez_rows, REAL);
     switch (W) {
-    case 1: return mf64_blocks_w<1>(CB, dyn);
-    case 2: return mf64_blocks_w<2>(CB, dyn);
-    case 3: return mf64_blocks_w<3>(CB, dyn);
-    default: return mf64_blocks_w<4>(CB, dyn);
+    case 1: return mf64_blocks_w<1, REAL>(CB, dyn);
+    case 2: return mf64_blocks_w<2, REAL>(CB, dyn);
+    case 3: return mf64_blocks_w<3, REAL>(CB, dyn);
+    default: return mf64_blocks_w<4, REAL>(CB, dyn);
     }
 }
 
-MovingShape moving_shape_f64(const CartesianTables &c, int64_t N, int V)
+// Shape over L rows and K kz rows; max_bytes bounds the partial tiles (0: no
+// bound).
+template <bool REAL>
+static MovingShape mf64_shape(const CartesianTables &c, int64_t L, int64_t K, int64_t N, int V, size_t max_bytes)
 {
     MovingShape s{};
     s.M = c.n_ro;
-    s.L = c.n_ln;
-    s.K = c.n_kz;
+    s.L = L;
+    s.K = K;
     s.V = V;
     s.KV = s.K * V;
     const int64_t nrb = cdiv(s.L, 16), ncb = cdiv(s.KV, 16);
@@ -313,50 +354,80 @@ MovingShape moving_shape_f64(const CartesianTables &c, int64_t N, int V)
     s.ez_rows = ez_rows_of(s.CB);
     // four workgroups per CU at least, in whole rounds of the workgroups the
     // device holds; FP64 accumulators need no bound on the split length
-    const int64_t capacity = (int64_t)mf64_blocks_per_cu(s.W, s.CB, s.ez_rows) * device_cu_count();
-    const int64_t splits = balanced_splits(N, chunk, base, cdiv(4 * (int64_t)device_cu_count(), base), capacity);
+    const size_t per_split = (size_t)s.M * (size_t)s.L * (size_t)s.KV * sizeof(double2);
+    const int64_t s_max = max_bytes ? (int64_t)(max_bytes / std::max<size_t>(per_split, 1)) : 0;
+    if (max_bytes && s_max < 1) return s;
+    const int64_t capacity = (int64_t)mf64_blocks_per_cu<REAL>(s.W, s.CB, s.ez_rows) * device_cu_count();
+    const int64_t splits =
+        balanced_splits(N, chunk, base, cdiv(4 * (int64_t)device_cu_count(), base), capacity, s_max);
     s.nodes_per_split = cdiv(cdiv(std::max<int64_t>(N, 1), splits), chunk) * chunk;
     s.n_splits = cdiv(std::max<int64_t>(N, 1), s.nodes_per_split);
-    s.part_bytes = (size_t)s.n_splits * (size_t)s.M * (size_t)s.L * (size_t)s.KV * sizeof(double2);
+    s.part_bytes = (size_t)s.n_splits * per_split;
+    s.pairs = REAL;
     return s;
 }
 
-template <int W, int CB>
+MovingShape moving_shape_f64(const CartesianTables &c, int64_t N, int V)
+{
+    return mf64_shape<false>(c, c.n_ln, c.n_kz, N, V, 0);
+}
+
+MovingShape moving_pairs_shape_f64(const CartesianTables &c, int64_t N, int V)
+{
+    // used where it runs fewer MFMAs (2 per block and k-step against 4),
+    // within the complex rows' workspace
+    const MovingShape g = moving_shape_f64(c, N, V);
+    if (!c.axis_aligned) return MovingShape{};
+    const MovingShape s = mf64_shape<true>(c, c.lines.n_rows, c.kzs.n_rows, N, V, g.part_bytes);
+    return s.n_rt * s.W * s.n_ct * s.CB < 2 * g.n_rt * g.W * g.n_ct * g.CB ? s : MovingShape{};
+}
+
+template <int W, int CB, bool REAL>
 static void launch_mf64_wc(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,
                            const float *modes, int R, const double *mcoef, double2 *part, hipStream_t st)
 {
     const int64_t grid = s.n_splits * s.M * s.n_rt * s.n_ct;
-    const size_t dyn = (size_t)s.ez_rows * kEz64Stride * sizeof(double2);
-    k_cart_moving_f64<W, CB><<<(unsigned)grid, 64 * W, dyn, st>>>(
-        packed, N, (int)s.V, modes, R, mcoef, c.d_ro_group, c.d_F, c.d_G, c.d_H, c.d_t, s.M, s.L, s.K, s.n_rt,
-        s.n_ct, s.n_splits, s.nodes_per_split, s.ez_rows, part);
+    const double *F = REAL ? c.d_F_pairs : c.d_F;
+    const double *G = REAL ? reinterpret_cast<const double *>(c.lines.d_rows) : c.d_G;
+    const double *H = REAL ? reinterpret_cast<const double *>(c.kzs.d_rows) : c.d_H;
+    k_cart_moving_f64<W, CB, REAL><<<(unsigned)grid, 64 * W, mf64_dyn(s.ez_rows, REAL), st>>>(
+        packed, N, (int)s.V, modes, R, mcoef, c.d_ro_group, F, G, H, c.d_t, s.M, s.L, s.K, s.n_rt, s.n_ct, s.n_splits,
+        s.nodes_per_split, s.ez_rows, part);
 }
 
 // Column-block counts instantiated per W: those <= min(2 W, 6) (the shape
 // never picks more).
-template <int W>
+template <int W, bool REAL>
 static void launch_mf64_w(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,
                           const float *modes, int R, const double *mcoef, double2 *part, hipStream_t st)
 {
     switch (s.CB) {
-    case 1: launch_mf64_wc<W, 1>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    case 2: launch_mf64_wc<W, 2>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    case 3: if constexpr (W >= 2) launch_mf64_wc<W, 3>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    case 4: if constexpr (W >= 2) launch_mf64_wc<W, 4>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    case 6: if constexpr (W >= 3) launch_mf64_wc<W, 6>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 1: launch_mf64_wc<W, 1, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 2: launch_mf64_wc<W, 2, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 3: if constexpr (W >= 2) launch_mf64_wc<W, 3, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 4: if constexpr (W >= 2) launch_mf64_wc<W, 4, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 6: if constexpr (W >= 3) launch_mf64_wc<W, 6, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
     default: break;
+    }
+}
+
+template <bool REAL>
+static void launch_mf64(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,
+                        const float *modes, int R, const double *mcoef, double2 *part, hipStream_t st)
+{
+    switch (s.W) {
+    case 1: launch_mf64_w<1, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 2: launch_mf64_w<2, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    case 3: launch_mf64_w<3, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
+    default: launch_mf64_w<4, REAL>(s, c, packed, N, modes, R, mcoef, part, st); break;
     }
 }
 
 void launch_cart_moving_f64(const MovingShape &s, const CartesianTables &c, const double *packed, int64_t N,
                             const float *modes, int R, const double *mcoef, double2 *part, hipStream_t st)
 {
-    switch (s.W) {
-    case 1: launch_mf64_w<1>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    case 2: launch_mf64_w<2>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    case 3: launch_mf64_w<3>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    default: launch_mf64_w<4>(s, c, packed, N, modes, R, mcoef, part, st); break;
-    }
+    if (s.pairs) launch_mf64<true>(s, c, packed, N, modes, R, mcoef, part, st);
+    else launch_mf64<false>(s, c, packed, N, modes, R, mcoef, part, st);
 }
 
 }  // namespace fm

@@ -62,21 +62,7 @@ static PairAxis pair_axis_about(const std::vector<double> &g, int64_t n, const d
         }
         return p < q;
     });
-    for (int d = 0; d < 3; ++d) a.c[d] = c[d];
-    std::vector<double> D;                 // per entity
-    std::vector<char> centred;
-    auto add = [&](int32_t p, int32_t q) {  // q = -1: no partner
-        bool zero = q < 0;
-        for (int d = 0; d < 3; ++d) {
-            const double gp = g[(size_t)(3 * p + d)];
-            const double v = q < 0 ? gp - c[d] : 0.5 * (gp - g[(size_t)(3 * q + d)]);
-            zero = zero && std::fabs(v) <= tol;
-            D.push_back(v);
-        }
-        if (zero) D[D.size() - 3] = D[D.size() - 2] = D[D.size() - 1] = 0.0;
-        centred.push_back(zero);
-        a.ent.insert(a.ent.end(), {p, q, 0, 0});
-    };
+    auto add = [&](int32_t p, int32_t q) { a.ent.insert(a.ent.end(), {p, q, 0, 0}); };  // q = -1: no partner
     int64_t lo = 0, hi = n - 1;
     while (lo <= hi) {
         const int32_t p = order[(size_t)lo], q = order[(size_t)hi];
@@ -103,8 +89,33 @@ static PairAxis pair_axis_about(const std::vector<double> &g, int64_t n, const d
             --hi;
         }
     }
-    // cosine rows first, then the sine rows
-    a.n_ent = (int64_t)centred.size();
+    a.n_ent = (int64_t)a.ent.size() / 4;
+    // the centre as the mean of the pairs' middles, which keeps c +- D within
+    // about one rounding of the given offsets (rms)
+    int64_t n_pair = 0;
+    long double mid[3] = {0.0L, 0.0L, 0.0L};
+    for (int64_t e = 0; e < a.n_ent; ++e) {
+        const int32_t p = a.ent[(size_t)(4 * e)], q = a.ent[(size_t)(4 * e + 1)];
+        if (q < 0) continue;
+        ++n_pair;
+        for (int d = 0; d < 3; ++d) mid[d] += 0.5L * ((long double)g[(size_t)(3 * p + d)] + (long double)g[(size_t)(3 * q + d)]);
+    }
+    for (int d = 0; d < 3; ++d) a.c[d] = n_pair ? (double)(mid[d] / (long double)n_pair) : c[d];
+    // rows: the cosines, then the sines
+    std::vector<double> D;
+    std::vector<char> centred;
+    for (int64_t e = 0; e < a.n_ent; ++e) {
+        const int32_t p = a.ent[(size_t)(4 * e)], q = a.ent[(size_t)(4 * e + 1)];
+        bool zero = q < 0;
+        for (int d = 0; d < 3; ++d) {
+            const double gp = g[(size_t)(3 * p + d)];
+            const double v = q < 0 ? gp - a.c[d] : 0.5 * (gp - g[(size_t)(3 * q + d)]);
+            zero = zero && std::fabs(v) <= tol;
+            D.push_back(v);
+        }
+        if (zero) D[D.size() - 3] = D[D.size() - 2] = D[D.size() - 1] = 0.0;
+        centred.push_back(zero);
+    }
     for (int64_t e = 0; e < a.n_ent; ++e) {
         a.ent[(size_t)(4 * e + 2)] = (int32_t)e;
         a.rows.insert(a.rows.end(), {D[(size_t)(3 * e)], D[(size_t)(3 * e + 1)], D[(size_t)(3 * e + 2)], 0.25});
@@ -277,7 +288,7 @@ static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, 
     s.pairs = pairs;
     const int rowblk = s.mixed ? 32 : 16;
     const int colblk = s.mixed ? 32 : 16;
-    const int max_rb = 4;
+    const int max_rb = !mixed && pairs ? 8 : 4;
     const int64_t outer = pairs ? c.n_ro : c.n_ln;  // the columns' outer index
     s.N = N;
     s.Np = cdiv(std::max<int64_t>(N, 1), 16) * 16;
@@ -285,6 +296,7 @@ static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, 
     const int64_t nrb = cdiv(s.M, rowblk);
     s.rb_per_wave = (int)std::min<int64_t>(max_rb, nrb);
     s.n_rt = cdiv(nrb, s.rb_per_wave);
+    if (!mixed && pairs) s.rb_per_wave = (int)cdiv(nrb, s.n_rt);  // tiles of equal height
     s.Mp = s.n_rt * s.rb_per_wave * rowblk;
     s.NC = outer * c.n_kz * V;
     s.n_ct = cdiv(s.NC, 4 * colblk);
@@ -325,14 +337,13 @@ static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, 
 }
 
 // Real rows where they take fewer MFMAs (half as many per row and column
-// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32) and no more
-// workspace than complex rows do.
+// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32; FP64 5.94 against
+// 11.69 ms at 150 001 nodes, 125 x 127 x 31) and no more workspace than complex rows do.
 static GemmShape gemm_shape(const fm_signal_plan *p, int precision, int64_t N, int V)
 {
     const CartesianTables &c = p->cart;
     const bool mixed = precision != FM_PREC_F64;
     const GemmShape g = gemm_shape_of(c, mixed, N, V, false);
-    if (!mixed) return g;
     const GemmShape s = gemm_shape_of(c, mixed, N, V, true);
     return s.Mp * s.NCp < 2 * g.Mp * g.NCp && s.total <= g.total ? s : g;
 }
@@ -523,6 +534,32 @@ __device__ __forceinline__ void cart_rows_bf16(int64_t t, const double *__restri
     }
 }
 
+// Real rows, FP64: tiles of (16 rows x 16 nodes), one plane in the lane order
+// of cart_E_f64.
+__device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
+                                              int64_t M, int64_t Mp, const double4 *__restrict__ rows,
+                                              double *__restrict__ E)
+{
+    // t over (Np / 16) * 4 * 64
+    if (t >= (Np / 16) * 256) return;
+    const int lane = (int)(t % 64);
+    const int st = (int)((t / 64) % 4);
+    const int64_t kb = t / 256;
+    const int64_t nrb = Mp / 16;
+    const int64_t n = kb * 16 + 4 * st + lane / 16;
+    const bool ok = n < N;
+    const double x = ok ? packed[n] : 0.0, y = ok ? packed[N + n] : 0.0, z = ok ? packed[2 * N + n] : 0.0;
+    for (int64_t rb = 0; rb < nrb; ++rb) {
+        const int64_t i = rb * 16 + (lane % 16);
+        double e = 0.0;
+        if (ok && i < M) {
+            const double4 d = rows[i];
+            e = sin_cycles_f64(fma(d.x, x, fma(d.y, y, fma(d.z, z, d.w))));
+        }
+        E[((kb * nrb + rb) * 4 + st) * 64 + lane] = e;
+    }
+}
+
 // The columns' outer rows -- complex rows: Ey, exp(-2 pi i (G_j . x_n)) of the
 // lines; real rows: Ex, exp(-t_i/T2) exp(i phi t_i) exp(-2 pi i F_i . x) of the
 // readout indices -- and Ezb rows exp(-2 pi i (H_k . x_n)) b_v[n] (the
@@ -605,6 +642,8 @@ __global__ __launch_bounds__(256) void k_cart_tables(const double *__restrict__ 
             cart_rows_bf16(t, packed, N, Np, M, Mp, lrows, reinterpret_cast<uint4 *>(E));
         else if (MIXED)
             cart_E_bf16(t, packed, N, Np, M, Mp, F, tr, reinterpret_cast<uint4 *>(E));
+        else if (PAIRS)
+            cart_rows_f64(t, packed, N, Np, M, Mp, lrows, reinterpret_cast<double *>(E));
         else
             cart_E_f64(t, packed, N, Np, M, Mp, F, tr, reinterpret_cast<double *>(E));
         return;
@@ -741,6 +780,7 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
                                                         c.d_G, c.d_H, ws + s.off_Ey, ws + s.off_Ez, nb_n)
         if (s.mixed && s.pairs) FM_TABLES(true, true);
         else if (s.mixed) FM_TABLES(true, false);
+        else if (s.pairs) FM_TABLES(false, true);
         else FM_TABLES(false, false);
 #undef FM_TABLES
         FM_LAUNCH_CHECK("k_cart_tables");
@@ -762,7 +802,10 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
         plan_timing_stop(p, st);
         FM_LAUNCH_CHECK("k_cart_gemm_f64");
         const int64_t MNC = s.M * s.NC;
-        k_cart_reduce<double2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(
+        if (s.pairs)
+            launch_reduce_pairs<double2, false>(reinterpret_cast<const double2 *>(ws + s.off_part), s.n_splits, n_kzV,
+                                                s.NC, V, c, reinterpret_cast<double2 *>(out), st);
+        else k_cart_reduce<double2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(
             reinterpret_cast<const double2 *>(ws + s.off_part), s.n_splits, MNC, reinterpret_cast<double2 *>(out));
     }
     FM_LAUNCH_CHECK("k_cart_reduce");
@@ -772,9 +815,8 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
 // The moving form a shape takes: real rows where the plan has them.
 static MovingShape moving_form(const CartesianTables &c, bool f64, int64_t N, int V)
 {
-    if (f64) return moving_shape_f64(c, N, V);
-    const MovingShape s = moving_pairs_shape(c, N, V);
-    return s.pairs ? s : moving_shape(c, N, V);
+    const MovingShape s = f64 ? moving_pairs_shape_f64(c, N, V) : moving_pairs_shape(c, N, V);
+    return s.pairs ? s : (f64 ? moving_shape_f64(c, N, V) : moving_shape(c, N, V));
 }
 
 size_t cartesian_moving_workspace(const fm_signal_plan *p, int precision, int64_t N, int V)
@@ -815,7 +857,10 @@ int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, 
         launch_cart_moving_f64(s, c, packed, N, modes, R, mcoef, part, st);
         plan_timing_stop(p, st);
         FM_LAUNCH_CHECK("k_cart_moving_f64");
-        k_cart_reduce<double2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
+        if (s.pairs)
+            launch_reduce_pairs<double2, true>(part, s.n_splits, s.L * s.KV, s.KV, s.V, c,
+                                               reinterpret_cast<double2 *>(out), st);
+        else k_cart_reduce<double2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
                                                                           reinterpret_cast<double2 *>(out));
     } else {
         float2 *part = reinterpret_cast<float2 *>(ws);
