@@ -76,6 +76,67 @@ __device__ inline double sin_cycles_f64(double u)
     return t * p;
 }
 
+// sin and cos of 2 pi u in FP64, u in cycles: u reduced exactly to t in
+// [-1/8, 1/8] and the octant's quarter turn, both Taylor series summed to t^17
+// and t^16 (the next terms are below 3e-18), swapped and signed by the quarter.
+// About 35 instructions, where the library's sincospi takes about 55.
+__device__ inline void sincos_cycles_f64(double u, double &s, double &c)
+{
+    const double r = u - __builtin_rint(u);
+    const double q = __builtin_rint(4.0 * r);
+    const double t = fma(-0.25, q, r);
+    const int iq = (int)q;
+    const double w = t * t;
+    double ps = 0.10422916220813984, pc = 0.28200596845579123;
+    ps = fma(ps, w, -0.71812230177850056);
+    pc = fma(pc, w, -1.714390711088672);
+    ps = fma(ps, w, 3.819952584848282);
+    pc = fma(pc, w, 7.9035363713184692);
+    ps = fma(ps, w, -15.09464257682299);
+    pc = fma(pc, w, -26.426256783374399);
+    ps = fma(ps, w, 42.058693944897655);
+    pc = fma(pc, w, 60.244641371876661);
+    ps = fma(ps, w, -76.705859753061389);
+    pc = fma(pc, w, -85.456817206693728);
+    ps = fma(ps, w, 81.605249276075057);
+    pc = fma(pc, w, 64.939394022668296);
+    ps = fma(ps, w, -41.341702240399762);
+    pc = fma(pc, w, -19.739208802178716);
+    ps = fma(ps, w, 6.2831853071795862);
+    pc = fma(pc, w, 1);
+    ps *= t;
+    const bool odd = iq & 1;
+    const unsigned long long ss = (unsigned long long)(iq & 2) << 62, sc = (unsigned long long)((iq + 1) & 2) << 62;
+    s = __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, odd ? pc : ps) ^ ss);
+    c = __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, odd ? ps : pc) ^ sc);
+}
+
+// The same in FP32, u reduced in FP64: Taylor series to t^9 and t^10 (the next
+// terms are below 2e-9), within an ulp or so of the rounded result where the
+// hardware sine and cosine have an absolute error of a few 1e-8.
+__device__ inline void sincos_cycles_f32(double u, float &s, float &c)
+{
+    const double r = u - __builtin_rint(u);
+    const double q = __builtin_rint(4.0 * r);
+    const float t = (float)fma(-0.25, q, r);
+    const int iq = (int)q;
+    const float w = t * t;
+    float ps = 42.0586939f, pc = -26.4262568f;
+    pc = fmaf(pc, w, 60.2446414f);
+    ps = fmaf(ps, w, -76.7058598f);
+    pc = fmaf(pc, w, -85.4568172f);
+    ps = fmaf(ps, w, 81.6052493f);
+    pc = fmaf(pc, w, 64.939394f);
+    ps = fmaf(ps, w, -41.3417022f);
+    pc = fmaf(pc, w, -19.7392088f);
+    ps = fmaf(ps, w, 6.28318531f);
+    pc = fmaf(pc, w, 1.0f);
+    ps *= t;
+    const bool odd = iq & 1;
+    s = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, odd ? pc : ps) ^ ((unsigned)(iq & 2) << 30));
+    c = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, odd ? ps : pc) ^ ((unsigned)((iq + 1) & 2) << 30));
+}
+
 // (double)(float)pi / pi: the reference forms 2*pi from a float constant
 // (cpp/feelmri/MRI.h:13), so every k.x phase carries this factor.
 constexpr double kPiFOverPi = static_cast<double>(static_cast<float>(3.14159265358979323846)) /
@@ -90,6 +151,13 @@ int device_cu_count();
 // cannot tell.
 template <typename F>
 int blocks_per_cu(F kernel, int threads, size_t dyn)
+{
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, dyn) != hipSuccess || n < 1) n = 1;
+    return n;
+}
+
+inline int blocks_per_cu(const void *kernel, int threads, size_t dyn)
 {
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, dyn) != hipSuccess || n < 1) n = 1;

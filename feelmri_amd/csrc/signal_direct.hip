@@ -4,21 +4,22 @@
 //
 // reference: cpp/feelmri/MRI.cpp:196-297 (static nodes), :38-159 (moving).
 //
-// Work decomposition.  Samples of equal t are grouped (the reference's t
-// cache) and cut into slots of up to 256 samples; a workgroup owns a tile of
-// two slots (2 samples per lane, the slots possibly of different t) and one
-// contiguous split of the nodes.  Nodes stream
-// through LDS in chunks of 256: each lane of the workgroup stages one node,
-// folding the t-dependent factors (T2* decay, off-resonance, and the POD
-// position update for moving nodes) into the staged coefficient, so the
-// inner loop per (node, sample) is just the k.x phase, one sincos and a
-// complex MAC.  All lanes read the same LDS node at the same time
-// (broadcast).  Node splits write partial sums that a second kernel adds in
-// a fixed order, so results do not depend on scheduling.
+// Work decomposition.  A workgroup owns a tile of samples and one contiguous
+// split of the nodes, which stream through LDS in chunks; all lanes read the
+// same LDS node at the same time (broadcast).  Node splits write partial sums
+// that a second kernel adds in a fixed order, so results do not depend on
+// scheduling.  Four kernels:
+//   * samples grouped by t (the reference's t cache): k_signal_groups
+//     (signal_groups.hip), all moving nodes, and static nodes whose t-groups
+//     are not tiny;
+//   * samples in any order, per-sample t: k_signal_consec, static nodes;
+//   * readouts linear in k and t: k_signal_runs and k_signal_runs_f64, static
+//     nodes;
+//   * whole lines linear in k and t: the per-line GEMM (signal_lines_bf16.hip).
 //
 // Phase handling.  u = k'.x is accumulated in FP64 in cycles (k' carries the
-// reference's float-pi factor).  FP64 form: r = u - rint(u) in [-1/2, 1/2],
-// sincospi(2r).  Mixed form: fract(u) in [0, 1) (one instruction, exact),
+// reference's float-pi factor).  FP64 form: exact range reduction, FP64 sine
+// and cosine.  Mixed form: fract(u) in [0, 1) (one instruction, exact),
 // rounded to FP32 and fed to the hardware v_sin_f32 / v_cos_f32, which take
 // revolutions; partial sums over a 256-node chunk are kept in FP32 and added
 // into FP64.
@@ -43,122 +44,47 @@ struct CoefT<false> {
     using T = double;
 };
 
-// A node staged in LDS.  Shared-t tiles carry one coefficient set per slot
-// (the slots of a tile may belong to different t-groups) or, in packed slots
-// of GP t-groups, one per (slot, group); for moving nodes one position per
-// slot.
-template <int VB, bool MIXED, bool SHARED_T, bool MOTION, int GP = 1, bool CONJ = false>
+// A node staged in LDS.
+template <int VB, bool MIXED>
 struct alignas(16) StagedNode {
     using CT = typename CoefT<MIXED>::T;
-    static constexpr int kPos = MOTION ? kDirectSPL : 1;
-    // conjugate-pair tiles: both slots hold the same GP t-groups
-    static constexpr int kCoef = SHARED_T ? (CONJ ? GP : kDirectSPL * GP) : 1;
-    static constexpr bool kPair = MIXED && GP > 1 && !CONJ;  // second slot's phase by FP32 offset
-    double x[kPos], y[kPos], z[kPos];
-    double dwc;                  // phi/(2 pi), cycles/ms   (per-sample-t kernel only)
-    double r2;                   // 1/T2, 1/ms              (per-sample-t kernel only)
-    CT c[kCoef][2 * VB];
-    float xf[kPair ? 4 : 1];     // packed mixed slots: x, y, z in FP32 and max |x|, |y|, |z|
+    double x, y, z;
+    double dwc;  // phi/(2 pi), cycles/ms
+    double r2;   // 1/T2, 1/ms
+    CT b[2 * VB];
 };
 
-// Tiles.  Shared-t ("grouped") tiles are kDirectSPL slot records
-// tiles[kDirectSPL * b + j]: slot j holds up to 256 samples of one t-group
-// (lane l takes sample perm[offset + l]).  Packed slots (GP > 1, static
-// nodes) hold GP consecutive t-groups of 256 / GP samples each, starting at
-// group `group`: lane l belongs to group + l / (256 / GP), and the
-// t-dependent factor exp(-t/T2) exp(i phi t) is staged per (node, slot,
-// group) instead of being formed per (node, sample).  Per-sample-t
-// ("consecutive") tiles are one record of up to 512 consecutive samples
-// (lane l takes offset + l + 256 j).
-//
-// In packed slots of the mixed form the two samples of a lane lie on one
-// line, GP readout indices apart.  When |k'1 - k'0|_1 max(|x|,|y|,|z|) <= 4
-// cycles for every node of a chunk (pair_dk is the plan's bound on the
-// first factor), the second phase is formed as the first one's FP64-reduced
-// phase plus (k'1 - k'0).x in FP32: an FP32 error of ~1e-6 cycles on top of
-// the FP64 range reduction.  PLANAR drops the kz.z term (every kz = 0).
-//
-// Conjugate-pair tiles (CONJ, mixed form): both slots hold the same GP
-// t-groups, and lane l's slot-1 sample has k'_b = -k'_a of its slot-0
-// sample (to 1e-12 of the largest |k'|, the plan checks; e.g. spiral
-// interleaves half a turn apart).  One phase and one sine/cosine then serve
-// both: exp(-2 pi i k'_b.x) = conj(exp(-2 pi i k'_a.x)), and the two share
-// the t-group's coefficient c, so the lane adds c e and c conj(e).
-template <int VB, bool MIXED, bool SHARED_T, bool MOTION, int GP = 1, bool PLANAR = false, bool CONJ = false>
-__global__ __launch_bounds__(kDirectThreads) void k_signal_direct(
-    const double *__restrict__ packed, int64_t N, int V, int v0,
-    const double4 *__restrict__ ks, const int32_t *__restrict__ perm,
-    const SignalTile *__restrict__ tiles, const double *__restrict__ tg_t,
-    const float *__restrict__ modes, int R, const double *__restrict__ mcoef,
-    int64_t nodes_per_split, double2 *__restrict__ dst, int64_t S, int write_final, double pair_dk)
+// Static nodes, tiles of up to 512 consecutive samples of any t (lane l takes
+// samples offset + l and offset + l + 256): the decay and the off-resonance
+// phase are formed per (node, sample).
+template <int VB, bool MIXED>
+__global__ __launch_bounds__(kDirectThreads) void k_signal_consec(
+    const double *__restrict__ packed, int64_t N, int V, int v0, const double4 *__restrict__ ks,
+    const SignalTile *__restrict__ tiles, int64_t nodes_per_split, double2 *__restrict__ dst, int64_t S,
+    int write_final)
 {
     using CT = typename CoefT<MIXED>::T;
-    using Node = StagedNode<VB, MIXED, SHARED_T, MOTION, GP, CONJ>;
-    static_assert(GP == 1 || (SHARED_T && !MOTION), "packed t-groups: shared-t tiles of static nodes");
-    static_assert(!CONJ || (MIXED && GP > 1 && kDirectSPL == 2), "conjugate pairs: mixed packed slots");
-    static_assert(!PLANAR || GP > 1, "planar phases: packed slots only");
-    constexpr bool kPair = Node::kPair && kDirectSPL == 2;
-    constexpr int kSlots = SHARED_T ? kDirectSPL : 1;
-    constexpr int kGSize = kDirectThreads / GP;  // samples per group of a packed slot
-    __shared__ Node snode[kDirectThreads];
-    __shared__ double scoef[MOTION ? kDirectSPL : 1][kMaxModes + 3];
-
+    __shared__ StagedNode<VB, MIXED> snode[kDirectThreads];
     const int64_t split = blockIdx.y;
     const int64_t n_begin = split * nodes_per_split;
     const int64_t n_end = (n_begin + nodes_per_split < N) ? n_begin + nodes_per_split : N;
     const int tid = threadIdx.x;
-
-    const double *px = packed;
-    const double *py = packed + N;
-    const double *pz = packed + 2 * N;
-    const double *pphi = packed + 3 * N;
-    const double *pr2 = packed + 4 * N;
-    const double *pb = packed + 5 * N;  // rows 2v, 2v+1
-
-    SignalTile tl[kSlots];
-#pragma unroll
-    for (int j = 0; j < kSlots; ++j) tl[j] = tiles[(int64_t)blockIdx.x * kSlots + j];
-    // slot (and group) times: uniform over the workgroup, kept in LDS
-    __shared__ double tg[kDirectSPL * GP];
-    bool same_group = GP == 1;  // both slots share one t-group (stage once)
-    if (SHARED_T) {
-        if (tid < kDirectSPL * GP) {
-            const int j = tid / GP, q = tid % GP;
-            tg[tid] = tl[j].count > q * kGSize ? tg_t[tl[j].group + q] : 0.0;
-        }
-#pragma unroll
-        for (int j = 1; j < kDirectSPL; ++j) same_group = same_group && (tl[j].group == tl[0].group || tl[j].count == 0);
-    }
-    const int gq = GP > 1 ? threadIdx.x / kGSize : 0;  // this lane's group in a packed slot
-    if (MOTION) {
-#pragma unroll
-        for (int j = 0; j < kDirectSPL; ++j)
-            for (int q = tid; q < R + 3; q += kDirectThreads)
-                scoef[j][q] = tl[j].count > 0 ? mcoef[(int64_t)tl[j].group * (R + 3) + q] : 0.0;
-    }
+    const SignalTile tl = tiles[blockIdx.x];
 
     int sid[kDirectSPL];
     bool valid[kDirectSPL];
     double kxs[kDirectSPL], kys[kDirectSPL], kzs[kDirectSPL], ts[kDirectSPL];
 #pragma unroll
     for (int j = 0; j < kDirectSPL; ++j) {
-        if (SHARED_T) {
-            valid[j] = tid < tl[j].count;
-            sid[j] = valid[j] ? perm[tl[j].offset + tid] : 0;
-        } else {
-            const int idx = tid + j * kDirectThreads;
-            valid[j] = idx < tl[0].count;
-            sid[j] = valid[j] ? tl[0].offset + idx : 0;
-        }
+        const int idx = tid + j * kDirectThreads;
+        valid[j] = idx < tl.count;
+        sid[j] = valid[j] ? tl.offset + idx : 0;
         const double4 k = ks[sid[j]];
         kxs[j] = k.x;
         kys[j] = k.y;
         kzs[j] = k.z;
         ts[j] = k.w;
     }
-    const float dkx = (float)(kxs[kSlots - 1] - kxs[0]), dky = (float)(kys[kSlots - 1] - kys[0]),
-                dkz = (float)(kzs[kSlots - 1] - kzs[0]);
-
     double tot_re[kDirectSPL][VB], tot_im[kDirectSPL][VB];
 #pragma unroll
     for (int j = 0; j < kDirectSPL; ++j)
@@ -166,103 +92,23 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_direct(
         for (int v = 0; v < VB; ++v) tot_re[j][v] = tot_im[j][v] = 0.0;
 
     for (int64_t base = n_begin; base < n_end; base += kDirectThreads) {
-        __syncthreads();  // previous chunk fully consumed (and scoef visible)
-        int far_node = 0;  // this thread's node too far out for the FP32 offset
+        __syncthreads();  // previous chunk fully consumed
         {
             const int64_t n = base + tid;
-            // staged in place: packed slots carry 2 GP coefficient sets per
-            // node, too many to assemble in registers first
-            Node &nd = snode[tid];
-            if (n < n_end) {
-                const double x0 = px[n], y0 = py[n], z0 = pz[n];
+            const bool ok = n < n_end;
+            StagedNode<VB, MIXED> &nd = snode[tid];
+            nd.x = ok ? packed[n] : 0.0;
+            nd.y = ok ? packed[N + n] : 0.0;
+            nd.z = ok ? packed[2 * N + n] : 0.0;
+            nd.dwc = (ok ? packed[3 * N + n] : 0.0) * (1.0 / kTwoPi);
+            nd.r2 = ok ? packed[4 * N + n] : 0.0;
 #pragma unroll
-                for (int j = 0; j < Node::kPos; ++j) {
-                    double x = x0, y = y0, z = z0;
-                    if (MOTION) {
-                        if (j > 0 && same_group) {
-                            x = nd.x[0];
-                            y = nd.y[0];
-                            z = nd.z[0];
-                        } else {
-                            double dx = scoef[j][R], dy = scoef[j][R + 1], dz = scoef[j][R + 2];
-                            for (int r = 0; r < R; ++r) {
-                                const double w = scoef[j][r];
-                                dx += (double)modes[(int64_t)(0 * R + r) * N + n] * w;
-                                dy += (double)modes[(int64_t)(1 * R + r) * N + n] * w;
-                                dz += (double)modes[(int64_t)(2 * R + r) * N + n] * w;
-                            }
-                            x += dx;
-                            y += dy;
-                            z += dz;
-                        }
-                    }
-                    nd.x[j] = x;
-                    nd.y[j] = y;
-                    nd.z[j] = z;
-                }
-                const double phi = pphi[n], r2 = pr2[n];
-                nd.dwc = phi * (1.0 / kTwoPi);
-                nd.r2 = r2;
-                if constexpr (kPair) {
-                    nd.xf[0] = (float)x0;
-                    nd.xf[1] = (float)y0;
-                    nd.xf[2] = PLANAR ? 0.0f : (float)z0;
-                    nd.xf[3] = (float)fmax(fabs(x0), fmax(fabs(y0), PLANAR ? 0.0 : fabs(z0)));
-                    far_node = fmax(fabs(x0), fmax(fabs(y0), PLANAR ? 0.0 : fabs(z0))) * pair_dk > 4.0;
-                }
-                for (int j = 0; j < Node::kCoef; ++j) {
-                    if (SHARED_T) {
-                        if (j > 0 && same_group) {
-#pragma unroll
-                            for (int v = 0; v < 2 * VB; ++v) nd.c[j][v] = nd.c[0][v];
-                            continue;
-                        }
-                        // c = b exp(-t/T2) exp(i phi t)   (MRI.cpp:264-271); the
-                        // mixed form reduces phi t / 2 pi in FP64 and takes the
-                        // FP32 hardware sine, cosine and exp2
-                        double fr, fi;
-                        if constexpr (MIXED) {
-                            const double u = phi * tg[j] * (1.0 / kTwoPi);
-                            const float r = turns_f32(u);
-                            const float d = __builtin_amdgcn_exp2f((float)(-tg[j] * r2 * 1.4426950408889634));
-                            fr = (double)(d * __builtin_amdgcn_cosf(r));
-                            fi = (double)(d * __builtin_amdgcn_sinf(r));
-                        } else {
-                            const double d = exp(-tg[j] * r2);
-                            double so, co;
-                            sincos(phi * tg[j], &so, &co);
-                            fr = d * co;
-                            fi = d * so;
-                        }
-#pragma unroll
-                        for (int v = 0; v < VB; ++v) {
-                            const double br = pb[(int64_t)(2 * (v0 + v)) * N + n];
-                            const double bi = pb[(int64_t)(2 * (v0 + v) + 1) * N + n];
-                            nd.c[j][2 * v] = (CT)(br * fr - bi * fi);
-                            nd.c[j][2 * v + 1] = (CT)(br * fi + bi * fr);
-                        }
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < VB; ++v) {
-                            nd.c[j][2 * v] = (CT)pb[(int64_t)(2 * (v0 + v)) * N + n];
-                            nd.c[j][2 * v + 1] = (CT)pb[(int64_t)(2 * (v0 + v) + 1) * N + n];
-                        }
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < Node::kPos; ++j) nd.x[j] = nd.y[j] = nd.z[j] = 0.0;
-                nd.dwc = nd.r2 = 0.0;
-                if constexpr (kPair) nd.xf[0] = nd.xf[1] = nd.xf[2] = nd.xf[3] = 0.0f;
-#pragma unroll
-                for (int j = 0; j < Node::kCoef; ++j)
-#pragma unroll
-                    for (int v = 0; v < 2 * VB; ++v) nd.c[j][v] = (CT)0;
+            for (int v = 0; v < VB; ++v) {
+                nd.b[2 * v] = ok ? (CT)packed[(int64_t)(5 + 2 * (v0 + v)) * N + n] : (CT)0;
+                nd.b[2 * v + 1] = ok ? (CT)packed[(int64_t)(6 + 2 * (v0 + v)) * N + n] : (CT)0;
             }
         }
-        bool pair_path = false;
-        if constexpr (kPair) pair_path = !__syncthreads_or(far_node);
-        else __syncthreads();
+        __syncthreads();
         const int cnt = (n_end - base < kDirectThreads) ? (int)(n_end - base) : kDirectThreads;
 
         CT acc_re[kDirectSPL][VB], acc_im[kDirectSPL][VB];
@@ -270,93 +116,33 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_direct(
         for (int j = 0; j < kDirectSPL; ++j)
 #pragma unroll
             for (int v = 0; v < VB; ++v) acc_re[j][v] = acc_im[j][v] = (CT)0;
-
-        if constexpr (CONJ) {
-            // one phase per pair; slot 1 takes the conjugate factor
-#pragma unroll 2
-            for (int m = 0; m < cnt; ++m) {
-                const Node &nd = snode[m];
-                const double u = PLANAR ? fma(kxs[0], nd.x[0], kys[0] * nd.y[0])
-                                        : fma(kxs[0], nd.x[0], fma(kys[0], nd.y[0], kzs[0] * nd.z[0]));
-                const float r = turns_f32(u);
-                const CT sn = __builtin_amdgcn_sinf(r), cs = __builtin_amdgcn_cosf(r);
-#pragma unroll
-                for (int v = 0; v < VB; ++v) {
-                    const CT cr = nd.c[gq][2 * v], ci = nd.c[gq][2 * v + 1];
-                    acc_re[0][v] = fma(cs, cr, fma(sn, ci, acc_re[0][v]));
-                    acc_im[0][v] = fma(cs, ci, fma(-sn, cr, acc_im[0][v]));
-                    acc_re[1][v] = fma(cs, cr, fma(-sn, ci, acc_re[1][v]));
-                    acc_im[1][v] = fma(cs, ci, fma(sn, cr, acc_im[1][v]));
-                }
-            }
-        } else if (pair_path) {
-            // first slot: FP64 phase, range-reduced; second: plus dk.x in FP32
-            if constexpr (kPair) {
-#pragma unroll 2
-            for (int m = 0; m < cnt; ++m) {
-                const Node &nd = snode[m];
-                const double u = PLANAR ? fma(kxs[0], nd.x[0], kys[0] * nd.y[0])
-                                        : fma(kxs[0], nd.x[0], fma(kys[0], nd.y[0], kzs[0] * nd.z[0]));
-                float r[2];
-                r[0] = turns_f32(u);
-                r[1] = turns_f32(r[0] + (PLANAR ? fmaf(dkx, nd.xf[0], dky * nd.xf[1])
-                                                : fmaf(dkx, nd.xf[0], fmaf(dky, nd.xf[1], dkz * nd.xf[2]))));
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const CT sn = __builtin_amdgcn_sinf(r[j]), cs = __builtin_amdgcn_cosf(r[j]);
-                    const int jc = j * GP + gq;
-#pragma unroll
-                    for (int v = 0; v < VB; ++v) {
-                        const CT cr = nd.c[jc][2 * v], ci = nd.c[jc][2 * v + 1];
-                        acc_re[j][v] = fma(cs, cr, fma(sn, ci, acc_re[j][v]));
-                        acc_im[j][v] = fma(cs, ci, fma(-sn, cr, acc_im[j][v]));
-                    }
-                }
-            }
-            }
-        } else {
 #pragma unroll 2
         for (int m = 0; m < cnt; ++m) {
-            const Node &nd = snode[m];
+            const StagedNode<VB, MIXED> &nd = snode[m];
 #pragma unroll
             for (int j = 0; j < kDirectSPL; ++j) {
-                const int jp = MOTION ? j : 0;
-                double u = PLANAR ? fma(kxs[j], nd.x[jp], kys[j] * nd.y[jp])
-                                  : fma(kxs[j], nd.x[jp], fma(kys[j], nd.y[jp], kzs[j] * nd.z[jp]));
-                if (!SHARED_T) u = fma(-nd.dwc, ts[j], u);  // phase - phi t, in cycles
-                CT cs, sn;
-                if (MIXED) {
+                // phase - phi t, in cycles
+                const double u = fma(-nd.dwc, ts[j], fma(kxs[j], nd.x, fma(kys[j], nd.y, kzs[j] * nd.z)));
+                CT cs, sn, d;
+                if constexpr (MIXED) {
                     const float rf = turns_f32(u);
                     sn = __builtin_amdgcn_sinf(rf);
                     cs = __builtin_amdgcn_cosf(rf);
+                    d = __builtin_amdgcn_exp2f((float)(-ts[j] * nd.r2 * 1.4426950408889634));
                 } else {
-                    const double rr = u - __builtin_rint(u);
-                    double s_, c_;
-                    sincospi(2.0 * rr, &s_, &c_);
-                    sn = (CT)s_;
-                    cs = (CT)c_;
+                    sincos_cycles_f64(u, sn, cs);
+                    d = exp(-ts[j] * nd.r2);
                 }
-                if (!SHARED_T) {
-                    // exp(-t/T2) per (node, sample)
-                    CT d;
-                    if (MIXED) {
-                        d = __builtin_amdgcn_exp2f((float)(-ts[j] * nd.r2 * 1.4426950408889634));
-                    } else {
-                        d = (CT)exp(-ts[j] * nd.r2);
-                    }
-                    cs *= d;
-                    sn *= d;
-                }
-                // e = cs - i sn ; acc += e * c
-                const int jc = SHARED_T ? j * GP + gq : 0;
+                cs *= d;
+                sn *= d;
+                // e = cs - i sn ; acc += e * b
 #pragma unroll
                 for (int v = 0; v < VB; ++v) {
-                    const CT cr = nd.c[jc][2 * v], ci = nd.c[jc][2 * v + 1];
+                    const CT cr = nd.b[2 * v], ci = nd.b[2 * v + 1];
                     acc_re[j][v] = fma(cs, cr, fma(sn, ci, acc_re[j][v]));
                     acc_im[j][v] = fma(cs, ci, fma(-sn, cr, acc_im[j][v]));
                 }
             }
-        }
         }
 #pragma unroll
         for (int j = 0; j < kDirectSPL; ++j)
@@ -366,7 +152,6 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_direct(
                 tot_im[j][v] += (double)acc_im[j][v];
             }
     }
-
 #pragma unroll
     for (int j = 0; j < kDirectSPL; ++j) {
         if (!valid[j]) continue;
@@ -384,7 +169,7 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_direct(
 //   q  = exp(-dt/T2) exp(-2 pi i (dk.x - phi dt / 2 pi))       (FP32)
 // and accumulates e0 q^m c for m = 0 .. kRunLen-1, advancing e (one
 // encoding: y = e c) by one complex multiply per sample.  FP32 partial sums over a 256-node chunk are
-// added into FP64, as in k_signal_direct.
+// added into FP64, as in k_signal_consec.
 template <int VB>
 struct alignas(16) RunNode {
     double x, y, z, dwc, r2;
@@ -765,14 +550,11 @@ struct DirectLaunch {
     int64_t nodes_per_split;
 };
 
-// Tilings of the direct path: 0 consecutive, 1 t-grouped, 2 readout runs,
-// 3 packed t-groups, 4 conjugate pairs in packed t-groups (mixed form).
+// Tilings of the direct path: 0 consecutive, 1 t-grouped, 2 readout runs.
 static int64_t direct_tiles(const fm_signal_plan *p, int tiling)
 {
-    if (tiling == 4) return p->n_tiles_conj;
-    if (tiling == 3) return p->n_tiles_packed;
     if (tiling == 2) return cdiv(p->n_runs, kDirectThreads);
-    return tiling == 1 ? p->n_tiles_grouped : p->n_tiles_consec;
+    return tiling == 1 ? p->n_tiles_pairs : p->n_tiles_consec;
 }
 
 static DirectLaunch direct_launch_shape(const fm_signal_plan *p, int64_t N, int tiling)
@@ -791,35 +573,27 @@ static DirectLaunch direct_launch_shape(const fm_signal_plan *p, int64_t N, int 
     return {splits, nps};
 }
 
-template <int VB, bool MIXED>
-static void launch_direct_vb(const fm_signal_plan *p, bool grouped, bool motion, dim3 grid,
-                             const double *packed, int64_t N, int V, int v0, const float *modes,
-                             int R, const double *mcoef, int64_t nps, double2 *dst, int write_final,
-                             hipStream_t st)
+// The t-grouped tiles' splits: whole rounds of the workgroups the device
+// holds, no more splits than the consecutive tiles (the fewest tiles) would
+// take, whose workspace the query reports.
+static DirectLaunch groups_launch_shape(const fm_signal_plan *p, bool mixed, bool motion, int64_t N, int V, int R)
 {
-    if (grouped) {
-        if (motion)
-            k_signal_direct<VB, MIXED, true, true><<<grid, kDirectThreads, 0, st>>>(
-                packed, N, V, v0, p->d_ks, p->d_perm, p->d_tiles_grouped, p->d_tg_t, modes, R, mcoef,
-                nps, dst, p->n_samples, write_final, 0.0);
-        else
-            k_signal_direct<VB, MIXED, true, false><<<grid, kDirectThreads, 0, st>>>(
-                packed, N, V, v0, p->d_ks, p->d_perm, p->d_tiles_grouped, p->d_tg_t, modes, R, mcoef,
-                nps, dst, p->n_samples, write_final, 0.0);
-    } else {
-        k_signal_direct<VB, MIXED, false, false><<<grid, kDirectThreads, 0, st>>>(
-            packed, N, V, v0, p->d_ks, p->d_perm, p->d_tiles_consec, p->d_tg_t, modes, R, mcoef, nps,
-            dst, p->n_samples, write_final, 0.0);
-    }
+    const int64_t most = direct_launch_shape(p, N, 0).n_splits;
+    const int64_t nt = p->n_tiles_pairs;
+    const int64_t capacity = (int64_t)groups_blocks_per_cu(p, mixed, motion, V, R) * device_cu_count();
+    const int64_t s_max = std::min(most, cdiv(N, 2048));
+    const int64_t splits = balanced_splits(N, kDirectThreads, nt, cdiv(capacity, nt), capacity, s_max);
+    const int64_t nps = cdiv(cdiv(N, splits), kDirectThreads) * kDirectThreads;
+    return {cdiv(N, nps), nps};
 }
 
 template <bool MIXED>
-static void launch_direct(const fm_signal_plan *p, bool grouped, bool motion, dim3 grid,
-                          const double *packed, int64_t N, int V, int v0, int vb, const float *modes,
-                          int R, const double *mcoef, int64_t nps, double2 *dst, int write_final,
-                          hipStream_t st)
+static void launch_consec(const fm_signal_plan *p, dim3 grid, const double *packed, int64_t N, int V, int v0, int vb,
+                          int64_t nps, double2 *dst, int write_final, hipStream_t st)
 {
-#define FM_LD(VBV) launch_direct_vb<VBV, MIXED>(p, grouped, motion, grid, packed, N, V, v0, modes, R, mcoef, nps, dst, write_final, st)
+#define FM_LD(VBV)                                                                                                  \
+    k_signal_consec<VBV, MIXED><<<grid, kDirectThreads, 0, st>>>(packed, N, V, v0, p->d_ks, p->d_tiles_consec, nps, \
+                                                                 dst, p->n_samples, write_final)
     switch (vb) {
     case 1: FM_LD(1); break;
     case 2: FM_LD(2); break;
@@ -829,63 +603,15 @@ static void launch_direct(const fm_signal_plan *p, bool grouped, bool motion, di
 #undef FM_LD
 }
 
-template <bool MIXED>
-static void launch_packed(const fm_signal_plan *p, dim3 grid, const double *packed, int64_t N, int V, int v0,
-                          int64_t nps, double2 *dst, int write_final, hipStream_t st)
-{
-#define FM_LP(GPV, PL)                                                                                      \
-    k_signal_direct<1, MIXED, true, false, GPV, PL><<<grid, kDirectThreads, 0, st>>>(                      \
-        packed, N, V, v0, p->d_ks, p->d_perm, p->d_tiles_packed, p->d_tg_t, nullptr, 0, nullptr, nps, dst, \
-        p->n_samples, write_final, p->packed_dk)
-    if (p->planar) {
-        switch (p->group_pack) {
-        case 2: FM_LP(2, true); break;
-        case 4: FM_LP(4, true); break;
-        default: FM_LP(8, true); break;
-        }
-    } else {
-        switch (p->group_pack) {
-        case 2: FM_LP(2, false); break;
-        case 4: FM_LP(4, false); break;
-        default: FM_LP(8, false); break;
-        }
-    }
-#undef FM_LP
-}
-
-static void launch_conj(const fm_signal_plan *p, dim3 grid, const double *packed, int64_t N, int V, int v0,
-                        int64_t nps, double2 *dst, int write_final, hipStream_t st)
-{
-#define FM_LQ(GPV, PL)                                                                                          \
-    k_signal_direct<1, true, true, false, GPV, PL, true><<<grid, kDirectThreads, 0, st>>>(                     \
-        packed, N, V, v0, p->d_ks, p->d_perm_conj, p->d_tiles_conj, p->d_tg_t, nullptr, 0, nullptr, nps, dst, \
-        p->n_samples, write_final, 0.0)
-    if (p->planar) {
-        switch (p->conj_pack) {
-        case 4: FM_LQ(4, true); break;
-        case 8: FM_LQ(8, true); break;
-        default: FM_LQ(16, true); break;
-        }
-    } else {
-        switch (p->conj_pack) {
-        case 4: FM_LQ(4, false); break;
-        case 8: FM_LQ(8, false); break;
-        default: FM_LQ(16, false); break;
-        }
-    }
-#undef FM_LQ
-}
-
 static size_t direct_workspace(const fm_signal_plan *p, int64_t N, int V)
 {
     if (N <= 0 || p->n_samples == 0) return 0;
-    // the largest of the tilings' needs (motion forces the grouped one) and
-    // of the per-line GEMM's partial samples (one encoding at a time)
+    // the largest of the tilings' needs (the t-grouped tiles take no more
+    // splits than the consecutive ones) and of the per-line GEMM's partial
+    // samples (one encoding at a time)
     size_t need = lines_workspace(p, N);
-    for (int g = 0; g < 5; ++g) {
+    for (int g = 0; g < 3; g += 2) {
         if (g == 2 && p->n_runs == 0) continue;
-        if (g == 3 && p->group_pack <= 1) continue;
-        if (g == 4 && p->conj_pack <= 1) continue;
         const DirectLaunch L = direct_launch_shape(p, N, g);
         if (L.n_splits > 1)
             need = std::max(need, (size_t)L.n_splits * (size_t)p->n_samples * (size_t)V * sizeof(double2));
@@ -909,13 +635,10 @@ static int direct_execute(const fm_signal_plan *p, int precision, int64_t N, int
     // static nodes take the readout runs when the plan has them (the FP64
     // form only when they are linear to 1e-14)
     const bool use_runs = !motion && p->n_runs > 0 && (precision != FM_PREC_F64 || p->runs_exact);
-    // static nodes with small equal-size t-groups: packed slots
-    const bool use_packed = !motion && !use_runs && p->group_pack > 1;
-    // mixed form: conjugate pairs when every packed group pairs up
-    const bool use_conj = use_packed && precision != FM_PREC_F64 && p->conj_pack > 1;
-    const bool grouped = motion || p->prefer_grouped;
-    const int tiling = use_runs ? 2 : (use_conj ? 4 : (use_packed ? 3 : (grouped ? 1 : 0)));
-    const DirectLaunch L = direct_launch_shape(p, N, tiling);
+    const bool grouped = motion || (!use_runs && p->prefer_grouped);
+    const int tiling = use_runs ? 2 : (grouped ? 1 : 0);
+    const DirectLaunch L = grouped ? groups_launch_shape(p, precision != FM_PREC_F64, motion, N, V, R)
+                                   : direct_launch_shape(p, N, tiling);
     const size_t need = L.n_splits > 1 ? (size_t)L.n_splits * (size_t)S * (size_t)V * sizeof(double2) : 0;
     if (need > ws_bytes) {
         set_error("signal workspace too small: need %zu bytes, got %zu", need, ws_bytes);
@@ -949,26 +672,19 @@ static int direct_execute(const fm_signal_plan *p, int precision, int64_t N, int
             FM_LAUNCH_CHECK("k_signal_runs");
         }
     }
-    if (use_packed) {
-        // one encoding per launch: the per-(slot, group) coefficients of a
-        // staged node take 2 * group_pack complex values per encoding
-        for (int v0 = 0; v0 < V; ++v0) {
-            if (precision == FM_PREC_F64)
-                launch_packed<false>(p, grid, packed, N, V, v0, L.nodes_per_split, dst, write_final, st);
-            else if (use_conj)
-                launch_conj(p, grid, packed, N, V, v0, L.nodes_per_split, dst, write_final, st);
-            else
-                launch_packed<true>(p, grid, packed, N, V, v0, L.nodes_per_split, dst, write_final, st);
-            FM_LAUNCH_CHECK("k_signal_direct (packed t-groups)");
-        }
-    }
-    for (int v0 = 0; v0 < V && !use_runs && !use_packed; v0 += kMaxVB) {
+    for (int v0 = 0; v0 < V && !use_runs; v0 += kMaxVB) {
         const int vb = (V - v0 < kMaxVB) ? V - v0 : kMaxVB;
+        if (grouped) {
+            const int rc = groups_launch(p, precision != FM_PREC_F64, motion, N, V, v0, vb, packed, modes, R, mcoef,
+                                         L.n_splits, L.nodes_per_split, dst, write_final, st);
+            if (rc != FM_OK) return rc;
+            continue;
+        }
         if (precision == FM_PREC_F64)
-            launch_direct<false>(p, grouped, motion, grid, packed, N, V, v0, vb, modes, R, mcoef, L.nodes_per_split, dst, write_final, st);
+            launch_consec<false>(p, grid, packed, N, V, v0, vb, L.nodes_per_split, dst, write_final, st);
         else
-            launch_direct<true>(p, grouped, motion, grid, packed, N, V, v0, vb, modes, R, mcoef, L.nodes_per_split, dst, write_final, st);
-        FM_LAUNCH_CHECK("k_signal_direct");
+            launch_consec<true>(p, grid, packed, N, V, v0, vb, L.nodes_per_split, dst, write_final, st);
+        FM_LAUNCH_CHECK("k_signal_consec");
     }
     plan_timing_stop(p, st);
     if (L.n_splits > 1) {
@@ -990,9 +706,10 @@ using namespace fm;
 namespace fm {
 // Host tables of a plan before upload.
 struct PlanHost {
-    std::vector<int32_t> perm;
-    std::vector<SignalTile> tiles_g, tiles_c, tiles_p, tiles_q;
-    std::vector<int32_t> perm_conj;
+    std::vector<SignalTile> tiles_c;
+    std::vector<int2> pairs;             // per lane: samples
+    std::vector<uint8_t> lane_group;     // per lane: group of its tile
+    std::vector<int4> tiles_p;
     std::vector<double4> ks;
     std::vector<RunDesc> runs;
     std::vector<RunDesc> lines;       // whole linear lines (per-line GEMM)
@@ -1037,136 +754,137 @@ static int plan_analyse(fm_signal_plan *p, const double *kx, const double *ky, c
         p->method = ok ? FM_METHOD_CARTESIAN : FM_METHOD_DIRECT;
     }
 
-    // Tilings.  Grouped: samples ordered by t-group, each tile within one
-    // group, so the t-dependent node factors are staged once per tile.
-    // Consecutive: plain runs of samples, per-sample t.  Static nodes prefer
-    // the grouped tiles when groups fill most of a 512-sample tile.
-    std::vector<int32_t> &perm = h.perm;
-    perm.resize((size_t)S);
-    std::vector<SignalTile> &tiles_g = h.tiles_g, &tiles_c = h.tiles_c;
-    {
-        std::vector<int64_t> count((size_t)p->n_tgroups + 1, 0);
-        for (int64_t s = 0; s < S; ++s) count[(size_t)p->sample_group[(size_t)s] + 1]++;
-        for (int64_t g = 0; g < p->n_tgroups; ++g) count[(size_t)g + 1] += count[(size_t)g];
-        std::vector<int64_t> fill(count.begin(), count.end() - 1);
-        for (int64_t s = 0; s < S; ++s) perm[(size_t)fill[(size_t)p->sample_group[(size_t)s]]++] = (int32_t)s;
-        // grouped: slot records of up to 256 samples of one group, packed
-        // kDirectSPL to a tile (slots of one tile may hold different groups)
-        for (int64_t g = 0; g < p->n_tgroups; ++g) {
-            for (int64_t o = count[(size_t)g]; o < count[(size_t)g + 1]; o += kDirectThreads) {
-                const int64_t c = std::min<int64_t>(kDirectThreads, count[(size_t)g + 1] - o);
-                tiles_g.push_back({(int32_t)g, (int32_t)o, (int32_t)c, 0});
-            }
-        }
-        while (tiles_g.size() % kDirectSPL) tiles_g.push_back({0, 0, 0, 0});
-        // packed slots: every t-group has the same size g in {32, 64, 128}
-        // (e.g. the interleaves of a spiral at one readout index), so a slot
-        // takes 256 / g whole groups
-        const int64_t g0 = p->n_tgroups > 0 ? count[1] - count[0] : 0;
-        bool uniform = g0 == 32 || g0 == 64 || g0 == 128;
-        for (int64_t g = 0; g < p->n_tgroups && uniform; ++g) uniform = count[(size_t)g + 1] - count[(size_t)g] == g0;
-        if (uniform) {
-            const int64_t gp = kDirectThreads / g0;
-            for (int64_t g = 0; g < p->n_tgroups; g += gp) {
-                const int64_t ng = std::min<int64_t>(gp, p->n_tgroups - g);
-                h.tiles_p.push_back({(int32_t)g, (int32_t)count[(size_t)g], (int32_t)(ng * g0), 0});
-            }
-            while (h.tiles_p.size() % kDirectSPL) h.tiles_p.push_back({0, 0, 0, 0});
-            p->group_pack = (int)gp;
-            p->n_tiles_packed = (int64_t)h.tiles_p.size() / kDirectSPL;
-        }
-        for (int64_t o = 0; o < S; o += kDirectTile)
-            tiles_c.push_back({-1, (int32_t)o, (int32_t)std::min<int64_t>(kDirectTile, S - o), 0});
-    }
-    const double avg_group = p->n_tgroups ? (double)S / (double)p->n_tgroups : 0.0;
-    p->prefer_grouped = avg_group >= 64.0;
-    p->n_tiles_grouped = (int64_t)tiles_g.size() / kDirectSPL;
-    p->n_tiles_consec = (int64_t)tiles_c.size();
-
     std::vector<double4> &ks = h.ks;
     ks.resize((size_t)S);
     for (int64_t s = 0; s < S; ++s)
         ks[(size_t)s] = make_double4(kx[s] * kPiFOverPi, ky[s] * kPiFOverPi, kz[s] * kPiFOverPi, t[s]);
     p->planar = 1;
     for (int64_t s = 0; s < S && p->planar; ++s) p->planar = ks[(size_t)s].z == 0.0;
-    // the two samples of a lane in a packed tile (same line, group_pack
-    // readout indices apart): the kernel may form the second one's phase as
-    // the first one's reduced phase plus dk.x in FP32 when |dk|_1 |x|_inf
-    // stays small; record the largest |dk|_1
-    p->packed_dk = 0.0;
-    for (size_t b = 0; b + 1 < h.tiles_p.size(); b += kDirectSPL) {
-        const SignalTile &s0 = h.tiles_p[b], &s1 = h.tiles_p[b + 1];
-        const int32_t c = std::min(s0.count, s1.count);
-        for (int32_t l = 0; l < c; ++l) {
-            const double4 a = ks[(size_t)perm[(size_t)(s0.offset + l)]];
-            const double4 q = ks[(size_t)perm[(size_t)(s1.offset + l)]];
-            p->packed_dk = std::max(p->packed_dk, std::fabs(q.x - a.x) + std::fabs(q.y - a.y) + std::fabs(q.z - a.z));
-        }
-    }
 
-    // Conjugate pairs (mixed form): in every packed t-group pair each sample
-    // with one whose k' is its negative, to 1e-12 of the largest |k'| (an
-    // O(g0^2) search per group of g0 <= 128 samples; k' = 0 pairs with
-    // another k' = 0).  All groups or none.
-    p->conj_pack = 1;
-    p->n_tiles_conj = 0;
-    p->conj_dk = 0.0;
-    if (p->group_pack > 1 && S > 0) {
-        const int64_t g0 = kDirectThreads / p->group_pack;
-        double kmax = 0.0;
-        for (int64_t s = 0; s < S; ++s)
-            kmax = std::max({kmax, std::fabs(ks[(size_t)s].x), std::fabs(ks[(size_t)s].y), std::fabs(ks[(size_t)s].z)});
+    // Tilings.  Consecutive: plain runs of samples, per-sample t.  Grouped:
+    // lanes of two samples of one t-group, in the order of the groups, cut
+    // into tiles of 256 lanes and at most kGroupCap groups, so the t-dependent
+    // node factors are staged once per tile and group.
+    for (int64_t o = 0; o < S; o += kDirectTile)
+        h.tiles_c.push_back({(int32_t)o, (int32_t)std::min<int64_t>(kDirectTile, S - o)});
+    p->n_tiles_consec = (int64_t)h.tiles_c.size();
+    std::vector<int64_t> first((size_t)p->n_tgroups + 1, 0);  // group g: perm[first[g] .. first[g + 1])
+    std::vector<int32_t> perm((size_t)S);
+    {
+        for (int64_t s = 0; s < S; ++s) first[(size_t)p->sample_group[(size_t)s] + 1]++;
+        for (int64_t g = 0; g < p->n_tgroups; ++g) first[(size_t)g + 1] += first[(size_t)g];
+        std::vector<int64_t> fill(first.begin(), first.end() - 1);
+        for (int64_t s = 0; s < S; ++s) perm[(size_t)fill[(size_t)p->sample_group[(size_t)s]]++] = (int32_t)s;
+    }
+    const double avg_group = p->n_tgroups ? (double)S / (double)p->n_tgroups : 0.0;
+    p->prefer_grouped = avg_group >= kGroupMin;
+
+    // Conjugate pairs: in every t-group pair each sample with one whose k' is
+    // its negative, to 1e-12 of the largest |k'| (an O(g^2) search per group
+    // of at most 128 samples, given up at the first sample without a partner;
+    // k' = 0 pairs with another k' = 0).  All groups or none.
+    std::vector<int32_t> mate;  // partner of perm[i] for the first of each pair, else -1
+    double worst = 0.0, kmax = 0.0;
+    for (int64_t s = 0; s < S; ++s)
+        kmax = std::max({kmax, std::fabs(ks[(size_t)s].x), std::fabs(ks[(size_t)s].y), std::fabs(ks[(size_t)s].z)});
+    p->pairs_conj = S > 0;
+    {
         const double tol = 1e-12 * (kmax > 0.0 ? kmax : 1.0);
-        std::vector<int32_t> first((size_t)S / 2), second((size_t)S / 2);  // per group: g0/2 pairs
-        bool ok = g0 % 2 == 0;
-        double worst = 0.0;
-        std::vector<char> used((size_t)g0);
-        for (int64_t g = 0; g < p->n_tgroups && ok; ++g) {
-            const int32_t *mem = &perm[(size_t)(g * g0)];  // uniform groups: group g at g * g0
-            std::fill(used.begin(), used.end(), 0);
-            int64_t np = 0;
-            for (int64_t a = 0; a < g0 && ok; ++a) {
+        std::vector<char> used;
+        for (int64_t g = 0; g < p->n_tgroups && p->pairs_conj; ++g) {
+            const int64_t n = first[(size_t)g + 1] - first[(size_t)g];
+            const int32_t *mem = &perm[(size_t)first[(size_t)g]];
+            p->pairs_conj = n % 2 == 0 && n <= 128;
+            if (!p->pairs_conj) break;
+            if (mate.empty()) mate.assign((size_t)S, -1);
+            used.assign((size_t)n, 0);
+            auto apart = [&](int64_t i, int64_t j) {
+                const double4 u = ks[(size_t)mem[i]], v = ks[(size_t)mem[j]];
+                return std::fabs(u.x + v.x) + std::fabs(u.y + v.y) + std::fabs(u.z + v.z);
+            };
+            for (int64_t a = 0; a < n && p->pairs_conj; ++a) {
                 if (used[(size_t)a]) continue;
-                const double4 ka = ks[(size_t)mem[a]];
                 int64_t best = -1;
                 double bd = 0.0;
-                for (int64_t b = a + 1; b < g0; ++b) {
+                // the sample half the group on (interleaves in order) at once
+                // where it is exact, else the nearest of the rest
+                const int64_t h = a + n / 2;
+                const bool opposite = h < n && !used[(size_t)h] && apart(a, h) <= 4e-15 * kmax;
+                if (opposite) {
+                    best = h;
+                    bd = apart(a, h);
+                }
+                for (int64_t b = a + 1; b < n && !opposite; ++b) {
                     if (used[(size_t)b]) continue;
-                    const double4 kb = ks[(size_t)mem[b]];
-                    const double d = std::fabs(ka.x + kb.x) + std::fabs(ka.y + kb.y) + std::fabs(ka.z + kb.z);
+                    const double d = apart(a, b);
                     if (d <= tol && (best < 0 || d < bd)) {
                         best = b;
                         bd = d;
                     }
                 }
                 if (best < 0) {
-                    ok = false;
+                    p->pairs_conj = false;
                     break;
                 }
                 used[(size_t)a] = used[(size_t)best] = 1;
-                first[(size_t)(g * g0 / 2 + np)] = mem[a];
-                second[(size_t)(g * g0 / 2 + np)] = mem[best];
+                mate[(size_t)(first[(size_t)g] + a)] = mem[best];
                 worst = std::max(worst, bd);
-                ++np;
             }
         }
-        if (ok) {
-            const int64_t half = g0 / 2, gpc = kDirectThreads / half;
-            std::vector<int32_t> &pc = h.perm_conj;
-            pc.clear();
-            for (int64_t g = 0; g < p->n_tgroups; g += gpc) {
-                const int64_t ng = std::min<int64_t>(gpc, p->n_tgroups - g);
-                const int32_t o0 = (int32_t)pc.size();
-                for (int64_t q = g * half; q < (g + ng) * half; ++q) pc.push_back(first[(size_t)q]);
-                const int32_t o1 = (int32_t)pc.size();
-                for (int64_t q = g * half; q < (g + ng) * half; ++q) pc.push_back(second[(size_t)q]);
-                h.tiles_q.push_back({(int32_t)g, o0, (int32_t)(ng * half), 0});
-                h.tiles_q.push_back({(int32_t)g, o1, (int32_t)(ng * half), 0});
+    }
+    p->pairs_exact = p->pairs_conj && worst <= 4e-15 * kmax;
+    // lanes and tiles
+    {
+        int32_t lane0 = 0, group0 = 0;
+        h.pairs.reserve((size_t)((S + p->n_tgroups) / 2));
+        h.lane_group.reserve((size_t)((S + p->n_tgroups) / 2));
+        auto close = [&](int64_t g_end) {  // the tile of groups [group0, g_end)
+            const int32_t n = (int32_t)h.pairs.size() - lane0;
+            if (n == 0) return;
+            h.tiles_p.push_back(make_int4(lane0, n, group0, (int32_t)g_end - group0));
+            p->groups_per_tile = std::max(p->groups_per_tile, (int)(g_end - group0));
+            lane0 = (int32_t)h.pairs.size();
+        };
+        for (int64_t g = 0; g < p->n_tgroups; ++g) {
+            const int64_t n = first[(size_t)g + 1] - first[(size_t)g], o = first[(size_t)g], half = (n + 1) / 2;
+            if (g - group0 >= kGroupCap) {
+                close(g);
+                group0 = (int32_t)g;
             }
-            p->conj_pack = (int)gpc;
-            p->n_tiles_conj = (int64_t)h.tiles_q.size() / kDirectSPL;
-            p->conj_dk = worst;
+            int64_t l = 0;  // lanes of the group so far
+            for (int64_t a = 0; l < half; ++a) {
+                int32_t s0 = perm[(size_t)(o + a)], s1 = a + half < n ? perm[(size_t)(o + a + half)] : -1;
+                if (p->pairs_conj) {
+                    s1 = mate[(size_t)(o + a)];
+                    if (s1 < 0) continue;  // the second of a pair
+                }
+                if ((int32_t)h.pairs.size() - lane0 == kDirectThreads) {
+                    close(l > 0 ? g + 1 : g);
+                    group0 = (int32_t)g;
+                }
+                h.pairs.push_back(make_int2(s0, s1));
+                h.lane_group.push_back((uint8_t)(g - group0));
+                ++l;
+            }
         }
+        close(p->n_tgroups);
+        p->n_tiles_pairs = (int64_t)h.tiles_p.size();
+    }
+    // reported facts: slots of up to 256 samples of one group, two to a tile;
+    // groups of one size of 32, 64 or 128 samples and how many fill 256 lanes,
+    // singly and as conjugate pairs
+    {
+        int64_t slots = 0;
+        const int64_t g0 = p->n_tgroups > 0 ? first[1] : 0;
+        bool uniform = g0 == 32 || g0 == 64 || g0 == 128;
+        for (int64_t g = 0; g < p->n_tgroups; ++g) {
+            const int64_t n = first[(size_t)g + 1] - first[(size_t)g];
+            slots += cdiv(n, kDirectThreads);
+            uniform = uniform && n == g0;
+        }
+        p->n_tiles_grouped = cdiv(slots, 2);
+        p->group_pack = uniform ? (int)(kDirectThreads / g0) : 1;
+        p->conj_pack = uniform && p->pairs_conj ? (int)(2 * kDirectThreads / g0) : 1;
     }
 
     // Readout runs: kRunLen consecutive readout samples of a line (stride
@@ -1175,9 +893,8 @@ static int plan_analyse(fm_signal_plan *p, const double *kx, const double *ky, c
     std::vector<RunDesc> &runs = h.runs;
     if (n_meas >= 2 && S > 0) {
         const int64_t stride = n_lines * n_kz;
-        double kmax = 0.0, tmax = 0.0;
+        double tmax = 0.0;
         for (int64_t s = 0; s < S; ++s) {
-            kmax = std::max({kmax, std::fabs(ks[(size_t)s].x), std::fabs(ks[(size_t)s].y), std::fabs(ks[(size_t)s].z)});
             tmax = std::max(tmax, std::fabs(ks[(size_t)s].w));
         }
         const double tolk = 1e-12 * (kmax > 0.0 ? kmax : 1.0), tolt = 1e-12 * (tmax > 0.0 ? tmax : 1.0);
@@ -1325,8 +1042,6 @@ extern "C" int fm_signal_plan_create(fm_signal_plan **plan, int64_t n_meas, int6
             return rc;
         }
     }
-    const std::vector<int32_t> &perm = h.perm;
-    const std::vector<SignalTile> &tiles_g = h.tiles_g, &tiles_c = h.tiles_c;
     const std::vector<double4> &ks = h.ks;
     const std::vector<RunDesc> &runs = h.runs;
 
@@ -1338,24 +1053,16 @@ extern "C" int fm_signal_plan_create(fm_signal_plan **plan, int64_t n_meas, int6
     hipError_t e;
     if (S > 0) {
         if ((e = hipMalloc(&p->d_ks, sizeof(double4) * (size_t)S)) != hipSuccess) return fail(e, "hipMalloc");
-        if ((e = hipMalloc(&p->d_perm, sizeof(int32_t) * (size_t)S)) != hipSuccess) return fail(e, "hipMalloc");
-        if ((e = hipMalloc(&p->d_tiles_grouped, sizeof(SignalTile) * tiles_g.size())) != hipSuccess) return fail(e, "hipMalloc");
-        if ((e = hipMalloc(&p->d_tiles_consec, sizeof(SignalTile) * tiles_c.size())) != hipSuccess) return fail(e, "hipMalloc");
+        if ((e = hipMalloc(&p->d_pairs, sizeof(int2) * h.pairs.size())) != hipSuccess) return fail(e, "hipMalloc");
+        if ((e = hipMalloc(&p->d_lane_group, h.lane_group.size())) != hipSuccess) return fail(e, "hipMalloc");
+        if ((e = hipMalloc(&p->d_tiles_pairs, sizeof(int4) * h.tiles_p.size())) != hipSuccess) return fail(e, "hipMalloc");
+        if ((e = hipMalloc(&p->d_tiles_consec, sizeof(SignalTile) * h.tiles_c.size())) != hipSuccess) return fail(e, "hipMalloc");
         if ((e = hipMalloc(&p->d_tg_t, sizeof(double) * (size_t)p->n_tgroups)) != hipSuccess) return fail(e, "hipMalloc");
         if ((e = hipMemcpy(p->d_ks, ks.data(), sizeof(double4) * (size_t)S, hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-        if ((e = hipMemcpy(p->d_perm, perm.data(), sizeof(int32_t) * (size_t)S, hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-        if ((e = hipMemcpy(p->d_tiles_grouped, tiles_g.data(), sizeof(SignalTile) * tiles_g.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-        if ((e = hipMemcpy(p->d_tiles_consec, tiles_c.data(), sizeof(SignalTile) * tiles_c.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-        if (!h.tiles_p.empty()) {
-            if ((e = hipMalloc(&p->d_tiles_packed, sizeof(SignalTile) * h.tiles_p.size())) != hipSuccess) return fail(e, "hipMalloc");
-            if ((e = hipMemcpy(p->d_tiles_packed, h.tiles_p.data(), sizeof(SignalTile) * h.tiles_p.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-        }
-        if (!h.tiles_q.empty()) {
-            if ((e = hipMalloc(&p->d_tiles_conj, sizeof(SignalTile) * h.tiles_q.size())) != hipSuccess) return fail(e, "hipMalloc");
-            if ((e = hipMemcpy(p->d_tiles_conj, h.tiles_q.data(), sizeof(SignalTile) * h.tiles_q.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-            if ((e = hipMalloc(&p->d_perm_conj, sizeof(int32_t) * h.perm_conj.size())) != hipSuccess) return fail(e, "hipMalloc");
-            if ((e = hipMemcpy(p->d_perm_conj, h.perm_conj.data(), sizeof(int32_t) * h.perm_conj.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
-        }
+        if ((e = hipMemcpy(p->d_pairs, h.pairs.data(), sizeof(int2) * h.pairs.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
+        if ((e = hipMemcpy(p->d_lane_group, h.lane_group.data(), h.lane_group.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
+        if ((e = hipMemcpy(p->d_tiles_pairs, h.tiles_p.data(), sizeof(int4) * h.tiles_p.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
+        if ((e = hipMemcpy(p->d_tiles_consec, h.tiles_c.data(), sizeof(SignalTile) * h.tiles_c.size(), hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
         if ((e = hipMemcpy(p->d_tg_t, p->tg_t.data(), sizeof(double) * (size_t)p->n_tgroups, hipMemcpyHostToDevice)) != hipSuccess) return fail(e, "hipMemcpy");
         if (p->n_runs > 0) {
             if ((e = hipMalloc(&p->d_runs, sizeof(RunDesc) * runs.size())) != hipSuccess) return fail(e, "hipMalloc");
@@ -1464,16 +1171,14 @@ extern "C" int fm_signal_plan_destroy(fm_signal_plan *p)
     for (hipEvent_t e : p->ev_start) (void)hipEventDestroy(e);
     for (hipEvent_t e : p->ev_stop) (void)hipEventDestroy(e);
     (void)hipFree(p->d_ks);
-    (void)hipFree(p->d_perm);
-    (void)hipFree(p->d_tiles_grouped);
+    (void)hipFree(p->d_pairs);
+    (void)hipFree(p->d_lane_group);
+    (void)hipFree(p->d_tiles_pairs);
     (void)hipFree(p->d_runs);
     (void)hipFree(p->d_lines);
     (void)hipFree(p->d_run_steps);
     (void)hipFree(p->d_run_nsteps);
     (void)hipFree(p->d_tiles_consec);
-    (void)hipFree(p->d_tiles_packed);
-    (void)hipFree(p->d_tiles_conj);
-    (void)hipFree(p->d_perm_conj);
     (void)hipFree(p->d_tg_t);
     cartesian_free(p);
     delete p;

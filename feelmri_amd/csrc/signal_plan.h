@@ -17,6 +17,13 @@ constexpr int kMaxModes = 32;
 // Encodings per launch of the moving-node Cartesian GEMM (node records in LDS).
 constexpr int kMovMaxV = 4;
 
+// t-groups of one tile, at most.
+constexpr int kGroupCap = 32;
+// Static nodes take the t-grouped tiles from this many samples per group on
+// average (32 groups then fill a tile's 256 lanes), else per-sample t (spiral,
+// 61 394 nodes, 568 x 16, FP64: 0.71 ms grouped, 1.80 ms per-sample t).
+constexpr double kGroupMin = 16.0;
+
 // Readout runs (mixed-form direct kernel for static nodes): kRunLen
 // consecutive readout samples of one line whose k and t are linear in the
 // readout index, so exp(-2 pi i k.x) exp((i phi - 1/T2) t) advances by one
@@ -40,10 +47,8 @@ constexpr int kLineMinLen = 128;
 constexpr int64_t kLineMaxNodes = int64_t(1) << 28;
 
 struct SignalTile {
-    int32_t group;   // t-group index (shared-t kernels) or -1
-    int32_t offset;  // first entry in perm
+    int32_t offset;  // first sample
     int32_t count;   // samples in the tile
-    int32_t pad;
 };
 
 // One axis of a Cartesian stack (its lines or its kz planes) as real rows.
@@ -91,35 +96,28 @@ struct fm_signal_plan {
     int device = 0;
     int64_t n_meas = 0, n_lines = 0, n_kz = 0, n_samples = 0;
     int method = FM_METHOD_DIRECT;
-    bool prefer_grouped = true;   // static nodes: use the t-grouped tiles
+    bool prefer_grouped = true;   // static nodes: take the t-grouped tiles
     int64_t n_tgroups = 0;
     std::vector<double> tg_t;     // distinct t, first-appearance order
     std::vector<int32_t> sample_group;
-    // Two tilings of the samples: t-grouped tiles (each tile one distinct t;
-    // always used for moving nodes) and consecutive tiles (any t per sample).
-    int64_t n_tiles_grouped = 0, n_tiles_consec = 0;
-    // packed slots of group_pack equal-size t-groups (1: none), static nodes
-    int group_pack = 1;
-    int64_t n_tiles_packed = 0;
-    // largest |k'(slot 1) - k'(slot 0)|_1 over the lanes of the packed tiles
-    // (cycles per unit length), and whether every sample has kz = 0
-    double packed_dk = 0.0;
-    int planar = 0;
-    // conjugate pairs (mixed form): within every packed t-group the samples
-    // pair up as k'_b = -k'_a (to 1e-12 of the largest |k'|); a conj tile
-    // holds one member of each pair in slot 0 and its partner in slot 1,
-    // lane for lane, conj_pack t-groups per tile (1: none)
-    int conj_pack = 1;
-    int64_t n_tiles_conj = 0;
-    double conj_dk = 0.0;  // largest |k'_a + k'_b|_1 over the pairs
-    int32_t *d_perm_conj = nullptr;
-    fm::SignalTile *d_tiles_conj = nullptr;
+    // Tilings of the samples: consecutive tiles (any t per sample) and tiles
+    // of lanes with two samples of one t-group each, in the order of the groups
+    // (signal_groups.hip; always used for moving nodes).
+    int64_t n_tiles_consec = 0, n_tiles_pairs = 0;
+    int groups_per_tile = 0;      // the most groups of one tile
+    // every lane's samples have k'_b = -k'_a: to 1e-12 of the largest |k'|
+    // (mixed form), to 4e-15 (FP64 form too)
+    bool pairs_conj = false, pairs_exact = false;
+    int planar = 0;               // every kz is 0
+    // reported by fm_signal_plan_analyse
+    int64_t n_tiles_grouped = 0;
+    int group_pack = 1, conj_pack = 1;
     // device tables
     double4 *d_ks = nullptr;      // per sample: kx', ky', kz' (cycles/m, pi_f-scaled), t
-    int32_t *d_perm = nullptr;    // samples ordered by t-group (grouped tiles index it)
-    fm::SignalTile *d_tiles_grouped = nullptr;
     fm::SignalTile *d_tiles_consec = nullptr;  // offsets are sample indices
-    fm::SignalTile *d_tiles_packed = nullptr;
+    int2 *d_pairs = nullptr;        // per lane: samples a, b (-1: none)
+    uint8_t *d_lane_group = nullptr;  // per lane: group within the tile
+    int4 *d_tiles_pairs = nullptr;  // first lane, lanes, first group, groups
     double *d_tg_t = nullptr;
     // readout runs (empty when some run is not linear in k and t)
     int64_t n_runs = 0, run_stride = 0;
@@ -172,6 +170,11 @@ bool lines_usable(const fm_signal_plan *p, int64_t n_nodes);
 size_t lines_workspace(const fm_signal_plan *p, int64_t n_nodes);
 int lines_execute(const fm_signal_plan *p, int64_t n_nodes, int n_enc, const double *packed, void *ws,
                   size_t ws_bytes, double *out, hipStream_t stream);
+// Samples grouped by t (signal_groups.hip).
+int groups_blocks_per_cu(const fm_signal_plan *p, bool mixed, bool motion, int n_enc, int n_modes);
+int groups_launch(const fm_signal_plan *p, bool mixed, bool motion, int64_t n_nodes, int n_enc, int v0, int vb,
+                  const double *packed, const float *modes, int n_modes, const double *motion_coef, int64_t n_splits,
+                  int64_t nodes_per_split, double2 *dst, int write_final, hipStream_t stream);
 // Moving nodes, per-readout GEMM in either form (n_enc <= kMovMaxV).
 size_t cartesian_moving_workspace(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc);
 int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc,

@@ -56,8 +56,8 @@ def _prec(precision) -> int:
 def analyse_trajectory(kloc, t, method: str = "auto") -> dict:
     """Host-only analysis of a trajectory (no device needed), as
     ``SignalPlan`` performs it: the method it would choose, the number of
-    distinct t, of readout runs and of t-grouped tiles, and the t-groups per
-    packed slot and per conjugate-pair tile (1: none)."""
+    distinct t, of readout runs and of t-grouped tiles, and the equal-size
+    t-groups that 256 lanes hold singly and as conjugate pairs (1: none)."""
     kx, ky, kz = (np.ascontiguousarray(np.asarray(k, dtype=np.float64)) for k in kloc)
     tt = np.ascontiguousarray(np.asarray(t, dtype=np.float64))
     if tt.ndim != 3 or any(k.shape != tt.shape for k in (kx, ky, kz)):

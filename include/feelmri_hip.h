@@ -80,11 +80,11 @@ int fm_signal_plan_destroy(fm_signal_plan *plan);
 /* Host-only analysis of a trajectory, as fm_signal_plan_create performs it,
  * without a device: the method it would choose, the number of distinct t,
  * of 16-sample readout runs and of t-grouped tiles, whether the runs are
- * linear to 1e-14 (runs_exact: the FP64 form takes them too), and how many
- * equal-size t-groups a packed slot holds (group_pack, 1 when the groups do
- * not pack), and how many a conjugate-pair tile holds (conj_pack, 1 when
- * some packed group's samples do not pair up as k and -k: the mixed form of
- * static nodes then takes the packed slots).  Out-pointers may be NULL.  No
+ * linear to 1e-14 (runs_exact: the FP64 form takes them too), and, where
+ * every t-group has the same size of 32, 64 or 128 samples, how many of them
+ * 256 lanes hold with one sample a lane (group_pack, else 1) and with a
+ * conjugate pair k, -k a lane (conj_pack, 1 when some group's samples do not
+ * pair up).  Out-pointers may be NULL.  No
  * counterpart in the reference (plan introspection; usable without a
  * GPU). */
 int fm_signal_plan_analyse(int64_t n_meas, int64_t n_lines, int64_t n_kz, const double *kx,
