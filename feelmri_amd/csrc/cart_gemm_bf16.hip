@@ -515,19 +515,25 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_cart_gemm_pairs_bf16(
     // that a copy in flight writes
     __shared__ uint4 sE0[kChunks * 64], sE1[kChunks * 64], sE2[kChunks * 64];
     __shared__ uint4 sY0[NP * kThreads], sY1[NP * kThreads], sY2[NP * kThreads];
-    int64_t split, rt, ct;
-    gemm_tile_ids(n_rt, n_ct, n_splits, split, rt, ct);
+    // tile ids as gemm_tile_ids gives them, in 32 bits (as the column indexes
+    // below): the 64-bit divisions took 2 us of a small call
+    const unsigned u_ct = (unsigned)n_ct, per_split = (unsigned)n_rt * u_ct, total = per_split * (unsigned)n_splits;
+    unsigned id = blockIdx.x;
+    if (total % kXcds == 0) id = (id % kXcds) * (total / kXcds) + id / kXcds;
+    const int64_t split = id / per_split;
+    const unsigned rem = id % per_split;
+    const int64_t rt = rem / u_ct, ct = rem % u_ct;
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int64_t nrb = Mp / 32;
     const int64_t k0 = split * steps_per_split;
     const int64_t k1 = (k0 + steps_per_split < ksteps) ? k0 + steps_per_split : ksteps;
 
-    const int64_t c0 = ct * kCols;
-    const int64_t clast = (c0 + kCols - 1 < NC) ? c0 + kCols - 1 : NC - 1;
-    const int64_t jf = c0 / n_kzV;
-    const int nJ = (int)(clast / n_kzV - jf) + 1;
-    const int nK = (int)(n_kzV < kCols ? n_kzV : kCols);
+    const unsigned kzV = (unsigned)n_kzV, c0 = (unsigned)ct * kCols;
+    const unsigned clast = (c0 + kCols - 1 < (unsigned)NC) ? c0 + kCols - 1 : (unsigned)NC - 1;
+    const unsigned jf = c0 / kzV;
+    const int nJ = (int)(clast / kzV - jf) + 1;
+    const int nK = (int)(kzV < kCols ? kzV : kCols);
     // kYZStride (nJ + nK) <= NP kThreads
 
     // staging: LDS slot s = tid + kThreads p holds piece s%9 of row s/9 (the
@@ -540,16 +546,16 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_cart_gemm_pairs_bf16(
         const int s = tid + kThreads * p;
         const int row = s / kYZStride;
         const int prt = (s % kYZStride) < 8 ? s % kYZStride : 7;
-        const float2 *base = Ex + jf * Np;
-        if (row < nJ + nK) base = row < nJ ? Ex + (jf + row) * Np : Ez + ((c0 + row - nJ) % n_kzV) * Np;
+        const float2 *base = Ex + (int64_t)jf * Np;
+        if (row < nJ + nK) base = row < nJ ? Ex + (int64_t)(jf + row) * Np : Ez + (int64_t)((c0 + row - nJ) % kzV) * Np;
         stg[p] = base + 2 * prt;
     }
 
     // this lane's output column (clamped for padding lanes; results discarded)
     const int64_t col = c0 + wave * 32 + (lane % 32);
-    const int64_t colc = col < NC ? col : NC - 1;
-    const int ys = (int)(colc / n_kzV - jf);
-    const int zs = nJ + (int)((colc - c0) % nK);
+    const unsigned colc = col < NC ? (unsigned)col : (unsigned)NC - 1;
+    const int ys = (int)(colc / kzV - jf);
+    const int zs = nJ + (int)((colc - c0) % (unsigned)nK);
     const int hb = lane / 32;
     const int yoff = ys * kYZStride + 4 * hb, zoff = zs * kYZStride + 4 * hb;
     const uint4 *const E_rt = E + rt * RB * 2 * 64;

@@ -281,7 +281,9 @@ void cartesian_free(fm_signal_plan *p)
 // Complex rows (pairs = false): rows are the readout indices, columns (line,
 // kz, encoding).  Real rows: the lines' cosine and sine rows, columns
 // (readout index, kz, encoding).
-static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, int V, bool pairs)
+// max_total: workspace that real rows may take (they fall back on fewer node
+// splits, and report total > max_total where even one does not fit).
+static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, int V, bool pairs, size_t max_total)
 {
     GemmShape s{};
     s.mixed = mixed;
@@ -296,12 +298,24 @@ static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, 
     const int64_t nrb = cdiv(s.M, rowblk);
     s.rb_per_wave = (int)std::min<int64_t>(max_rb, nrb);
     s.n_rt = cdiv(nrb, s.rb_per_wave);
-    if (!mixed && pairs) s.rb_per_wave = (int)cdiv(nrb, s.n_rt);  // tiles of equal height
+    if (pairs) s.rb_per_wave = (int)cdiv(nrb, s.n_rt);  // tiles of equal height
     s.Mp = s.n_rt * s.rb_per_wave * rowblk;
     s.NC = outer * c.n_kz * V;
     s.n_ct = cdiv(s.NC, 4 * colblk);
     s.NCp = s.n_ct * 4 * colblk;
     s.ksteps = s.Np / 16;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        size_t o = off;
+        off += (bytes + 255) & ~size_t(255);
+        return o;
+    };
+    const size_t real = s.mixed ? sizeof(float) : sizeof(double);
+    // E: Re (and Im) planes, in the mixed form each as bf16 hi, lo
+    s.off_E = take((size_t)s.Mp * s.Np * (pairs ? 1 : 2) * real);
+    s.off_Ey = take((size_t)outer * s.Np * 2 * real);
+    s.off_Ez = take((size_t)c.n_kz * V * s.Np * 2 * real);
+    const size_t per_split = (size_t)s.M * s.NC * 2 * real;
     const int64_t base = s.n_rt * s.n_ct;
     // mixed: one round of workgroups (one 8-wave or two 4-wave workgroups
     // per CU); FP64: two rounds (two 4-wave workgroups per CU, measured faster)
@@ -310,42 +324,36 @@ static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, 
     // mixed: FP32 accumulators sum at most 8192 steps (131 072 nodes) per
     // split before the FP64 split reduction, bounding the accumulation error
     // for large meshes
-    if (s.mixed) splits = std::max<int64_t>(splits, cdiv(s.ksteps, 8192));
-    splits = std::max<int64_t>(1, std::min<int64_t>(splits, cdiv(s.ksteps, 8)));
+    const int64_t s_acc = s.mixed ? cdiv(s.ksteps, 8192) : 1;
+    splits = std::max(splits, s_acc);
+    // small meshes: a split keeps at least 8 steps, with real rows 3 (half as
+    // long a step, and more workgroups hide more of the memory latency: 4 110
+    // nodes, 45 x 123, 3 encodings: GEMM 18.0 -> 15.3 us; 10 007 nodes, 64 x 64: 11.5
+    // -> 8.1 us)
+    splits = std::max<int64_t>(1, std::min<int64_t>(splits, cdiv(s.ksteps, pairs ? 3 : 8)));
+    if (pairs) {
+        const int64_t fit = off < max_total ? (int64_t)((max_total - off) / std::max<size_t>(per_split, 1)) : 0;
+        splits = std::max(s_acc, std::min(splits, std::max<int64_t>(fit, 1)));
+    }
     s.steps_per_split = cdiv(s.ksteps, splits);
     s.n_splits = cdiv(s.ksteps, s.steps_per_split);
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        size_t o = off;
-        off += (bytes + 255) & ~size_t(255);
-        return o;
-    };
-    const size_t planes = pairs ? 1 : 2;                                     // Re (and Im)
-    if (s.mixed) {
-        s.off_E = take((size_t)s.Mp * s.Np * planes * 2 * sizeof(uint16_t));  // each as bf16 hi, lo
-        s.off_Ey = take((size_t)outer * s.Np * sizeof(float2));
-        s.off_Ez = take((size_t)c.n_kz * V * s.Np * sizeof(float2));
-        s.off_part = take((size_t)s.n_splits * s.M * s.NC * sizeof(float2));
-    } else {
-        s.off_E = take((size_t)s.Mp * s.Np * planes * sizeof(double));
-        s.off_Ey = take((size_t)outer * s.Np * sizeof(double2));
-        s.off_Ez = take((size_t)c.n_kz * V * s.Np * sizeof(double2));
-        s.off_part = take((size_t)s.n_splits * s.M * s.NC * sizeof(double2));
-    }
+    s.off_part = take((size_t)s.n_splits * per_split);
     s.total = off;
     return s;
 }
 
 // Real rows where they take fewer MFMAs (half as many per row and column
-// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32; FP64 5.94 against
-// 11.69 ms at 150 001 nodes, 125 x 127 x 31) and no more workspace than complex rows do.
+// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32; FP64 5.94
+// against 11.69 ms at 150 001 nodes, 125 x 127 x 31) and no more workspace than
+// complex rows do.
 static GemmShape gemm_shape(const fm_signal_plan *p, int precision, int64_t N, int V)
 {
     const CartesianTables &c = p->cart;
     const bool mixed = precision != FM_PREC_F64;
-    const GemmShape g = gemm_shape_of(c, mixed, N, V, false);
-    const GemmShape s = gemm_shape_of(c, mixed, N, V, true);
-    return s.Mp * s.NCp < 2 * g.Mp * g.NCp && s.total <= g.total ? s : g;
+    const GemmShape g = gemm_shape_of(c, mixed, N, V, false, 0);
+    const GemmShape s = gemm_shape_of(c, mixed, N, V, true, g.total);
+    const bool fits = s.total <= g.total && s.NCp < (int64_t(1) << 31);  // column indexes in 32 bits
+    return fits && s.Mp * s.NCp < 2 * g.Mp * g.NCp ? s : g;
 }
 
 size_t cartesian_workspace(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc)
@@ -386,7 +394,7 @@ __device__ inline void cis_neg_cycles(double u, double &c, double &s)
 // node n = 16 kb + 4 st + l/16 and walks the row blocks (row 16 rb + l%16),
 // so a wave writes 512 contiguous bytes per plane.
 __device__ __forceinline__ void cart_E_f64(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
-                                           int64_t M, int64_t Mp, const double *__restrict__ F,
+                                           int64_t M, int64_t Mp, int64_t rb0, int64_t rb1, const double *__restrict__ F,
                                            const double *__restrict__ tr, double *__restrict__ E)
 {
     // t over (Np / 16) * 4 * 64
@@ -399,7 +407,7 @@ __device__ __forceinline__ void cart_E_f64(int64_t t, const double *__restrict__
     const bool ok = n < N;
     const double x = ok ? packed[n] : 0.0, y = ok ? packed[N + n] : 0.0, z = ok ? packed[2 * N + n] : 0.0;
     const double phi = ok ? packed[3 * N + n] : 0.0, r2 = ok ? packed[4 * N + n] : 0.0;
-    for (int64_t rb = 0; rb < nrb; ++rb) {
+    for (int64_t rb = rb0; rb < rb1; ++rb) {
         const int64_t i = rb * 16 + (lane % 16);
         double er = 0.0, ei = 0.0;
         if (ok && i < M) {
@@ -425,7 +433,7 @@ __device__ __forceinline__ void cart_E_f64(int64_t t, const double *__restrict__
 // 1 KB contiguous per plane).  Phase in FP64 with range reduction, then the
 // hardware FP32 sine/cosine and exp2.
 __device__ __forceinline__ void cart_E_bf16(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
-                                            int64_t M, int64_t Mp, const double *__restrict__ F,
+                                            int64_t M, int64_t Mp, int64_t rb0, int64_t rb1, const double *__restrict__ F,
                                             const double *__restrict__ tr, uint4 *__restrict__ E)
 {
     // t over (Np / 16) * 64
@@ -446,7 +454,7 @@ __device__ __forceinline__ void cart_E_bf16(int64_t t, const double *__restrict_
         r2[q] = ok ? packed[4 * N + n] : 0.0;
     }
     const int nvalid = (int)(N - n0 < 8 ? (N - n0 > 0 ? N - n0 : 0) : 8);
-    for (int64_t rb = 0; rb < nrb; ++rb) {
+    for (int64_t rb = rb0; rb < rb1; ++rb) {
         const int64_t i = rb * 32 + (lane % 32);
         const bool row_ok = i < M;
         const double fx = row_ok ? F[3 * i] : 0.0, fy = row_ok ? F[3 * i + 1] : 0.0,
@@ -487,7 +495,7 @@ __device__ __forceinline__ void cart_E_bf16(int64_t t, const double *__restrict_
 // lane order of cart_E_bf16; row r holds sin 2 pi (D_r . x + quarter turn of a
 // cosine row).
 __device__ __forceinline__ void cart_rows_bf16(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
-                                               int64_t M, int64_t Mp, const double4 *__restrict__ rows,
+                                               int64_t M, int64_t Mp, int64_t rb0, int64_t rb1, const double4 *__restrict__ rows,
                                                uint4 *__restrict__ E)
 {
     // t over (Np / 16) * 64
@@ -506,7 +514,7 @@ __device__ __forceinline__ void cart_rows_bf16(int64_t t, const double *__restri
         z[q] = ok ? packed[2 * N + n] : 0.0;
     }
     const int nvalid = (int)(N - n0 < 8 ? (N - n0 > 0 ? N - n0 : 0) : 8);
-    for (int64_t rb = 0; rb < nrb; ++rb) {
+    for (int64_t rb = rb0; rb < rb1; ++rb) {
         const int64_t i = rb * 32 + (lane % 32);
         const bool row_ok = i < M;
         const double4 d = rows[row_ok ? i : 0];
@@ -537,7 +545,7 @@ __device__ __forceinline__ void cart_rows_bf16(int64_t t, const double *__restri
 // Real rows, FP64: tiles of (16 rows x 16 nodes), one plane in the lane order
 // of cart_E_f64.
 __device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
-                                              int64_t M, int64_t Mp, const double4 *__restrict__ rows,
+                                              int64_t M, int64_t Mp, int64_t rb0, int64_t rb1, const double4 *__restrict__ rows,
                                               double *__restrict__ E)
 {
     // t over (Np / 16) * 4 * 64
@@ -549,7 +557,7 @@ __device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restric
     const int64_t n = kb * 16 + 4 * st + lane / 16;
     const bool ok = n < N;
     const double x = ok ? packed[n] : 0.0, y = ok ? packed[N + n] : 0.0, z = ok ? packed[2 * N + n] : 0.0;
-    for (int64_t rb = 0; rb < nrb; ++rb) {
+    for (int64_t rb = rb0; rb < rb1; ++rb) {
         const int64_t i = rb * 16 + (lane % 16);
         double e = 0.0;
         if (ok && i < M) {
@@ -564,19 +572,17 @@ __device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restric
 // lines; real rows: Ex, exp(-t_i/T2) exp(i phi t_i) exp(-2 pi i F_i . x) of the
 // readout indices -- and Ezb rows exp(-2 pi i (H_k . x_n)) b_v[n] (the
 // encoding's weighted magnetisation folded into the kz factor).  One thread
-// per node keeps its position in registers and walks a block of
-// kYZRowsPerBlock rows (outer rows first, then Ezb).
-constexpr int kYZRowsPerBlock = 16;
-
+// per node keeps its position in registers and walks a block of rows_blk rows
+// (outer rows first, then Ezb).
 template <bool MIXED, bool PAIRS>
-__device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, const double *__restrict__ packed, int64_t N,
+__device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, int rows_blk, const double *__restrict__ packed, int64_t N,
                                         int64_t Np, int V, int64_t n_out, int64_t n_kz,
                                         const double *__restrict__ G, const double *__restrict__ tr,
                                         const double *__restrict__ H, void *__restrict__ Ey, void *__restrict__ Ez)
 {
     if (n >= Np) return;
-    const int64_t r0 = rblk * kYZRowsPerBlock;
-    const int64_t r1 = (r0 + kYZRowsPerBlock < n_out + n_kz) ? r0 + kYZRowsPerBlock : n_out + n_kz;
+    const int64_t r0 = rblk * rows_blk;
+    const int64_t r1 = (r0 + rows_blk < n_out + n_kz) ? r0 + rows_blk : n_out + n_kz;
     const bool ok = n < N;
     const double x = ok ? packed[n] : 0.0, y = ok ? packed[N + n] : 0.0, z = ok ? packed[2 * N + n] : 0.0;
     double phi = 0.0, r2 = 0.0;
@@ -633,23 +639,28 @@ __global__ __launch_bounds__(256) void k_cart_tables(const double *__restrict__ 
                                                      const double *__restrict__ tr, void *__restrict__ E,
                                                      int64_t nb_E, int V, int64_t n_out, int64_t n_kz,
                                                      const double *__restrict__ G, const double *__restrict__ H,
-                                                     void *__restrict__ Ey, void *__restrict__ Ez, int64_t nb_n)
+                                                     void *__restrict__ Ey, void *__restrict__ Ez, int64_t nb_n,
+                                                     int e_parts, int rows_blk)
 {
-    const int64_t b = blockIdx.x;
-    if (b < nb_E) {
-        const int64_t t = b * 256 + threadIdx.x;
+    // the grid is below 2^31 blocks: 32-bit divisions
+    const unsigned b = blockIdx.x, nE = (unsigned)nb_E;
+    if (b < nE * (unsigned)e_parts) {
+        const int64_t t = (int64_t)(b % nE) * 256 + threadIdx.x;
+        // this block's share of the row blocks
+        const int64_t nrb = Mp / (MIXED ? 32 : 16), ep = b / nE;
+        const int64_t rb0 = (unsigned)(nrb * ep) / (unsigned)e_parts, rb1 = (unsigned)(nrb * (ep + 1)) / (unsigned)e_parts;
         if (MIXED && PAIRS)
-            cart_rows_bf16(t, packed, N, Np, M, Mp, lrows, reinterpret_cast<uint4 *>(E));
+            cart_rows_bf16(t, packed, N, Np, M, Mp, rb0, rb1, lrows, reinterpret_cast<uint4 *>(E));
         else if (MIXED)
-            cart_E_bf16(t, packed, N, Np, M, Mp, F, tr, reinterpret_cast<uint4 *>(E));
+            cart_E_bf16(t, packed, N, Np, M, Mp, rb0, rb1, F, tr, reinterpret_cast<uint4 *>(E));
         else if (PAIRS)
-            cart_rows_f64(t, packed, N, Np, M, Mp, lrows, reinterpret_cast<double *>(E));
+            cart_rows_f64(t, packed, N, Np, M, Mp, rb0, rb1, lrows, reinterpret_cast<double *>(E));
         else
-            cart_E_f64(t, packed, N, Np, M, Mp, F, tr, reinterpret_cast<double *>(E));
+            cart_E_f64(t, packed, N, Np, M, Mp, rb0, rb1, F, tr, reinterpret_cast<double *>(E));
         return;
     }
-    const int64_t c = b - nb_E;
-    cart_yz<MIXED, PAIRS>((c % nb_n) * 256 + threadIdx.x, c / nb_n, packed, N, Np, V, n_out, n_kz, PAIRS ? F : G, tr,
+    const unsigned c = b - nE * (unsigned)e_parts, nn = (unsigned)nb_n;
+    cart_yz<MIXED, PAIRS>((int64_t)(c % nn) * 256 + threadIdx.x, c / nn, rows_blk, packed, N, Np, V, n_out, n_kz, PAIRS ? F : G, tr,
                           H, Ey, Ez);
 }
 
@@ -675,64 +686,106 @@ __global__ void k_cart_reduce(const P *__restrict__ part, int64_t n_splits, int6
 // encoding) in FP64, each thread a contiguous share of them, the shares added
 // in order, and writes the entity's up to four samples:
 //   (C_a -+ i S_a) (C_b -+ i S_b) = CC - s_a s_b SS - i (s_b CS + s_a SC).
-template <typename P, int G, bool KPAIR>
+template <typename P, int OL, bool KPAIR>
 __global__ __launch_bounds__(256) void k_cart_reduce_pairs(
     const P *__restrict__ part, int64_t n_splits, int64_t M, int64_t per_split, int64_t si, int64_t sr, int64_t V,
     const int4 *__restrict__ lent, int64_t n_lent, const int4 *__restrict__ kent, int64_t n_kent, int64_t L, int64_t K,
     double2 *__restrict__ out)
 {
-    constexpr int kOut = 256 / G;
-    __shared__ double2 sum[4][G][kOut];
-    const int o = threadIdx.x % kOut, g = threadIdx.x / kOut;
-    const int64_t t = (int64_t)blockIdx.x * kOut + o;
-    const bool live = t < M * n_lent * n_kent * V;
-    const int64_t tc = live ? t : 0;
-    const int64_t v = tc % V, e = (tc / V) % n_kent, f = (tc / (V * n_kent)) % n_lent, i = tc / (V * n_kent * n_lent);
+    constexpr int GL = 64 / OL, G = 4 * GL;  // shares in a wave, in the workgroup
+    constexpr int NC = KPAIR ? 4 : 2;        // sums per group: (line cosine, sine) x (kz cosine, sine)
+    __shared__ double2 sum[4][NC][OL];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int o = lane % OL, g = wave * GL + lane / OL;
+    const int64_t t = (int64_t)blockIdx.x * OL + o;
+    const int64_t n_out = M * n_lent * n_kent * V;
+    const bool live = t < n_out;
+    // the index that is contiguous in `part` runs first (7 434 nodes, 121 x 140,
+    // 4 encodings: 22.5 -> 14.4 us): after (kz, encoding)
+    // the line rows of a readout index (KPAIR), or the readout indices of a row
+    const int64_t na = KPAIR ? n_lent : M;
+    int64_t v, e, a, b;
+    if (n_out < (int64_t(1) << 31)) {  // 32-bit division: a fifth of the instructions
+        unsigned r = live ? (unsigned)t : 0u;
+        v = r % (unsigned)V;
+        r /= (unsigned)V;
+        e = r % (unsigned)n_kent;
+        r /= (unsigned)n_kent;
+        a = r % (unsigned)na;
+        b = r / (unsigned)na;
+    } else {
+        const int64_t r = live ? t : 0;
+        v = r % V;
+        e = (r / V) % n_kent;
+        a = (r / (V * n_kent)) % na;
+        b = r / (V * n_kent * na);
+    }
+    const int64_t f = KPAIR ? a : b, i = KPAIR ? b : a;
     const int4 le = lent[f];
     const int4 ke = KPAIR ? kent[e] : make_int4((int)e, -1, (int)e, -1);
     const int rows[2] = {le.z, le.w}, cols[2] = {ke.z, ke.w};
     const int64_t s0 = n_splits * g / G, s1 = n_splits * (g + 1) / G;
+    // the sums advance together, so their loads overlap
+    double re[NC], im[NC];
+    const P *src[NC];
+    bool on[NC];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int r = rows[c / 2], q = cols[c % 2];
-        double re = 0.0, im = 0.0;
-        if (live && r >= 0 && q >= 0) {
-            const P *src = part + i * si + r * sr + q * V + v;
+    for (int c = 0; c < NC; ++c) {
+        const int r = rows[KPAIR ? c / 2 : c], q = cols[KPAIR ? c % 2 : 0];
+        re[c] = im[c] = 0.0;
+        on[c] = live && r >= 0 && q >= 0;
+        src[c] = part + (on[c] ? i * si + r * sr + q * V + v : 0) + s0 * per_split;
+    }
 #pragma unroll 4
-            for (int64_t s = s0; s < s1; ++s) {
-                const P x = src[s * per_split];
-                re += (double)x.x;
-                im += (double)x.y;
+    for (int64_t s = s0; s < s1; ++s) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (on[c]) {
+                const P x = *src[c];
+                re[c] += (double)x.x;
+                im[c] += (double)x.y;
+                src[c] += per_split;
             }
         }
-        sum[c][g][o] = make_double2(re, im);
+    }
+    // shares of a wave, then of the four waves, each in a fixed order
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+#pragma unroll
+        for (int d = OL; d < 64; d *= 2) {
+            re[c] += __shfl_xor(re[c], d, 64);
+            im[c] += __shfl_xor(im[c], d, 64);
+        }
+        if (lane < OL) sum[wave][c][o] = make_double2(re[c], im[c]);
     }
     __syncthreads();
-    if (g != 0 || !live) return;
+    // one thread per sample of the group
+    const int c = threadIdx.x / OL;
+    if (c >= 4 || !live) return;
+    const int j = c / 2 ? le.y : le.x, k = c % 2 ? ke.y : ke.x;
+    if (j < 0 || k < 0) return;
     double2 w[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        w[c] = sum[c][0][o];
+    for (int q = 0; q < 4; ++q) {
+        w[q] = make_double2(0.0, 0.0);
+        if (!KPAIR && q % 2) continue;
 #pragma unroll
-        for (int q = 1; q < G; ++q) {
-            w[c].x += sum[c][q][o].x;
-            w[c].y += sum[c][q][o].y;
+        for (int x = 0; x < 4; ++x) {
+            const double2 y = sum[x][KPAIR ? q : q / 2][o];
+            w[q].x += y.x;
+            w[q].y += y.y;
         }
     }
     // w: CC, CS (kz sine), SC (line sine), SS
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int j = c / 2 ? le.y : le.x, k = c % 2 ? ke.y : ke.x;
-        if (j < 0 || k < 0) continue;
-        const double sa = c / 2 ? -1.0 : 1.0, sb = c % 2 ? -1.0 : 1.0;
-        const double ar = w[0].x - sa * sb * w[3].x, ai = w[0].y - sa * sb * w[3].y;
-        const double br = sb * w[1].x + sa * w[2].x, bi = sb * w[1].y + sa * w[2].y;
-        out[((i * L + j) * K + k) * V + v] = make_double2(ar + bi, ai - br);
-    }
+    const double sa = c / 2 ? -1.0 : 1.0, sb = c % 2 ? -1.0 : 1.0;
+    const double ar = w[0].x - sa * sb * w[3].x, ai = w[0].y - sa * sb * w[3].y;
+    const double br = sb * w[1].x + sa * w[2].x, bi = sb * w[1].y + sa * w[2].y;
+    out[((i * L + j) * K + k) * V + v] = make_double2(ar + bi, ai - br);
 }
 
-// Threads per sample group: 16 where the samples alone would leave most of
-// the device idle in a long chain of loads, else 4.
+// 16 groups of samples to a workgroup (16 shares of the splits) where the
+// samples alone would leave most of the device idle in a long chain of loads,
+// else 64 (4 shares).
 template <typename P, bool KPAIR>
 static void launch_reduce_pairs(const P *part, int64_t n_splits, int64_t si, int64_t sr, int64_t V,
                                 const CartesianTables &c, double2 *out, hipStream_t st)
@@ -743,10 +796,12 @@ static void launch_reduce_pairs(const P *part, int64_t n_splits, int64_t si, int
     const int64_t n = M * c.lines.n_ent * n_kent * V;
     if (n < 64 * 1024)
         k_cart_reduce_pairs<P, 16, KPAIR><<<(unsigned)cdiv(n, 16), 256, 0, st>>>(
-            part, n_splits, M, per_split, si, sr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
+            part, n_splits, M, per_split, si, sr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz,
+            out);
     else
-        k_cart_reduce_pairs<P, 4, KPAIR><<<(unsigned)cdiv(n, 64), 256, 0, st>>>(
-            part, n_splits, M, per_split, si, sr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz, out);
+        k_cart_reduce_pairs<P, 64, KPAIR><<<(unsigned)cdiv(n, 64), 256, 0, st>>>(
+            part, n_splits, M, per_split, si, sr, V, c.lines.d_ent, c.lines.n_ent, c.kzs.d_ent, n_kent, c.n_ln, c.n_kz,
+            out);
 }
 
 int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, const double *packed, void *wsv,
@@ -769,7 +824,13 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
         const int64_t nb_E = s.mixed ? cdiv(s.Np / 16 * 64, 256) : cdiv(s.Np / 16 * 256, 256);
         const int64_t nb_n = cdiv(s.Np, 256);
         const int64_t n_out = s.pairs ? c.n_ro : c.n_ln;
-        const int64_t nb = nb_E + nb_n * cdiv(n_out + c.n_kz, kYZRowsPerBlock);
+        // small meshes: the row blocks and rows shared among more blocks, until
+        // there are some 4 per CU (4 110 nodes, 45 x 123: 9.9 -> 6.0 us)
+        const int64_t nrb = s.Mp / (s.mixed ? 32 : 16), want = 4 * (int64_t)device_cu_count();
+        const int e_parts = (int)std::max<int64_t>(1, std::min(nrb, want / std::max<int64_t>(2 * nb_E, 1)));
+        int rows_blk = 16;
+        while (rows_blk > 2 && nb_n * cdiv(n_out + c.n_kz, rows_blk) < want) rows_blk /= 2;
+        const int64_t nb = nb_E * e_parts + nb_n * cdiv(n_out + c.n_kz, rows_blk);
         if (nb > (int64_t)0x7fffffff) {
             set_error("Cartesian operand tables exceed the launch grid (%lld blocks)", (long long)nb);
             return FM_ERR_UNSUPPORTED;
@@ -777,7 +838,8 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
 #define FM_TABLES(MX, PR)                                                                                            \
     k_cart_tables<MX, PR><<<(unsigned)nb, 256, 0, st>>>(packed, N, s.Np, s.M, s.Mp, PR ? c.d_F_lines : c.d_F,       \
                                                         c.lines.d_rows, c.d_t, ws + s.off_E, nb_E, V, n_out, c.n_kz, \
-                                                        c.d_G, c.d_H, ws + s.off_Ey, ws + s.off_Ez, nb_n)
+                                                        c.d_G, c.d_H, ws + s.off_Ey, ws + s.off_Ez, nb_n, e_parts, \
+                                                        rows_blk)
         if (s.mixed && s.pairs) FM_TABLES(true, true);
         else if (s.mixed) FM_TABLES(true, false);
         else if (s.pairs) FM_TABLES(false, true);
