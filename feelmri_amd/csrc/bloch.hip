@@ -5,7 +5,7 @@
 //
 // One lane per node; node attributes come from an SoA table (coalesced).
 // The event table is walked in chunks of 256 events: each lane of the
-// workgroup stages one event (rf, |rf|^2, -gamma dt / 2, G, dt and, for
+// workgroup stages one event (rf, |rf|^2, G, dt, flags and, for
 // moving nodes, the POD weights of that step) into LDS, then every lane
 // integrates its node through the chunk reading the events by broadcast.
 // Step i -> i+1 uses event i+1; e1/e2 are refreshed only when dt changes;
@@ -16,6 +16,28 @@
 // so Mxy turns by -gamma dt Bz and the rotation leaves Mz alone.  This skips
 // |B|, its reciprocal and the Cayley-Klein products; the result departs from
 // the general step by rounding only (|alpha|^2 is 1 to an ulp).
+//
+// What an event needs is found once, by the thread that stages it, and stored
+// as flags that every lane branches on together:
+//   * the gradient axes that are on: a position along an axis (and the modes of
+//     moving nodes) enters only where its gradient is not 0, since the other
+//     products are 0 (all three axes where a coefficient or a position is not
+//     finite, whose products are not);
+//   * whether RF and field repeat the previous step's (hard pulses, gradient
+//     plateaus and delays; moving nodes: no gradient): the lane then keeps the
+//     rotation it formed.  FP32 form: where dt is the same, to the last bit the
+//     same results.  FP64 form: dt = diff(times) varies by roundings (~1e-15
+//     ms) within such a run; to 1e-12 ms the kept sine and cosine and the decay
+//     factors are corrected to first order (the second order is below 1e-16).
+// A run's steps are an inner loop that applies the rotation and relaxes: the
+// rotation is local to it (kept across the outer loop it was copied on every
+// path).  FP64 rotations are formed as a 3 x 3 matrix and applied in 9
+// instructions; formed and applied as (alpha, beta) products they took 45 a
+// step.  The mode loop is unrolled for 1, 2, 5, 10 or 16 modes (zero padded; it
+// was one loop of 16 with a test each), and the next event's record is read
+// from LDS in wide reads while the current one relaxes.  Bound by VALU issue.
+// 1 948 800 moving nodes, 1 mode, 11 255 events, FP32: 22.5 ms (before: 52.6);
+// 512 000 nodes, 33 blocks, 419 steps in all, FP64: 0.367 ms (0.929).
 #include <algorithm>
 #include <type_traits>
 
@@ -44,21 +66,16 @@ struct NoChain {};
 
 template <typename T>
 struct alignas(16) Event {
-    T rf_re, rf_im, rf2, kappa;
-    T gx, gy, gz, dt;
+    T rf_re, rf_im, rf2, dt;
+    T gx, gy, gz;
+    int flags;  // kEv...; of a block's end 1 + its code, negated
 };
+// Event flags: axes with a gradient, RF on, rotation as the previous step's,
+// dt as the previous step's.
+constexpr int kEvAxes = 7, kEvRf = 8, kEvSame = 16, kEvDt = 32;
+// FP64: largest departure of dt (ms) that is corrected to first order.
+constexpr double kDtNear = 1e-12;
 
-template <typename T>
-__device__ inline void dev_sincos(T x, T *s, T *c);
-// FP64 form: sincospi of x / pi.  Its range reduction is exact (x/pi -
-// rint), where sincos of a many-radian argument takes the general reduction;
-// the one extra rounding of x / pi is 1.1e-16 relative.  7 % faster on the
-// 1000-event, 512k-node integrator.
-template <>
-__device__ inline void dev_sincos<double>(double x, double *s, double *c)
-{
-    sincospi(x * 0.31830988618379067154, s, c);
-}
 // FP32 form: the hardware sine/cosine, which take revolutions, after
 // reducing the argument to [-1/2, 1/2] revolution.  Their error is absolute
 // (a few 1e-7), which is large relative to the small per-event rotations of
@@ -67,8 +84,7 @@ __device__ inline void dev_sincos<double>(double x, double *s, double *c)
 // (truncation < 1e-10) is used instead.  The choice is per lane; the wave
 // evaluates only the form(s) its lanes need (series only, hardware only, or
 // both and a select).
-template <>
-__device__ inline void dev_sincos<float>(float x, float *s, float *c)
+__device__ inline void sincos_f32(float x, float *s, float *c)
 {
     float r = x * 0.159154943091895336f;
     r -= __builtin_rintf(r);
@@ -107,74 +123,169 @@ __device__ inline float dev_exp<float>(float x) { return __builtin_amdgcn_exp2f(
 // E1 / (1 - E1) (~200 for TR 5 ms, T1 1 s), so e1 rounded to FP32 (or 1 - e1
 // formed in FP32) would bias Mz by ~1e-5; om1 carries the recovery with full
 // FP32 relative precision.  Evaluated only when dt changes.
-template <typename T>
-__device__ inline T one_minus_exp(T x, T e);
-template <>
-__device__ inline double one_minus_exp<double>(double, double e) { return 1.0 - e; }
-template <>
-__device__ inline float one_minus_exp<float>(float x, float) { return (float)(-expm1((double)x)); }
-
-template <typename T>
-__device__ inline T relax_mz(T mz, T e1, T om1, T M0);
-template <>
-__device__ inline double relax_mz<double>(double mz, double e1, double om1, double M0) { return fma(mz, e1, om1 * M0); }
-template <>
-__device__ inline float relax_mz<float>(float mz, float, float om1, float M0) { return mz - om1 * (mz - M0); }
-
-// Mz coefficient |alpha|^2 - |beta|^2 of the rotation.  FP64 form: the
-// reference's expression (BlochSimulator.cpp:262, :133).  FP32 form: 1 - 2
-// |beta|^2, equal to it for a unitary (alpha, beta).  In FP32, c^2 + s^2
-// misses 1 by up to an ulp, the same way on every event of a readout (same
-// node, same gradient), so a2 - b2 scales Mz systematically during free
-// precession; 1 - 2 b2 is exactly 1 there (beta = 0).
-template <typename T>
-__device__ inline T mz_coef(T a2, T b2);
-template <>
-__device__ inline double mz_coef<double>(double a2, double b2) { return a2 - b2; }
-template <>
-__device__ inline float mz_coef<float>(float, float b2) { return fmaf(-2.0f, b2, 1.0f); }
-
-template <typename T>
-__device__ inline T dev_sqrt(T x);
-template <>
-__device__ inline double dev_sqrt<double>(double x) { return sqrt(x); }
-template <>
-__device__ inline float dev_sqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
-
-template <typename T>
-__device__ inline T dev_rcp(T x);
-template <>
-__device__ inline double dev_rcp<double>(double x) { return 1.0 / x; }
-template <>
-__device__ inline float dev_rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
-
-// a != b for values that are equal across the wave, decided on the scalar
-// unit (first lane's bits).
-__device__ inline bool uniform_ne(double a, double b)
+__device__ inline float one_minus_exp(float x)
 {
-    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a);
-    const unsigned long long ub = __builtin_bit_cast(unsigned long long, b);
-    const unsigned alo = __builtin_amdgcn_readfirstlane((unsigned)ua);
-    const unsigned ahi = __builtin_amdgcn_readfirstlane((unsigned)(ua >> 32));
-    const unsigned blo = __builtin_amdgcn_readfirstlane((unsigned)ub);
-    const unsigned bhi = __builtin_amdgcn_readfirstlane((unsigned)(ub >> 32));
-    return alo != blo || ahi != bhi;
+    const double w = (double)x;
+    double p;
+    if (__all(__builtin_fabsf(x) < 1.0f / 64.0f)) {  // an event against T1: the series to w^7, within 3e-15
+        p = fma(w, 1.0 / 5040.0, 1.0 / 720.0);
+        p = fma(w, p, 1.0 / 120.0);
+        p = fma(w, p, 1.0 / 24.0);
+        p = fma(w, p, 1.0 / 6.0);
+        p = fma(w, p, 0.5);
+        p = w * fma(w, p, 1.0);
+    } else {
+        p = exp(w) - 1.0;  // loses no more than 6 of 53 bits
+    }
+    return (float)-p;
 }
-__device__ inline bool uniform_ne(float a, float b)
+
+// The FP32 rotation of an event with RF: alpha = c - i nz s, beta = -i (rf/|B|)
+// s (BlochSimulator.cpp:251-262), as the coefficients of Mz, Mxy and conj(Mxy).
+// The Mz coefficient is 1 - 2 |beta|^2, equal to |alpha|^2 - |beta|^2 for a
+// unitary (alpha, beta): in FP32 c^2 + s^2 misses 1 by up to an ulp, the same
+// way on every event of a readout.
+struct Rot32 {
+    float zr, zi;      // 2 conj(alpha) beta: Mz into Mxy
+    float ar, ai;      // conj(alpha)^2: Mxy into Mxy
+    float br, bi;      // beta^2: conj(Mxy) into Mxy (subtracted)
+    float m, abr, abi; // Mz into Mz; alpha beta: 2 Re(alpha beta conj(Mxy)) out of Mz
+};
+__device__ inline void rot_make(Rot32 &r, float Bz, float rf_re, float rf_im, float rf2, float gamma, float dt)
 {
-    return __builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, a)) !=
-           __builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, b));
+    float Bn = __builtin_amdgcn_sqrtf(fmaf(Bz, Bz, rf2));
+    if (Bn < 1e-12f) Bn = 1e-12f;
+    const float inv = __builtin_amdgcn_rcpf(Bn);
+    const float nz = Bz * inv;
+    float s, c;
+    sincos_f32(Bn * (-0.5f * gamma * dt), &s, &c);
+    const float ar = c, ai = -nz * s;
+    const float br = rf_im * inv * s, bi = -rf_re * inv * s;
+    // every sum of two products is written as one fma and one product, so that
+    // each instantiation of the kernel rounds alike (a free contraction may
+    // fuse either product)
+    const float b2 = fmaf(br, br, bi * bi);
+    const float car = ar, cai = -ai;
+    r.zr = 2.0f * fmaf(car, br, -(cai * bi));
+    r.zi = 2.0f * fmaf(car, bi, cai * br);
+    r.ar = fmaf(car, car, -(cai * cai));
+    r.ai = (2.0f * car) * cai;
+    r.br = fmaf(br, br, -(bi * bi));
+    r.bi = (2.0f * br) * bi;
+    r.m = fmaf(-2.0f, b2, 1.0f);
+    r.abr = fmaf(ar, br, -(ai * bi));
+    r.abi = fmaf(ar, bi, ai * br);
 }
-// a == 0 for a value that is equal across the wave (first lane's bits,
-// either sign of zero)
-__device__ inline bool uniform_zero(double a)
+__device__ inline void rot_apply(const Rot32 &r, bool, float, float &mxr, float &mxi, float &mz)
 {
-    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a) << 1;
-    return (__builtin_amdgcn_readfirstlane((unsigned)ua) | __builtin_amdgcn_readfirstlane((unsigned)(ua >> 32))) == 0;
+    const float cmr = mxr, cmi = -mxi;
+    const float nmr = fmaf(r.zr, mz, fmaf(r.ar, mxr, -(r.ai * mxi)) - fmaf(r.br, cmr, -(r.bi * cmi)));
+    const float nmi = fmaf(r.zi, mz, fmaf(r.ar, mxi, r.ai * mxr) - fmaf(r.br, cmi, r.bi * cmr));
+    mz = fmaf(r.m, mz, -(2.0f * fmaf(r.abr, cmr, -(r.abi * cmi))));
+    mxr = nmr;
+    mxi = nmi;
 }
-__device__ inline bool uniform_zero(float a)
+// Free precession: Mxy exp(-i gamma dt Bz).
+struct Pre32 {
+    float s, c;
+};
+__device__ inline void pre_make(Pre32 &r, float Bz, float gamma, float dt)
 {
-    return (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, a)) << 1) == 0;
+    sincos_f32(-gamma * dt * Bz, &r.s, &r.c);
+}
+__device__ inline void pre_apply(const Pre32 &r, bool, float, float &mxr, float &mxi)
+{
+    const float nmr = fmaf(r.c, mxr, -(r.s * mxi));
+    mxi = fmaf(r.c, mxi, r.s * mxr);
+    mxr = nmr;
+}
+
+// 1 / sqrt(x) for x in [1e-24, 1e24]: the hardware's estimate and two Newton
+// steps (error below an ulp or so).
+__device__ inline double rsqrt_f64(double x)
+{
+    double r = __builtin_amdgcn_rsq(x);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const double e = fma(-x * r, r, 1.0);
+        r = fma(0.5 * r, e, r);
+    }
+    return r;
+}
+
+// FP64: the rotation matrix about the axis n = (rf, Bz) / |B|, and the angle's
+// rate om per ms of dt: for a dt that is off by d the rotation by om d about n
+// follows, to first order.
+struct Rot64 {
+    double m[9], nx, ny, nz, om;
+};
+// -gamma dt B in cycles.  gamma / 2 pi enters as two doubles: its rounding
+// would be the same on every event, and add up over a sequence.
+__device__ inline double cycles_f64(double B, double gamma, double dt)
+{
+    constexpr double kHi = 0.15915494309189535, kLo = -9.839338337591243e-18;  // 1 / 2 pi
+    const double hi = gamma * kHi, lo = fma(gamma, kLo, fma(gamma, kHi, -hi));
+    const double u = -dt * B;
+    return fma(u, hi, u * lo);
+}
+__device__ inline void rot_make(Rot64 &r, double Bz, double rf_re, double rf_im, double rf2, double gamma, double dt)
+{
+    const double B2 = fma(Bz, Bz, rf2);
+    const double B2c = B2 < 1e-24 ? 1e-24 : B2;  // |B| floored at 1e-12
+    const double inv = rsqrt_f64(B2c), B0 = B2c * inv;
+    const double Bn = fma(0.5 * inv, fma(-B0, B0, B2c), B0);
+    double sh, ch;
+    sincos_cycles_f64(0.5 * cycles_f64(Bn, gamma, dt), sh, ch);  // of the half angle
+    const double x = rf_re * inv, y = rf_im * inv, z = Bz * inv;
+    r.nx = x;
+    r.ny = y;
+    r.nz = z;
+    const double s = 2.0 * sh * ch, k = 2.0 * sh * sh;  // v + s n x v + k n x (n x v)
+    const double kx = k * x, ky = k * y, kz = k * z;
+    r.m[0] = 1.0 - fma(ky, y, kz * z);
+    r.m[1] = fma(kx, y, -(s * z));
+    r.m[2] = fma(kx, z, s * y);
+    r.m[3] = fma(kx, y, s * z);
+    r.m[4] = 1.0 - fma(kx, x, kz * z);
+    r.m[5] = fma(ky, z, -(s * x));
+    r.m[6] = fma(kx, z, -(s * y));
+    r.m[7] = fma(ky, z, s * x);
+    r.m[8] = 1.0 - fma(kx, x, ky * y);
+    r.om = -gamma * Bn;
+}
+__device__ inline void rot_apply(const Rot64 &r, bool off, double d, double &mxr, double &mxi, double &mz)
+{
+    const double a = fma(r.m[0], mxr, fma(r.m[1], mxi, r.m[2] * mz));
+    const double b = fma(r.m[3], mxr, fma(r.m[4], mxi, r.m[5] * mz));
+    const double c = fma(r.m[6], mxr, fma(r.m[7], mxi, r.m[8] * mz));
+    mxr = a;
+    mxi = b;
+    mz = c;
+    if (off) {
+        const double th = r.om * d;
+        mxr = fma(th, fma(r.ny, c, -(r.nz * b)), a);
+        mxi = fma(th, fma(r.nz, a, -(r.nx * c)), b);
+        mz = fma(th, fma(r.nx, b, -(r.ny * a)), c);
+    }
+}
+struct Pre64 {
+    double s, c, om;
+};
+__device__ inline void pre_make(Pre64 &r, double Bz, double gamma, double dt)
+{
+    sincos_cycles_f64(cycles_f64(Bz, gamma, dt), r.s, r.c);
+    r.om = -gamma * Bz;
+}
+__device__ inline void pre_apply(const Pre64 &r, bool off, double d, double &mxr, double &mxi)
+{
+    const double a = fma(r.c, mxr, -(r.s * mxi)), b = fma(r.c, mxi, r.s * mxr);
+    mxr = a;
+    mxi = b;
+    if (off) {
+        const double th = r.om * d;
+        mxr = fma(-th, b, a);
+        mxi = fma(th, a, b);
+    }
 }
 
 template <typename T>
@@ -182,10 +293,14 @@ struct Cplx2;
 template <>
 struct Cplx2<double> {
     using type = double2;
+    using Rot = Rot64;
+    using Pre = Pre64;
 };
 template <>
 struct Cplx2<float> {
     using type = float2;
+    using Rot = Rot32;
+    using Pre = Pre32;
 };
 
 // Chained blocks: kChainHost takes the block boundaries from a ChainDesc
@@ -195,8 +310,18 @@ struct Cplx2<float> {
 // read from device memory as well.
 constexpr int kChainNone = 0, kChainHost = 1, kChainMarks = 2;
 
-template <typename T, bool MOTION, bool HISTORY, int CHAIN = kChainNone>
-__global__ __launch_bounds__(kBlochThreads) void k_bloch(
+// Waves per SIMD: one event is a chain of dependent operations, so waves that
+// overlap it are worth the few registers spilled on the paths seldom taken.
+// The moving FP32 sequence above: 26.9 ms at 5, 24.4 at 6, 22.5 at 8; the
+// static FP64 one: 0.43 ms at 3 and at 5 (29 registers spilled), 0.40 at 4.
+constexpr int bloch_waves(bool f64, int RB)
+{
+    return f64 ? (RB <= 1 ? 4 : 2) : (RB <= 2 ? 8 : RB <= 5 ? 6 : 4);
+}
+
+// RB: modes per component, 0 for static nodes (R <= RB; the rest are zero).
+template <typename T, int RB, bool HISTORY, int CHAIN = kChainNone>
+__global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) void k_bloch(
     const double *__restrict__ packed, int64_t N, int64_t n_time, double M0d, double gammad,
     const double *__restrict__ rf, const double *__restrict__ G, const double *__restrict__ dt,
     const double *mxy_in, const double *mz_in,  // may alias mxy_fin / mz_fin
@@ -208,10 +333,11 @@ __global__ __launch_bounds__(kBlochThreads) void k_bloch(
     int64_t n_store = 0)
 {
     using C2 = typename Cplx2<T>::type;
+    constexpr bool MOTION = RB > 0, F64 = sizeof(T) == 8;
     static_assert(CHAIN == kChainNone || !HISTORY, "chained blocks keep the final state only");
-    __shared__ Event<T> sev[kBlochChunk];
-    __shared__ T scoef[MOTION ? kBlochChunk * (kBlochMaxModes + 3) : 1];
-    __shared__ int32_t smark[CHAIN != kChainNone ? kBlochChunk : 1];  // 0: a step; else 1 + block-end code
+    constexpr int kRow = RB + 3;                     // mode weights, translation
+    __shared__ Event<T> sev[kBlochChunk + 1];        // one more: the read ahead
+    __shared__ T scoef[MOTION ? (kBlochChunk + 1) * kRow : 1];
     if constexpr (CHAIN == kChainMarks) {
         // the event count is produced on the device; n_time is the capacity
         const int64_t ne = *n_events;
@@ -223,28 +349,30 @@ __global__ __launch_bounds__(kBlochThreads) void k_bloch(
     const bool active = p < N;
     const T M0 = (T)M0d, gamma = (T)gammad;
 
-    T x = 0, y = 0, z = 0, invT1 = 0, invT2 = 0, dB = 0;
+    T pos[3] = {0, 0, 0}, invT1 = 0, invT2 = 0, dB = 0;
     T mxr = 0, mxi = 0, mz = 0;
-    float md[MOTION ? 3 * kBlochMaxModes : 1];
+    float md[MOTION ? 3 * RB : 1];
+    bool finite = true;  // position and modes: a gradient of 0 leaves nothing of them
     if (active) {
-        x = (T)packed[p];
-        y = (T)packed[N + p];
-        z = (T)packed[2 * N + p];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            pos[c] = (T)packed[c * N + p];
+            finite = finite && __builtin_isfinite(pos[c]);
+        }
         invT1 = (T)packed[3 * N + p];
         invT2 = (T)packed[4 * N + p];
         dB = (T)packed[5 * N + p];
         mxr = (T)mxy_in[2 * p];
         mxi = (T)mxy_in[2 * p + 1];
         mz = (T)mz_in[p];
-        if (MOTION) {
+        if constexpr (MOTION) {
 #pragma unroll
-            for (int r = 0; r < kBlochMaxModes; ++r) {
-                if (r < R) {
-                    md[r] = modes[(int64_t)r * N + p];
-                    md[kBlochMaxModes + r] = modes[(int64_t)(R + r) * N + p];
-                    md[2 * kBlochMaxModes + r] = modes[(int64_t)(2 * R + r) * N + p];
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    md[c * RB + r] = r < R ? modes[(int64_t)(c * R + r) * N + p] : 0.0f;
+                    finite = finite && __builtin_isfinite(md[c * RB + r]);
                 }
-            }
         }
         if (HISTORY) {
             C2 o;
@@ -254,148 +382,223 @@ __global__ __launch_bounds__(kBlochThreads) void k_bloch(
             mz_out[p] = mz;
         }
     }
-    T e1 = 0, e2 = 0, om1 = 0, dt_prev = (T)-1;
+    const int all_axes = __all(finite) ? 0 : kEvAxes;  // the same for the wave
+    T e1 = 0, e2 = 0, dt_e = (T)-1;                    // decay factors (FP32: e1 is 1 - exp(-dt / T1)), their dt
+    T dt_r = (T)-1;                                    // dt of the rotation
     const int64_t n_steps = n_time > 0 ? n_time - 1 : 0;
     const int RC = R + 3;
+    if (tid == 0) sev[kBlochChunk].flags = 0;
 
     for (int64_t base = 0; base < n_steps; base += kBlochChunk) {
         __syncthreads();
         {
             const int64_t i = base + tid;  // step i uses event i + 1
             Event<T> ev;
+            int mk = 0, fl = 0;
             if (i < n_steps) {
                 const double rr = rf[2 * (i + 1)], ri = rf[2 * (i + 1) + 1];
+                const double g0 = G[3 * (i + 1)], g1 = G[3 * (i + 1) + 1], g2 = G[3 * (i + 1) + 2];
                 ev.rf_re = (T)rr;
                 ev.rf_im = (T)ri;
                 ev.rf2 = ev.rf_re * ev.rf_re + ev.rf_im * ev.rf_im;
                 ev.dt = (T)dt[i + 1];
-                ev.kappa = -(T)0.5 * gamma * ev.dt;
-                ev.gx = (T)G[3 * (i + 1)];
-                ev.gy = (T)G[3 * (i + 1) + 1];
-                ev.gz = (T)G[3 * (i + 1) + 2];
-            } else {
-                ev.rf_re = ev.rf_im = ev.rf2 = ev.kappa = ev.gx = ev.gy = ev.gz = ev.dt = 0;
-            }
-            sev[tid] = ev;
-            if constexpr (CHAIN == kChainMarks) {
-                smark[tid] = i < n_steps ? marks[i + 1] : 0;
-            }
-            if constexpr (CHAIN == kChainHost) {
-                // event i + 1 starts block b > 0: it ends block b - 1
-                int mk = 0;
-                if (i < n_steps) {
-                    int lo = 1, hi = chain.n - 1;
-                    while (lo <= hi) {
-                        const int mid = (lo + hi) / 2;
-                        if (chain.offset[mid] == i + 1) {
-                            mk = 1 + chain.code[mid - 1];
-                            break;
-                        }
-                        if (chain.offset[mid] < i + 1) lo = mid + 1;
-                        else hi = mid - 1;
-                    }
+                ev.gx = (T)g0;
+                ev.gy = (T)g1;
+                ev.gz = (T)g2;
+                fl = (ev.gx != (T)0 ? 1 : 0) | (ev.gy != (T)0 ? 2 : 0) | (ev.gz != (T)0 ? 4 : 0) |
+                     (ev.rf2 != (T)0 ? kEvRf : 0);
+                // the previous event (a step unless it starts a block or is the first)
+                bool prev_step = i >= 1;
+                if constexpr (CHAIN == kChainMarks) {
+                    mk = marks[i + 1];
+                    prev_step = prev_step && marks[i] == 0;
                 }
-                smark[tid] = mk;
+                if constexpr (CHAIN == kChainHost) {
+                    // event q starts block b > 0: it ends block b - 1
+                    auto starts = [&](int64_t q) {
+                        int lo = 1, hi = chain.n - 1;
+                        while (lo <= hi) {
+                            const int mid = (lo + hi) / 2;
+                            if (chain.offset[mid] == q) return 1 + chain.code[mid - 1];
+                            if (chain.offset[mid] < q) lo = mid + 1;
+                            else hi = mid - 1;
+                        }
+                        return 0;
+                    };
+                    mk = starts(i + 1);
+                    prev_step = prev_step && starts(i) == 0;
+                }
+                if (prev_step && (T)dt[i] == ev.dt) fl |= kEvDt;
+                if (prev_step && (F64 || (fl & kEvDt)) && (!MOTION || (fl & kEvAxes) == 0) && rf[2 * i] == rr &&
+                    rf[2 * i + 1] == ri && G[3 * i] == g0 && G[3 * i + 1] == g1 && G[3 * i + 2] == g2)
+                    fl |= kEvSame;
+            } else {
+                ev.rf_re = ev.rf_im = ev.rf2 = ev.gx = ev.gy = ev.gz = ev.dt = 0;
             }
-            if (MOTION) {
-                for (int q = 0; q < RC; ++q)
-                    scoef[tid * RC + q] = (i < n_steps) ? (T)mcoef[i * RC + q] : (T)0;
+            if constexpr (MOTION) {
+                bool fin = true;
+                for (int q = 0; q < kRow; ++q) {
+                    // weights 0 .. R - 1, zeros up to RB, translation
+                    const int src = q < R ? q : (q >= RB ? q - RB + R : -1);
+                    const T w = i < n_steps && src >= 0 ? (T)mcoef[i * RC + src] : (T)0;
+                    scoef[tid * kRow + q] = w;
+                    fin = fin && __builtin_isfinite(w);
+                }
+                if (!fin) fl = (fl | kEvAxes) & ~kEvSame;
             }
+            ev.flags = mk != 0 ? -mk : fl;
+            sev[tid] = ev;
         }
         __syncthreads();
         const int cnt = (n_steps - base < kBlochChunk) ? (int)(n_steps - base) : kBlochChunk;
         if (active) {
-            for (int e = 0; e < cnt; ++e) {
+            int e = 0;
+            Event<T> ev;
+            T cf[RB > 0 && RB <= 2 ? kRow : 1];
+            // event e, and its weights where they are few, in wide reads kept together
+            auto fetch = [&]() {
+                ev = sev[e];
+                if constexpr (RB > 0 && RB <= 2)
+#pragma unroll
+                    for (int q = 0; q < kRow; ++q) cf[q] = scoef[e * kRow + q];
+            };
+            auto fetched = [&]() {
+                if constexpr (!F64) {
+                    asm volatile("" : "+v"(ev.rf_re), "+v"(ev.rf_im), "+v"(ev.rf2), "+v"(ev.dt), "+v"(ev.gx), "+v"(ev.gy),
+                                 "+v"(ev.gz), "+v"(ev.flags));
+                    if constexpr (RB > 0 && RB <= 2)
+#pragma unroll
+                        for (int q = 0; q < kRow; ++q) asm volatile("" : "+v"(cf[q]));
+                }
+            };
+            fetch();
+            fetched();
+            T de = 0, d = 0;  // FP64: departures of dt from that of the decay factors and of the rotation
+            bool off = false;  // either is not 0
+            // the end of a step: the next event's record, then relaxation
+            auto relax = [&]() {
+                ++e;
+                fetch();  // one past the last: the spare entry, which is not a step
+                if constexpr (F64) {
+                    T f2 = e2, f1 = e1;
+                    if (off) {
+                        f2 = fma(-de * invT2, e2, e2);
+                        f1 = fma(-de * invT1, e1, e1);
+                    }
+                    mxr *= f2;
+                    mxi *= f2;
+                    mz = fma(mz, f1, (1.0 - f1) * M0);
+                } else {
+                    mxr *= e2;
+                    mxi *= e2;
+                    mz = mz - e1 * (mz - M0);
+                }
+                fetched();
+                if (HISTORY) {
+                    const int64_t o = p + (base + e) * N;
+                    C2 v;
+                    v.x = mxr;
+                    v.y = mxi;
+                    mxy_out[o] = v;
+                    mz_out[o] = mz;
+                }
+            };
+            // the next step has the rotation and decay at hand
+            auto more = [&]() {
+                const int fl = __builtin_amdgcn_readfirstlane(ev.flags);
+                if (fl < 0 || !(fl & kEvSame)) return false;
+                if constexpr (F64) {
+                    de = ev.dt - dt_e;
+                    d = ev.dt - dt_r;
+                    const T m = __builtin_fabs(de) + __builtin_fabs(d);
+                    off = __any(m != 0);
+                    return __all(m <= kDtNear) != 0;
+                }
+                return true;
+            };
+            while (e < cnt) {
+                const int flags = __builtin_amdgcn_readfirstlane(ev.flags);
+                const int fl = flags | all_axes;
                 if constexpr (CHAIN != kChainNone) {
-                    const int mk = smark[e];
-                    if (mk != 0) {  // the same for every lane: a block ends here
+                    if (flags < 0) {  // the same for every lane: a block ends here
+                        const int mk = -flags;
                         const int col = ((mk - 1) >> 1) - 1;
                         if (col >= 0 && (CHAIN == kChainHost || col < n_store)) {
                             store_xy[p + col * N] = make_float2((float)mxr, (float)mxi);
                             store_z[p + col * N] = (float)mz;
                         }
                         if ((mk - 1) & 1) mxr = mxi = 0;
+                        ++e;
+                        fetch();
+                        fetched();
                         continue;
                     }
                 }
-                const Event<T> ev = sev[e];
                 // BlochSimulator.cpp:207-214: e1/e2 only when dt changes.  dt
-                // is the same for every lane (LDS broadcast), so test it on
-                // the scalar unit: a real branch, not two exp per event
-                // under a lane mask.
-                if (uniform_ne(ev.dt, dt_prev)) {
-                    e1 = dev_exp<T>(-ev.dt * invT1);
-                    e2 = dev_exp<T>(-ev.dt * invT2);
-                    om1 = one_minus_exp<T>(-ev.dt * invT1, e1);
-                    dt_prev = ev.dt;
+                // is the same for every lane, so these are real branches.
+                if constexpr (F64) {
+                    de = ev.dt - dt_e;
+                    if (!__all(__builtin_fabs(de) <= kDtNear)) {
+                        e1 = dev_exp<T>(-ev.dt * invT1);
+                        e2 = dev_exp<T>(-ev.dt * invT2);
+                        dt_e = ev.dt;
+                        de = 0;
+                    }
+                    // a run of equal steps that a chunk cuts keeps its dt
+                    d = ev.dt - dt_r;
+                    if (!((fl & kEvSame) && __all(__builtin_fabs(d) <= kDtNear))) {
+                        dt_r = ev.dt;
+                        d = 0;
+                    }
+                    off = __any(de != 0 || d != 0);
+                } else {
+                    if (!(fl & kEvDt)) {
+                        e1 = one_minus_exp(-ev.dt * invT1);
+                        e2 = dev_exp<T>(-ev.dt * invT2);
+                    }
+                    dt_r = ev.dt;
                 }
-                T px = x, py = y, pz = z;
-                if (MOTION) {
-                    const T *cf = &scoef[e * RC];
-                    T dx = cf[R], dy = cf[R + 1], dz = cf[R + 2];
+                T Bz = 0;
+                {
+#pragma clang fp contract(off)
+                    // field along z: only the axes that are on; rounded as the
+                    // sum over all three would be
+                    const T *w = RB > 0 && RB <= 2 ? cf : &scoef[MOTION ? e * kRow : 0];
+                    auto at = [&](auto axis) {
+                        constexpr int c = decltype(axis)::value;
+                        T q = pos[c];
+                        if constexpr (MOTION) {
+                            T dq = w[RB + c];
 #pragma unroll
-                    for (int r = 0; r < kBlochMaxModes; ++r) {
-                        if (r < R) {
-                            dx = fma((T)md[r], cf[r], dx);
-                            dy = fma((T)md[kBlochMaxModes + r], cf[r], dy);
-                            dz = fma((T)md[2 * kBlochMaxModes + r], cf[r], dz);
+                            for (int r = 0; r < RB; ++r) dq = fma((T)md[c * RB + r], w[r], dq);
+                            q += dq;
                         }
-                    }
-                    px += dx;
-                    py += dy;
-                    pz += dz;
+                        return q;
+                    };
+                    using X = std::integral_constant<int, 0>;
+                    using Y = std::integral_constant<int, 1>;
+                    using Z = std::integral_constant<int, 2>;
+                    const int axes = fl & kEvAxes;
+                    if (axes == 1) Bz = at(X{}) * ev.gx;
+                    else if (axes == 2) Bz = at(Y{}) * ev.gy;
+                    else if (axes == 4) Bz = at(Z{}) * ev.gz;
+                    else if (axes != 0) Bz = fma(at(Z{}), ev.gz, fma(at(Y{}), ev.gy, at(X{}) * ev.gx));
+                    Bz = Bz + dB;
                 }
-                const T Bz = fma(pz, ev.gz, fma(py, ev.gy, px * ev.gx)) + dB;
-                if (uniform_zero(ev.rf2)) {
-                    // free precession: Mxy exp(-i gamma dt Bz); kappa = -gamma dt / 2
-                    T s, c;
-                    dev_sincos<T>((ev.kappa + ev.kappa) * Bz, &s, &c);
-                    const T nmr = fma(c, mxr, -(s * mxi)), nmi = fma(c, mxi, s * mxr);
-                    mxr = nmr * e2;
-                    mxi = nmi * e2;
-                    mz = relax_mz<T>(mz, e1, om1, M0);
-                    if (HISTORY) {
-                        const int64_t o = p + (base + e + 1) * N;
-                        C2 v;
-                        v.x = mxr;
-                        v.y = mxi;
-                        mxy_out[o] = v;
-                        mz_out[o] = mz;
-                    }
-                    continue;
-                }
-                T Bn = dev_sqrt<T>(fma(Bz, Bz, ev.rf2));
-                if (Bn < (T)1e-12) Bn = (T)1e-12;
-                const T inv = dev_rcp<T>(Bn);
-                const T nz = Bz * inv;
-                T s, c;
-                dev_sincos<T>(Bn * ev.kappa, &s, &c);
-                // alpha = c - i nz s ; beta = -i (rf/|B|) s
-                const T ar = c, ai = -nz * s;
-                const T br = ev.rf_im * inv * s, bi = -ev.rf_re * inv * s;
-                // every sum of two products is written as one fma and one
-                // product, so that each instantiation of this kernel rounds
-                // alike (a free contraction may fuse either product)
-                const T a2 = fma(ar, ar, ai * ai), b2 = fma(br, br, bi * bi);
-                const T car = ar, cai = -ai;
-                const T cab_r = fma(car, br, -(cai * bi)), cab_i = fma(car, bi, cai * br);
-                const T ca2_r = fma(car, car, -(cai * cai)), ca2_i = ((T)2 * car) * cai;
-                const T bb_r = fma(br, br, -(bi * bi)), bb_i = ((T)2 * br) * bi;
-                const T cmr = mxr, cmi = -mxi;
-                const T nmr = fma((T)2 * cab_r, mz, fma(ca2_r, mxr, -(ca2_i * mxi)) - fma(bb_r, cmr, -(bb_i * cmi)));
-                const T nmi = fma((T)2 * cab_i, mz, fma(ca2_r, mxi, ca2_i * mxr) - fma(bb_r, cmi, bb_i * cmr));
-                const T ab_r = fma(ar, br, -(ai * bi)), ab_i = fma(ar, bi, ai * br);
-                const T nmz = fma(mz_coef<T>(a2, b2), mz, -((T)2 * fma(ab_r, cmr, -(ab_i * cmi))));
-                mxr = nmr * e2;
-                mxi = nmi * e2;
-                mz = relax_mz<T>(nmz, e1, om1, M0);
-                if (HISTORY) {
-                    const int64_t o = p + (base + e + 1) * N;
-                    C2 v;
-                    v.x = mxr;
-                    v.y = mxi;
-                    mxy_out[o] = v;
-                    mz_out[o] = mz;
+                if (fl & kEvRf) {
+                    typename Cplx2<T>::Rot rot;
+                    rot_make(rot, Bz, ev.rf_re, ev.rf_im, ev.rf2, gamma, dt_r);
+                    do {
+                        rot_apply(rot, off, d, mxr, mxi, mz);
+                        relax();
+                    } while (more());
+                } else {  // the precession leaves Mz alone
+                    typename Cplx2<T>::Pre pre;
+                    pre_make(pre, Bz, gamma, dt_r);
+                    do {
+                        pre_apply(pre, off, d, mxr, mxi);
+                        relax();
+                    } while (more());
                 }
             }
         }
@@ -447,6 +650,17 @@ __global__ void k_store_spoil(int64_t N, double2 *__restrict__ mxy, const double
     if (spoil) mxy[n] = make_double2(0.0, 0.0);
 }
 
+// Instantiated mode counts: the smallest that holds R.
+#define FM_BLOCH_MODES(R, CALL)             \
+    do {                                    \
+        if ((R) <= 0) CALL(0);              \
+        else if ((R) <= 1) CALL(1);         \
+        else if ((R) <= 2) CALL(2);         \
+        else if ((R) <= 5) CALL(5);         \
+        else if ((R) <= 10) CALL(10);       \
+        else CALL(16);                      \
+    } while (0)
+
 template <typename T>
 static int launch_bloch(bool motion, bool history, int64_t N, int64_t n_time, const double *packed,
                         double M0, double gamma, const double *rf, const double *G, const double *dt,
@@ -459,18 +673,14 @@ static int launch_bloch(bool motion, bool history, int64_t N, int64_t n_time, co
     T *zo = reinterpret_cast<T *>(mz_out);
     double2 *mf = reinterpret_cast<double2 *>(mxy_out);
     double *zf = reinterpret_cast<double *>(mz_out);
-#define FM_BLOCH_ARGS packed, N, n_time, M0, gamma, rf, G, dt, mxy_in, mz_in, modes, R, mcoef, mo, zo, mf, zf
-    if (motion) {
-        if (history)
-            k_bloch<T, true, true><<<blocks, kBlochThreads, 0, st>>>(FM_BLOCH_ARGS);
-        else
-            k_bloch<T, true, false><<<blocks, kBlochThreads, 0, st>>>(FM_BLOCH_ARGS);
-    } else {
-        if (history)
-            k_bloch<T, false, true><<<blocks, kBlochThreads, 0, st>>>(FM_BLOCH_ARGS);
-        else
-            k_bloch<T, false, false><<<blocks, kBlochThreads, 0, st>>>(FM_BLOCH_ARGS);
-    }
+    const int RR = motion ? R : 0;
+#define FM_BLOCH_ARGS packed, N, n_time, M0, gamma, rf, G, dt, mxy_in, mz_in, modes, RR, mcoef, mo, zo, mf, zf
+#define FM_BLOCH_H(RB) k_bloch<T, RB, true><<<blocks, kBlochThreads, 0, st>>>(FM_BLOCH_ARGS)
+#define FM_BLOCH_F(RB) k_bloch<T, RB, false><<<blocks, kBlochThreads, 0, st>>>(FM_BLOCH_ARGS)
+    if (history) FM_BLOCH_MODES(RR, FM_BLOCH_H);
+    else FM_BLOCH_MODES(RR, FM_BLOCH_F);
+#undef FM_BLOCH_H
+#undef FM_BLOCH_F
 #undef FM_BLOCH_ARGS
     FM_LAUNCH_CHECK("k_bloch");
     return FM_OK;
@@ -483,7 +693,7 @@ static void launch_bloch_chain(int64_t N, int64_t n_time, const double *packed, 
                                float2 *store_xy, float *store_z, hipStream_t st)
 {
     const unsigned blocks = (unsigned)cdiv(N, kBlochThreads);
-    k_bloch<T, false, false, kChainHost><<<blocks, kBlochThreads, 0, st>>>(
+    k_bloch<T, 0, false, kChainHost><<<blocks, kBlochThreads, 0, st>>>(
         packed, N, n_time, M0, gamma, rf, G, dt, mxy_in, mz_in, nullptr, 0, nullptr, nullptr, nullptr,
         reinterpret_cast<double2 *>(mxy_out), mz_out, cd, store_xy, store_z);
 }
@@ -497,14 +707,13 @@ static void launch_bloch_marked(bool motion, int64_t N, int64_t capacity, const 
 {
     const unsigned blocks = (unsigned)cdiv(N, kBlochThreads);
     double2 *mf = reinterpret_cast<double2 *>(mxy_out);
-    if (motion)
-        k_bloch<T, true, false, kChainMarks><<<blocks, kBlochThreads, 0, st>>>(
-            packed, N, capacity, M0, gamma, rf, G, dt, mxy_in, mz_in, modes, R, mcoef, nullptr, nullptr, mf, mz_out,
-            NoChain{}, store_xy, store_z, marks, n_events, n_store);
-    else
-        k_bloch<T, false, false, kChainMarks><<<blocks, kBlochThreads, 0, st>>>(
-            packed, N, capacity, M0, gamma, rf, G, dt, mxy_in, mz_in, nullptr, 0, nullptr, nullptr, nullptr, mf,
-            mz_out, NoChain{}, store_xy, store_z, marks, n_events, n_store);
+    const int RR = motion ? R : 0;
+#define FM_BLOCH_M(RB)                                                                                             \
+    k_bloch<T, RB, false, kChainMarks><<<blocks, kBlochThreads, 0, st>>>(                                         \
+        packed, N, capacity, M0, gamma, rf, G, dt, mxy_in, mz_in, modes, RR, mcoef, nullptr, nullptr, mf, mz_out, \
+        NoChain{}, store_xy, store_z, marks, n_events, n_store)
+    FM_BLOCH_MODES(RR, FM_BLOCH_M);
+#undef FM_BLOCH_M
 }
 
 }  // namespace fm
