@@ -53,6 +53,17 @@ __host__ __device__ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 
 __device__ inline float turns_f32(double u) { return (float)__builtin_amdgcn_fract(u); }
 __device__ inline float turns_f32(float u) { return __builtin_amdgcn_fractf(u); }
 
+// Workgroup b of a launch of ceil(n / 8) * 8 workgroups takes range
+// (b % 8) * ceil(n / 8) + b / 8 of n ranges: workgroups are dealt onto the
+// 8 XCDs round-robin, so each XCD runs one contiguous eighth of the ranges.
+__device__ inline int64_t xcd_range(int64_t n_ranges)
+{
+    const int64_t per = (n_ranges + 7) / 8;
+    return (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
+}
+
+inline unsigned xcd_grid(int64_t n_ranges) { return (unsigned)(((n_ranges + 7) / 8) * 8); }
+
 // sin 2 pi u in FP64, u in cycles.  u is reduced exactly to t in [-1/4, 1/4]
 // (whole turns, then sin(pi - x) = sin x) and the Taylor series in t summed to
 // t^21 (the next term is below 2e-18): about 17 FP64 instructions, where a

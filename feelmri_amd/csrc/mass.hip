@@ -71,17 +71,6 @@ __global__ void k_lumped_colour(int64_t begin, int64_t end, const int32_t *__res
     for (int i = 0; i < 4; ++i) w[ids[i]] = fma(det, 1.0 / 24.0, w[ids[i]]);  // += |T|/4
 }
 
-// Workgroup b of a launch of ceil(n / 8) * 8 workgroups takes range
-// (b % 8) * ceil(n / 8) + b / 8 of n ranges: workgroups are dealt onto the
-// 8 XCDs round-robin, so each XCD runs one contiguous eighth of the ranges.
-__device__ inline int64_t xcd_range(int64_t n_ranges)
-{
-    const int64_t per = (n_ranges + 7) / 8;
-    return (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-}
-
-inline unsigned xcd_grid(int64_t n_ranges) { return (unsigned)(((n_ranges + 7) / 8) * 8); }
-
 template <typename T>
 __global__ __launch_bounds__(256) void k_abs_dets(int64_t E, const int32_t *__restrict__ elems,
                                                   const int32_t *__restrict__ pos, const T *__restrict__ nodes,
@@ -92,6 +81,11 @@ __global__ __launch_bounds__(256) void k_abs_dets(int64_t E, const int32_t *__re
     int32_t ids[4];
     dets[pos ? (int64_t)pos[e] : e] = tet_abs_det<T>(elems + 4 * e, nodes, ids);
 }
+
+// Bound by the latency of the two dependent loads of a term, so the loads of
+// kGatherAhead terms are in flight together: 13.4 us for 215 940 nodes of 1 231
+// 920 elements, 4.7 TB/s (24.5 us one term at a time).
+constexpr int kGatherAhead = 8;
 
 // Positions >= n_elems are skipped: with the identity order on a mesh whose
 // elements are ordered by their largest node id, the first n_nodes nodes and
@@ -108,25 +102,40 @@ __global__ __launch_bounds__(256) void k_lumped_gather(int64_t n_nodes, int64_t 
     const int32_t *ids = incident + chunk_offsets[n / 64] + n % 64;
     const int d = degree[n];
     double acc = 0.0;
-    for (int j = 0; j < d; ++j) {
-        const int32_t k = ids[64 * j];
-        if (k < n_elems) acc = fma(dets[k], 1.0 / 24.0, acc);  // += |T|/4
+    for (int j0 = 0; j0 < d; j0 += kGatherAhead) {
+        int32_t k[kGatherAhead];
+        double det[kGatherAhead];
+#pragma unroll
+        for (int u = 0; u < kGatherAhead; ++u) k[u] = j0 + u < d ? ids[64 * (j0 + u)] : -1;
+#pragma unroll
+        for (int u = 0; u < kGatherAhead; ++u) det[u] = k[u] >= 0 && k[u] < n_elems ? dets[k[u]] : 0.0;
+#pragma unroll
+        for (int u = 0; u < kGatherAhead; ++u) acc = fma(det[u], 1.0 / 24.0, acc);  // += |T|/4 (nothing: + 0)
     }
     w[n] = acc;
 }
 
+// Bound by the 128 bytes an element writes.  A wave writes its 64 matrices in
+// 8 stores of 1 KB each: lane l holds 16-byte piece l % 8 of element 8 s +
+// l / 8 in store s, whose determinant it takes from that element's lane.
+// 1 231 920 elements: 37 us, 4.8 TB/s (60 us where a lane wrote its own matrix).
 template <typename T>
-__global__ void k_element_matrices(int64_t E, const int32_t *__restrict__ elems, const T *__restrict__ nodes,
-                                   double *__restrict__ vals)
+__global__ __launch_bounds__(256) void k_element_matrices(int64_t E, const int32_t *__restrict__ elems,
+                                                          const T *__restrict__ nodes, double *__restrict__ vals)
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= E) return;
+    const int lane = threadIdx.x % 64, piece = lane % 8;
+    const int64_t e0 = xcd_range(cdiv(E, 256)) * 256 + threadIdx.x - lane;  // the wave's first element
+    if (e0 >= E) return;
     int32_t ids[4];
-    const double m = tet_abs_det<T>(elems + 4 * e, nodes, ids) * (1.0 / 120.0);  // |T|/20
+    // lanes past the last element work on it and write nothing
+    const double m = tet_abs_det<T>(elems + 4 * (e0 + lane < E ? e0 + lane : E - 1), nodes, ids) * (1.0 / 120.0);  // |T|/20
+    const double fx = piece == 0 || piece == 5 ? 2.0 : 1.0, fy = piece == 2 || piece == 7 ? 2.0 : 1.0;  // diagonal
+    double2 *out = reinterpret_cast<double2 *>(vals + 16 * e0) + lane;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vals[16 * e + 4 * i + j] = (i == j) ? 2.0 * m : m;
+    for (int s = 0; s < 8; ++s) {
+        const double q = __shfl(m, 8 * s + lane / 8);
+        if (e0 + 8 * s + lane / 8 < E) out[64 * s] = make_double2(fx * q, fy * q);
+    }
 }
 
 __global__ void k_fill_f64(int64_t n, double v, double *__restrict__ x)
@@ -301,7 +310,7 @@ extern "C" int fm_mass_p1_element_matrices(int64_t n_elems, const int32_t *elems
     FM_CHECK_ARG(dtype == FM_DTYPE_F32 || dtype == FM_DTYPE_F64, "unknown dtype %d", dtype);
     if (n_elems == 0) return FM_OK;
     FM_CHECK_ARG(elems && nodes && vals, "NULL array");
-    const unsigned blocks = (unsigned)cdiv(n_elems, 256);
+    const unsigned blocks = xcd_grid(cdiv(n_elems, 256));
     hipStream_t st = as_stream(stream);
     if (dtype == FM_DTYPE_F64)
         k_element_matrices<double><<<blocks, 256, 0, st>>>(n_elems, elems, (const double *)nodes, vals);

@@ -496,49 +496,95 @@ __global__ void k_nodes_pack(int64_t N, int V, const T *__restrict__ r0, const T
     }
 }
 
-// CSR SpMV, G lanes per row (G a power of two, at most 64): lane j of a
-// row's group adds the row's terms j, j + G, ... for up to 4 encodings at a
-// time (the row's values and column indices read once per pass, coalesced
-// across the group), then the group sums its lanes in a fixed butterfly, so
-// a result does not depend on the launch.  Groups past the last row work on
-// the last row and write nothing.
-template <int G>
-__global__ __launch_bounds__(256) void k_csr_spmv_c128(int64_t n_rows, int V, const int64_t *__restrict__ indptr,
-                                                        const int64_t *__restrict__ indices,
-                                                        const double *__restrict__ data,
-                                                        const double2 *__restrict__ x, double2 *__restrict__ y)
+// Sum over the 16 lanes of a row group by a fixed butterfly (lane ^ 8, 4, 2,
+// 1; a rotation by 8, 4, 2, 1 reaches the same value, as lanes that far apart
+// hold equal sums by then).
+__device__ inline double sum_group16(double v)
 {
-    const int64_t g = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / G;
-    const int j = threadIdx.x % G;
-    const bool live = g < n_rows;
-    const int64_t r = live ? g : n_rows - 1;
-    const int64_t k0 = indptr[r], k1 = indptr[r + 1];
-    for (int v0 = 0; v0 < V; v0 += 4) {
-        double re[4] = {0.0, 0.0, 0.0, 0.0}, im[4] = {0.0, 0.0, 0.0, 0.0};
-        for (int64_t k = k0 + j; k < k1; k += G) {
-            const double a = data[k];
-            const double2 *xr = x + indices[k] * V + v0;
+    auto step = [&](auto ctrl) {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+        const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)b, decltype(ctrl)::value, 0xf, 0xf, true);
+        const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, true);
+        v += __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+    };
+    step(std::integral_constant<int, 0x128>{});  // row_ror:8
+    step(std::integral_constant<int, 0x124>{});
+    step(std::integral_constant<int, 0x122>{});
+    step(std::integral_constant<int, 0x121>{});
+    return v;
+}
+
+// CSR SpMV, 16 lanes per row (P1 mass rows hold ~15 entries on tetrahedral
+// meshes): lane j of a row's group adds the row's terms j, j + 16, ... for VB
+// encodings at a time (the row's values and column indices read once per pass,
+// coalesced across the group), then the group sums its lanes in a fixed
+// butterfly, so a result does not depend on the launch.  Rows past the last
+// one work on it and write nothing.
+// Bound by the latency of three dependent loads (row, entry, x), so a group
+// takes kSpmvRows rows together, and the rows of a workgroup's XCD are one
+// range, whose part of x stays in that L2.  215 940 rows of 15, two encodings:
+// 20 us, 3.3 TB/s (42 us with a row a group, sums for four encodings through
+// LDS).
+constexpr int kSpmvRows = 4, kSpmvBlockRows = 16 * kSpmvRows;
+
+template <int VB>
+__global__ __launch_bounds__(256) void k_csr_spmv_c128(int64_t n_rows, int V, const int64_t *__restrict__ indptr,
+                                                       const int64_t *__restrict__ indices,
+                                                       const double *__restrict__ data,
+                                                       const double2 *__restrict__ x, double2 *__restrict__ y)
+{
+    const int64_t r0 = xcd_range(cdiv(n_rows, kSpmvBlockRows)) * kSpmvBlockRows + threadIdx.x / 16;
+    const int j = threadIdx.x % 16;
+    int64_t k0[kSpmvRows], k1[kSpmvRows];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (v0 + u < V) {
-                    const double2 xv = xr[u];
-                    re[u] = fma(a, xv.x, re[u]);
-                    im[u] = fma(a, xv.y, im[u]);
+    for (int q = 0; q < kSpmvRows; ++q) {
+        const int64_t r = r0 + 16 * q < n_rows ? r0 + 16 * q : n_rows - 1;
+        k0[q] = indptr[r] + j;
+        k1[q] = indptr[r + 1];
+    }
+    for (int v0 = 0; v0 < V; v0 += VB) {
+        double re[kSpmvRows][VB], im[kSpmvRows][VB], a[kSpmvRows];
+        int64_t c[kSpmvRows];
+#pragma unroll
+        for (int q = 0; q < kSpmvRows; ++q) {
+            a[q] = 0.0;
+            c[q] = -1;
+            if (k0[q] < k1[q]) {
+                a[q] = data[k0[q]];
+                c[q] = indices[k0[q]];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kSpmvRows; ++q)
+#pragma unroll
+            for (int u = 0; u < VB; ++u) {
+                double2 xv = make_double2(0.0, 0.0);
+                if (c[q] >= 0 && v0 + u < V) xv = x[c[q] * V + v0 + u];
+                re[q][u] = fma(a[q], xv.x, 0.0);
+                im[q][u] = fma(a[q], xv.y, 0.0);
+            }
+#pragma unroll
+        for (int q = 0; q < kSpmvRows; ++q) {
+            for (int64_t k = k0[q] + 16; k < k1[q]; k += 16) {
+                const double ak = data[k];
+                const double2 *xr = x + indices[k] * V + v0;
+#pragma unroll
+                for (int u = 0; u < VB; ++u) {
+                    if (v0 + u < V) {
+                        re[q][u] = fma(ak, xr[u].x, re[q][u]);
+                        im[q][u] = fma(ak, xr[u].y, im[q][u]);
+                    }
                 }
             }
         }
 #pragma unroll
-        for (int off = G / 2; off > 0; off >>= 1)
+        for (int q = 0; q < kSpmvRows; ++q)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                re[u] += __shfl_xor(re[u], off, G);
-                im[u] += __shfl_xor(im[u], off, G);
+            for (int u = 0; u < VB; ++u) {
+                const double sr = sum_group16(re[q][u]), si = sum_group16(im[q][u]);
+                if (j == 0 && v0 + u < V && r0 + 16 * q < n_rows)
+                    y[(r0 + 16 * q) * V + v0 + u] = make_double2(sr, si);
             }
-        if (live && j == 0) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (v0 + u < V) y[r * V + v0 + u] = make_double2(re[u], im[u]);
-        }
     }
 }
 
@@ -1285,13 +1331,16 @@ extern "C" int fm_csr_spmv_c128(int64_t n_rows, int n_enc, const int64_t *indptr
     FM_CHECK_ARG(n_rows >= 0 && n_enc >= 1, "bad sizes");
     if (n_rows == 0) return FM_OK;
     FM_CHECK_ARG(indptr && indices && data && x && y, "NULL array");
-    // 16 lanes per row: P1 mass rows hold ~15 entries on tetrahedral meshes
-    // (longer rows take more passes)
-    constexpr int G = 16;
-    const int64_t threads = n_rows * G;
-    FM_CHECK_ARG(cdiv(threads, 256) <= 0x7fffffff, "too many rows for one launch");
-    k_csr_spmv_c128<G><<<(unsigned)cdiv(threads, 256), 256, 0, as_stream(stream)>>>(
-        n_rows, n_enc, indptr, indices, data, reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y));
+    FM_CHECK_ARG(cdiv(n_rows * 16, 256) <= 0x7fffffff, "too many rows for one launch");
+    const unsigned grid = xcd_grid(cdiv(n_rows, kSpmvBlockRows));
+    auto launch = [&](auto vb) {
+        k_csr_spmv_c128<decltype(vb)::value><<<grid, 256, 0, as_stream(stream)>>>(
+            n_rows, n_enc, indptr, indices, data, reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y));
+    };
+    if (n_enc == 1) launch(std::integral_constant<int, 1>{});
+    else if (n_enc == 2) launch(std::integral_constant<int, 2>{});
+    else if (n_enc == 3) launch(std::integral_constant<int, 3>{});
+    else launch(std::integral_constant<int, 4>{});
     FM_LAUNCH_CHECK("k_csr_spmv_c128");
     return FM_OK;
 }
