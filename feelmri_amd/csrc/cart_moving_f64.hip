@@ -11,9 +11,9 @@
 //   * per chunk of 64 W nodes each thread forms one node record in LDS: the
 //     position x0 + sum_r modes_r w_r(t_i) + translation (FP64) and
 //     c_i[n, 0..V) = b_v exp(-t_i/T2) exp(i phi t_i) exp(-2 pi i F_i . x)
-//     (FP64 phase, range reduction, sincospi, exp);
+//     (FP64 phase, sine and cosine, exp);
 //   * per 16-node step (4 k-steps), wave w builds its A fragments (16 lines
-//     of row block W rt + w) in registers, one FP64 sincospi per (line, node);
+//     of row block W rt + w) in registers, one FP64 sine and cosine per (line, node);
 //     the kz factors exp(-2 pi i H_k . x) of the step's nodes are in LDS
 //     (one buffer, written during the previous step's products) and the
 //     workgroup forms the B fragments (16 (k,v) columns per column block,
@@ -26,9 +26,9 @@
 // cart_moving_pairs_bf16.hip): A is one sine per row and node, B the kz row
 // times c_i (two products per entry), and a k-step takes 2 MFMAs per column
 // block: Re += A Re B, Im += A Im B.  150 001 nodes, 63 x 65 x 17, 3
-// encodings, 6 modes: 6.25 ms against 13.1 ms with complex rows, error against
+// encodings, 6 modes: 6.15 ms against 13.1 ms with complex rows, error against
 // 64 bits 1.7e-15 against 1.6e-15.  Real rows need few enough registers for 3
-// waves per SIMD up to 4 column blocks: 6.25 ms against 7.28 ms with 2 (MFMA 41 %
+// waves per SIMD up to 4 column blocks: 6.15 ms against 7.28 ms with 2 (MFMA 41 %
 // busy, the waves waiting at the step barriers).
 // FP64 accumulators need no bound on the split length; node splits exist for
 // parallelism only and are summed in FP64 by k_cart_reduce.
@@ -39,14 +39,11 @@
 
 namespace fm {
 
-// exp(-2 pi i u), u in cycles: exact range reduction, FP64 sincospi.
+// exp(-2 pi i u), u in cycles.
 __device__ inline void cis_neg_f64(double u, double &c, double &s)
 {
-    const double r = u - __builtin_rint(u);
-    double sn, cs;
-    sincospi(2.0 * r, &sn, &cs);
-    c = cs;
-    s = -sn;
+    sincos_cycles_f64(u, s, c);
+    s = -s;
 }
 
 // kz rows of the kz-factor buffer: 16 nodes + 1 entry of pad

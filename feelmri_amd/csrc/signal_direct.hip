@@ -328,10 +328,13 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_runs(
 }
 
 // FP64 form, static nodes, readout runs: the same recurrence in FP64
-// (FP64 phase and sincospi for the anchor and the step, FP64 products and
+// (FP64 phase, sine and cosine for the anchor and the step, FP64 products and
 // accumulators).  Taken only when every run is linear to 1e-14 of the
 // largest |k'| and |t|; 15 FP64 complex products then leave the result
-// ~1e-15 from the per-sample sum of MRI.cpp:260-288.
+// ~1e-15 from the per-sample sum of MRI.cpp:260-288.  Bound by FP64 issue: 96
+// instructions for a run's 16 samples, 35 for a sine and cosine, an exponential.
+// 212 765 nodes, 150 x 188, radial: 3.52 ms (3.88 with the library's sincospi);
+// 70 479 nodes, 140 x 118: 0.94 (1.07).
 template <int VB>
 struct alignas(16) RunNode64 {
     double x, y, z, dwc, r2, pad;
@@ -387,10 +390,9 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_runs_f64(
             if constexpr (SHQ) {
                 for (int j = 0; j < nst; ++j) {
                     const double *st = &run_steps[((int64_t)blockIdx.x * kRunSteps + j) * 4];
-                    double du = fma(st[0], nd.x, fma(st[1], nd.y, fma(st[2], nd.z, -nd.dwc * st[3])));
-                    du -= __builtin_rint(du);
+                    const double du = fma(st[0], nd.x, fma(st[1], nd.y, fma(st[2], nd.z, -nd.dwc * st[3])));
                     double qs, qc;
-                    sincospi(2.0 * du, &qs, &qc);
+                    sincos_cycles_f64(du, qs, qc);
                     const double ds = exp(-st[3] * nd.r2);
                     sq64[j * kSqStride + tid] = make_double2(ds * qc, -ds * qs);
                 }
@@ -402,9 +404,8 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_runs_f64(
             const RunNode64<VB> &nd = snode[i];
             // anchor: the first sample's term, as the per-sample sum forms it
             const double u = fma(rd.k0x, nd.x, fma(rd.k0y, nd.y, fma(rd.k0z, nd.z, -nd.dwc * rd.t0)));
-            const double r = u - __builtin_rint(u);
             double sn, cs;
-            sincospi(2.0 * r, &sn, &cs);
+            sincos_cycles_f64(u, sn, cs);
             const double d0 = exp(-rd.t0 * nd.r2);
             double er = d0 * cs, ei = -d0 * sn;
             // step factor
@@ -414,10 +415,9 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_runs_f64(
                 qr = q.x;
                 qi = q.y;
             } else {
-                double du = fma(rd.dkx, nd.x, fma(rd.dky, nd.y, fma(rd.dkz, nd.z, -nd.dwc * rd.dt)));
-                du -= __builtin_rint(du);
+                const double du = fma(rd.dkx, nd.x, fma(rd.dky, nd.y, fma(rd.dkz, nd.z, -nd.dwc * rd.dt)));
                 double qs, qc;
-                sincospi(2.0 * du, &qs, &qc);
+                sincos_cycles_f64(du, qs, qc);
                 const double ds = exp(-rd.dt * nd.r2);
                 qr = ds * qc;
                 qi = -ds * qs;

@@ -365,21 +365,18 @@ size_t cartesian_workspace(const fm_signal_plan *p, int precision, int64_t n_nod
 // ---------------------------------------------------------------------------
 // Operand tables
 // ---------------------------------------------------------------------------
-// exp(-2 pi i u) for u in cycles: FP64 range reduction, then FP64 sincospi
-// (FP64 form) or the hardware FP32 sine/cosine, which take revolutions.
+// exp(-2 pi i u) for u in cycles: in FP64 (FP64 form), or reduced in FP64 for the
+// hardware FP32 sine/cosine, which take revolutions.
 template <bool MIXED>
 __device__ inline void cis_neg_cycles(double u, double &c, double &s)
 {
-    const double r = u - __builtin_rint(u);
     if (MIXED) {
-        const float rf = (float)r;
+        const float rf = (float)(u - __builtin_rint(u));
         c = (double)__builtin_amdgcn_cosf(rf);
         s = -(double)__builtin_amdgcn_sinf(rf);
     } else {
-        double sn, cs;
-        sincospi(2.0 * r, &sn, &cs);
-        c = cs;
-        s = -sn;
+        sincos_cycles_f64(u, s, c);
+        s = -s;
     }
 }
 
