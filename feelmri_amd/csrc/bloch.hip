@@ -314,9 +314,13 @@ constexpr int kChainNone = 0, kChainHost = 1, kChainMarks = 2;
 // overlap it are worth the few registers spilled on the paths seldom taken.
 // The moving FP32 sequence above: 26.9 ms at 5, 24.4 at 6, 22.5 at 8; the
 // static FP64 one: 0.43 ms at 3 and at 5 (29 registers spilled), 0.40 at 4.
+// Moving FP64, 800 000 / 60 000 nodes, 2500 events, ms at 2, 3 and 4: 2 modes
+// 7.6, 7.6, 7.1 / 1.34, 1.33, 1.43; 5 modes 7.6, 7.6, 8.8 / 1.3, 1.3, 1.7; 10
+// modes 11.0, 10.1, 10.0 / 1.56, 1.77, 1.43; 16 modes 12.5, 10.7, 10.8 / 1.78,
+// 1.49, 1.49.
 constexpr int bloch_waves(bool f64, int RB)
 {
-    return f64 ? (RB <= 1 ? 4 : 2) : (RB <= 2 ? 8 : RB <= 5 ? 6 : 4);
+    return f64 ? (RB <= 2 || RB == 10 ? 4 : 3) : (RB <= 2 ? 8 : RB <= 5 ? 6 : 4);
 }
 
 // RB: modes per component, 0 for static nodes (R <= RB; the rest are zero).
