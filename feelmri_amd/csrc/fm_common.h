@@ -157,6 +157,62 @@ constexpr double kTwoPi = 6.283185307179586476925286766559;
 // Number of CUs on the current device (cached per device).
 int device_cu_count();
 
+// Sum of n split partials, `stride` apart, in FP64 and in order, 8 loads in
+// flight together (past the last: + 0).
+template <typename P>
+__device__ inline double2 sum_splits(const P *__restrict__ p, int64_t stride, int64_t n)
+{
+    double re = 0.0, im = 0.0;
+    for (int64_t s = 0; s < n; s += 8) {
+        P v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            v[u].x = v[u].y = 0;
+            if (s + u < n) v[u] = p[(s + u) * stride];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            re += (double)v[u].x;
+            im += (double)v[u].y;
+        }
+    }
+    return make_double2(re, im);
+}
+
+// Reductions over splits: G threads of a workgroup of 256 share an output, each
+// sums a contiguous range of its splits, and the ranges are added in order.
+// Few outputs of many splits leave most CUs idle and a thread waits for one
+// round of loads after the other, so G is 8 where the outputs alone fill less
+// than 4 waves a CU and there are splits to share.  Radial, mixed, 342 x 55
+// samples of 52 splits, 19 838 nodes: the call 60.6 -> 50.0 us.
+inline int reduce_group(int64_t n_out, int64_t n_splits)
+{
+    return n_splits >= 16 && n_out < (int64_t)256 * device_cu_count() ? 8 : 1;
+}
+inline unsigned reduce_grid(int64_t n_out, int G) { return (unsigned)cdiv(n_out, 256 / G); }
+// The output of this thread, and its sum: of all splits in the thread with
+// tid < 256 / G, whose result it is.
+template <int G>
+__device__ inline int64_t reduce_output() { return (int64_t)blockIdx.x * (256 / G) + threadIdx.x % (256 / G); }
+template <int G, typename P>
+__device__ inline double2 reduce_sum(const P *__restrict__ p, int64_t stride, int64_t n, bool live)
+{
+    if constexpr (G == 1) return live ? sum_splits(p, stride, n) : make_double2(0.0, 0.0);
+    constexpr int kOut = 256 / G;
+    __shared__ double2 sums[G][kOut];
+    const int g = threadIdx.x / kOut, o = threadIdx.x % kOut;
+    const int64_t share = (n + G - 1) / G, s0 = g * share, s1 = s0 + share < n ? s0 + share : n;
+    sums[g][o] = live && s0 < s1 ? sum_splits(p + s0 * stride, stride, s1 - s0) : make_double2(0.0, 0.0);
+    __syncthreads();
+    double2 t = sums[0][o];
+#pragma unroll
+    for (int q = 1; q < G; ++q) {
+        t.x += sums[q][o].x;
+        t.y += sums[q][o].y;
+    }
+    return t;
+}
+
 // Workgroups of `kernel` (a __global__ function) that one CU holds at once
 // with `threads` threads and `dyn` bytes of dynamic LDS; 1 when the runtime
 // cannot tell.

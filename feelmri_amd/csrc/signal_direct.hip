@@ -463,18 +463,13 @@ __global__ __launch_bounds__(kDirectThreads) void k_signal_runs_f64(
 }
 
 // out[s, v] = sum over splits, in split order.
-__global__ void k_reduce_splits(const double2 *__restrict__ part, int64_t n_splits, int64_t SV,
-                                double2 *__restrict__ out)
+template <int G>
+__global__ __launch_bounds__(256) void k_reduce_splits(const double2 *__restrict__ part, int64_t n_splits, int64_t SV,
+                                                       double2 *__restrict__ out)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= SV) return;
-    double re = 0.0, im = 0.0;
-    for (int64_t s = 0; s < n_splits; ++s) {
-        const double2 p = part[s * SV + i];
-        re += p.x;
-        im += p.y;
-    }
-    out[i] = make_double2(re, im);
+    const int64_t i = reduce_output<G>();
+    const double2 sum = reduce_sum<G>(part + i, SV, n_splits, i < SV);
+    if (i < SV && threadIdx.x < 256 / G) out[i] = sum;
 }
 
 template <typename T>
@@ -735,8 +730,9 @@ static int direct_execute(const fm_signal_plan *p, int precision, int64_t N, int
     plan_timing_stop(p, st);
     if (L.n_splits > 1) {
         const int64_t SV = S * V;
-        k_reduce_splits<<<(unsigned)cdiv(SV, 256), 256, 0, st>>>(dst, L.n_splits, SV,
-                                                               reinterpret_cast<double2 *>(out));
+        const int G = reduce_group(SV, L.n_splits);
+        auto *reduce = G == 8 ? k_reduce_splits<8> : k_reduce_splits<1>;
+        reduce<<<reduce_grid(SV, G), 256, 0, st>>>(dst, L.n_splits, SV, reinterpret_cast<double2 *>(out));
         FM_LAUNCH_CHECK("k_reduce_splits");
     }
     return FM_OK;

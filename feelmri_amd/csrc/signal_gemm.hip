@@ -661,18 +661,22 @@ __global__ __launch_bounds__(256) void k_cart_tables(const double *__restrict__ 
                           H, Ey, Ez);
 }
 
-template <typename P>
-__global__ void k_cart_reduce(const P *__restrict__ part, int64_t n_splits, int64_t MNC, double2 *__restrict__ out)
+template <typename P, int G>
+__global__ __launch_bounds__(256) void k_cart_reduce(const P *__restrict__ part, int64_t n_splits, int64_t MNC,
+                                                     double2 *__restrict__ out)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= MNC) return;
-    double re = 0.0, im = 0.0;
-    for (int64_t s = 0; s < n_splits; ++s) {
-        const P v = part[s * MNC + i];
-        re += (double)v.x;
-        im += (double)v.y;
-    }
-    out[i] = make_double2(re, im);
+    const int64_t i = reduce_output<G>();
+    const double2 sum = reduce_sum<G>(part + i, MNC, n_splits, i < MNC);
+    if (i < MNC && threadIdx.x < 256 / G) out[i] = sum;
+}
+
+template <typename P>
+static void launch_cart_reduce(const void *part, int64_t n_splits, int64_t MNC, void *out, hipStream_t st)
+{
+    const int G = reduce_group(MNC, n_splits);
+    auto *reduce = G == 8 ? k_cart_reduce<P, 8> : k_cart_reduce<P, 1>;
+    reduce<<<reduce_grid(MNC, G), 256, 0, st>>>(reinterpret_cast<const P *>(part), n_splits, MNC,
+                                                reinterpret_cast<double2 *>(out));
 }
 
 // Samples from the partial sums over real rows: Lr cosine and sine rows of the
@@ -853,8 +857,7 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
         if (s.pairs)
             launch_reduce_pairs<float2, false>(reinterpret_cast<const float2 *>(ws + s.off_part), s.n_splits, n_kzV,
                                                s.NC, V, c, reinterpret_cast<double2 *>(out), st);
-        else k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(
-            reinterpret_cast<const float2 *>(ws + s.off_part), s.n_splits, MNC, reinterpret_cast<double2 *>(out));
+        else launch_cart_reduce<float2>(ws + s.off_part, s.n_splits, MNC, out, st);
     } else {
         plan_timing_start(p, st);
         launch_cart_gemm_f64(s, ws, n_kzV, st);
@@ -864,8 +867,7 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
         if (s.pairs)
             launch_reduce_pairs<double2, false>(reinterpret_cast<const double2 *>(ws + s.off_part), s.n_splits, n_kzV,
                                                 s.NC, V, c, reinterpret_cast<double2 *>(out), st);
-        else k_cart_reduce<double2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(
-            reinterpret_cast<const double2 *>(ws + s.off_part), s.n_splits, MNC, reinterpret_cast<double2 *>(out));
+        else launch_cart_reduce<double2>(ws + s.off_part, s.n_splits, MNC, out, st);
     }
     FM_LAUNCH_CHECK("k_cart_reduce");
     return FM_OK;
@@ -919,8 +921,7 @@ int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, 
         if (s.pairs)
             launch_reduce_pairs<double2, true>(part, s.n_splits, s.L * s.KV, s.KV, s.V, c,
                                                reinterpret_cast<double2 *>(out), st);
-        else k_cart_reduce<double2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
-                                                                          reinterpret_cast<double2 *>(out));
+        else launch_cart_reduce<double2>(part, s.n_splits, MNC, out, st);
     } else {
         float2 *part = reinterpret_cast<float2 *>(ws);
         if (s.pairs) launch_cart_moving_pairs_bf16(s, c, packed, N, modes, R, mcoef, part, st);
@@ -930,8 +931,7 @@ int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t N, 
         if (s.pairs)
             launch_reduce_pairs<float2, true>(part, s.n_splits, s.L * s.KV, s.KV, s.V, c,
                                               reinterpret_cast<double2 *>(out), st);
-        else k_cart_reduce<float2><<<(unsigned)cdiv(MNC, 256), 256, 0, st>>>(part, s.n_splits, MNC,
-                                                                         reinterpret_cast<double2 *>(out));
+        else launch_cart_reduce<float2>(part, s.n_splits, MNC, out, st);
     }
     FM_LAUNCH_CHECK("k_cart_reduce");
     return FM_OK;

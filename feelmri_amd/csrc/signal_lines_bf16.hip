@@ -263,21 +263,17 @@ __global__ __launch_bounds__(64) void k_signal_lines_bf16(const double *__restri
 }
 
 // out[(m stride + line) V + v] = sum over splits of the partial samples, FP64.
-__global__ void k_lines_reduce(const float2 *__restrict__ part, int64_t n_splits, int64_t n_lines, int64_t PQ,
-                               int64_t L, const RunDesc *__restrict__ lines, int64_t stride, int V, int v,
-                               double2 *__restrict__ out)
+template <int G>
+__global__ __launch_bounds__(256) void k_lines_reduce(const float2 *__restrict__ part, int64_t n_splits,
+                                                      int64_t n_lines, int64_t PQ, int64_t L,
+                                                      const RunDesc *__restrict__ lines, int64_t stride, int V, int v,
+                                                      double2 *__restrict__ out)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_lines * L) return;
+    const int64_t i = reduce_output<G>();
+    const bool live = i < n_lines * L;
     const int64_t line = i / L, m = i % L;
-    double re = 0.0, im = 0.0;
-    for (int64_t s = 0; s < n_splits; ++s) {
-        const float2 p = part[(s * n_lines + line) * PQ + m];
-        re += (double)p.x;
-        im += (double)p.y;
-    }
-    const int64_t sid = (int64_t)lines[line].s0 + m * stride;
-    out[sid * V + v] = make_double2(re, im);
+    const double2 sum = reduce_sum<G>(part + line * PQ + m, n_lines * PQ, n_splits, live);
+    if (live && threadIdx.x < 256 / G) out[((int64_t)lines[line].s0 + m * stride) * V + v] = sum;
 }
 
 struct LineShape {
@@ -378,9 +374,10 @@ int lines_execute(const fm_signal_plan *p, int64_t N, int V, const double *packe
         plan_timing_stop(p, st);
         FM_LAUNCH_CHECK("k_signal_lines_bf16");
         const int64_t n_out = p->n_line_tabs * L;
-        k_lines_reduce<<<(unsigned)cdiv(n_out, 256), 256, 0, st>>>(part, s.n_splits, p->n_line_tabs, s.PQ, L,
-                                                                   p->d_lines, p->n_lines * p->n_kz, V, v,
-                                                                   reinterpret_cast<double2 *>(out));
+        const int G = reduce_group(n_out, s.n_splits);
+        auto *reduce = G == 8 ? k_lines_reduce<8> : k_lines_reduce<1>;
+        reduce<<<reduce_grid(n_out, G), 256, 0, st>>>(part, s.n_splits, p->n_line_tabs, s.PQ, L, p->d_lines,
+                                                      p->n_lines * p->n_kz, V, v, reinterpret_cast<double2 *>(out));
         FM_LAUNCH_CHECK("k_lines_reduce");
     }
     return FM_OK;
