@@ -19,10 +19,11 @@
 //
 // What an event needs is found once, by the thread that stages it, and stored
 // as flags that every lane branches on together:
-//   * the gradient axes that are on: a position along an axis (and the modes of
-//     moving nodes) enters only where its gradient is not 0, since the other
-//     products are 0 (all three axes where a coefficient or a position is not
-//     finite, whose products are not);
+//   * the gradient axes that are on: with more than two modes a position along an
+//     axis is formed only where its gradient is not 0, since the other products
+//     are 0 (all three axes where a coefficient or a position is not finite,
+//     whose products are not); with fewer the tests cost more than they save;
+//   * whether dt is the previous step's;
 //   * whether RF and field repeat the previous step's (hard pulses, gradient
 //     plateaus and delays; moving nodes: no gradient): the lane then keeps the
 //     rotation it formed.  FP32 form: where dt is the same, to the last bit the
@@ -36,8 +37,12 @@
 // step.  The mode loop is unrolled for 1, 2, 5, 10 or 16 modes (zero padded; it
 // was one loop of 16 with a test each), and the next event's record is read
 // from LDS in wide reads while the current one relaxes.  Bound by VALU issue.
-// 1 948 800 moving nodes, 1 mode, 11 255 events, FP32: 22.5 ms (before: 52.6);
-// 512 000 nodes, 33 blocks, 419 steps in all, FP64: 0.367 ms (0.929).
+// 1 948 800 moving nodes, 1 mode, 11 255 events, FP32: 21.5-22.8 ms (before: 52.6);
+// 512 000 nodes, 33 blocks, 419 steps in all, FP64: 0.29 ms (0.929).  1000 events
+// that all differ (no runs): 512 000 nodes, FP64 1.13 ms (1.13), with RF 1.88
+// (2.17), FP32 0.63 (0.57), 1.03 (0.98); 30 000 nodes, where the latency of one
+// event counts, FP64 0.35 (0.24), FP32 0.26 (0.23); 20-event plateaus instead: 0.14
+// (0.24), 0.08 (0.23).
 #include <algorithm>
 #include <type_traits>
 
@@ -235,7 +240,7 @@ __device__ inline void rot_make(Rot64 &r, double Bz, double rf_re, double rf_im,
     const double inv = rsqrt_f64(B2c), B0 = B2c * inv;
     const double Bn = fma(0.5 * inv, fma(-B0, B0, B2c), B0);
     double sh, ch;
-    sincos_cycles_f64(0.5 * cycles_f64(Bn, gamma, dt), sh, ch);  // of the half angle
+    sincos_cycles_f64<true>(0.5 * cycles_f64(Bn, gamma, dt), sh, ch);  // of the half angle
     const double x = rf_re * inv, y = rf_im * inv, z = Bz * inv;
     r.nx = x;
     r.ny = y;
@@ -262,6 +267,7 @@ __device__ inline void rot_apply(const Rot64 &r, bool off, double d, double &mxr
     mxi = b;
     mz = c;
     if (off) {
+        asm volatile("");  // a branch, not a select
         const double th = r.om * d;
         mxr = fma(th, fma(r.ny, c, -(r.nz * b)), a);
         mxi = fma(th, fma(r.nz, a, -(r.nx * c)), b);
@@ -273,7 +279,7 @@ struct Pre64 {
 };
 __device__ inline void pre_make(Pre64 &r, double Bz, double gamma, double dt)
 {
-    sincos_cycles_f64(cycles_f64(Bz, gamma, dt), r.s, r.c);
+    sincos_cycles_f64<true>(cycles_f64(Bz, gamma, dt), r.s, r.c);
     r.om = -gamma * Bz;
 }
 __device__ inline void pre_apply(const Pre64 &r, bool off, double d, double &mxr, double &mxi)
@@ -282,6 +288,7 @@ __device__ inline void pre_apply(const Pre64 &r, bool off, double d, double &mxr
     mxr = a;
     mxi = b;
     if (off) {
+        asm volatile("");
         const double th = r.om * d;
         mxr = fma(-th, b, a);
         mxi = fma(th, a, b);
@@ -310,17 +317,16 @@ struct Cplx2<float> {
 // read from device memory as well.
 constexpr int kChainNone = 0, kChainHost = 1, kChainMarks = 2;
 
+// Modes above which a gradient axis that is off is skipped.
+constexpr int kSkipFrom = 2;
+
 // Waves per SIMD: one event is a chain of dependent operations, so waves that
 // overlap it are worth the few registers spilled on the paths seldom taken.
-// The moving FP32 sequence above: 26.9 ms at 5, 24.4 at 6, 22.5 at 8; the
-// static FP64 one: 0.43 ms at 3 and at 5 (29 registers spilled), 0.40 at 4.
-// Moving FP64, 800 000 / 60 000 nodes, 2500 events, ms at 2, 3 and 4: 2 modes
-// 7.6, 7.6, 7.1 / 1.34, 1.33, 1.43; 5 modes 7.6, 7.6, 8.8 / 1.3, 1.3, 1.7; 10
-// modes 11.0, 10.1, 10.0 / 1.56, 1.77, 1.43; 16 modes 12.5, 10.7, 10.8 / 1.78,
-// 1.49, 1.49.
+// The moving FP32 sequence above: 26.9 ms at 5, 24.4 at 6, 22.5 at 8.  512 000
+// static nodes, FP64, 1000 events that all differ: 1.20 ms at 4, 1.13 at 5.
 constexpr int bloch_waves(bool f64, int RB)
 {
-    return f64 ? (RB <= 2 || RB == 10 ? 4 : 3) : (RB <= 2 ? 8 : RB <= 5 ? 6 : 4);
+    return f64 ? (RB == 0 ? 5 : RB <= 2 ? 4 : RB <= 10 ? 3 : 2) : (RB <= 2 ? 8 : RB <= 5 ? 6 : 4);
 }
 
 // RB: modes per component, 0 for static nodes (R <= RB; the rest are zero).
@@ -337,7 +343,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
     int64_t n_store = 0)
 {
     using C2 = typename Cplx2<T>::type;
-    constexpr bool MOTION = RB > 0, F64 = sizeof(T) == 8;
+    constexpr bool MOTION = RB > 0, F64 = sizeof(T) == 8, kSkip = RB > kSkipFrom;
     static_assert(CHAIN == kChainNone || !HISTORY, "chained blocks keep the final state only");
     constexpr int kRow = RB + 3;                     // mode weights, translation
     __shared__ Event<T> sev[kBlochChunk + 1];        // one more: the read ahead
@@ -387,7 +393,8 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
         }
     }
     const int all_axes = __all(finite) ? 0 : kEvAxes;  // the same for the wave
-    T e1 = 0, e2 = 0, dt_e = (T)-1;                    // decay factors (FP32: e1 is 1 - exp(-dt / T1)), their dt
+    // decay factors (FP32: e1 is 1 - exp(-dt / T1); FP64: om1 = (1 - e1) M0) and their dt
+    T e1 = 0, e2 = 0, om1 = 0, dt_e = (T)-1;
     T dt_r = (T)-1;                                    // dt of the rotation
     const int64_t n_steps = n_time > 0 ? n_time - 1 : 0;
     const int RC = R + 3;
@@ -467,7 +474,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     for (int q = 0; q < kRow; ++q) cf[q] = scoef[e * kRow + q];
             };
             auto fetched = [&]() {
-                if constexpr (!F64) {
+                {
                     asm volatile("" : "+v"(ev.rf_re), "+v"(ev.rf_im), "+v"(ev.rf2), "+v"(ev.dt), "+v"(ev.gx), "+v"(ev.gy),
                                  "+v"(ev.gz), "+v"(ev.flags));
                     if constexpr (RB > 0 && RB <= 2)
@@ -478,20 +485,23 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
             fetch();
             fetched();
             T de = 0, d = 0;  // FP64: departures of dt from that of the decay factors and of the rotation
-            bool off = false;  // either is not 0
+            bool off = false, off_e = false;  // either, the first is not 0
             // the end of a step: the next event's record, then relaxation
             auto relax = [&]() {
                 ++e;
                 fetch();  // one past the last: the spare entry, which is not a step
                 if constexpr (F64) {
-                    T f2 = e2, f1 = e1;
                     if (off) {
-                        f2 = fma(-de * invT2, e2, e2);
-                        f1 = fma(-de * invT1, e1, e1);
+                        asm volatile("");
+                        const T f2 = fma(-de * invT2, e2, e2), f1 = fma(-de * invT1, e1, e1);
+                        mxr *= f2;
+                        mxi *= f2;
+                        mz = fma(mz, f1, (1.0 - f1) * M0);
+                    } else {
+                        mxr *= e2;
+                        mxi *= e2;
+                        mz = fma(mz, e1, om1);
                     }
-                    mxr *= f2;
-                    mxi *= f2;
-                    mz = fma(mz, f1, (1.0 - f1) * M0);
                 } else {
                     mxr *= e2;
                     mxi *= e2;
@@ -511,12 +521,13 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
             auto more = [&]() {
                 const int fl = __builtin_amdgcn_readfirstlane(ev.flags);
                 if (fl < 0 || !(fl & kEvSame)) return false;
-                if constexpr (F64) {
+                if (F64 && !(fl & kEvDt)) {
                     de = ev.dt - dt_e;
                     d = ev.dt - dt_r;
                     const T m = __builtin_fabs(de) + __builtin_fabs(d);
                     off = __any(m != 0);
-                    return __all(m <= kDtNear) != 0;
+                    off_e = __any(de != 0);
+                    return __all(m <= (T)kDtNear) != 0;
                 }
                 return true;
             };
@@ -541,20 +552,27 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                 // BlochSimulator.cpp:207-214: e1/e2 only when dt changes.  dt
                 // is the same for every lane, so these are real branches.
                 if constexpr (F64) {
-                    de = ev.dt - dt_e;
-                    if (!__all(__builtin_fabs(de) <= kDtNear)) {
-                        e1 = dev_exp<T>(-ev.dt * invT1);
-                        e2 = dev_exp<T>(-ev.dt * invT2);
-                        dt_e = ev.dt;
-                        de = 0;
+                    if (!(fl & kEvDt)) {
+                        de = ev.dt - dt_e;
+                        if (!__all(__builtin_fabs(de) <= kDtNear)) {
+                            e1 = dev_exp<T>(-ev.dt * invT1);
+                            e2 = dev_exp<T>(-ev.dt * invT2);
+                            om1 = (1.0 - e1) * M0;
+                            dt_e = ev.dt;
+                            de = 0;
+                        }
+                        off_e = __any(de != 0);
                     }
                     // a run of equal steps that a chunk cuts keeps its dt
-                    d = ev.dt - dt_r;
-                    if (!((fl & kEvSame) && __all(__builtin_fabs(d) <= kDtNear))) {
+                    off = off_e;
+                    const T dr = ev.dt - dt_r;
+                    if ((fl & kEvSame) && __all(__builtin_fabs(dr) <= kDtNear)) {
+                        d = dr;
+                        off = true;
+                    } else {
                         dt_r = ev.dt;
                         d = 0;
                     }
-                    off = __any(de != 0 || d != 0);
                 } else {
                     if (!(fl & kEvDt)) {
                         e1 = one_minus_exp(-ev.dt * invT1);
@@ -582,11 +600,13 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     using X = std::integral_constant<int, 0>;
                     using Y = std::integral_constant<int, 1>;
                     using Z = std::integral_constant<int, 2>;
-                    const int axes = fl & kEvAxes;
-                    if (axes == 1) Bz = at(X{}) * ev.gx;
-                    else if (axes == 2) Bz = at(Y{}) * ev.gy;
-                    else if (axes == 4) Bz = at(Z{}) * ev.gz;
-                    else if (axes != 0) Bz = fma(at(Z{}), ev.gz, fma(at(Y{}), ev.gy, at(X{}) * ev.gx));
+                    if constexpr (kSkip) {
+                        if (fl & 1) Bz = at(X{}) * ev.gx;
+                        if (fl & 2) Bz = fma(at(Y{}), ev.gy, Bz);
+                        if (fl & 4) Bz = fma(at(Z{}), ev.gz, Bz);
+                    } else {
+                        Bz = fma(at(Z{}), ev.gz, fma(at(Y{}), ev.gy, at(X{}) * ev.gx));
+                    }
                     Bz = Bz + dB;
                 }
                 if (fl & kEvRf) {
