@@ -80,23 +80,22 @@ __device__ inline double coef_f64(double c)
 // (whole turns, then sin(pi - x) = sin x) and the Taylor series in t summed to
 // t^21 (the next term is below 2e-18): about 17 FP64 instructions, where a
 // sine and cosine pair takes about 45.
-template <bool SCALAR = false>
 __device__ inline double sin_cycles_f64(double u)
 {
     const double r = u - __builtin_rint(u);
     const double t = __builtin_fabs(r) > 0.25 ? __builtin_copysign(0.5, r) - r : r;
     const double q = t * t;
     double p = 0.0011309237482517963;
-    p = fma(p, q, coef_f64<SCALAR>(-0.012031585942120627));
-    p = fma(p, q, coef_f64<SCALAR>(0.10422916220813984));
-    p = fma(p, q, coef_f64<SCALAR>(-0.71812230177850056));
-    p = fma(p, q, coef_f64<SCALAR>(3.819952584848282));
-    p = fma(p, q, coef_f64<SCALAR>(-15.09464257682299));
-    p = fma(p, q, coef_f64<SCALAR>(42.058693944897655));
-    p = fma(p, q, coef_f64<SCALAR>(-76.705859753061389));
-    p = fma(p, q, coef_f64<SCALAR>(81.605249276075057));
-    p = fma(p, q, coef_f64<SCALAR>(-41.341702240399762));
-    p = fma(p, q, coef_f64<SCALAR>(6.2831853071795862));
+    p = fma(p, q, -0.012031585942120627);
+    p = fma(p, q, 0.10422916220813984);
+    p = fma(p, q, -0.71812230177850056);
+    p = fma(p, q, 3.819952584848282);
+    p = fma(p, q, -15.09464257682299);
+    p = fma(p, q, 42.058693944897655);
+    p = fma(p, q, -76.705859753061389);
+    p = fma(p, q, 81.605249276075057);
+    p = fma(p, q, -41.341702240399762);
+    p = fma(p, q, 6.2831853071795862);
     return t * p;
 }
 
