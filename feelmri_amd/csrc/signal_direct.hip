@@ -821,15 +821,25 @@ static int plan_analyse(fm_signal_plan *p, const double *kx, const double *ky, c
     const double avg_group = p->n_tgroups ? (double)S / (double)p->n_tgroups : 0.0;
     p->prefer_grouped = avg_group >= kGroupMin;
 
+    // Pairs and runs are found to a tolerance taken from the largest |k'| and
+    // |t|.  Where a coordinate is infinite or NaN nothing is: every sample is
+    // then summed by itself, and only those coordinates' samples are not finite.
+    double kmax = 0.0, tmax = 0.0;
+    bool finite = true;
+    for (int64_t s = 0; s < S; ++s) {
+        const double4 v = ks[(size_t)s];
+        kmax = std::max({kmax, std::fabs(v.x), std::fabs(v.y), std::fabs(v.z)});
+        tmax = std::max(tmax, std::fabs(v.w));
+        finite = finite && std::isfinite(v.x) && std::isfinite(v.y) && std::isfinite(v.z) && std::isfinite(v.w);
+    }
+
     // Conjugate pairs: in every t-group pair each sample with one whose k' is
     // its negative, to 1e-12 of the largest |k'| (an O(g^2) search per group
     // of at most 128 samples, given up at the first sample without a partner;
     // k' = 0 pairs with another k' = 0).  All groups or none.
     std::vector<int32_t> mate;  // partner of perm[i] for the first of each pair, else -1
-    double worst = 0.0, kmax = 0.0;
-    for (int64_t s = 0; s < S; ++s)
-        kmax = std::max({kmax, std::fabs(ks[(size_t)s].x), std::fabs(ks[(size_t)s].y), std::fabs(ks[(size_t)s].z)});
-    p->pairs_conj = S > 0;
+    double worst = 0.0;
+    p->pairs_conj = S > 0 && finite;
     {
         const double tol = 1e-12 * (kmax > 0.0 ? kmax : 1.0);
         std::vector<char> used;
@@ -933,12 +943,8 @@ static int plan_analyse(fm_signal_plan *p, const double *kx, const double *ky, c
     // lines * kz in the sample index) whose k' and t are linear in the
     // readout index to 1e-12 of the largest |k'| / |t|.  All runs or none.
     std::vector<RunDesc> &runs = h.runs;
-    if (n_meas >= 2 && S > 0) {
+    if (n_meas >= 2 && S > 0 && finite) {
         const int64_t stride = n_lines * n_kz;
-        double tmax = 0.0;
-        for (int64_t s = 0; s < S; ++s) {
-            tmax = std::max(tmax, std::fabs(ks[(size_t)s].w));
-        }
         const double tolk = 1e-12 * (kmax > 0.0 ? kmax : 1.0), tolt = 1e-12 * (tmax > 0.0 ? tmax : 1.0);
         bool linear = true;
         double devk = 0.0, devt = 0.0;  // largest departure from the linear model

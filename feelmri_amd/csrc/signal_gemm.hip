@@ -132,6 +132,19 @@ static PairAxis pair_axis_about(const std::vector<double> &g, int64_t n, const d
     return a;
 }
 
+// Every offset as an entity of its own, about 0.
+static PairAxis unpaired_axis(const std::vector<double> &g, int64_t n)
+{
+    PairAxis a;
+    for (int row = 0; row < 2; ++row)  // the cosines, then the sines
+        for (int64_t j = 0; j < n; ++j)
+            a.rows.insert(a.rows.end(), {g[(size_t)(3 * j)], g[(size_t)(3 * j + 1)], g[(size_t)(3 * j + 2)], row ? 0.0 : 0.25});
+    for (int64_t j = 0; j < n; ++j) a.ent.insert(a.ent.end(), {(int32_t)j, -1, (int32_t)j, (int32_t)(n + j)});
+    a.n_ent = n;
+    a.n_rows = 2 * n;
+    return a;
+}
+
 // The centre that leaves the fewest rows: the middle of the offsets (an even
 // count -n/2 .. n/2 - 1 pairs up completely about its half step), or 0 (where
 // single-precision offsets are symmetric to the last bit).
@@ -139,6 +152,10 @@ static PairAxis pair_axis(const std::vector<double> &g, int64_t n)
 {
     double mid[3] = {0.0, 0.0, 0.0};
     const double zero[3] = {0.0, 0.0, 0.0};
+    // an offset that is not finite has no partner, and no tolerance can be
+    // taken from it: no pairs, every offset with rows of its own
+    for (double v : g)
+        if (!std::isfinite(v)) return unpaired_axis(g, n);
     for (int d = 0; d < 3; ++d) {
         double lo = g[(size_t)d], hi = lo;
         for (int64_t j = 1; j < n; ++j) {
