@@ -552,7 +552,8 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                 // BlochSimulator.cpp:207-214: e1/e2 only when dt changes.  dt
                 // is the same for every lane, so these are real branches.
                 if constexpr (F64) {
-                    if (!(fl & kEvDt)) {
+                    // (a chunk begins without the departure of the one before)
+                    if (!(fl & kEvDt) || e == 0) {
                         de = ev.dt - dt_e;
                         if (!__all(__builtin_fabs(de) <= kDtNear)) {
                             e1 = dev_exp<T>(-ev.dt * invT1);

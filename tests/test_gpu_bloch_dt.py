@@ -1,0 +1,64 @@
+"""Steps whose dt departs by roundings from that of the decay factors at hand (FP64 form), against the
+same steps in 80 bits: the departure's correction holds wherever the 256-event chunks cut the table."""
+import numpy as np
+import pytest
+
+from feelmri_amd import sequences
+
+pytestmark = pytest.mark.gpu
+GAMMA = sequences.GAMMA
+LD, CLD = np.longdouble, np.clongdouble
+
+
+def _steps(r0, T1, T2, dB, rf, G, dt, mxy, mz):
+    r, x, z = r0.astype(LD), mxy.astype(CLD), mz.astype(LD)
+    with np.errstate(divide="ignore"):
+        R1, R2 = 1 / T1.astype(LD), 1 / T2.astype(LD)
+    for i in range(1, dt.size):
+        h, B = LD(dt[i]), r @ G[i].astype(LD) + dB.astype(LD)
+        q = CLD(rf[i])
+        Bn = np.maximum(np.sqrt(B * B + abs(q) ** 2), LD(1e-12))
+        th = -LD(GAMMA) * h * Bn / 2
+        a, b = np.cos(th) - 1j * (B / Bn * np.sin(th)), -1j * (q / Bn * np.sin(th))
+        nx = 2 * a.conj() * b * z + a.conj() ** 2 * x - b ** 2 * x.conj()
+        nz = (abs(a) ** 2 - abs(b) ** 2) * z - 2 * (a * b * x.conj()).real
+        e1 = np.exp(-h * R1)
+        x, z = nx * np.exp(-h * R2), nz * e1 + (1 - e1)
+    return x, z
+
+
+def _run(gpu, r0, T1, T2, dB, rf, G, dt, mxy, mz):
+    import torch
+
+    from feelmri_amd import device
+
+    nodes = device.BlochNodes.from_arrays(r0, T1, T2, dB)
+    x, z = device.bloch(nodes, device.EventTable(rf, G, dt), 1.0, GAMMA, torch.tensor(mxy, device=gpu),
+                        torch.tensor(mz, device=gpu), precision="f64")
+    return x.cpu().numpy(), z.cpu().numpy()
+
+
+def _inputs(n, T, seed=1):
+    r = np.random.default_rng(seed)
+    return (r.uniform(-0.1, 0.1, (n, 3)), r.normal(0, 1e-3, n), np.zeros(T, complex), np.zeros((T, 3)),
+            r.normal(size=n) + 1j * r.normal(size=n), r.uniform(0.2, 1.0, n))
+
+
+@pytest.mark.parametrize("shift", [0, 3, 250])
+@pytest.mark.parametrize("rf_on", [False, True])
+def test_departure_survives_the_end_of_a_chunk(gpu, shift, rf_on):
+    """dt departs by 5e-13 ms once and then stays, over the end of a chunk (step 257); T2 of 1 us make a
+    departure that is dropped worth 5e-10 a step, 1e-7 of the result.  Steps of exactly the same dt in
+    80 bits; the FP64 steps round at 1e-16 each, 300 of them: bound 1e-12."""
+    n, T = 70, 300
+    r0, dB, rf, G, mxy, mz = _inputs(n, T)
+    T1, T2 = np.full(n, 2e-3), np.full(n, 1e-3)
+    dt = np.full(T, 1e-5)
+    dt[0] = 0.0
+    dt[2 + shift:] += 5e-13
+    if rf_on:
+        rf[:] = 1e-3 * (1 + 0.5j)
+    want = _steps(r0, T1, T2, dB, rf, G, dt, mxy, mz)
+    got = _run(gpu, r0, T1, T2, dB, rf, G, dt, mxy, mz)
+    for g, w in zip(got, want):
+        assert np.linalg.norm(g - w) <= 1e-12 * np.linalg.norm(w)
