@@ -78,8 +78,10 @@ struct alignas(16) Event {
 // Event flags: axes with a gradient, RF on, rotation as the previous step's,
 // dt as the previous step's.
 constexpr int kEvAxes = 7, kEvRf = 8, kEvSame = 16, kEvDt = 32;
-// FP64: largest departure of dt (ms) that is corrected to first order.
-constexpr double kDtNear = 1e-12;
+// FP64: largest departure of dt (ms) that is corrected to first order, and the
+// largest 1/T1, 1/T2 (1/ms) of a wave that does so: the second order of the decay
+// is then below 1e-16.  (At T = 0 the rate is infinite and has no first order.)
+constexpr double kDtNear = 1e-12, kRateNear = 1e4;
 
 // FP32 form: the hardware sine/cosine, which take revolutions, after
 // reducing the argument to [-1/2, 1/2] revolution.  Their error is absolute
@@ -393,6 +395,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
         }
     }
     const int all_axes = __all(finite) ? 0 : kEvAxes;  // the same for the wave
+    const T dt_near = __all(__builtin_fabs(invT1) <= kRateNear && __builtin_fabs(invT2) <= kRateNear) ? (T)kDtNear : (T)0;
     // decay factors (FP32: e1 is 1 - exp(-dt / T1); FP64: om1 = (1 - e1) M0) and their dt
     T e1 = 0, e2 = 0, om1 = 0, dt_e = (T)-1;
     T dt_r = (T)-1;                                    // dt of the rotation
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     const T m = __builtin_fabs(de) + __builtin_fabs(d);
                     off = __any(m != 0);
                     off_e = __any(de != 0);
-                    return __all(m <= (T)kDtNear) != 0;
+                    return __all(m <= dt_near) != 0;
                 }
                 return true;
             };
@@ -555,7 +558,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     // (a chunk begins without the departure of the one before)
                     if (!(fl & kEvDt) || e == 0) {
                         de = ev.dt - dt_e;
-                        if (!__all(__builtin_fabs(de) <= kDtNear)) {
+                        if (!__all(__builtin_fabs(de) <= dt_near)) {
                             e1 = dev_exp<T>(-ev.dt * invT1);
                             e2 = dev_exp<T>(-ev.dt * invT2);
                             om1 = (1.0 - e1) * M0;
@@ -567,7 +570,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     // a run of equal steps that a chunk cuts keeps its dt
                     off = off_e;
                     const T dr = ev.dt - dt_r;
-                    if ((fl & kEvSame) && __all(__builtin_fabs(dr) <= kDtNear)) {
+                    if ((fl & kEvSame) && __all(__builtin_fabs(dr) <= dt_near)) {
                         d = dr;
                         off = true;
                     } else {

@@ -62,3 +62,25 @@ def test_departure_survives_the_end_of_a_chunk(gpu, shift, rf_on):
     got = _run(gpu, r0, T1, T2, dB, rf, G, dt, mxy, mz)
     for g, w in zip(got, want):
         assert np.linalg.norm(g - w) <= 1e-12 * np.linalg.norm(w)
+
+
+@pytest.mark.parametrize("zero", ["T1", "T2", "both", "tiny"])
+def test_nodes_that_relax_at_once(gpu, zero):
+    """T1 or T2 of 0 (or far below dt): the factor is exp(-inf) = 0 on every step, also where dt departs by
+    roundings from the step before.  Other nodes of the wave keep their values (1e-12, as above)."""
+    n, T = 70, 300
+    r0, dB, rf, G, mxy, mz = _inputs(n, T)
+    r = np.random.default_rng(3)
+    T1, T2 = r.uniform(500, 1500, n), r.uniform(40, 100, n)
+    short = 1e-9 if zero == "tiny" else 0.0
+    if zero != "T2":
+        T1[5] = short
+    if zero != "T1":
+        T2[[5, 64]] = short
+    G[:] = np.repeat(r.normal(0, 5, (T // 50, 3)), 50, 0)
+    rf[:] = 1e-3 * np.repeat(r.normal(size=T // 50), 50)
+    dt = np.diff(1000.0 + np.arange(T) * 0.01, prepend=1000.0 - 0.01)
+    want = _steps(r0, T1, T2, dB, rf, G, dt, mxy, mz)
+    got = _run(gpu, r0, T1, T2, dB, rf, G, dt, mxy, mz)
+    for g, w in zip(got, want):
+        assert np.isfinite(g).all() and np.linalg.norm(g - w) <= 1e-12 * np.linalg.norm(w)
