@@ -130,20 +130,19 @@ __device__ inline float dev_exp<float>(float x) { return __builtin_amdgcn_exp2f(
 // E1 / (1 - E1) (~200 for TR 5 ms, T1 1 s), so e1 rounded to FP32 (or 1 - e1
 // formed in FP32) would bias Mz by ~1e-5; om1 carries the recovery with full
 // FP32 relative precision.  Evaluated only when dt changes.
+// Every lane takes the form its own x asks for, so that a node's result does not
+// depend on its neighbours in the wave; the exponential runs where some lane needs it.
 __device__ inline float one_minus_exp(float x)
 {
     const double w = (double)x;
-    double p;
-    if (__all(__builtin_fabsf(x) < 1.0f / 64.0f)) {  // an event against T1: the series to w^7, within 3e-15
-        p = fma(w, 1.0 / 5040.0, 1.0 / 720.0);
-        p = fma(w, p, 1.0 / 120.0);
-        p = fma(w, p, 1.0 / 24.0);
-        p = fma(w, p, 1.0 / 6.0);
-        p = fma(w, p, 0.5);
-        p = w * fma(w, p, 1.0);
-    } else {
-        p = exp(w) - 1.0;  // loses no more than 6 of 53 bits
-    }
+    const bool small = __builtin_fabsf(x) < 1.0f / 64.0f;  // an event against T1: the series to w^7, within 3e-15
+    double p = fma(w, 1.0 / 5040.0, 1.0 / 720.0);
+    p = fma(w, p, 1.0 / 120.0);
+    p = fma(w, p, 1.0 / 24.0);
+    p = fma(w, p, 1.0 / 6.0);
+    p = fma(w, p, 0.5);
+    p = w * fma(w, p, 1.0);
+    if (!__all(small)) p = small ? p : exp(w) - 1.0;  // from 1/64 on: loses no more than 6 of 53 bits
     return (float)-p;
 }
 

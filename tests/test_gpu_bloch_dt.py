@@ -84,3 +84,30 @@ def test_nodes_that_relax_at_once(gpu, zero):
     got = _run(gpu, r0, T1, T2, dB, rf, G, dt, mxy, mz)
     for g, w in zip(got, want):
         assert np.isfinite(g).all() and np.linalg.norm(g - w) <= 1e-12 * np.linalg.norm(w)
+
+
+def test_fp32_recovery_does_not_depend_on_the_neighbours(gpu):
+    """FP32 form: 1 - exp(-dt/T1) of a node is the same number whatever T1 the other nodes of its wave
+    have, and Mz recovers by it: to 4 roundings of FP32 over 3 steps of dt/T1 = 1.3e-11."""
+    import torch
+
+    from feelmri_amd import device
+
+    n, T = 64, 4
+    r0, dB, rf, G, mxy, _ = _inputs(n, T)
+    dt = np.array([0.0, 1.3e-8, 1.3e-8, 1.3e-8])
+    mz = np.zeros(n)
+
+    def run(T1):
+        nodes = device.BlochNodes.from_arrays(r0, T1, np.full(n, 50.0), dB)
+        return device.bloch(nodes, device.EventTable(rf, G, dt), 1.0, GAMMA, torch.tensor(mxy, device=gpu),
+                            torch.tensor(mz, device=gpu), precision="f32")[1].cpu().numpy()
+
+    T1 = np.full(n, 1000.0)
+    alone = run(T1)
+    T1[7] = 1.3e-8                     # exp(-1) for this node
+    mixed = run(T1)
+    other = np.arange(n) != 7
+    assert np.array_equal(alone[other], mixed[other])
+    assert np.abs(mixed[other] / 3.9e-11 - 1.0).max() <= 4 * 2.0 ** -24
+    assert abs(mixed[7] - (1 - np.exp(-3.0))) <= 4 * 2.0 ** -24
