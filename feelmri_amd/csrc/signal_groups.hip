@@ -22,6 +22,8 @@
 // per node and encoding, and the samples are P -+ i Q.
 //
 // Phases are FP64, in cycles (k' carries the reference's float-pi factor).
+// PLANAR: every kz is 0, so z is neither staged nor multiplied; 0 z joins x where
+// it is staged, which makes a node with an infinite z what the product would (NaN).
 // FP64 form: sincos_cycles_f64.  Mixed form: one fract, FP32 hardware sine and
 // cosine, partial sums of a chunk in FP32, added into FP64.
 //
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
             }
             if constexpr (!MOTION) {
                 if (g0 == 0) {
-                    sxy[nl] = make_double2(x0, y0);
+                    sxy[nl] = make_double2(PLANAR ? fma(0.0, z0, x0) : x0, y0);
                     if (!PLANAR) sz[nl] = z0;
                 }
             } else {
@@ -209,8 +211,10 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
                     for (int q = 0; q < kB; ++q) {
                         const int g = gb + q * gstep;
                         if (g < ng) {
-                            sxy[nl * off.ps + g] = ok ? make_double2(x0 + dx[q], y0 + dy[q]) : make_double2(0.0, 0.0);
-                            if (!PLANAR) sz[nl * off.ps + g] = ok ? z0 + dz[q] : 0.0;
+                            const double x = x0 + dx[q], z = z0 + dz[q];
+                            sxy[nl * off.ps + g] =
+                                ok ? make_double2(PLANAR ? fma(0.0, z, x) : x, y0 + dy[q]) : make_double2(0.0, 0.0);
+                            if (!PLANAR) sz[nl * off.ps + g] = ok ? z : 0.0;
                         }
                     }
                 }

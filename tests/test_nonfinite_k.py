@@ -80,3 +80,37 @@ def test_other_samples_keep_their_values(kind, precision, moving):
     assert np.isnan(got[bad]).all()
     tol = 1e-12 if precision == "f64" else 2e-5
     assert np.linalg.norm(got[~bad] - want[~bad]) <= tol * np.linalg.norm(want[~bad])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("moving", [False, True])
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+@pytest.mark.parametrize("size", [20, 32])
+@pytest.mark.parametrize("paired", [False, True])
+def test_infinite_z_shows_where_kz_is_zero(size, precision, moving, paired):
+    """kz z is 0 times infinity: a node with an infinite z makes every sample NaN, in a plane too."""
+    import torch
+
+    from feelmri_amd import device
+
+    kloc, t = _random_groups(40, size)
+    kloc[2][:] = 0.0
+    if paired:
+        for k in kloc:
+            k[:, size // 2:] = -k[:, :size // 2]
+    r = np.random.default_rng(8)
+    N, R = 300, 2
+    r0 = r.uniform(-0.1, 0.1, (N, 3))
+    plan = device.SignalPlan(kloc, t, method="direct")
+    motion = None
+    if moving:
+        motion = (torch.zeros((3 * R, N), dtype=torch.float32, device=plan.device),
+                  torch.zeros((plan.n_tgroups, R + 3), dtype=torch.float64, device=plan.device))
+
+    def run():
+        nodes = device.SignalNodes.from_arrays(r0, np.zeros(N), np.full(N, 50.0), np.ones((N, 1), complex))
+        return plan.execute(nodes, precision=precision, motion=motion).cpu().numpy()
+
+    assert np.isfinite(run()).all()
+    r0[123, 2] = np.inf
+    assert np.isnan(run()).all()
