@@ -169,11 +169,11 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
             const bool ok = n < n_end;
             const double x0 = ok ? packed[n] : 0.0, y0 = ok ? packed[N + n] : 0.0, z0 = ok ? packed[2 * N + n] : 0.0;
             const double phc = (ok ? packed[3 * N + n] : 0.0) * (1.0 / kTwoPi), r2 = ok ? packed[4 * N + n] : 0.0;
-            CT br[VB], bi[VB];
+            double br[VB], bi[VB];
 #pragma unroll
             for (int v = 0; v < VB; ++v) {
-                br[v] = ok ? (CT)packed[(int64_t)(5 + 2 * (v0 + v)) * N + n] : (CT)0;
-                bi[v] = ok ? (CT)packed[(int64_t)(6 + 2 * (v0 + v)) * N + n] : (CT)0;
+                br[v] = ok ? packed[(int64_t)(5 + 2 * (v0 + v)) * N + n] : 0.0;
+                bi[v] = ok ? packed[(int64_t)(6 + 2 * (v0 + v)) * N + n] : 0.0;
             }
             if constexpr (!MOTION) {
                 if (g0 == 0) {
@@ -219,32 +219,33 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
                     }
                 }
             }
-            // b exp(-t/T2) and phi t, or c = b exp(-t/T2) exp(i phi t)   (MRI.cpp:264-271)
+            // b exp(-t/T2) and phi t, or c = b exp(-t/T2) exp(i phi t)   (MRI.cpp:264-271);
+            // products in FP64, rounded once
             for (int g = g0; g < ng; g += gstep) {
                 const double t = st[g];
                 CT d;
                 if constexpr (MIXED) d = __builtin_amdgcn_exp2f((float)(-t * r2 * 1.4426950408889634));
                 else d = exp(-t * r2);
-                CT fr = d, fi = (CT)0;
+                double fr = (double)d, fi = 0.0;
                 if constexpr (CONJ) {
                     CT so, co;
                     if constexpr (MIXED) sincos_cycles_f32(phc * t, so, co);
                     else sincos_cycles_f64(phc * t, so, co);
-                    fr = d * co;
-                    fi = d * so;
+                    fr = (double)(d * co);
+                    fi = (double)(d * so);
                 } else {
                     sph[nl * (gs | 1) + g] = -phc * t;
                 }
 #pragma unroll
                 for (int v = 0; v < VB; ++v) {
-                    CT cr = br[v] * fr, ci = bi[v] * fr;
+                    double cr = br[v] * fr, ci = bi[v] * fr;
                     if constexpr (CONJ) {
                         cr = fma(-bi[v], fi, cr);
                         ci = fma(br[v], fi, ci);
                     }
                     CT2 c;
-                    c.x = ok ? cr : (CT)0;
-                    c.y = ok ? ci : (CT)0;
+                    c.x = ok ? (CT)cr : (CT)0;
+                    c.y = ok ? (CT)ci : (CT)0;
                     sc[nl * off.cs + g * VB + v] = c;
                 }
             }
