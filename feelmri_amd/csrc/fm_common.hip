@@ -27,13 +27,15 @@ int64_t balanced_splits(int64_t N, int64_t chunk, int64_t base, int64_t s_min, i
     s_min = std::max<int64_t>(1, std::min(s_min, s_top));
     capacity = std::max<int64_t>(capacity, 1);
     int64_t best = s_min, best_cost = -1;
-    for (int64_t s = s_min; s <= std::min(2 * s_min, s_top); ++s) {
+    for (int64_t s = s_min; s <= std::min(2 * s_min, s_top);) {
         const int64_t nps = cdiv(cdiv(n, s), chunk) * chunk;
         const int64_t cost = cdiv(base * cdiv(n, nps), capacity) * nps;
         if (best_cost < 0 || cost < best_cost) {
             best = s;
             best_cost = cost;
         }
+        if (nps == chunk) break;
+        s = std::max(s + 1, cdiv(n, nps - chunk));  // the next count of fewer chunks a split
     }
     return best;
 }

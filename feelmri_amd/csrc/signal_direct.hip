@@ -614,18 +614,46 @@ static DirectLaunch direct_launch_shape(const fm_signal_plan *p, int64_t N, int 
     return {splits, nps};
 }
 
-// The t-grouped tiles' splits: whole rounds of the workgroups the device
-// holds, no more splits than the consecutive tiles (the fewest tiles) would
-// take, whose workspace the query reports.
-static DirectLaunch groups_launch_shape(const fm_signal_plan *p, bool mixed, bool motion, int64_t N, int V, int R)
+// Workspace that the t-grouped tiles may take for node splits beyond the least
+// (below the array of fm_signal_execute_noalloc).
+constexpr size_t kFineSplitBytes = size_t(32) << 20;
+
+// The t-grouped tiles' splits.  The least, which the workspace has to hold: whole
+// rounds of the workgroups the device holds, of at least 2048 nodes, no more
+// splits than the consecutive tiles (the fewest tiles) would take.  Where that
+// leaves the device idle (few tiles, small meshes) the splits are as fine as 256
+// nodes, as far as kFineSplitBytes and the workspace at hand go: tiles of many
+// groups are few, and one workgroup alone on a CU waits for its loads.
+// Mixed form, 20 011 nodes: 40 x 31 moving, 32 modes: 1.04 -> 0.13 ms (one group to
+// a slot, more tiles: 0.24); 200 x 16, 4 encodings: 0.52 -> 0.11 ms (0.31 with per-sample
+// t); 64 x 64 of one t: 0.16 -> 0.05 ms.  200 003 nodes, 200 x 17: 0.52 -> 0.40 ms.
+static DirectLaunch groups_launch_shape(const fm_signal_plan *p, bool mixed, bool motion, int64_t N, int V, int R,
+                                        size_t ws_bytes)
 {
     const int64_t most = direct_launch_shape(p, N, 0).n_splits;
     const int64_t nt = p->n_tiles_pairs;
     const int64_t capacity = (int64_t)groups_blocks_per_cu(p, mixed, motion, V, R) * device_cu_count();
-    const int64_t s_max = std::min(most, cdiv(N, 2048));
-    const int64_t splits = balanced_splits(N, kDirectThreads, nt, cdiv(capacity, nt), capacity, s_max);
-    const int64_t nps = cdiv(cdiv(N, splits), kDirectThreads) * kDirectThreads;
-    return {cdiv(N, nps), nps};
+    const size_t per_split = (size_t)p->n_samples * (size_t)V * sizeof(double2);
+    auto shape = [&](int64_t s_max) -> DirectLaunch {
+        const int64_t splits = balanced_splits(N, kDirectThreads, nt, cdiv(capacity, nt), capacity, s_max);
+        const int64_t nps = cdiv(cdiv(N, splits), kDirectThreads) * kDirectThreads;
+        return {cdiv(N, nps), nps};
+    };
+    const DirectLaunch least = shape(std::min(most, cdiv(N, 2048)));
+    const int64_t fits = (int64_t)(std::min(ws_bytes, kFineSplitBytes) / per_split);
+    if (fits <= least.n_splits) return least;
+    return shape(std::min(cdiv(N, kDirectThreads), fits));
+}
+
+// Workspace of the t-grouped tiles with the finest splits they may take
+// (balanced_splits takes at most twice its least count).
+static size_t groups_fine_workspace(const fm_signal_plan *p, int64_t N, int V)
+{
+    const size_t per_split = (size_t)p->n_samples * (size_t)V * sizeof(double2);
+    const int64_t most = 2 * cdiv(8 * (int64_t)device_cu_count(), std::max<int64_t>(p->n_tiles_pairs, 1));
+    const int64_t fits = (int64_t)(kFineSplitBytes / per_split);
+    const int64_t splits = std::min({cdiv(N, kDirectThreads), most, fits});
+    return splits > 1 ? (size_t)splits * per_split : 0;
 }
 
 template <bool MIXED>
@@ -647,10 +675,10 @@ static void launch_consec(const fm_signal_plan *p, dim3 grid, const double *pack
 static size_t direct_workspace(const fm_signal_plan *p, int64_t N, int V)
 {
     if (N <= 0 || p->n_samples == 0) return 0;
-    // the largest of the tilings' needs (the t-grouped tiles take no more
-    // splits than the consecutive ones) and of the per-line GEMM's partial
-    // samples (one encoding at a time)
-    size_t need = lines_workspace(p, N);
+    // the largest of the tilings' needs (the t-grouped tiles' least is no more
+    // than the consecutive ones') and of the per-line GEMM's partial samples
+    // (one encoding at a time)
+    size_t need = std::max(lines_workspace(p, N), groups_fine_workspace(p, N, V));
     for (int g = 0; g < 3; g += 2) {
         if (g == 2 && p->n_runs == 0) continue;
         const DirectLaunch L = direct_launch_shape(p, N, g);
@@ -678,7 +706,7 @@ static int direct_execute(const fm_signal_plan *p, int precision, int64_t N, int
     const bool use_runs = !motion && p->n_runs > 0 && (precision != FM_PREC_F64 || p->runs_exact);
     const bool grouped = motion || (!use_runs && p->prefer_grouped);
     const int tiling = use_runs ? 2 : (grouped ? 1 : 0);
-    const DirectLaunch L = grouped ? groups_launch_shape(p, precision != FM_PREC_F64, motion, N, V, R)
+    const DirectLaunch L = grouped ? groups_launch_shape(p, precision != FM_PREC_F64, motion, N, V, R, ws ? ws_bytes : 0)
                                    : direct_launch_shape(p, N, tiling);
     const size_t need = L.n_splits > 1 ? (size_t)L.n_splits * (size_t)S * (size_t)V * sizeof(double2) : 0;
     if (need > ws_bytes) {

@@ -27,8 +27,8 @@
 // FP64 form: sincos_cycles_f64.  Mixed form: one fract, FP32 hardware sine and
 // cosine, partial sums of a chunk in FP32, added into FP64.
 //
-// Bound by VALU issue.  LDS is kept small (chunks of 16 to 128 nodes) so that
-// 6 or more waves share a SIMD.  Measured, whole calls (before: tiles of two
+// Bound by VALU issue.  LDS is kept small (chunks of 16 to 128 nodes, group_chunk)
+// so that several waves share a SIMD.  Measured, whole calls (before: tiles of two
 // 256-sample slots, one group to a slot or 32, 64, 128-sample groups packed,
 // 3 waves per SIMD):
 //   spiral, 973 000 nodes, 2048 x 32, mixed: 15.07 -> 13.1 ms (the FP32 series
@@ -39,6 +39,7 @@
 //   2.67 ms;
 //   spiral, 138 519 nodes, 1504 x 48, mixed (per-sample t before): 5.49 -> 1.9 ms.
 #include <algorithm>
+#include <type_traits>
 
 #include "signal_plan.h"
 
@@ -53,7 +54,7 @@ struct GroupLds {
     int ps, cs;             // entries from node to node: positions, c
     int total;
 };
-__host__ __device__ inline GroupLds group_lds(int vb, bool mixed, bool motion, bool conj, bool planar, int chunk,
+__host__ __device__ constexpr GroupLds group_lds(int vb, bool mixed, bool motion, bool conj, bool planar, int chunk,
                                               int gs, int R)
 {
     GroupLds l{};
@@ -77,6 +78,11 @@ __host__ __device__ inline GroupLds group_lds(int vb, bool mixed, bool motion, b
     l.total = off;
     return l;
 }
+
+// The most a tile can ask for, at the fewest nodes to a chunk: 59 136 bytes.
+constexpr int kGroupChunkMin = 16, kGroupChunkMax = 128;
+static_assert(group_lds(kMaxVB, false, true, false, false, kGroupChunkMin, kGroupCap, kMaxModes).total <= 64 * 1024,
+              "the records of the fewest nodes fit the LDS of a workgroup");
 
 template <bool MIXED>
 struct GroupCT;
@@ -181,14 +187,15 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
                     if (!PLANAR) sz[nl] = z0;
                 }
             } else {
-                constexpr int kB = 4;  // groups per pass over the modes
-                for (int gb = g0; gb < ng; gb += kB * gstep) {
-                    double dx[kB], dy[kB], dz[kB];
-                    int cg[kB];
+                // one pass over the modes for B groups of the thread (gb, gb + gstep, ...)
+                auto place = [&](int gb, auto count) {
+                    constexpr int B = decltype(count)::value;
+                    double dx[B], dy[B], dz[B];
+                    int cg[B];
 #pragma unroll
-                    for (int q = 0; q < kB; ++q) {
+                    for (int q = 0; q < B; ++q) {
                         const int g = gb + q * gstep;
-                        cg[q] = (g < ng ? g : gb) * (R + 3);
+                        cg[q] = (g < ng ? g : ng - 1) * (R + 3);
                         dx[q] = scoef[cg[q] + R];
                         dy[q] = scoef[cg[q] + R + 1];
                         dz[q] = scoef[cg[q] + R + 2];
@@ -199,7 +206,7 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
                             const double my = (double)modes[(int64_t)(1 * R + r) * N + n];
                             const double mz = (double)modes[(int64_t)(2 * R + r) * N + n];
 #pragma unroll
-                            for (int q = 0; q < kB; ++q) {
+                            for (int q = 0; q < B; ++q) {
                                 const double w = scoef[cg[q] + r];
                                 dx[q] = fma(mx, w, dx[q]);
                                 dy[q] = fma(my, w, dy[q]);
@@ -208,7 +215,7 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
                         }
                     }
 #pragma unroll
-                    for (int q = 0; q < kB; ++q) {
+                    for (int q = 0; q < B; ++q) {
                         const int g = gb + q * gstep;
                         if (g < ng) {
                             const double x = x0 + dx[q], z = z0 + dz[q];
@@ -216,6 +223,19 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
                                 ok ? make_double2(PLANAR ? fma(0.0, z, x) : x, y0 + dy[q]) : make_double2(0.0, 0.0);
                             if (!PLANAR) sz[nl * off.ps + g] = ok ? z : 0.0;
                         }
+                    }
+                };
+                // the same passes for every thread of the workgroup: 4, 2 or 1 groups by what is left
+                for (int k0 = 0; k0 < ng;) {
+                    if (ng - k0 > 2 * gstep) {
+                        place(k0 + g0, std::integral_constant<int, 4>{});
+                        k0 += 4 * gstep;
+                    } else if (ng - k0 > gstep) {
+                        place(k0 + g0, std::integral_constant<int, 2>{});
+                        k0 += 2 * gstep;
+                    } else {
+                        place(k0 + g0, std::integral_constant<int, 1>{});
+                        k0 += gstep;
                     }
                 }
             }
@@ -334,12 +354,14 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
 static bool group_conj(const fm_signal_plan *p, bool mixed) { return p->pairs_conj && (mixed || p->pairs_exact); }
 
 // Nodes per chunk: the most, a power of two from 16 to 128, whose records take
-// at most 24 KB (6 workgroups of 4 waves per CU).
+// at most 24 KB (6 workgroups of 4 waves per CU).  16 where even those take
+// more: FP64 moving nodes, 4 encodings, 32 groups and modes ask for 58 KB and run 2
+// workgroups per CU.
 static int group_chunk(const fm_signal_plan *p, int vb, bool mixed, bool motion, int R)
 {
     const bool conj = group_conj(p, mixed);
-    int c = 128;
-    while (c > 16 && group_lds(vb, mixed, motion, conj, p->planar != 0, c, p->groups_per_tile, R).total > 24 * 1024) c /= 2;
+    int c = kGroupChunkMax;
+    while (c > kGroupChunkMin && group_lds(vb, mixed, motion, conj, p->planar != 0, c, p->groups_per_tile, R).total > 24 * 1024) c /= 2;
     return c;
 }
 
