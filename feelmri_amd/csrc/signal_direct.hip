@@ -515,71 +515,46 @@ __device__ inline double sum_group16(double v)
 // coalesced across the group), then the group sums its lanes in a fixed
 // butterfly, so a result does not depend on the launch.  Rows past the last
 // one work on it and write nothing.
-// Bound by the latency of three dependent loads (row, entry, x), so a group
-// takes kSpmvRows rows together, and the rows of a workgroup's XCD are one
-// range, whose part of x stays in that L2.  215 940 rows of 15, two encodings:
-// 20 us, 3.3 TB/s (42 us with a row a group, sums for four encodings through
-// LDS).
-constexpr int kSpmvRows = 4, kSpmvBlockRows = 16 * kSpmvRows;
-
+// Bound by the latency of three dependent loads (row, entry, x).  The rows of a
+// workgroup's XCD are one range, whose part of x stays in that L2.  215 940 rows
+// of 15, two encodings: 16.6 us, 4 TB/s (38.7 us with sums for four encodings
+// through LDS and the rows dealt over the XCDs).  One row a group: with four rows a
+// group their loads overlap, but a call of few or long rows leaves CUs idle (2000
+// rows of 500, one encoding: 12.8 us, 21.8 with four), and long meshes gain nothing
+// (17.1 us).  The x of all encodings is loaded before it is used: 200 000 rows of 40, four
+// encodings 205 -> 139 us.
 template <int VB>
 __global__ __launch_bounds__(256) void k_csr_spmv_c128(int64_t n_rows, int V, const int64_t *__restrict__ indptr,
                                                        const int64_t *__restrict__ indices,
                                                        const double *__restrict__ data,
                                                        const double2 *__restrict__ x, double2 *__restrict__ y)
 {
-    const int64_t r0 = xcd_range(cdiv(n_rows, kSpmvBlockRows)) * kSpmvBlockRows + threadIdx.x / 16;
+    const int64_t row = xcd_range(cdiv(n_rows, 16)) * 16 + threadIdx.x / 16;
     const int j = threadIdx.x % 16;
-    int64_t k0[kSpmvRows], k1[kSpmvRows];
-#pragma unroll
-    for (int q = 0; q < kSpmvRows; ++q) {
-        const int64_t r = r0 + 16 * q < n_rows ? r0 + 16 * q : n_rows - 1;
-        k0[q] = indptr[r] + j;
-        k1[q] = indptr[r + 1];
-    }
+    const bool live = row < n_rows;
+    const int64_t r = live ? row : n_rows - 1;
+    const int64_t k0 = indptr[r] + j, k1 = indptr[r + 1];
     for (int v0 = 0; v0 < V; v0 += VB) {
-        double re[kSpmvRows][VB], im[kSpmvRows][VB], a[kSpmvRows];
-        int64_t c[kSpmvRows];
+        double re[VB], im[VB];
 #pragma unroll
-        for (int q = 0; q < kSpmvRows; ++q) {
-            a[q] = 0.0;
-            c[q] = -1;
-            if (k0[q] < k1[q]) {
-                a[q] = data[k0[q]];
-                c[q] = indices[k0[q]];
+        for (int u = 0; u < VB; ++u) re[u] = im[u] = 0.0;
+        for (int64_t k = k0; k < k1; k += 16) {
+            const double a = data[k];
+            const double2 *xr = x + indices[k] * V + v0;
+            double2 xv[VB];  // loaded together
+#pragma unroll
+            for (int u = 0; u < VB; ++u) xv[u] = v0 + u < V ? xr[u] : make_double2(0.0, 0.0);
+#pragma unroll
+            for (int u = 0; u < VB; ++u) {
+                re[u] = fma(a, xv[u].x, re[u]);
+                im[u] = fma(a, xv[u].y, im[u]);
             }
         }
 #pragma unroll
-        for (int q = 0; q < kSpmvRows; ++q)
-#pragma unroll
-            for (int u = 0; u < VB; ++u) {
-                double2 xv = make_double2(0.0, 0.0);
-                if (c[q] >= 0 && v0 + u < V) xv = x[c[q] * V + v0 + u];
-                re[q][u] = fma(a[q], xv.x, 0.0);
-                im[q][u] = fma(a[q], xv.y, 0.0);
-            }
-#pragma unroll
-        for (int q = 0; q < kSpmvRows; ++q) {
-            for (int64_t k = k0[q] + 16; k < k1[q]; k += 16) {
-                const double ak = data[k];
-                const double2 *xr = x + indices[k] * V + v0;
-#pragma unroll
-                for (int u = 0; u < VB; ++u) {
-                    if (v0 + u < V) {
-                        re[q][u] = fma(ak, xr[u].x, re[q][u]);
-                        im[q][u] = fma(ak, xr[u].y, im[q][u]);
-                    }
-                }
-            }
+        for (int u = 0; u < VB; ++u) {
+            const double sr = sum_group16(re[u]), si = sum_group16(im[u]);
+            if (j == 0 && v0 + u < V && live) y[r * V + v0 + u] = make_double2(sr, si);
         }
-#pragma unroll
-        for (int q = 0; q < kSpmvRows; ++q)
-#pragma unroll
-            for (int u = 0; u < VB; ++u) {
-                const double sr = sum_group16(re[q][u]), si = sum_group16(im[q][u]);
-                if (j == 0 && v0 + u < V && r0 + 16 * q < n_rows)
-                    y[(r0 + 16 * q) * V + v0 + u] = make_double2(sr, si);
-            }
     }
 }
 
@@ -1362,7 +1337,7 @@ extern "C" int fm_csr_spmv_c128(int64_t n_rows, int n_enc, const int64_t *indptr
     if (n_rows == 0) return FM_OK;
     FM_CHECK_ARG(indptr && indices && data && x && y, "NULL array");
     FM_CHECK_ARG(cdiv(n_rows * 16, 256) <= 0x7fffffff, "too many rows for one launch");
-    const unsigned grid = xcd_grid(cdiv(n_rows, kSpmvBlockRows));
+    const unsigned grid = xcd_grid(cdiv(n_rows, 16));
     auto launch = [&](auto vb) {
         k_csr_spmv_c128<decltype(vb)::value><<<grid, 256, 0, as_stream(stream)>>>(
             n_rows, n_enc, indptr, indices, data, reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y));
