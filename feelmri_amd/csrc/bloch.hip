@@ -34,15 +34,27 @@
 // rotation is local to it (kept across the outer loop it was copied on every
 // path).  FP64 rotations are formed as a 3 x 3 matrix and applied in 9
 // instructions; formed and applied as (alpha, beta) products they took 45 a
-// step.  The mode loop is unrolled for 1, 2, 5, 10 or 16 modes (zero padded; it
-// was one loop of 16 with a test each), and the next event's record is read
-// from LDS in wide reads while the current one relaxes.  Bound by VALU issue.
-// 1 948 800 moving nodes, 1 mode, 11 255 events, FP32: 21.5-22.8 ms (before: 52.6);
+// step.  The next event's record is read from LDS in wide reads while the current
+// one relaxes.
+//
+// Finding out whether the next step is of the run costs a single event more than
+// forming its rotation again would (30 000 nodes, 400 events that all differ: 134
+// against 85 us in FP64, 95 against 87 in FP32), so a chunk with few like steps takes a
+// loop without runs.  Few is less than a half in FP64 (runs of 2: 92 against 85 us at
+// 30 000 nodes, 258 against 308 at 400 000) and less than a sixth in FP32 (runs of 2: 63
+// against 87 us; all different 210 against 187 at 400 000).
+//
+// Bound by VALU issue, and by the latency of one event's chain of operations where
+// the nodes do not fill the device.  The mode loop is unrolled for some mode counts
+// (it was one loop of 16 with a test each).
+// Before: one loop over the events, every rotation formed and applied as products.
+// 1 948 800 moving nodes, 1 mode, 11 255 events, FP32: 21.0-22.1 ms (before: 52.6);
 // 512 000 nodes, 33 blocks, 419 steps in all, FP64: 0.29 ms (0.929).  1000 events
-// that all differ (no runs): 512 000 nodes, FP64 1.13 ms (1.13), with RF 1.88
-// (2.17), FP32 0.63 (0.57), 1.03 (0.98); 30 000 nodes, where the latency of one
-// event counts, FP64 0.35 (0.24), FP32 0.26 (0.23); 20-event plateaus instead: 0.14
-// (0.24), 0.08 (0.23).
+// that all differ: 512 000 nodes, FP64 0.88 ms (1.10), with RF 1.63 (2.19), FP32 0.52
+// (0.56), 0.95 (1.00); 30 000 nodes, FP64 0.22 (0.23), 0.30 (0.37), FP32 0.22 (0.22), 0.29
+// (0.29); 20-event plateaus instead: 0.14 (0.23), 0.08 (0.22).  Slower than before: events
+// of which every one has another dt, FP64, 30 000 nodes, 0.35 (0.33; at 512 000 1.67
+// against 1.78).
 #include <algorithm>
 #include <type_traits>
 
@@ -123,6 +135,15 @@ __device__ inline double dev_exp<double>(double x) { return exp(x); }
 template <>
 __device__ inline float dev_exp<float>(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
+// An FP64 constant of the FP32 form's seldom taken decay update, in scalar registers:
+// left to the compiler these are hoisted into some 20 vector registers of the event
+// loop, which then spills (static nodes: 14 of 64).
+__device__ inline double seldom(double c)
+{
+    asm("" : "+s"(c));
+    return c;
+}
+
 // T1 recovery Mz' = Mz e1 + (1 - e1) M0.  FP64 form: exactly the reference's
 // expression (BlochSimulator.cpp:271).  FP32 form: Mz - om1 (Mz - M0) with
 // om1 = 1 - e1 = -expm1(x) evaluated in FP64 and rounded once.  The spoiled
@@ -131,18 +152,29 @@ __device__ inline float dev_exp<float>(float x) { return __builtin_amdgcn_exp2f(
 // formed in FP32) would bias Mz by ~1e-5; om1 carries the recovery with full
 // FP32 relative precision.  Evaluated only when dt changes.
 // Every lane takes the form its own x asks for, so that a node's result does not
-// depend on its neighbours in the wave; the exponential runs where some lane needs it.
+// depend on its neighbours in the wave.
 __device__ inline float one_minus_exp(float x)
 {
     const double w = (double)x;
     const bool small = __builtin_fabsf(x) < 1.0f / 64.0f;  // an event against T1: the series to w^7, within 3e-15
-    double p = fma(w, 1.0 / 5040.0, 1.0 / 720.0);
-    p = fma(w, p, 1.0 / 120.0);
-    p = fma(w, p, 1.0 / 24.0);
-    p = fma(w, p, 1.0 / 6.0);
+    double p = fma(w, seldom(1.0 / 5040.0), seldom(1.0 / 720.0));
+    p = fma(w, p, seldom(1.0 / 120.0));
+    p = fma(w, p, seldom(1.0 / 24.0));
+    p = fma(w, p, seldom(1.0 / 6.0));
     p = fma(w, p, 0.5);
     p = w * fma(w, p, 1.0);
-    if (!__all(small)) p = small ? p : exp(w) - 1.0;  // from 1/64 on: loses no more than 6 of 53 bits
+    if (!__all(small)) {
+        // x = n ln 2 + r, |r| <= ln 2 / 2, the series of exp(r) to r^13; exp(x) - 1
+        // loses no more than 6 of 53 bits.  0 or infinity beyond +-800.
+        const double v = w < -800.0 ? -800.0 : w > 800.0 ? 800.0 : w;
+        const double n = __builtin_rint(v * seldom(1.4426950408889634));
+        const double r = fma(-n, seldom(2.3190468138462996e-17), fma(-n, seldom(0.6931471805599453), v));
+        double e = 1.0;
+#pragma unroll
+        for (int i = 13; i > 0; --i) e = fma(r * seldom(1.0 / i), e, 1.0);
+        e = __builtin_amdgcn_ldexp(e, (int)n) - 1.0;
+        p = small ? p : e;
+    }
     return (float)-p;
 }
 
@@ -151,13 +183,14 @@ __device__ inline float one_minus_exp(float x)
 // The Mz coefficient is 1 - 2 |beta|^2, equal to |alpha|^2 - |beta|^2 for a
 // unitary (alpha, beta): in FP32 c^2 + s^2 misses 1 by up to an ulp, the same
 // way on every event of a readout.
+struct NoCoefs {};
 struct Rot32 {
     float zr, zi;      // 2 conj(alpha) beta: Mz into Mxy
     float ar, ai;      // conj(alpha)^2: Mxy into Mxy
     float br, bi;      // beta^2: conj(Mxy) into Mxy (subtracted)
     float m, abr, abi; // Mz into Mz; alpha beta: 2 Re(alpha beta conj(Mxy)) out of Mz
 };
-__device__ inline void rot_make(Rot32 &r, float Bz, float rf_re, float rf_im, float rf2, float gamma, float dt)
+__device__ inline void rot_make(Rot32 &r, float Bz, float rf_re, float rf_im, float rf2, float gamma, float dt, NoCoefs)
 {
     float Bn = __builtin_amdgcn_sqrtf(fmaf(Bz, Bz, rf2));
     if (Bn < 1e-12f) Bn = 1e-12f;
@@ -195,7 +228,7 @@ __device__ inline void rot_apply(const Rot32 &r, bool, float, float &mxr, float 
 struct Pre32 {
     float s, c;
 };
-__device__ inline void pre_make(Pre32 &r, float Bz, float gamma, float dt)
+__device__ inline void pre_make(Pre32 &r, float Bz, float gamma, float dt, NoCoefs)
 {
     sincos_f32(-gamma * dt * Bz, &r.s, &r.c);
 }
@@ -234,14 +267,15 @@ __device__ inline double cycles_f64(double B, double gamma, double dt)
     const double u = -dt * B;
     return fma(u, hi, u * lo);
 }
-__device__ inline void rot_make(Rot64 &r, double Bz, double rf_re, double rf_im, double rf2, double gamma, double dt)
+__device__ inline void rot_make(Rot64 &r, double Bz, double rf_re, double rf_im, double rf2, double gamma, double dt,
+                                const TrigCoefs &trig)
 {
     const double B2 = fma(Bz, Bz, rf2);
     const double B2c = B2 < 1e-24 ? 1e-24 : B2;  // |B| floored at 1e-12
     const double inv = rsqrt_f64(B2c), B0 = B2c * inv;
     const double Bn = fma(0.5 * inv, fma(-B0, B0, B2c), B0);
     double sh, ch;
-    sincos_cycles_f64<true>(0.5 * cycles_f64(Bn, gamma, dt), sh, ch);  // of the half angle
+    sincos_cycles_f64(0.5 * cycles_f64(Bn, gamma, dt), sh, ch, trig);  // of the half angle
     const double x = rf_re * inv, y = rf_im * inv, z = Bz * inv;
     r.nx = x;
     r.ny = y;
@@ -278,9 +312,9 @@ __device__ inline void rot_apply(const Rot64 &r, bool off, double d, double &mxr
 struct Pre64 {
     double s, c, om;
 };
-__device__ inline void pre_make(Pre64 &r, double Bz, double gamma, double dt)
+__device__ inline void pre_make(Pre64 &r, double Bz, double gamma, double dt, const TrigCoefs &trig)
 {
-    sincos_cycles_f64<true>(cycles_f64(Bz, gamma, dt), r.s, r.c);
+    sincos_cycles_f64(cycles_f64(Bz, gamma, dt), r.s, r.c, trig);
     r.om = -gamma * Bz;
 }
 __device__ inline void pre_apply(const Pre64 &r, bool off, double d, double &mxr, double &mxi)
@@ -321,18 +355,24 @@ constexpr int kChainNone = 0, kChainHost = 1, kChainMarks = 2;
 // Modes above which a gradient axis that is off is skipped.
 constexpr int kSkipFrom = 2;
 
-// Waves per SIMD: one event is a chain of dependent operations, so waves that
-// overlap it are worth the few registers spilled on the paths seldom taken.
-// The moving FP32 sequence above: 26.9 ms at 5, 24.4 at 6, 22.5 at 8.  512 000
-// static nodes, FP64, 1000 events that all differ: 1.20 ms at 4, 1.13 at 5.
-constexpr int bloch_waves(bool f64, int RB)
+// Waves per SIMD: one event is a chain of dependent operations that waves overlap,
+// until registers spill.  400 events that all differ, with one wave fewer and one
+// more (us, 200 000 nodes unless named):
+//   FP64, static  192, 195, 196; 800 000 nodes 559, 551, 544; chained blocks spill 22
+//                 registers at 5 (33 blocks: 0.297 ms at 5, 0.291 at 4);
+//   FP64, 1 mode  222, 221, 224;  2 modes 256, 233, 236;  5 modes 290, 269 (3, 4 waves);
+//   FP64, 10      392, 358, 391;  16 445, 445, 445;
+//   FP32, 1 mode  139, 137;  2 modes 144, 144 (7, 8: the most there are);
+//   FP32, 5       174, 173, 171 and 800 000 nodes 453, 455, 434;
+//   FP32, 10      210, 209, 210;  16 249, 245, 264.
+constexpr int bloch_waves(bool f64, int RB, bool chain)
 {
-    return f64 ? (RB == 0 ? 5 : RB <= 2 ? 4 : RB <= 10 ? 3 : 2) : (RB <= 2 ? 8 : RB <= 5 ? 6 : 4);
+    return f64 ? (RB == 0 && !chain ? 5 : RB <= 5 ? 4 : RB <= 10 ? 3 : 2) : (RB <= 2 ? 8 : RB <= 5 ? 7 : 4);
 }
 
 // RB: modes per component, 0 for static nodes (R <= RB; the rest are zero).
 template <typename T, int RB, bool HISTORY, int CHAIN = kChainNone>
-__global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) void k_bloch(
+__global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB, CHAIN != kChainNone)) void k_bloch(
     const double *__restrict__ packed, int64_t N, int64_t n_time, double M0d, double gammad,
     const double *__restrict__ rf, const double *__restrict__ G, const double *__restrict__ dt,
     const double *mxy_in, const double *mz_in,  // may alias mxy_fin / mz_fin
@@ -349,6 +389,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
     constexpr int kRow = RB + 3;                     // mode weights, translation
     __shared__ Event<T> sev[kBlochChunk + 1];        // one more: the read ahead
     __shared__ T scoef[MOTION ? (kBlochChunk + 1) * kRow : 1];
+    __shared__ int slike[kBlochThreads / 64];
     if constexpr (CHAIN == kChainMarks) {
         // the event count is produced on the device; n_time is the capacity
         const int64_t ne = *n_events;
@@ -359,6 +400,8 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
     const int64_t p = (int64_t)blockIdx.x * kBlochThreads + tid;
     const bool active = p < N;
     const T M0 = (T)M0d, gamma = (T)gammad;
+    std::conditional_t<F64, TrigCoefs, NoCoefs> trig;
+    if constexpr (F64) trig = scalar_trig_coefs();
 
     T pos[3] = {0, 0, 0}, invT1 = 0, invT2 = 0, dB = 0;
     T mxr = 0, mxi = 0, mz = 0;
@@ -402,8 +445,10 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
     const int RC = R + 3;
     if (tid == 0) sev[kBlochChunk].flags = 0;
 
+    int64_t kept = p + N;                              // HISTORY: where the next state goes
     for (int64_t base = 0; base < n_steps; base += kBlochChunk) {
         __syncthreads();
+        bool like;  // a step like the one before
         {
             const int64_t i = base + tid;  // step i uses event i + 1
             Event<T> ev;
@@ -411,6 +456,9 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
             if (i < n_steps) {
                 const double rr = rf[2 * (i + 1)], ri = rf[2 * (i + 1) + 1];
                 const double g0 = G[3 * (i + 1)], g1 = G[3 * (i + 1) + 1], g2 = G[3 * (i + 1) + 2];
+                // the event before, loaded with it (one wait for both)
+                const double pr = rf[2 * i], pi = rf[2 * i + 1], p0 = G[3 * i], p1 = G[3 * i + 1], p2 = G[3 * i + 2];
+                const T pdt = (T)dt[i];
                 ev.rf_re = (T)rr;
                 ev.rf_im = (T)ri;
                 ev.rf2 = ev.rf_re * ev.rf_re + ev.rf_im * ev.rf_im;
@@ -441,10 +489,9 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     mk = starts(i + 1);
                     prev_step = prev_step && starts(i) == 0;
                 }
-                if (prev_step && (T)dt[i] == ev.dt) fl |= kEvDt;
-                if (prev_step && (F64 || (fl & kEvDt)) && (!MOTION || (fl & kEvAxes) == 0) && rf[2 * i] == rr &&
-                    rf[2 * i + 1] == ri && G[3 * i] == g0 && G[3 * i + 1] == g1 && G[3 * i + 2] == g2)
-                    fl |= kEvSame;
+                if (prev_step & (pdt == ev.dt)) fl |= kEvDt;
+                const bool same = (pr == rr) & (pi == ri) & (p0 == g0) & (p1 == g1) & (p2 == g2);
+                if (prev_step & same & (F64 || (fl & kEvDt)) & (!MOTION || (fl & kEvAxes) == 0)) fl |= kEvSame;
             } else {
                 ev.rf_re = ev.rf_im = ev.rf2 = ev.gx = ev.gy = ev.gz = ev.dt = 0;
             }
@@ -461,10 +508,139 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
             }
             ev.flags = mk != 0 ? -mk : fl;
             sev[tid] = ev;
+            like = mk == 0 && (fl & kEvSame);
+        }
+        {   // how many of the chunk's steps are like the one before: a wave's count each
+            const int wave_like = __builtin_popcountll(__ballot(like));
+            if (tid % 64 == 0) slike[tid / 64] = wave_like;
         }
         __syncthreads();
+        int n_like = 0;
+#pragma unroll
+        for (int w = 0; w < kBlochThreads / 64; ++w) n_like += slike[w];
+        n_like = __builtin_amdgcn_readfirstlane(n_like);
         const int cnt = (n_steps - base < kBlochChunk) ? (int)(n_steps - base) : kBlochChunk;
-        if (active) {
+        // field along z: rounded as the sum over all three axes would be
+        auto field = [&](const Event<T> &ev, int fl, const T *w) {
+#pragma clang fp contract(off)
+            auto at = [&](auto axis) {
+                constexpr int c = decltype(axis)::value;
+                T q = pos[c];
+                if constexpr (MOTION) {
+                    T dq = w[RB + c];
+#pragma unroll
+                    for (int r = 0; r < RB; ++r) dq = fma((T)md[c * RB + r], w[r], dq);
+                    q += dq;
+                }
+                return q;
+            };
+            using X = std::integral_constant<int, 0>;
+            using Y = std::integral_constant<int, 1>;
+            using Z = std::integral_constant<int, 2>;
+            T Bz = 0;
+            if (!kSkip || (fl & kEvAxes) == kEvAxes) {
+                Bz = fma(at(Z{}), ev.gz, fma(at(Y{}), ev.gy, at(X{}) * ev.gx));
+            } else {  // only the axes that are on
+                if (fl & 1) Bz = at(X{}) * ev.gx;
+                if (fl & 2) Bz = fma(at(Y{}), ev.gy, Bz);
+                if (fl & 4) Bz = fma(at(Z{}), ev.gz, Bz);
+            }
+            return Bz + dB;
+        };
+        // a block ends at an event whose flags are the negated mark (the same for every lane)
+        auto block_end = [&](int mk) {
+            const int col = ((mk - 1) >> 1) - 1;
+            if (col >= 0 && (CHAIN == kChainHost || col < n_store)) {
+                store_xy[p + col * N] = make_float2((float)mxr, (float)mxi);
+                store_z[p + col * N] = (float)mz;
+            }
+            if ((mk - 1) & 1) mxr = mxi = 0;
+        };
+        auto keep = [&]() {  // the state after one more event
+            if constexpr (HISTORY) {
+                C2 v;
+                v.x = mxr;
+                v.y = mxi;
+                mxy_out[kept] = v;
+                mz_out[kept] = mz;
+                kept += N;
+            }
+        };
+        if (active && n_like * (F64 ? 2 : 6) < cnt) {
+            // few like steps: every event by itself
+            T de = 0;
+            bool off_e = false;
+            auto step = [&](int e, const Event<T> &ev) {
+                const int flags = __builtin_amdgcn_readfirstlane(ev.flags);
+                if constexpr (CHAIN != kChainNone) {
+                    if (flags < 0) {
+                        block_end(-flags);
+                        return;
+                    }
+                }
+                const int fl = flags | all_axes;
+                if constexpr (F64) {
+                    if (!(fl & kEvDt) || e == 0) {
+                        de = ev.dt - dt_e;
+                        if (!__all(__builtin_fabs(de) <= dt_near)) {
+                            e1 = dev_exp<T>(-ev.dt * invT1);
+                            e2 = dev_exp<T>(-ev.dt * invT2);
+                            om1 = (1.0 - e1) * M0;
+                            dt_e = ev.dt;
+                            de = 0;
+                            off_e = false;
+                        } else {
+                            off_e = __any(de != 0);
+                        }
+                    }
+                } else if (!(fl & kEvDt)) {
+                    e1 = one_minus_exp(-ev.dt * invT1);
+                    e2 = dev_exp<T>(-ev.dt * invT2);
+                }
+                const T Bz = field(ev, fl, &scoef[MOTION ? e * kRow : 0]);
+                if (fl & kEvRf) {
+                    typename Cplx2<T>::Rot rot;
+                    rot_make(rot, Bz, ev.rf_re, ev.rf_im, ev.rf2, gamma, ev.dt, trig);
+                    rot_apply(rot, false, (T)0, mxr, mxi, mz);
+                } else {
+                    typename Cplx2<T>::Pre pre;
+                    pre_make(pre, Bz, gamma, ev.dt, trig);
+                    pre_apply(pre, false, (T)0, mxr, mxi);
+                }
+                if constexpr (F64) {
+                    if (off_e) {
+                        asm volatile("");
+                        const T f2 = fma(-de * invT2, e2, e2), f1 = fma(-de * invT1, e1, e1);
+                        mxr *= f2;
+                        mxi *= f2;
+                        mz = fma(mz, f1, (1.0 - f1) * M0);
+                    } else {
+                        mxr *= e2;
+                        mxi *= e2;
+                        mz = fma(mz, e1, om1);
+                    }
+                } else {
+                    mxr *= e2;
+                    mxi *= e2;
+                    mz = mz - e1 * (mz - M0);
+                }
+                keep();
+            };
+            if constexpr (F64 || HISTORY) {
+                for (int e = 0; e < cnt; ++e) {
+                    const Event<T> a = sev[e];
+                    step(e, a);
+                }
+            } else {
+                // two events read at a time: the second's latency passes behind the first's step
+                for (int e = 0; e < cnt; e += 2) {
+                    const Event<T> a = sev[e], b = sev[e + 1];
+                    asm volatile("");
+                    step(e, a);
+                    if (e + 1 < cnt) step(e + 1, b);
+                }
+            }
+        } else if (active) {
             int e = 0;
             Event<T> ev;
             T cf[RB > 0 && RB <= 2 ? kRow : 1];
@@ -510,14 +686,7 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     mz = mz - e1 * (mz - M0);
                 }
                 fetched();
-                if (HISTORY) {
-                    const int64_t o = p + (base + e) * N;
-                    C2 v;
-                    v.x = mxr;
-                    v.y = mxi;
-                    mxy_out[o] = v;
-                    mz_out[o] = mz;
-                }
+                keep();
             };
             // the next step has the rotation and decay at hand
             auto more = [&]() {
@@ -537,14 +706,8 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                 const int flags = __builtin_amdgcn_readfirstlane(ev.flags);
                 const int fl = flags | all_axes;
                 if constexpr (CHAIN != kChainNone) {
-                    if (flags < 0) {  // the same for every lane: a block ends here
-                        const int mk = -flags;
-                        const int col = ((mk - 1) >> 1) - 1;
-                        if (col >= 0 && (CHAIN == kChainHost || col < n_store)) {
-                            store_xy[p + col * N] = make_float2((float)mxr, (float)mxi);
-                            store_z[p + col * N] = (float)mz;
-                        }
-                        if ((mk - 1) & 1) mxr = mxi = 0;
+                    if (flags < 0) {
+                        block_end(-flags);
                         ++e;
                         fetch();
                         fetched();
@@ -563,8 +726,10 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                             om1 = (1.0 - e1) * M0;
                             dt_e = ev.dt;
                             de = 0;
+                            off_e = false;
+                        } else {
+                            off_e = __any(de != 0);
                         }
-                        off_e = __any(de != 0);
                     }
                     // a run of equal steps that a chunk cuts keeps its dt
                     off = off_e;
@@ -583,45 +748,17 @@ __global__ __launch_bounds__(kBlochThreads, bloch_waves(sizeof(T) == 8, RB)) voi
                     }
                     dt_r = ev.dt;
                 }
-                T Bz = 0;
-                {
-#pragma clang fp contract(off)
-                    // field along z: only the axes that are on; rounded as the
-                    // sum over all three would be
-                    const T *w = RB > 0 && RB <= 2 ? cf : &scoef[MOTION ? e * kRow : 0];
-                    auto at = [&](auto axis) {
-                        constexpr int c = decltype(axis)::value;
-                        T q = pos[c];
-                        if constexpr (MOTION) {
-                            T dq = w[RB + c];
-#pragma unroll
-                            for (int r = 0; r < RB; ++r) dq = fma((T)md[c * RB + r], w[r], dq);
-                            q += dq;
-                        }
-                        return q;
-                    };
-                    using X = std::integral_constant<int, 0>;
-                    using Y = std::integral_constant<int, 1>;
-                    using Z = std::integral_constant<int, 2>;
-                    if constexpr (kSkip) {
-                        if (fl & 1) Bz = at(X{}) * ev.gx;
-                        if (fl & 2) Bz = fma(at(Y{}), ev.gy, Bz);
-                        if (fl & 4) Bz = fma(at(Z{}), ev.gz, Bz);
-                    } else {
-                        Bz = fma(at(Z{}), ev.gz, fma(at(Y{}), ev.gy, at(X{}) * ev.gx));
-                    }
-                    Bz = Bz + dB;
-                }
+                const T Bz = field(ev, fl, RB > 0 && RB <= 2 ? cf : &scoef[MOTION ? e * kRow : 0]);
                 if (fl & kEvRf) {
                     typename Cplx2<T>::Rot rot;
-                    rot_make(rot, Bz, ev.rf_re, ev.rf_im, ev.rf2, gamma, dt_r);
+                    rot_make(rot, Bz, ev.rf_re, ev.rf_im, ev.rf2, gamma, dt_r, trig);
                     do {
                         rot_apply(rot, off, d, mxr, mxi, mz);
                         relax();
                     } while (more());
                 } else {  // the precession leaves Mz alone
                     typename Cplx2<T>::Pre pre;
-                    pre_make(pre, Bz, gamma, dt_r);
+                    pre_make(pre, Bz, gamma, dt_r, trig);
                     do {
                         pre_apply(pre, off, d, mxr, mxi);
                         relax();
@@ -677,7 +814,12 @@ __global__ void k_store_spoil(int64_t N, double2 *__restrict__ mxy, const double
     if (spoil) mxy[n] = make_double2(0.0, 0.0);
 }
 
-// Instantiated mode counts: the smallest that holds R.
+// Instantiated mode counts: the smallest that holds R.  The counts between run the
+// next one's zero modes too, which costs less than the tests of a loop over them did:
+// 1000 events, 300 000 nodes, FP64, 3 modes (as 5) 0.82 ms (1.63 before), 6 (as 10) 1.05
+// (1.95), 11 (as 16) 1.39 (2.45); FP32 0.49 (1.07), 0.60 (1.28), 0.81 (1.64).  More
+// counts would save up to a third of that and cost a kernel for each of the
+// six forms.
 #define FM_BLOCH_MODES(R, CALL)             \
     do {                                    \
         if ((R) <= 0) CALL(0);              \

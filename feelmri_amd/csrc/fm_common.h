@@ -64,18 +64,6 @@ __device__ inline int64_t xcd_range(int64_t n_ranges)
 
 inline unsigned xcd_grid(int64_t n_ranges) { return (unsigned)(((n_ranges + 7) / 8) * 8); }
 
-// A coefficient of a series, for SCALAR in scalar registers: the compiler keeps
-// those of a loop in vector registers, 30 or more of them.  Where registers
-// bound the waves that pays (Bloch, FP64: 128 with 19 spilled -> 121 with none,
-// 0.367 -> 0.345 ms for the sequence named there); where they do not it
-// costs (spiral, FP64: 3.03 -> 3.32 ms; radial runs 0.94 -> 1.08 ms).
-template <bool SCALAR>
-__device__ inline double coef_f64(double c)
-{
-    if (SCALAR) asm("" : "+s"(c));
-    return c;
-}
-
 // sin 2 pi u in FP64, u in cycles.  u is reduced exactly to t in [-1/4, 1/4]
 // (whole turns, then sin(pi - x) = sin x) and the Taylor series in t summed to
 // t^21 (the next term is below 2e-18): about 17 FP64 instructions, where a
@@ -99,35 +87,48 @@ __device__ inline double sin_cycles_f64(double u)
     return t * p;
 }
 
+// Coefficients of the series below, in t: s t + s[7] t^3 + ... and 1 + c[7] t^2 + ...
+struct TrigCoefs {
+    double s[9] = {0.10422916220813984, -0.71812230177850056, 3.819952584848282,   -15.09464257682299, 42.058693944897655,
+                   -76.705859753061389, 81.605249276075057,   -41.341702240399762, 6.2831853071795862};
+    double c[8] = {0.28200596845579123, -1.714390711088672,  7.9035363713184692, -26.426256783374399,
+                   60.244641371876661,  -85.456817206693728, 64.939394022668296, -19.739208802178716};
+};
+// The same held in scalar registers: the compiler keeps the constants of a loop in
+// vector registers, 30 or more of them.  Where registers bound the waves that pays
+// (Bloch, FP64: 128 with 19 spilled -> 121 with none, 0.367 -> 0.345 ms for the
+// sequence named there); where they do not it costs (spiral, FP64: 3.03 -> 3.32 ms;
+// radial runs 0.94 -> 1.08 ms).  Formed once, before the loop: an operand pinned in
+// the loop is copied before each use, which one wave alone on a SIMD waits for.
+__device__ inline TrigCoefs scalar_trig_coefs()
+{
+    TrigCoefs k;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) asm volatile("" : "+s"(k.s[i]));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) asm volatile("" : "+s"(k.c[i]));
+    return k;
+}
+
 // sin and cos of 2 pi u in FP64, u in cycles: u reduced exactly to t in
 // [-1/8, 1/8] and the octant's quarter turn, both Taylor series summed to t^17
 // and t^16 (the next terms are below 3e-18), swapped and signed by the quarter.
 // About 35 instructions, where the library's sincospi takes about 55.
-template <bool SCALAR = false>
-__device__ inline void sincos_cycles_f64(double u, double &s, double &c)
+__device__ inline void sincos_cycles_f64(double u, double &s, double &c, const TrigCoefs &k = TrigCoefs())
 {
     const double r = u - __builtin_rint(u);
     const double q = __builtin_rint(4.0 * r);
     const double t = fma(-0.25, q, r);
     const int iq = (int)q;
     const double w = t * t;
-    double ps = coef_f64<SCALAR>(0.10422916220813984), pc = coef_f64<SCALAR>(0.28200596845579123);
-    ps = fma(ps, w, coef_f64<SCALAR>(-0.71812230177850056));
-    pc = fma(pc, w, coef_f64<SCALAR>(-1.714390711088672));
-    ps = fma(ps, w, coef_f64<SCALAR>(3.819952584848282));
-    pc = fma(pc, w, coef_f64<SCALAR>(7.9035363713184692));
-    ps = fma(ps, w, coef_f64<SCALAR>(-15.09464257682299));
-    pc = fma(pc, w, coef_f64<SCALAR>(-26.426256783374399));
-    ps = fma(ps, w, coef_f64<SCALAR>(42.058693944897655));
-    pc = fma(pc, w, coef_f64<SCALAR>(60.244641371876661));
-    ps = fma(ps, w, coef_f64<SCALAR>(-76.705859753061389));
-    pc = fma(pc, w, coef_f64<SCALAR>(-85.456817206693728));
-    ps = fma(ps, w, coef_f64<SCALAR>(81.605249276075057));
-    pc = fma(pc, w, coef_f64<SCALAR>(64.939394022668296));
-    ps = fma(ps, w, coef_f64<SCALAR>(-41.341702240399762));
-    pc = fma(pc, w, coef_f64<SCALAR>(-19.739208802178716));
-    ps = fma(ps, w, coef_f64<SCALAR>(6.2831853071795862));
-    pc = fma(pc, w, 1);
+    double ps = k.s[0], pc = k.c[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+        ps = fma(ps, w, k.s[i]);
+        pc = fma(pc, w, k.c[i]);
+    }
+    ps = fma(ps, w, k.s[8]);
+    pc = fma(pc, w, 1.0);
     ps *= t;
     const bool odd = iq & 1;
     const unsigned long long ss = (unsigned long long)(iq & 2) << 62, sc = (unsigned long long)((iq + 1) & 2) << 62;

@@ -10,12 +10,13 @@ GAMMA = sequences.GAMMA
 LD, CLD = np.longdouble, np.clongdouble
 
 
-def _steps(r0, T1, T2, dB, rf, G, dt, mxy, mz):
+def _steps(r0, T1, T2, dB, rf, G, dt, mxy, mz, disp=None):
     r, x, z = r0.astype(LD), mxy.astype(CLD), mz.astype(LD)
     with np.errstate(divide="ignore"):
         R1, R2 = 1 / T1.astype(LD), 1 / T2.astype(LD)
     for i in range(1, dt.size):
-        h, B = LD(dt[i]), r @ G[i].astype(LD) + dB.astype(LD)
+        h = LD(dt[i])
+        B = (r if disp is None else r + disp[i - 1].astype(LD)) @ G[i].astype(LD) + dB.astype(LD)
         q = CLD(rf[i])
         Bn = np.maximum(np.sqrt(B * B + abs(q) ** 2), LD(1e-12))
         th = -LD(GAMMA) * h * Bn / 2
@@ -111,3 +112,51 @@ def test_fp32_recovery_does_not_depend_on_the_neighbours(gpu):
     assert np.array_equal(alone[other], mixed[other])
     assert np.abs(mixed[other] / 3.9e-11 - 1.0).max() <= 4 * 2.0 ** -24
     assert abs(mixed[7] - (1 - np.exp(-3.0))) <= 4 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("R", [0, 1, 3])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("order", [(0, 128, 255), (255, 0, 64), (42, 43, 127), (128, 129, 0)])
+def test_chunks_with_few_and_many_like_steps(gpu, order, precision, R):
+    """Three chunks of 256 steps of which order[i] repeat the step before, spread over the chunk: the loop
+    for single events and the one for runs follow each other in every order and carry dt, its departure
+    and the state over.  FP64: 768 steps of up to 40 rad each in 80 bits, whose angle rounds at 40 x 1.1e-16 a
+    step: 768 x 5e-15 = 4e-12.  FP32: 4 times the error of the same steps in plain FP32."""
+    import torch
+
+    from feelmri_amd import device
+    from test_gpu_bloch_runs import _plain_f32
+
+    n, T = 70, 769
+    r0, dB, rf, G, mxy, mz = _inputs(n, T)
+    r = np.random.default_rng(sum(order))
+    T1, T2 = r.uniform(500, 1500, n), r.uniform(40, 100, n)
+    like = np.zeros(T, bool)
+    for c, k in enumerate(order):
+        like[1 + 256 * c + np.sort(r.permutation(256)[:k])] = True
+    like[1] = False
+    dt = np.zeros(T)
+    for i in range(1, T):
+        if like[i]:
+            rf[i], G[i], dt[i] = rf[i - 1], G[i - 1], dt[i - 1] + r.choice([0.0, 2e-15, -1e-13])
+        else:
+            rf[i] = r.choice([0.0, 1e-4]) * (r.normal() + 1j * r.normal())
+            G[i] = r.normal(0, 5, 3) * (r.random(3) < 0.7) * (R == 0 or i % 3 == 0)
+            dt[i] = r.choice([0.01, 0.01 + 1e-14, 0.004])
+    motion, disp = None, None
+    if R:
+        modes = r.normal(0, 1e-3, (3 * R, n)).astype(np.float32)
+        coef = np.concatenate([r.normal(size=(T - 1, R)), np.zeros((T - 1, 3))], axis=1)
+        motion = (torch.tensor(modes, device=gpu), torch.tensor(coef, device=gpu))
+        disp = np.einsum("crn,tr->tnc", modes.astype(float).reshape(3, R, n), coef[:, :R])
+    nodes = device.BlochNodes.from_arrays(r0, T1, T2, dB)
+    x, z = device.bloch(nodes, device.EventTable(rf, G, dt), 1.0, GAMMA, torch.tensor(mxy, device=gpu),
+                        torch.tensor(mz, device=gpu), precision=precision, motion=motion)
+    got = np.concatenate([x.cpu().numpy(), z.cpu().numpy()])
+    want = np.concatenate(_steps(r0, T1, T2, dB, rf, G, dt, mxy, mz, disp))
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    if precision == "f64":
+        assert err <= 4e-12
+    else:
+        plain = np.concatenate(_plain_f32(r0, T1, T2, dB, 1.0, rf, G, dt, mxy, mz, disp))
+        assert err <= 4 * np.linalg.norm(plain - want) / np.linalg.norm(want)
