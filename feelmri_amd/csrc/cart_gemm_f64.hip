@@ -22,9 +22,10 @@ namespace fm {
 // k-step instead of 4.  Up to 8 row blocks then share a column operand (RB = 8:
 // 128 accumulator registers, as RB = 4 needs for E's two planes and their
 // products).  150 001 nodes, 125 x 127 x 31, whole call:
-// 5.94 ms against 11.69 ms with complex rows (99 against 50 TFLOP/s of 8 flops
-// per node * sample), error against 64 bits 6.4e-15 against 4.7e-15 (both at
-// the rounding of the phases).  Bound by the FP64 MFMAs.
+// 5.93 ms against 11.69 ms with complex rows (99 against 50 TFLOP/s of 8 flops
+// per node * sample); 300 nodes, 61 x 63 x 5, error against the sums in 80 bits 1.3e-15
+// against 2.1e-15 (the offsets and phases of real rows are held beyond a double).
+// Bound by the FP64 MFMAs.
 template <int CHUNKS>
 __device__ inline void stage_E64_to_lds(const double *__restrict__ src, double *dst, int wave, int lane)
 {

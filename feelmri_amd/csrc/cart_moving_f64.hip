@@ -26,8 +26,9 @@
 // cart_moving_pairs_bf16.hip): A is one sine per row and node, B the kz row
 // times c_i (two products per entry), and a k-step takes 2 MFMAs per column
 // block: Re += A Re B, Im += A Im B.  150 001 nodes, 63 x 65 x 17, 3
-// encodings, 6 modes: 6.15 ms against 13.1 ms with complex rows, error against
-// 64 bits 1.7e-15 against 1.6e-15.  Real rows need few enough registers for 3
+// encodings, 6 modes: 6.27 ms against 13.1 ms with complex rows (6.15 with phases
+// rounded as products); 300 nodes, 9 x 65 x 17, error against the sums in 80 bits
+// 1.9e-15 against 2.2e-15.  Real rows need few enough registers for 3
 // waves per SIMD up to 4 column blocks: 6.15 ms against 7.28 ms with 2 (MFMA 41 %
 // busy, the waves waiting at the step barriers).
 // FP64 accumulators need no bound on the split length; node splits exist for
@@ -49,12 +50,14 @@ __device__ inline void cis_neg_f64(double u, double &c, double &s)
 // kz rows of the kz-factor buffer: 16 nodes + 1 entry of pad
 constexpr int kEz64Stride = 17;
 
-// G and H: line and kz offsets (3 a row), REAL: real rows (4 a row).
+// G and H: line and kz offsets (3 a row), REAL: real rows (4 a row); F_lo, G_lo and
+// H_lo: their second doubles (REAL only).
 template <int W, int CB, bool REAL>
 __global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving_f64(
     const double *__restrict__ packed, int64_t N, int V, const float *__restrict__ modes, int R,
     const double *__restrict__ mcoef, const int32_t *__restrict__ ro_group, const double *__restrict__ F,
-    const double *__restrict__ G, const double *__restrict__ H, const double *__restrict__ tr, int64_t M,
+    const double *__restrict__ F_lo, const double *__restrict__ G, const double *__restrict__ G_lo,
+    const double *__restrict__ H, const double *__restrict__ H_lo, const double *__restrict__ tr, int64_t M,
     int64_t L, int64_t K, int64_t n_rt, int64_t n_ct, int64_t n_splits, int64_t nodes_per_split, int ez_rows,
     double2 *__restrict__ part)
 {
@@ -100,7 +103,8 @@ __global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving
     const bool row_ok = row < L;
     constexpr int kG = REAL ? 4 : 3;
     const double Gx = row_ok ? G[kG * row] : 0.0, Gy = row_ok ? G[kG * row + 1] : 0.0,
-                 Gz = row_ok ? G[kG * row + (REAL ? 3 : 2)] : 0.0;  // REAL: the quarter turn
+                 Gz = row_ok ? G[kG * row + (REAL ? 3 : 2)] : 0.0,  // REAL: the quarter turn
+                 Gl = REAL && row_ok ? G_lo[kG * row + 1] : 0.0;
 
     // the column tile's kz rows
     const int64_t c0 = ct * kCols;
@@ -108,7 +112,10 @@ __global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving
     const int64_t kmax = std::min<int64_t>(K - 1, (c0 + kCols - 1) / V);
     const int nk = (int)(kmax - kmin + 1);  // <= ez_rows
     if constexpr (REAL) {
-        for (int q = tid; q < 2 * nk; q += kThreads) sH[q] = H[4 * kmin + 4 * (q / 2) + 2 + q % 2];
+        for (int q = tid; q < 3 * nk; q += kThreads) {  // z, its second double, the quarter turn
+            const int64_t r = 4 * (kmin + q / 3);
+            sH[q] = q % 3 == 0 ? H[r + 2] : q % 3 == 1 ? H_lo[r + 2] : H[r + 3];
+        }
     } else {
         for (int q = tid; q < 3 * nk; q += kThreads) sH[q] = H[3 * kmin + q];
     }
@@ -138,7 +145,7 @@ __global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving
         for (int e = tid; e < nk * 16; e += kThreads) {
             const int kk = e / 16, m = s * 16 + e % 16;
             if constexpr (REAL) {
-                sKz64[kk * kEz64Stride + e % 16] = sin_cycles_f64(fma(sH[2 * kk], sz[m], sH[2 * kk + 1]));
+                sKz64[kk * kEz64Stride + e % 16] = sin_turns_f64(sH[3 * kk], sH[3 * kk + 1], sz[m], sH[3 * kk + 2]);
             } else {
                 const double u = fma(sH[3 * kk], sx[m], fma(sH[3 * kk + 1], sy[m], sH[3 * kk + 2] * sz[m]));
                 double c, sn;
@@ -169,7 +176,13 @@ __global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving
                 z = packed[2 * N + n] + dz;
                 const double phi = packed[3 * N + n], r2 = packed[4 * N + n];
                 // c = b exp(-t/T2) exp(i phi t) exp(-2 pi i F.x)   (MRI.cpp:124-146)
-                const double u = fma(Fx, x, fma(Fy, y, Fz * z)) - phi * ti * (1.0 / kTwoPi);
+                double u;
+                if constexpr (REAL)
+                    u = turns_f64(Fx, F_lo[3 * i], x) + turns_f64(Fy, F_lo[3 * i + 1], y) +
+                        turns_f64(Fz, F_lo[3 * i + 2], z);
+                else
+                    u = fma(Fx, x, fma(Fy, y, Fz * z));
+                u -= phi * ti * (1.0 / kTwoPi);
                 double ec, es;
                 cis_neg_f64(u, ec, es);
                 const double d = exp(-ti * r2);
@@ -225,7 +238,7 @@ __global__ __launch_bounds__(64 * W, REAL && CB <= 4 ? 3 : 2) void k_cart_moving
             for (int st = 0; st < 4; ++st) {
                 const int m = s * 16 + 4 * st + lane / 16;
                 if constexpr (REAL) {
-                    ar[st] = sin_cycles_f64(fma(Gy, sy[m], Gz));
+                    ar[st] = sin_turns_f64(Gy, Gl, sy[m], Gz);
                 } else {
                     const double u = fma(Gx, sx[m], fma(Gy, sy[m], Gz * sz[m]));
                     cis_neg_f64(u, ar[st], ai[st]);
@@ -372,9 +385,9 @@ MovingShape moving_shape_f64(const CartesianTables &c, int64_t N, int V)
 MovingShape moving_pairs_shape_f64(const CartesianTables &c, int64_t N, int V)
 {
     // used where it runs fewer MFMAs (2 per block and k-step against 4),
-    // within the complex rows' workspace
+    // within the complex rows' workspace, and is no less exact
     const MovingShape g = moving_shape_f64(c, N, V);
-    if (!c.axis_aligned) return MovingShape{};
+    if (!c.axis_aligned || !c.pairs_f64_moving) return MovingShape{};
     const MovingShape s = mf64_shape<true>(c, c.lines.n_rows, c.kzs.n_rows, N, V, g.part_bytes);
     return s.n_rt * s.W * s.n_ct * s.CB < 2 * g.n_rt * g.W * g.n_ct * g.CB ? s : MovingShape{};
 }
@@ -387,9 +400,11 @@ static void launch_mf64_wc(const MovingShape &s, const CartesianTables &c, const
     const double *F = REAL ? c.d_F_pairs : c.d_F;
     const double *G = REAL ? reinterpret_cast<const double *>(c.lines.d_rows) : c.d_G;
     const double *H = REAL ? reinterpret_cast<const double *>(c.kzs.d_rows) : c.d_H;
+    const double *G_lo = reinterpret_cast<const double *>(c.lines.d_rows_lo);
+    const double *H_lo = reinterpret_cast<const double *>(c.kzs.d_rows_lo);
     k_cart_moving_f64<W, CB, REAL><<<(unsigned)grid, 64 * W, mf64_dyn(s.ez_rows, REAL), st>>>(
-        packed, N, (int)s.V, modes, R, mcoef, c.d_ro_group, F, G, H, c.d_t, s.M, s.L, s.K, s.n_rt, s.n_ct, s.n_splits,
-        s.nodes_per_split, s.ez_rows, part);
+        packed, N, (int)s.V, modes, R, mcoef, c.d_ro_group, F, c.d_F_pairs_lo, G, G_lo, H, H_lo, c.d_t, s.M, s.L, s.K,
+        s.n_rt, s.n_ct, s.n_splits, s.nodes_per_split, s.ez_rows, part);
 }
 
 // Column-block counts instantiated per W: those <= min(2 W, 6) (the shape

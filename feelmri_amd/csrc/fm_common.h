@@ -64,13 +64,19 @@ __device__ inline int64_t xcd_range(int64_t n_ranges)
 
 inline unsigned xcd_grid(int64_t n_ranges) { return (unsigned)(((n_ranges + 7) / 8) * 8); }
 
-// sin 2 pi u in FP64, u in cycles.  u is reduced exactly to t in [-1/4, 1/4]
-// (whole turns, then sin(pi - x) = sin x) and the Taylor series in t summed to
-// t^21 (the next term is below 2e-18): about 17 FP64 instructions, where a
-// sine and cosine pair takes about 45.
-__device__ inline double sin_cycles_f64(double u)
+// (h + l) v less a whole number of turns, l far below h: the product's rounding
+// is that of the fraction left, 2^-54 of a turn, not of the product.
+__device__ inline double turns_f64(double h, double l, double v)
 {
-    const double r = u - __builtin_rint(u);
+    return fma(l, v, fma(h, v, -__builtin_rint(h * v)));
+}
+
+// sin 2 pi r, |r| <= 3/4, in FP64: r is reduced exactly to t in [-1/4, 1/4] (sin(pi - x)
+// = sin x) and the Taylor series in t summed to t^21 (the next term is below
+// 2e-18): with the reductions below about 20 FP64 instructions, where a sine and
+// cosine pair takes about 45.
+__device__ inline double sin_fraction_f64(double r)
+{
     const double t = __builtin_fabs(r) > 0.25 ? __builtin_copysign(0.5, r) - r : r;
     const double q = t * t;
     double p = 0.0011309237482517963;
@@ -85,6 +91,17 @@ __device__ inline double sin_cycles_f64(double u)
     p = fma(p, q, -41.341702240399762);
     p = fma(p, q, 6.2831853071795862);
     return t * p;
+}
+// sin 2 pi (u + quarter), quarter 0 or 1/4 (a cosine; what the sum rounds then lies
+// at the top of the sine).
+__device__ inline double sin_cycles_f64(double u, double quarter)
+{
+    return sin_fraction_f64((u - __builtin_rint(u + quarter)) + quarter);
+}
+// The same of (h + l) v + quarter, the product as turns_f64 takes it.
+__device__ inline double sin_turns_f64(double h, double l, double v, double quarter)
+{
+    return sin_fraction_f64(fma(l, v, fma(h, v, quarter - __builtin_rint(fma(h, v, quarter)))));
 }
 
 // Coefficients of the series below, in t: s t + s[7] t^3 + ... and 1 + c[7] t^2 + ...

@@ -43,11 +43,77 @@ namespace fm {
 // ---------------------------------------------------------------------------
 // Sampling analysis (host)
 // ---------------------------------------------------------------------------
-// Real rows of the n offsets of one axis (PairAxis) about the centre c: the
-// offsets sorted, partners found from both ends.  Partners lie within 4e-15
-// of the largest |offset| of c +- D, a few roundings, so the phases differ
-// from the given ones by no more than their own rounding.
-static PairAxis pair_axis_about(const std::vector<double> &g, int64_t n, const double (&c)[3])
+// k as the kernels' phases take it, k' = k (float)pi / pi, in extended precision.
+static long double kprime(double k)
+{
+    return (long double)k * ((long double)(float)3.14159265358979323846 / 3.14159265358979323846264338327950288L);
+}
+
+// A value as two doubles.
+static void two_doubles(long double v, double &hi, double &lo)
+{
+    hi = (double)v;
+    lo = std::isfinite(hi) ? (double)(v - (long double)hi) : 0.0;
+}
+
+// Rows of the entities in a.ent (index, partner or -1): first the cosines, then the
+// sines; the centre a.c is that of the pairs (their middles' mean), or as given.
+static void pair_rows(PairAxis &a, const std::vector<double> &k, double tol)
+{
+    const int64_t n = a.n_ent = (int64_t)a.ent.size() / 4;
+    auto at = [&](int32_t j, int d) { return kprime(k[(size_t)(3 * j + d)]); };
+    int64_t n_pair = 0;
+    long double mid[3] = {0.0L, 0.0L, 0.0L};
+    for (int64_t e = 0; e < n; ++e) {
+        const int32_t p = a.ent[(size_t)(4 * e)], q = a.ent[(size_t)(4 * e + 1)];
+        if (q < 0) continue;
+        ++n_pair;
+        for (int d = 0; d < 3; ++d) mid[d] += 0.5L * (at(p, d) + at(q, d));
+    }
+    for (int d = 0; d < 3 && n_pair; ++d) a.c[d] = mid[d] / (long double)n_pair;
+    std::vector<long double> D;
+    int64_t n_lines = 0;
+    long double departs = 0.0L;
+    std::vector<char> centred;
+    for (int64_t e = 0; e < n; ++e) {
+        const int32_t p = a.ent[(size_t)(4 * e)], q = a.ent[(size_t)(4 * e + 1)];
+        bool zero = q < 0;
+        for (int d = 0; d < 3; ++d) {
+            const long double v = q < 0 ? at(p, d) - a.c[d] : 0.5L * (at(p, d) - at(q, d));
+            zero = zero && std::fabs((double)v) <= tol;
+            D.push_back(v);
+            const long double off = q < 0 ? 0.0L : 0.5L * (at(p, d) + at(q, d)) - a.c[d];
+            departs += 2.0L * off * off;  // of both
+        }
+        if (zero)
+            for (int d = 0; d < 3; ++d) {
+                departs += D[D.size() - 3 + (size_t)d] * D[D.size() - 3 + (size_t)d];
+                D[D.size() - 3 + (size_t)d] = 0.0L;
+            }
+        centred.push_back(zero);
+        n_lines += q < 0 ? 1 : 2;
+    }
+    a.departs2 = (double)(departs / (long double)std::max<int64_t>(n_lines, 1));
+    auto row = [&](int64_t e, double quarter) {
+        double lo[3];
+        for (int d = 0; d < 3; ++d) {
+            double hi;
+            two_doubles(D[(size_t)(3 * e + d)], hi, lo[d]);
+            a.rows.push_back(hi);
+        }
+        a.rows.push_back(quarter);
+        a.rows_lo.insert(a.rows_lo.end(), {lo[0], lo[1], lo[2], 0.0});
+        return (int32_t)a.n_rows++;
+    };
+    a.n_rows = 0;
+    for (int64_t e = 0; e < n; ++e) a.ent[(size_t)(4 * e + 2)] = row(e, 0.25);
+    for (int64_t e = 0; e < n; ++e) a.ent[(size_t)(4 * e + 3)] = centred[(size_t)e] ? -1 : row(e, 0.0);
+}
+
+// Real rows of the n offsets of one axis (PairAxis; g as k', k as given) about the
+// centre c: the offsets sorted, partners found from both ends.  Partners' middles
+// lie within 2e-15 of the largest |offset| of c.
+static PairAxis pair_axis_about(const std::vector<double> &g, const std::vector<double> &k, int64_t n, const double (&c)[3])
 {
     PairAxis a;
     double gmax = 0.0;
@@ -89,73 +155,27 @@ static PairAxis pair_axis_about(const std::vector<double> &g, int64_t n, const d
             --hi;
         }
     }
-    a.n_ent = (int64_t)a.ent.size() / 4;
-    // the centre as the mean of the pairs' middles, which keeps c +- D within
-    // about one rounding of the given offsets (rms)
-    int64_t n_pair = 0;
-    long double mid[3] = {0.0L, 0.0L, 0.0L};
-    for (int64_t e = 0; e < a.n_ent; ++e) {
-        const int32_t p = a.ent[(size_t)(4 * e)], q = a.ent[(size_t)(4 * e + 1)];
-        if (q < 0) continue;
-        ++n_pair;
-        for (int d = 0; d < 3; ++d) mid[d] += 0.5L * ((long double)g[(size_t)(3 * p + d)] + (long double)g[(size_t)(3 * q + d)]);
-    }
-    for (int d = 0; d < 3; ++d) a.c[d] = n_pair ? (double)(mid[d] / (long double)n_pair) : c[d];
-    // rows: the cosines, then the sines
-    std::vector<double> D;
-    std::vector<char> centred;
-    for (int64_t e = 0; e < a.n_ent; ++e) {
-        const int32_t p = a.ent[(size_t)(4 * e)], q = a.ent[(size_t)(4 * e + 1)];
-        bool zero = q < 0;
-        for (int d = 0; d < 3; ++d) {
-            const double gp = g[(size_t)(3 * p + d)];
-            const double v = q < 0 ? gp - a.c[d] : 0.5 * (gp - g[(size_t)(3 * q + d)]);
-            zero = zero && std::fabs(v) <= tol;
-            D.push_back(v);
-        }
-        if (zero) D[D.size() - 3] = D[D.size() - 2] = D[D.size() - 1] = 0.0;
-        centred.push_back(zero);
-    }
-    for (int64_t e = 0; e < a.n_ent; ++e) {
-        a.ent[(size_t)(4 * e + 2)] = (int32_t)e;
-        a.rows.insert(a.rows.end(), {D[(size_t)(3 * e)], D[(size_t)(3 * e + 1)], D[(size_t)(3 * e + 2)], 0.25});
-    }
-    a.n_rows = a.n_ent;
-    for (int64_t e = 0; e < a.n_ent; ++e) {
-        if (centred[(size_t)e]) {
-            a.ent[(size_t)(4 * e + 3)] = -1;
-            continue;
-        }
-        a.ent[(size_t)(4 * e + 3)] = (int32_t)a.n_rows++;
-        a.rows.insert(a.rows.end(), {D[(size_t)(3 * e)], D[(size_t)(3 * e + 1)], D[(size_t)(3 * e + 2)], 0.0});
-    }
-    return a;
-}
-
-// Every offset as an entity of its own, about 0.
-static PairAxis unpaired_axis(const std::vector<double> &g, int64_t n)
-{
-    PairAxis a;
-    for (int row = 0; row < 2; ++row)  // the cosines, then the sines
-        for (int64_t j = 0; j < n; ++j)
-            a.rows.insert(a.rows.end(), {g[(size_t)(3 * j)], g[(size_t)(3 * j + 1)], g[(size_t)(3 * j + 2)], row ? 0.0 : 0.25});
-    for (int64_t j = 0; j < n; ++j) a.ent.insert(a.ent.end(), {(int32_t)j, -1, (int32_t)j, (int32_t)(n + j)});
-    a.n_ent = n;
-    a.n_rows = 2 * n;
+    for (int d = 0; d < 3; ++d) a.c[d] = c[d];
+    pair_rows(a, k, tol);
     return a;
 }
 
 // The centre that leaves the fewest rows: the middle of the offsets (an even
 // count -n/2 .. n/2 - 1 pairs up completely about its half step), or 0 (where
 // single-precision offsets are symmetric to the last bit).
-static PairAxis pair_axis(const std::vector<double> &g, int64_t n)
+static PairAxis pair_axis(const std::vector<double> &g, const std::vector<double> &k, int64_t n)
 {
     double mid[3] = {0.0, 0.0, 0.0};
     const double zero[3] = {0.0, 0.0, 0.0};
     // an offset that is not finite has no partner, and no tolerance can be
-    // taken from it: no pairs, every offset with rows of its own
+    // taken from it: no pairs, every offset with rows of its own about 0
     for (double v : g)
-        if (!std::isfinite(v)) return unpaired_axis(g, n);
+        if (!std::isfinite(v)) {
+            PairAxis a;
+            for (int64_t j = 0; j < n; ++j) a.ent.insert(a.ent.end(), {(int32_t)j, -1, 0, 0});
+            pair_rows(a, k, -1.0);
+            return a;
+        }
     for (int d = 0; d < 3; ++d) {
         double lo = g[(size_t)d], hi = lo;
         for (int64_t j = 1; j < n; ++j) {
@@ -164,8 +184,20 @@ static PairAxis pair_axis(const std::vector<double> &g, int64_t n)
         }
         mid[d] = 0.5 * (lo + hi);
     }
-    PairAxis a = pair_axis_about(g, n, mid), b = pair_axis_about(g, n, zero);
+    PairAxis a = pair_axis_about(g, k, n, mid), b = pair_axis_about(g, k, n, zero);
     return b.n_rows < a.n_rows ? b : a;
+}
+
+// What complex rows round on the offsets k (mean square, as an offset): k' to a
+// double, and the product with a position, 0.42 of 2^-53 of it (rms over the mantissas).
+static double complex_rounding2(const std::vector<double> &k, int64_t n)
+{
+    long double sum = 0.0L;
+    for (double v : k) {
+        const long double e = kprime(v) - (long double)(v * kPiFOverPi), r = 0.42L * 0x1p-53L * kprime(v);
+        sum += e * e + r * r;
+    }
+    return (double)(sum / (long double)std::max<int64_t>(n, 1));
 }
 
 bool cartesian_analyse(fm_signal_plan *p, const double *kx, const double *ky, const double *kz,
@@ -224,20 +256,28 @@ bool cartesian_analyse(fm_signal_plan *p, const double *kx, const double *ky, co
                     }
         }
     }
+    const std::vector<double> kF = c.F, kG = c.G, kH = c.H;
     for (auto *v : {&c.F, &c.G, &c.H})
         for (double &x : *v) x *= kPiFOverPi;
     c.axis_aligned = true;
     for (int64_t j = 0; j < L; ++j) c.axis_aligned &= c.G[(size_t)(3 * j)] == 0.0 && c.G[(size_t)(3 * j + 2)] == 0.0;
     for (int64_t k = 0; k < K; ++k) c.axis_aligned &= c.H[(size_t)(3 * k)] == 0.0 && c.H[(size_t)(3 * k + 1)] == 0.0;
-    c.lines = pair_axis(c.G, L);
-    c.kzs = pair_axis(c.H, K);
+    c.lines = pair_axis(c.G, kG, L);
+    c.kzs = pair_axis(c.H, kH, K);
     c.F_pairs.assign((size_t)R * 6, 0.0);
+    c.F_pairs_lo.assign((size_t)R * 6, 0.0);
     for (int64_t i = 0; i < R; ++i)
         for (int d = 0; d < 3; ++d) {
-            const double f = c.F[(size_t)(3 * i + d)] + c.lines.c[d];
-            c.F_pairs[(size_t)(3 * i + d)] = f;
-            c.F_pairs[(size_t)(3 * (R + i) + d)] = f + c.kzs.c[d];
+            const long double f = kprime(kF[(size_t)(3 * i + d)]) + c.lines.c[d];
+            two_doubles(f, c.F_pairs[(size_t)(3 * i + d)], c.F_pairs_lo[(size_t)(3 * i + d)]);
+            two_doubles(f + c.kzs.c[d], c.F_pairs[(size_t)(3 * (R + i) + d)], c.F_pairs_lo[(size_t)(3 * (R + i) + d)]);
         }
+    c.H_lo.assign((size_t)K * 3, 0.0);
+    for (size_t q = 0; q < c.H_lo.size(); ++q) c.H_lo[q] = std::isfinite(c.H[q]) ? (double)(kprime(kH[q]) - (long double)c.H[q]) : 0.0;
+    // (the box of the nodes is taken to be as wide along each axis)
+    const double rounds = complex_rounding2(kF, R) + complex_rounding2(kG, L) + complex_rounding2(kH, K);
+    c.pairs_f64 = c.lines.departs2 <= rounds;
+    c.pairs_f64_moving = c.lines.departs2 + c.kzs.departs2 <= rounds;
     c.ok = true;
     return true;
 }
@@ -253,25 +293,35 @@ int cartesian_upload(fm_signal_plan *p)
     FM_HIP(hipMemcpy(c.d_G, c.G.data(), sizeof(double) * c.G.size(), hipMemcpyHostToDevice));
     FM_HIP(hipMemcpy(c.d_H, c.H.data(), sizeof(double) * c.H.size(), hipMemcpyHostToDevice));
     FM_HIP(hipMemcpy(c.d_t, c.t.data(), sizeof(double) * c.t.size(), hipMemcpyHostToDevice));
-    {   // the pair tables in one allocation: rows (32 B each), entities (16 B), F
-        size_t off[6] = {0, 0, 0, 0, 0, 0};
-        const void *src[5] = {c.lines.rows.data(), c.kzs.rows.data(), c.lines.ent.data(), c.kzs.ent.data(),
-                              c.F_pairs.data()};
-        const size_t len[5] = {sizeof(double) * c.lines.rows.size(), sizeof(double) * c.kzs.rows.size(),
-                               sizeof(int32_t) * c.lines.ent.size(), sizeof(int32_t) * c.kzs.ent.size(),
-                               sizeof(double) * c.F_pairs.size()};
-        for (int q = 0; q < 5; ++q) off[q + 1] = off[q] + len[q];
-        std::vector<char> host(off[5]);
-        for (int q = 0; q < 5; ++q) std::memcpy(host.data() + off[q], src[q], len[q]);
-        FM_HIP(hipMalloc(&c.d_pairs, off[5]));
-        FM_HIP(hipMemcpy(c.d_pairs, host.data(), off[5], hipMemcpyHostToDevice));
+    {   // the pair tables in one allocation: rows (32 B each), entities (16 B), F, H
+        const std::vector<double> *src[7] = {&c.lines.rows, &c.lines.rows_lo, &c.kzs.rows, &c.kzs.rows_lo,
+                                             &c.F_pairs, &c.F_pairs_lo, &c.H_lo};
+        const std::vector<int32_t> *ent[2] = {&c.lines.ent, &c.kzs.ent};
+        size_t off[9], total = 0;
+        auto place = [&](size_t bytes) {
+            const size_t o = total;
+            total += (bytes + 31) & ~size_t(31);
+            return o;
+        };
+        for (int q = 0; q < 7; ++q) off[q] = place(sizeof(double) * src[q]->size());
+        for (int q = 0; q < 2; ++q) off[7 + q] = place(sizeof(int32_t) * ent[q]->size());
+        std::vector<char> host(total);
+        for (int q = 0; q < 7; ++q) std::memcpy(host.data() + off[q], src[q]->data(), sizeof(double) * src[q]->size());
+        for (int q = 0; q < 2; ++q) std::memcpy(host.data() + off[7 + q], ent[q]->data(), sizeof(int32_t) * ent[q]->size());
+        FM_HIP(hipMalloc(&c.d_pairs, total));
+        FM_HIP(hipMemcpy(c.d_pairs, host.data(), total, hipMemcpyHostToDevice));
         char *d = reinterpret_cast<char *>(c.d_pairs);
         c.lines.d_rows = reinterpret_cast<double4 *>(d + off[0]);
-        c.kzs.d_rows = reinterpret_cast<double4 *>(d + off[1]);
-        c.lines.d_ent = reinterpret_cast<int4 *>(d + off[2]);
-        c.kzs.d_ent = reinterpret_cast<int4 *>(d + off[3]);
+        c.lines.d_rows_lo = reinterpret_cast<double4 *>(d + off[1]);
+        c.kzs.d_rows = reinterpret_cast<double4 *>(d + off[2]);
+        c.kzs.d_rows_lo = reinterpret_cast<double4 *>(d + off[3]);
         c.d_F_lines = reinterpret_cast<double *>(d + off[4]);
         c.d_F_pairs = c.d_F_lines + 3 * c.n_ro;
+        c.d_F_lines_lo = reinterpret_cast<double *>(d + off[5]);
+        c.d_F_pairs_lo = c.d_F_lines_lo + 3 * c.n_ro;
+        c.d_H_lo = reinterpret_cast<double *>(d + off[6]);
+        c.lines.d_ent = reinterpret_cast<int4 *>(d + off[7]);
+        c.kzs.d_ent = reinterpret_cast<int4 *>(d + off[8]);
     }
     FM_HIP(hipMalloc(&c.d_ro_group, sizeof(int32_t) * c.ro_group.size()));
     FM_HIP(hipMemcpy(c.d_ro_group, c.ro_group.data(), sizeof(int32_t) * c.ro_group.size(), hipMemcpyHostToDevice));
@@ -360,14 +410,15 @@ static GemmShape gemm_shape_of(const CartesianTables &c, bool mixed, int64_t N, 
 }
 
 // Real rows where they take fewer MFMAs (half as many per row and column
-// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32; FP64 5.94
+// block: 2.64 against 4.67 ms at 512 000 nodes, 128 x 128 x 32; FP64 5.93
 // against 11.69 ms at 150 001 nodes, 125 x 127 x 31) and no more workspace than
-// complex rows do.
+// complex rows do; the FP64 form where they are no less exact (pairs_f64).
 static GemmShape gemm_shape(const fm_signal_plan *p, int precision, int64_t N, int V)
 {
     const CartesianTables &c = p->cart;
     const bool mixed = precision != FM_PREC_F64;
     const GemmShape g = gemm_shape_of(c, mixed, N, V, false, 0);
+    if (!mixed && !c.pairs_f64) return g;
     const GemmShape s = gemm_shape_of(c, mixed, N, V, true, g.total);
     const bool fits = s.total <= g.total && s.NCp < (int64_t(1) << 31);  // column indexes in 32 bits
     return fits && s.Mp * s.NCp < 2 * g.Mp * g.NCp ? s : g;
@@ -557,10 +608,12 @@ __device__ __forceinline__ void cart_rows_bf16(int64_t t, const double *__restri
 }
 
 // Real rows, FP64: tiles of (16 rows x 16 nodes), one plane in the lane order
-// of cart_E_f64.
+// of cart_E_f64.  Offsets in two doubles, products to about 2^-54 of a cycle
+// (turns_f64), which takes the rounding of the phases (2e-15 cycles at 16 cycles)
+// out of the sum.
 __device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restrict__ packed, int64_t N, int64_t Np,
                                               int64_t M, int64_t Mp, int64_t rb0, int64_t rb1, const double4 *__restrict__ rows,
-                                              double *__restrict__ E)
+                                              const double4 *__restrict__ rows_lo, double *__restrict__ E)
 {
     // t over (Np / 16) * 4 * 64
     if (t >= (Np / 16) * 256) return;
@@ -575,8 +628,8 @@ __device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restric
         const int64_t i = rb * 16 + (lane % 16);
         double e = 0.0;
         if (ok && i < M) {
-            const double4 d = rows[i];
-            e = sin_cycles_f64(fma(d.x, x, fma(d.y, y, fma(d.z, z, d.w))));
+            const double4 d = rows[i], l = rows_lo[i];
+            e = sin_cycles_f64(turns_f64(d.x, l.x, x) + turns_f64(d.y, l.y, y) + turns_f64(d.z, l.z, z), d.w);
         }
         E[((kb * nrb + rb) * 4 + st) * 64 + lane] = e;
     }
@@ -591,8 +644,9 @@ __device__ __forceinline__ void cart_rows_f64(int64_t t, const double *__restric
 template <bool MIXED, bool PAIRS>
 __device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, int rows_blk, const double *__restrict__ packed, int64_t N,
                                         int64_t Np, int V, int64_t n_out, int64_t n_kz,
-                                        const double *__restrict__ G, const double *__restrict__ tr,
-                                        const double *__restrict__ H, void *__restrict__ Ey, void *__restrict__ Ez)
+                                        const double *__restrict__ G, const double *__restrict__ G_lo,
+                                        const double *__restrict__ tr, const double *__restrict__ H,
+                                        const double *__restrict__ H_lo, void *__restrict__ Ey, void *__restrict__ Ez)
 {
     if (n >= Np) return;
     const int64_t r0 = rblk * rows_blk;
@@ -609,7 +663,13 @@ __device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, int rows_blk, c
         const double *kv = outer ? &G[3 * row] : &H[3 * (row - n_out)];
         double c = 0.0, s = 0.0;
         if (ok) {
-            double u = fma(kv[0], x, fma(kv[1], y, kv[2] * z));
+            double u;
+            if constexpr (PAIRS && !MIXED) {
+                const double *lv = outer ? &G_lo[3 * row] : &H_lo[3 * (row - n_out)];
+                u = turns_f64(kv[0], lv[0], x) + turns_f64(kv[1], lv[1], y) + turns_f64(kv[2], lv[2], z);
+            } else {
+                u = fma(kv[0], x, fma(kv[1], y, kv[2] * z));
+            }
             const double ti = PAIRS && outer ? tr[row] : 0.0;
             if (PAIRS && outer) u -= phi * ti * (1.0 / kTwoPi);
             cis_neg_cycles<MIXED>(u, c, s);
@@ -649,11 +709,13 @@ __device__ __forceinline__ void cart_yz(int64_t n, int64_t rblk, int rows_blk, c
 template <bool MIXED, bool PAIRS>
 __global__ __launch_bounds__(256) void k_cart_tables(const double *__restrict__ packed, int64_t N, int64_t Np,
                                                      int64_t M, int64_t Mp, const double *__restrict__ F,
-                                                     const double4 *__restrict__ lrows,
+                                                     const double *__restrict__ F_lo, const double4 *__restrict__ lrows,
+                                                     const double4 *__restrict__ lrows_lo,
                                                      const double *__restrict__ tr, void *__restrict__ E,
                                                      int64_t nb_E, int V, int64_t n_out, int64_t n_kz,
                                                      const double *__restrict__ G, const double *__restrict__ H,
-                                                     void *__restrict__ Ey, void *__restrict__ Ez, int64_t nb_n,
+                                                     const double *__restrict__ H_lo, void *__restrict__ Ey,
+                                                     void *__restrict__ Ez, int64_t nb_n,
                                                      int e_parts, int rows_blk)
 {
     // the grid is below 2^31 blocks: 32-bit divisions
@@ -668,14 +730,14 @@ __global__ __launch_bounds__(256) void k_cart_tables(const double *__restrict__ 
         else if (MIXED)
             cart_E_bf16(t, packed, N, Np, M, Mp, rb0, rb1, F, tr, reinterpret_cast<uint4 *>(E));
         else if (PAIRS)
-            cart_rows_f64(t, packed, N, Np, M, Mp, rb0, rb1, lrows, reinterpret_cast<double *>(E));
+            cart_rows_f64(t, packed, N, Np, M, Mp, rb0, rb1, lrows, lrows_lo, reinterpret_cast<double *>(E));
         else
             cart_E_f64(t, packed, N, Np, M, Mp, rb0, rb1, F, tr, reinterpret_cast<double *>(E));
         return;
     }
     const unsigned c = b - nE * (unsigned)e_parts, nn = (unsigned)nb_n;
-    cart_yz<MIXED, PAIRS>((int64_t)(c % nn) * 256 + threadIdx.x, c / nn, rows_blk, packed, N, Np, V, n_out, n_kz, PAIRS ? F : G, tr,
-                          H, Ey, Ez);
+    cart_yz<MIXED, PAIRS>((int64_t)(c % nn) * 256 + threadIdx.x, c / nn, rows_blk, packed, N, Np, V, n_out, n_kz, PAIRS ? F : G,
+                          F_lo, tr, H, H_lo, Ey, Ez);
 }
 
 template <typename P, int G>
@@ -855,9 +917,9 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t N, int V, 
         }
 #define FM_TABLES(MX, PR)                                                                                            \
     k_cart_tables<MX, PR><<<(unsigned)nb, 256, 0, st>>>(packed, N, s.Np, s.M, s.Mp, PR ? c.d_F_lines : c.d_F,       \
-                                                        c.lines.d_rows, c.d_t, ws + s.off_E, nb_E, V, n_out, c.n_kz, \
-                                                        c.d_G, c.d_H, ws + s.off_Ey, ws + s.off_Ez, nb_n, e_parts, \
-                                                        rows_blk)
+                                                        c.d_F_lines_lo, c.lines.d_rows, c.lines.d_rows_lo, c.d_t,    \
+                                                        ws + s.off_E, nb_E, V, n_out, c.n_kz, c.d_G, c.d_H, c.d_H_lo, \
+                                                        ws + s.off_Ey, ws + s.off_Ez, nb_n, e_parts, rows_blk)
         if (s.mixed && s.pairs) FM_TABLES(true, true);
         else if (s.mixed) FM_TABLES(true, false);
         else if (s.pairs) FM_TABLES(false, true);

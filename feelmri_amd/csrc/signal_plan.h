@@ -60,12 +60,20 @@ struct SignalTile {
 // multiplications of one with the complex factors; the centre's phase joins
 // another factor.  An offset without a partner takes both rows for itself, an
 // offset at the centre the cosine row only.
+//
+// The centre and D are held in two doubles each, formed in extended precision from
+// the given offsets; the mixed form uses the first of them.  What is left of an
+// offset is the pair's departure from the common centre.  The FP64 form takes the
+// rows where that departure (rms) is no larger than what complex rows round
+// (pairs_f64): k' and the products are then the less exact way.
 struct PairAxis {
-    double c[3] = {0.0, 0.0, 0.0};
+    long double c[3] = {0.0L, 0.0L, 0.0L};
     int64_t n_rows = 0, n_ent = 0;
     std::vector<double> rows;    // (n_rows, 4): D, then the quarter turn added to D.x: 1/4 cosine, 0 sine
+    std::vector<double> rows_lo; // (n_rows, 4): what D is more than that, 0
     std::vector<int32_t> ent;    // (n_ent, 4): index of c + D, of c - D or -1, cosine row, sine row or -1
-    double4 *d_rows = nullptr;
+    double departs2 = 0.0;       // mean square of the departures
+    double4 *d_rows = nullptr, *d_rows_lo = nullptr;
     int4 *d_ent = nullptr;
 };
 
@@ -85,8 +93,11 @@ struct CartesianTables {
     // lines and kz planes as real rows, and F plus the lines' centre (R
     // entries), then F plus both centres
     PairAxis lines, kzs;
-    std::vector<double> F_pairs;
-    double *d_F_lines = nullptr, *d_F_pairs = nullptr;
+    std::vector<double> F_pairs, F_pairs_lo, H_lo;  // _lo: second doubles (H as it is: first double c.H)
+    double *d_F_lines = nullptr, *d_F_pairs = nullptr, *d_F_lines_lo = nullptr, *d_F_pairs_lo = nullptr, *d_H_lo = nullptr;
+    // the FP64 form's choice of real rows: for the lines (static nodes), for lines
+    // and kz planes (moving nodes)
+    bool pairs_f64 = false, pairs_f64_moving = false;
     void *d_pairs = nullptr;     // one allocation behind the pair tables
 };
 
