@@ -134,9 +134,10 @@ __device__ inline TrigCoefs scalar_trig_coefs()
 __device__ inline void sincos_cycles_f64(double u, double &s, double &c, const TrigCoefs &k = TrigCoefs())
 {
     const double r = u - __builtin_rint(u);
-    const double q = __builtin_rint(4.0 * r);
-    const double t = fma(-0.25, q, r);
-    const int iq = (int)q;
+    constexpr double kWhole = 6755399441055744.0;  // 1.5 2^52: the sum's low bits are the integer
+    const double qw = fma(4.0, r, kWhole);
+    const double t = fma(-0.25, qw - kWhole, r);
+    const int iq = (int)__builtin_bit_cast(unsigned long long, qw);
     const double w = t * t;
     double ps = k.s[0], pc = k.c[0];
 #pragma unroll

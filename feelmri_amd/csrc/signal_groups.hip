@@ -19,7 +19,12 @@
 // CONJ: the two samples of a lane have k' = m and -m (every group pairs up,
 // e.g. spiral interleaves half a turn apart); c is staged, so that one phase and one sine and
 // cosine serve both: P = sum cos c and Q = sum sin c are accumulated, 4 FMAs
-// per node and encoding, and the samples are P -+ i Q.
+// per node and encoding, and the samples are P -+ i Q.  The mixed form takes k' to be
+// +-m; in FP64 the pair's k' are mid +- m with a mid of a few roundings, whose phase
+// turns c (to first order: its square is below 1e-24), and m is held in two
+// doubles: without either the error against the sums in 80 bits is 2.1 times that of
+// single samples (spiral, 300 x 32, 600 nodes: 2.8e-15 against 1.3e-15), with both 0.97
+// times, for 8 % of the time.
 //
 // Phases are FP64, in cycles (k' carries the reference's float-pi factor).
 // PLANAR: every kz is 0, so z is neither staged nor multiplied; 0 z joins x where
@@ -34,7 +39,7 @@
 //   spiral, 973 000 nodes, 2048 x 32, mixed: 15.07 -> 13.1 ms (the FP32 series
 //   for the staged factors, 0.9 ms of it less with the hardware sine and
 //   cosine, takes the error against 64 bits from 7.8e-8 to 4.2e-8);
-//   spiral, 120 011 nodes, 1024 x 32, FP64: 6.53 -> 3.00 ms;
+//   spiral, 120 011 nodes, 1024 x 32, FP64: 6.53 -> 3.23 ms;
 //   radial, 200 003 moving nodes, 256 x 96, 8 modes, 2 encodings, mixed: 5.70 ->
 //   2.67 ms;
 //   spiral, 138 519 nodes, 1504 x 48, mixed (per-sample t before): 5.49 -> 1.9 ms.
@@ -110,6 +115,15 @@ __device__ inline void group_sincos(double u, typename GroupCT<MIXED>::T &s, typ
     }
 }
 
+// m + lo = (a - b) / 2 exactly (the rounding of a - b is a double), and (a + b) / 2.
+__device__ inline void half_difference(double a, double b, double &m, double &lo, double &mid)
+{
+    const double s = a - b, t = s - a;
+    m = 0.5 * s;
+    lo = 0.5 * ((a - (s - t)) - (b + t));
+    mid = 0.5 * (a + b);
+}
+
 template <int VB, bool MIXED, bool MOTION, bool CONJ, bool PLANAR>
 __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups(
     const double *__restrict__ packed, int64_t N, int V, int v0, const double4 *__restrict__ ks,
@@ -142,13 +156,24 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
     const int2 pr = pairs[tile.x + (live ? tid : 0)];  // samples (second -1: none)
     const int lg = lane_group[tile.x + (live ? tid : 0)];
     double kx[2], ky[2], kz[2];
+    constexpr int kFix = CONJ && !MIXED ? 3 : 0;
+    double klo[kFix ? kFix : 1], kmid[kFix ? kFix : 1];  // FP64 pairs: of m, of the middle
     {
         const double4 a = ks[pr.x], b = ks[pr.y >= 0 ? pr.y : pr.x];
         if (CONJ) {
-            kx[0] = 0.5 * (a.x - b.x);
-            ky[0] = 0.5 * (a.y - b.y);
-            kz[0] = 0.5 * (a.z - b.z);
+            double m[3], lo[3], sum[3];
+            half_difference(a.x, b.x, m[0], lo[0], sum[0]);
+            half_difference(a.y, b.y, m[1], lo[1], sum[1]);
+            half_difference(a.z, b.z, m[2], lo[2], sum[2]);
+            kx[0] = m[0];
+            ky[0] = m[1];
+            kz[0] = m[2];
             kx[1] = ky[1] = kz[1] = 0.0;
+#pragma unroll
+            for (int d = 0; d < kFix; ++d) {
+                klo[d] = lo[d];
+                kmid[d] = kTwoPi * sum[d];
+            }
         } else {
             kx[0] = a.x;
             ky[0] = a.y;
@@ -301,7 +326,21 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
 #pragma unroll
             for (int j = 0; j < (CONJ ? 1 : 2); ++j) {
                 double u;
-                if constexpr (CONJ) {
+                if constexpr (kFix) {
+                    double lo = fma(klo[0], xy.x, klo[1] * xy.y), eps = fma(kmid[0], xy.x, kmid[1] * xy.y);
+                    if (!PLANAR) {
+                        lo = fma(klo[2], z, lo);
+                        eps = fma(kmid[2], z, eps);
+                        lo = fma(kz[j], z, lo);
+                    }
+                    u = fma(kx[j], xy.x, fma(ky[j], xy.y, lo));
+#pragma unroll
+                    for (int v = 0; v < VB; ++v) {
+                        const CT2 w = c[v];
+                        c[v].x = fma(eps, w.y, w.x);
+                        c[v].y = fma(-eps, w.x, w.y);
+                    }
+                } else if constexpr (CONJ) {
                     u = PLANAR ? fma(kx[j], xy.x, ky[j] * xy.y) : fma(kx[j], xy.x, fma(ky[j], xy.y, kz[j] * z));
                 } else {
                     u = PLANAR ? fma(kx[j], xy.x, fma(ky[j], xy.y, ph))

@@ -72,6 +72,32 @@ def test_moving_cartesian(gpu, shape):
     _check(gpu, kloc, t, R=3)
 
 
+def _spiral(m, l):
+    fov, res = (0.24, 0.24, 0.24), (256, l, 1)
+    T_ms = trajectories.spiral_stack(fov, res, density_exponent=2.0, dtype=np.float64)[2]
+    kloc, t, _ = trajectories.spiral_stack(fov, res, oversampling=2, t_start=0.5, density_exponent=2.0,
+                                           receiver_bw=(m // 2) / (T_ms * 1e-3), dtype=np.float64)
+    return kloc, t
+
+
+@pytest.mark.parametrize("moving", [False, True])
+@pytest.mark.parametrize("m,l", [(300, 32), (200, 31), (160, 48), (90, 16)])
+def test_spiral(gpu, m, l, moving):
+    """Interleaves half a turn apart (an even number of them) pair up as k and -k to a rounding."""
+    kloc, t = _spiral(m, l)
+    _check(gpu, kloc, t, R=3 if moving else 0)
+
+
+def test_pairs_in_three_dimensions(gpu):
+    """Pairs k, -k + a rounding, with kz."""
+    r = np.random.default_rng(6)
+    kloc = [r.uniform(-250.0, 250.0, (60, 24, 1)) for _ in range(3)]
+    for k in kloc:
+        k[:, 12:] = -k[:, :12] * (1 + 2.0 ** -52 * r.integers(-1, 2, (60, 12, 1)))
+    t = np.broadcast_to(np.linspace(0.5, 4.0, 60)[:, None, None], (60, 24, 1)).copy()
+    _check(gpu, kloc, t, method="direct")
+
+
 def test_stack_far_from_the_centre(gpu):
     """(A rotated stack is left out: its split into axes rounds before any form is taken.)"""
     (kx, ky, kz), t = trajectories.cartesian((0.22, 0.22, 0.22), (24, 48, 4), t_first=1.0)
