@@ -663,6 +663,27 @@ static size_t direct_workspace(const fm_signal_plan *p, int64_t N, int V)
     return need;
 }
 
+// The direct kernels' route.  Mixed form, static nodes, whole linear lines: the
+// per-line GEMM.  Positions depend on t, so moving nodes always take the t-grouped
+// tiles; static nodes take the readout runs when the plan has them (the FP64
+// form only when they are linear to 1e-14).
+static int direct_route(const fm_signal_plan *p, int precision, int64_t N, bool motion)
+{
+    const bool mixed = precision != FM_PREC_F64;
+    if (!motion && mixed && lines_usable(p, N)) return FM_ROUTE_LINES;
+    if (!motion && p->n_runs > 0 && (mixed || p->runs_exact)) return FM_ROUTE_RUNS;
+    if (!motion && !p->prefer_grouped) return FM_ROUTE_CONSECUTIVE;
+    return groups_in_pairs(p, mixed) ? FM_ROUTE_GROUP_PAIRS : FM_ROUTE_GROUPS;
+}
+
+static DirectLaunch direct_launch(const fm_signal_plan *p, int route, int precision, int64_t N, int V, int R,
+                                  size_t ws_bytes)
+{
+    if (route == FM_ROUTE_RUNS) return direct_launch_shape(p, N, 2);
+    if (route == FM_ROUTE_CONSECUTIVE) return direct_launch_shape(p, N, 0);
+    return groups_launch_shape(p, precision != FM_PREC_F64, R > 0, N, V, R, ws_bytes);
+}
+
 static int direct_execute(const fm_signal_plan *p, int precision, int64_t N, int V,
                           const double *packed, const float *modes, int R, const double *mcoef,
                           void *ws, size_t ws_bytes, double *out, hipStream_t st)
@@ -673,16 +694,11 @@ static int direct_execute(const fm_signal_plan *p, int precision, int64_t N, int
         return zero_f64_async(out, 2 * S * V, st);
     }
     const bool motion = modes != nullptr && R > 0;
-    // mixed form, static nodes, whole linear lines: the per-line GEMM
-    if (!motion && precision != FM_PREC_F64 && lines_usable(p, N)) return lines_execute(p, N, V, packed, ws, ws_bytes, out, st);
-    // positions depend on t, so moving nodes always take the t-grouped tiles;
-    // static nodes take the readout runs when the plan has them (the FP64
-    // form only when they are linear to 1e-14)
-    const bool use_runs = !motion && p->n_runs > 0 && (precision != FM_PREC_F64 || p->runs_exact);
-    const bool grouped = motion || (!use_runs && p->prefer_grouped);
+    const int route = direct_route(p, precision, N, motion);
+    if (route == FM_ROUTE_LINES) return lines_execute(p, N, V, packed, ws, ws_bytes, out, st);
+    const bool use_runs = route == FM_ROUTE_RUNS, grouped = !use_runs && route != FM_ROUTE_CONSECUTIVE;
     const int tiling = use_runs ? 2 : (grouped ? 1 : 0);
-    const DirectLaunch L = grouped ? groups_launch_shape(p, precision != FM_PREC_F64, motion, N, V, R, ws ? ws_bytes : 0)
-                                   : direct_launch_shape(p, N, tiling);
+    const DirectLaunch L = direct_launch(p, route, precision, N, V, motion ? R : 0, ws ? ws_bytes : 0);
     const size_t need = L.n_splits > 1 ? (size_t)L.n_splits * (size_t)S * (size_t)V * sizeof(double2) : 0;
     if (need > ws_bytes) {
         set_error("signal workspace too small: need %zu bytes, got %zu", need, ws_bytes);
@@ -925,7 +941,7 @@ static int plan_analyse(fm_signal_plan *p, const double *kx, const double *ky, c
         close(p->n_tgroups);
         p->n_tiles_pairs = (int64_t)h.tiles_p.size();
     }
-    // reported facts: slots of up to 256 samples of one group, two to a tile;
+    // facts reported by the analysis: slots of up to 256 samples of one group, two to a tile;
     // groups of one size of 32, 64 or 128 samples and how many fill 256 lanes,
     // singly and as conjugate pairs
     {
@@ -1278,6 +1294,26 @@ extern "C" int fm_signal_workspace_size(const fm_signal_plan *p, int precision, 
         *bytes = cartesian_moving_workspace(p, precision, n_nodes, n_enc);
     else
         *bytes = direct_workspace(p, n_nodes, n_enc);
+    return FM_OK;
+}
+
+extern "C" int fm_signal_route(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc, int n_modes,
+                               int *route, int64_t *n_splits)
+{
+    FM_CHECK_ARG(p != nullptr && route != nullptr && n_splits != nullptr, "NULL argument");
+    FM_CHECK_ARG(precision == FM_PREC_F64 || precision == FM_PREC_MIXED,
+                 "signal precision must be FM_PREC_F64 or FM_PREC_MIXED (got %d)", precision);
+    FM_CHECK_ARG(n_nodes >= 1 && n_enc >= 1 && p->n_samples >= 1, "no nodes, encodings or samples");
+    FM_CHECK_ARG(n_modes >= 0 && n_modes <= kMaxModes, "n_modes must be in [0, %d]", kMaxModes);
+    const bool motion = n_modes > 0;
+    if (p->method == FM_METHOD_CARTESIAN && (!motion || n_enc <= kMovMaxV)) {
+        *route = cartesian_route(p, precision, n_nodes, n_enc, motion, n_splits);
+        return FM_OK;
+    }
+    *route = direct_route(p, precision, n_nodes, motion);
+    *n_splits = *route == FM_ROUTE_LINES
+                    ? lines_splits(p, n_nodes)
+                    : direct_launch(p, *route, precision, n_nodes, n_enc, n_modes, direct_workspace(p, n_nodes, n_enc)).n_splits;
     return FM_OK;
 }
 

@@ -959,6 +959,21 @@ static MovingShape moving_form(const CartesianTables &c, bool f64, int64_t N, in
     return s.pairs ? s : (f64 ? moving_shape_f64(c, N, V) : moving_shape(c, N, V));
 }
 
+int cartesian_route(const fm_signal_plan *p, int precision, int64_t N, int V, bool moving, int64_t *n_splits)
+{
+    bool pairs;
+    if (moving) {
+        const MovingShape s = moving_form(p->cart, precision == FM_PREC_F64, N, V);
+        pairs = s.pairs;
+        *n_splits = s.n_splits;
+    } else {
+        const GemmShape s = gemm_shape(p, precision, N, V);
+        pairs = s.pairs;
+        *n_splits = s.n_splits;
+    }
+    return pairs ? FM_ROUTE_CARTESIAN_REAL : FM_ROUTE_CARTESIAN;
+}
+
 size_t cartesian_moving_workspace(const fm_signal_plan *p, int precision, int64_t N, int V)
 {
     if (p->n_samples == 0 || N == 0 || V > kMovMaxV) return 0;

@@ -390,7 +390,8 @@ __global__ __launch_bounds__(kDirectThreads, MIXED ? 4 : 3) void k_signal_groups
 }
 
 // Conjugate pairs serve the FP64 form where they are exact to a few roundings.
-static bool group_conj(const fm_signal_plan *p, bool mixed) { return p->pairs_conj && (mixed || p->pairs_exact); }
+
+bool groups_in_pairs(const fm_signal_plan *p, bool mixed) { return p->pairs_conj && (mixed || p->pairs_exact); }
 
 // Nodes per chunk: the most, a power of two from 16 to 128, whose records take
 // at most 24 KB (6 workgroups of 4 waves per CU).  16 where even those take
@@ -398,7 +399,7 @@ static bool group_conj(const fm_signal_plan *p, bool mixed) { return p->pairs_co
 // workgroups per CU.
 static int group_chunk(const fm_signal_plan *p, int vb, bool mixed, bool motion, int R)
 {
-    const bool conj = group_conj(p, mixed);
+    const bool conj = groups_in_pairs(p, mixed);
     int c = kGroupChunkMax;
     while (c > kGroupChunkMin && group_lds(vb, mixed, motion, conj, p->planar != 0, c, p->groups_per_tile, R).total > 24 * 1024) c /= 2;
     return c;
@@ -433,8 +434,8 @@ int groups_blocks_per_cu(const fm_signal_plan *p, bool mixed, bool motion, int V
 {
     const int vb = std::min(V, kMaxVB);
     const int chunk = group_chunk(p, vb, mixed, motion, R);
-    const int lds = group_lds(vb, mixed, motion, group_conj(p, mixed), p->planar != 0, chunk, p->groups_per_tile, R).total;
-    return blocks_per_cu(group_kernel_of(vb, mixed, motion, group_conj(p, mixed), p->planar != 0), kDirectThreads,
+    const int lds = group_lds(vb, mixed, motion, groups_in_pairs(p, mixed), p->planar != 0, chunk, p->groups_per_tile, R).total;
+    return blocks_per_cu(group_kernel_of(vb, mixed, motion, groups_in_pairs(p, mixed), p->planar != 0), kDirectThreads,
                          (size_t)lds);
 }
 
@@ -443,7 +444,7 @@ int groups_launch(const fm_signal_plan *p, bool mixed, bool motion, int64_t N, i
                   int64_t nodes_per_split, double2 *dst, int write_final, hipStream_t st)
 {
     int chunk = group_chunk(p, vb, mixed, motion, R), gs = p->groups_per_tile, vv = V, vfirst = v0, RR = R;
-    const int lds = group_lds(vb, mixed, motion, group_conj(p, mixed), p->planar != 0, chunk, gs, R).total;
+    const int lds = group_lds(vb, mixed, motion, groups_in_pairs(p, mixed), p->planar != 0, chunk, gs, R).total;
     int64_t S = p->n_samples, nn = N, nps = nodes_per_split;
     const double4 *ks = p->d_ks;
     const int2 *pairs = p->d_pairs;
@@ -452,7 +453,7 @@ int groups_launch(const fm_signal_plan *p, bool mixed, bool motion, int64_t N, i
     const double *tg = p->d_tg_t;
     void *args[] = {&packed, &nn, &vv, &vfirst, &ks, &pairs, &lane_group, &tiles, &tg, &modes, &RR, &mcoef, &chunk, &gs, &nps,
                     &dst, &S, &write_final};
-    FM_HIP(hipLaunchKernel(group_kernel_of(vb, mixed, motion, group_conj(p, mixed), p->planar != 0),
+    FM_HIP(hipLaunchKernel(group_kernel_of(vb, mixed, motion, groups_in_pairs(p, mixed), p->planar != 0),
                            dim3((unsigned)p->n_tiles_pairs, (unsigned)n_splits), dim3(kDirectThreads), args,
                            (size_t)lds, st));
     return FM_OK;

@@ -323,6 +323,8 @@ bool lines_usable(const fm_signal_plan *p, int64_t N)
            N < kLineMaxNodes;
 }
 
+int64_t lines_splits(const fm_signal_plan *p, int64_t N) { return line_shape(p, N).n_splits; }
+
 size_t lines_workspace(const fm_signal_plan *p, int64_t N)
 {
     if (!lines_usable(p, N) || N <= 0) return 0;

@@ -179,6 +179,7 @@ int cartesian_execute(const fm_signal_plan *p, int precision, int64_t n_nodes, i
 // (signal_lines_bf16.hip).
 bool lines_usable(const fm_signal_plan *p, int64_t n_nodes);
 size_t lines_workspace(const fm_signal_plan *p, int64_t n_nodes);
+int64_t lines_splits(const fm_signal_plan *p, int64_t n_nodes);
 int lines_execute(const fm_signal_plan *p, int64_t n_nodes, int n_enc, const double *packed, void *ws,
                   size_t ws_bytes, double *out, hipStream_t stream);
 // Samples grouped by t (signal_groups.hip).
@@ -186,6 +187,9 @@ int groups_blocks_per_cu(const fm_signal_plan *p, bool mixed, bool motion, int n
 int groups_launch(const fm_signal_plan *p, bool mixed, bool motion, int64_t n_nodes, int n_enc, int v0, int vb,
                   const double *packed, const float *modes, int n_modes, const double *motion_coef, int64_t n_splits,
                   int64_t nodes_per_split, double2 *dst, int write_final, hipStream_t stream);
+bool groups_in_pairs(const fm_signal_plan *p, bool mixed);
+// Route and splits of the Cartesian GEMM (fm_signal_route), static or moving.
+int cartesian_route(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc, bool moving, int64_t *n_splits);
 // Moving nodes, per-readout GEMM in either form (n_enc <= kMovMaxV).
 size_t cartesian_moving_workspace(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc);
 int cartesian_moving_execute(const fm_signal_plan *p, int precision, int64_t n_nodes, int n_enc,

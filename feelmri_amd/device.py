@@ -56,8 +56,10 @@ def _prec(precision) -> int:
 def analyse_trajectory(kloc, t, method: str = "auto") -> dict:
     """Host-only analysis of a trajectory (no device needed), as
     ``SignalPlan`` performs it: the method it would choose, the number of
-    distinct t, of readout runs and of t-grouped tiles, and the equal-size
-    t-groups that 256 lanes hold singly and as conjugate pairs (1: none)."""
+    distinct t and of readout runs; and of the samples of equal t, how many
+    512-sample tiles slots of 256 would fill, and how many equal-size groups
+    256 lanes hold singly and as conjugate pairs (1: none).
+    ``SignalPlan.route`` tells what an evaluation runs."""
     kx, ky, kz = (np.ascontiguousarray(np.asarray(k, dtype=np.float64)) for k in kloc)
     tt = np.ascontiguousarray(np.asarray(t, dtype=np.float64))
     if tt.ndim != 3 or any(k.shape != tt.shape for k in (kx, ky, kz)):
@@ -151,6 +153,15 @@ class SignalPlan:
         _lib.call("fm_signal_workspace_size", self._h, _prec(precision), int(n_nodes), int(n_enc),
                   int(bool(moving)), ctypes.byref(out))
         return int(out.value)
+
+    ROUTES = ("consecutive", "groups", "group_pairs", "runs", "lines", "cartesian", "cartesian_real")
+
+    def route(self, precision, n_nodes: int, n_enc: int, n_modes: int = 0) -> tuple[str, int]:
+        """(kernel family, node splits) that ``execute`` runs for these sizes."""
+        kind, splits = ctypes.c_int(), ctypes.c_int64()
+        _lib.call("fm_signal_route", self._h, _prec(precision), int(n_nodes), int(n_enc), int(n_modes),
+                  ctypes.byref(kind), ctypes.byref(splits))
+        return self.ROUTES[kind.value], splits.value
 
     def execute(self, nodes: "SignalNodes", precision="f64", motion=None, out=None,
                 workspace=None, stream=None) -> torch.Tensor:

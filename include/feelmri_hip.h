@@ -79,14 +79,16 @@ int fm_signal_plan_create(fm_signal_plan **plan, int64_t n_meas, int64_t n_lines
 int fm_signal_plan_destroy(fm_signal_plan *plan);
 /* Host-only analysis of a trajectory, as fm_signal_plan_create performs it,
  * without a device: the method it would choose, the number of distinct t,
- * of 16-sample readout runs and of t-grouped tiles, whether the runs are
- * linear to 1e-14 (runs_exact: the FP64 form takes them too), and, where
- * every t-group has the same size of 32, 64 or 128 samples, how many of them
- * 256 lanes hold with one sample a lane (group_pack, else 1) and with a
- * conjugate pair k, -k a lane (conj_pack, 1 when some group's samples do not
- * pair up).  Out-pointers may be NULL.  No
- * counterpart in the reference (plan introspection; usable without a
- * GPU). */
+ * of 16-sample readout runs, and whether the runs are linear to 1e-14
+ * (runs_exact: the FP64 form takes them too).  The last three describe the
+ * samples of equal t, not a launch (fm_signal_route tells what an evaluation
+ * runs): n_tiles_grouped is the number of 512-sample tiles that would hold
+ * slots of up to 256 samples of one t each, two to a tile; where every t
+ * has the same number of 32, 64 or 128 samples, group_pack is how many of
+ * those groups 256 lanes hold with one sample a lane (else 1), and conj_pack
+ * the same with a conjugate pair k, -k a lane (1 when some group's samples
+ * do not pair up).  Out-pointers may be NULL.  No counterpart in the reference
+ * (plan introspection; usable without a GPU). */
 int fm_signal_plan_analyse(int64_t n_meas, int64_t n_lines, int64_t n_kz, const double *kx,
                            const double *ky, const double *kz, const double *t, int method,
                            int *method_out, int64_t *n_tgroups, int64_t *n_runs,
@@ -117,6 +119,20 @@ int fm_signal_plan_lines(const fm_signal_plan *plan, int64_t *n_lines, int *line
  * query on the device that will execute. */
 int fm_signal_workspace_size(const fm_signal_plan *plan, int precision, int64_t n_nodes,
                              int n_enc, int moving, size_t *bytes);
+
+/* What fm_signal_execute launches for these sizes (n_modes 0: static nodes) with
+ * a workspace of the size fm_signal_workspace_size reports: the kernel family
+ * and the number of node splits.  Query on the device that will execute.  No
+ * counterpart in the reference (plan introspection). */
+#define FM_ROUTE_CONSECUTIVE 0  /* samples in any order, t per sample */
+#define FM_ROUTE_GROUPS 1       /* samples grouped by t */
+#define FM_ROUTE_GROUP_PAIRS 2  /* the same, two samples k, -k to a phase */
+#define FM_ROUTE_RUNS 3         /* 16-sample readout runs */
+#define FM_ROUTE_LINES 4        /* whole lines, matrix cores */
+#define FM_ROUTE_CARTESIAN 5    /* Cartesian GEMM, complex rows */
+#define FM_ROUTE_CARTESIAN_REAL 6 /* Cartesian GEMM, paired lines as real rows */
+int fm_signal_route(const fm_signal_plan *plan, int precision, int64_t n_nodes, int n_enc, int n_modes,
+                    int *route, int64_t *n_splits);
 
 /* Pack reference-layout node inputs into the SoA table fm_signal_execute
  * reads: rows x, y, z, phi_dB0 (rad/ms), 1/T2, then Re/Im of (w .* Mxy)[:, v]
