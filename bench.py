@@ -252,6 +252,24 @@ def load_traffic(kernel: str, config: str, form: str):
     return None if rec is None else rec.get("bytes_per_launch")
 
 
+def signal_kernel(route: str, form: str, moving: bool) -> str:
+    """The kernel behind ``SignalPlan.route``'s answer."""
+    mixed = form == "mixed"
+    return {"cartesian": ("k_cart_moving_bf16" if mixed else "k_cart_moving_f64") if moving
+            else ("k_cart_gemm_bf16" if mixed else "k_cart_gemm_f64"),
+            "cartesian_real": ("k_cart_moving_pairs_bf16" if mixed else "k_cart_moving_f64") if moving
+            else ("k_cart_gemm_pairs_bf16" if mixed else "k_cart_gemm_f64"),
+            "lines": "k_signal_lines_bf16", "runs": "k_signal_runs" if mixed else "k_signal_runs_f64",
+            "groups": "k_signal_groups", "group_pairs": "k_signal_groups", "consecutive": "k_signal_consec"}[route]
+
+
+def products_per_complex_mac(route: str) -> float:
+    """Real products that the matrix cores form, over the 4 of a complex one,
+    times the 3 bf16 products of the mixed form: lines that pair up are real
+    rows, half the products."""
+    return 1.5 if route == "cartesian_real" else 3.0
+
+
 def cpu_baseline(wl, w_h, mxy_h, target_s: float, motion=None):
     """The FP64 oracle run the reference's way (``oracle.cpu_ranks``): forked
     ranks, one per host core, each owning one block of elements and the
@@ -526,30 +544,34 @@ def run_flow(args, dev) -> dict:
     err_or = rel_l2(out0[idx], ref)
     log(f"relL2 vs FP64 oracle on {idx.size} sampled k-points of phase 0: {err_or:.2e}")
     k_s = (k_ms or ms / n_ph) * 1e-3   # dominant kernel, per phase
+    route = plan.route(args.form, m.n_nodes, 4, modes.shape[0] // 3)[0]
+    kernel = signal_kernel(route, args.form, True)
+    rows = "real (line, kz) rows" if route == "cartesian_real" else "complex (line, kz) rows"
     if plan.method == "cartesian" and args.form == "mixed":
         # 8 flops per complex MAC per node*k-sample*encoding; the kernel
-        # executes 3 bf16 products per real product (24)
+        # executes 3 bf16 products per real product, of which real rows need half
         achieved = 8.0 * m.n_nodes * wl.n_samples * 4 / k_s / 1e12
-        roof = {"bound": "mfma", "kernel": "k_cart_moving_bf16", "achieved": achieved,
+        roof = {"bound": "mfma", "kernel": kernel, "achieved": achieved,
                 "peak": PEAKS["bf16_mfma_tflops"], "unit": "TFLOP/s",
                 "frac": achieved / PEAKS["bf16_mfma_tflops"],
-                "traffic": load_traffic("k_cart_moving_bf16", "c3", "mixed"), "kernel_ms": k_ms,
-                "executed": 3.0 * achieved,
+                "traffic": load_traffic(kernel, "c3", "mixed"), "kernel_ms": k_ms,
+                "executed": products_per_complex_mac(route) * achieved,
                 "per_unit": "8 flops per node*k-sample*encoding (complex MAC); one launch is one cardiac phase "
                             "(1948800 nodes x 221184 k-samples x 4 encodings); operands generated in the kernel "
-                            "(FP64 phase, FP32 sin/cos per node and line / kz, bf16 hi+lo split)"}
+                            f"(FP64 phase, FP32 sine per node and row, bf16 hi+lo split), {rows}"}
     elif plan.method == "cartesian":
         achieved = 8.0 * m.n_nodes * wl.n_samples * 4 / k_s / 1e12
-        roof = {"bound": "mfma", "kernel": "k_cart_moving_f64", "achieved": achieved,
+        roof = {"bound": "mfma", "kernel": kernel, "achieved": achieved,
                 "peak": PEAKS["fp64_mfma_tflops"], "unit": "TFLOP/s",
                 "frac": achieved / PEAKS["fp64_mfma_tflops"],
-                "traffic": load_traffic("k_cart_moving_f64", "c3", "f64"), "kernel_ms": k_ms,
+                "traffic": load_traffic(kernel, "c3", "f64"), "kernel_ms": k_ms,
+                "executed": products_per_complex_mac(route) / 3.0 * achieved,
                 "per_unit": "8 flops per node*k-sample*encoding (complex MAC) on FP64 MFMA; operands "
-                            "generated in the kernel (FP64 sincospi per node and line / kz)"}
+                            f"generated in the kernel (FP64 sines per node and row), {rows}"}
     else:
         peak = PEAKS["fp32_valu_tflops"] if args.form == "mixed" else PEAKS["fp64_valu_tflops"]
         achieved = (8.0 + 8.0 * 4) * m.n_nodes * wl.n_samples / k_s / 1e12
-        roof = {"bound": "valu", "kernel": "k_signal_direct (moving nodes)", "achieved": achieved, "peak": peak,
+        roof = {"bound": "valu", "kernel": f"{kernel} (moving nodes)", "achieved": achieved, "peak": peak,
                 "unit": "TFLOP/s", "frac": achieved / peak, "traffic": None,
                 "per_unit": "8 flops + 8 per encoding and 2 transcendentals per node*k-sample"}
 
@@ -661,36 +683,27 @@ def measure_static(args, dev, wl, form: str, with_cpu: bool) -> dict:
     log(f"relL2 vs FP64 oracle on sampled k-points: {err_oracle:.2e}")
 
     # roofline of the dominant kernel
-    if plan.method == "cartesian":
+    route = plan.route(form, wl.n_nodes, wl.n_enc)[0]
+    dom = signal_kernel(route, form, False)
+    if route.startswith("cartesian") or route == "lines":
         bound, unit = "mfma", "TFLOP/s"
         flops = 8.0 * work
         peak = PEAKS["bf16_mfma_tflops"] if form == "mixed" else PEAKS["fp64_mfma_tflops"]
-        dom = "k_cart_gemm"
-    elif form == "mixed" and plan.line_gemm:
-        bound, unit = "mfma", "TFLOP/s"
-        flops = 8.0 * work
-        peak = PEAKS["bf16_mfma_tflops"]
-        dom = "k_signal_lines_bf16"
-    elif form == "mixed" and plan.n_runs > 0:
-        bound, unit = "valu", "TFLOP/s"
-        flops = (8.0 + 8.0 * wl.n_enc) * wl.n_nodes * wl.n_samples
-        peak = PEAKS["fp32_valu_tflops"]
-        dom = "k_signal_runs"
     else:
         bound, unit = "valu", "TFLOP/s"
         flops = (8.0 + 8.0 * wl.n_enc) * wl.n_nodes * wl.n_samples
         peak = PEAKS["fp64_valu_tflops"] if form == "f64" else PEAKS["fp32_valu_tflops"]
-        dom = "k_signal_direct"
     ms_dom = ms_kernel if ms_kernel else ms_ev
     achieved = flops / (ms_dom * 1e-3) / 1e12
     roof = {"bound": bound, "kernel": dom, "achieved": achieved, "peak": peak, "unit": unit,
             "frac": achieved / peak, "traffic": load_traffic(dom, wl.name, form), "kernel_ms": ms_dom,
             "per_unit": ("8 flops per node*k-sample*encoding (complex MAC); the mixed GEMM executes 3 bf16 "
-                         "products (hi*hi + hi*lo + lo*hi) per real product, i.e. 24" if bound == "mfma"
+                         "products (hi*hi + hi*lo + lo*hi) per real product, and half the real products "
+                         "where lines are real rows (cartesian_real): 24 or 12" if bound == "mfma"
                          else "8 flops (k.x 3 FMA + phi t 1 FMA) + 8 per encoding (complex MAC) and 2 "
                               "transcendentals per node*k-sample")}
     if bound == "mfma" and form == "mixed":
-        roof["executed"] = 3.0 * achieved
+        roof["executed"] = products_per_complex_mac(route) * achieved
     cpu = None
     err_cpu = {}
     if with_cpu:
