@@ -518,44 +518,78 @@ __device__ inline double sum_group16(double v)
 // Bound by the latency of three dependent loads (row, entry, x).  The rows of a
 // workgroup's XCD are one range, whose part of x stays in that L2.  215 940 rows
 // of 15, two encodings: 16.6 us, 4 TB/s (38.7 us with sums for four encodings
-// through LDS and the rows dealt over the XCDs).  One row a group: with four rows a
-// group their loads overlap, but a call of few or long rows leaves CUs idle (2000
-// rows of 500, one encoding: 12.8 us, 21.8 with four), and long meshes gain nothing
-// (17.1 us).  The x of all encodings is loaded before it is used: 200 000 rows of 40, four
-// encodings 205 -> 139 us.
-template <int VB>
+// through LDS and the rows dealt over the XCDs).  The x of all encodings is loaded before
+// it is used: 200 000 rows of 40, four encodings 205 -> 139 us.
+// ROWS: rows of a lane group, whose loads overlap; csr_two_rows tells when that is two.
+template <int VB, int ROWS>
 __global__ __launch_bounds__(256) void k_csr_spmv_c128(int64_t n_rows, int V, const int64_t *__restrict__ indptr,
                                                        const int64_t *__restrict__ indices,
                                                        const double *__restrict__ data,
                                                        const double2 *__restrict__ x, double2 *__restrict__ y)
 {
-    const int64_t row = xcd_range(cdiv(n_rows, 16)) * 16 + threadIdx.x / 16;
+    const int64_t row = xcd_range(cdiv(n_rows, 16 * ROWS)) * 16 * ROWS + threadIdx.x / 16;
     const int j = threadIdx.x % 16;
-    const bool live = row < n_rows;
-    const int64_t r = live ? row : n_rows - 1;
-    const int64_t k0 = indptr[r] + j, k1 = indptr[r + 1];
+    int64_t k0[ROWS], k1[ROWS], longest = 0;
+#pragma unroll
+    for (int q = 0; q < ROWS; ++q) {
+        const int64_t r = row + 16 * q < n_rows ? row + 16 * q : n_rows - 1;
+        k0[q] = indptr[r] + j;
+        k1[q] = indptr[r + 1];
+        longest = k1[q] - k0[q] > longest ? k1[q] - k0[q] : longest;
+    }
     for (int v0 = 0; v0 < V; v0 += VB) {
-        double re[VB], im[VB];
+        double re[ROWS][VB], im[ROWS][VB];
 #pragma unroll
-        for (int u = 0; u < VB; ++u) re[u] = im[u] = 0.0;
-        for (int64_t k = k0; k < k1; k += 16) {
-            const double a = data[k];
-            const double2 *xr = x + indices[k] * V + v0;
-            double2 xv[VB];  // loaded together
+        for (int q = 0; q < ROWS; ++q)
 #pragma unroll
-            for (int u = 0; u < VB; ++u) xv[u] = v0 + u < V ? xr[u] : make_double2(0.0, 0.0);
+            for (int u = 0; u < VB; ++u) re[q][u] = im[q][u] = 0.0;
+        for (int64_t t = 0; t < longest; t += 16) {
+            double a[ROWS];
+            int64_t c[ROWS];
+            double2 xv[ROWS][VB];  // loaded together
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q) {
+                c[q] = -1;
+                if (ROWS == 1 || k0[q] + t < k1[q]) {
+                    a[q] = data[k0[q] + t];
+                    c[q] = indices[k0[q] + t];
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q)
+#pragma unroll
+                for (int u = 0; u < VB; ++u)
+                    if ((ROWS == 1 || c[q] >= 0) && v0 + u < V) xv[q][u] = x[c[q] * V + v0 + u];
+                    else xv[q][u] = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int q = 0; q < ROWS; ++q)
+                if (ROWS == 1 || c[q] >= 0)
+#pragma unroll
+                    for (int u = 0; u < VB; ++u) {
+                        re[q][u] = fma(a[q], xv[q][u].x, re[q][u]);
+                        im[q][u] = fma(a[q], xv[q][u].y, im[q][u]);
+                    }
+        }
+#pragma unroll
+        for (int q = 0; q < ROWS; ++q)
 #pragma unroll
             for (int u = 0; u < VB; ++u) {
-                re[u] = fma(a, xv[u].x, re[u]);
-                im[u] = fma(a, xv[u].y, im[u]);
+                const double sr = sum_group16(re[q][u]), si = sum_group16(im[q][u]);
+                if (j == 0 && v0 + u < V && row + 16 * q < n_rows)
+                    y[(row + 16 * q) * V + v0 + u] = make_double2(sr, si);
             }
-        }
-#pragma unroll
-        for (int u = 0; u < VB; ++u) {
-            const double sr = sum_group16(re[u]), si = sum_group16(im[u]);
-            if (j == 0 && v0 + u < V && live) y[r * V + v0 + u] = make_double2(sr, si);
-        }
     }
+}
+
+// Two rows a lane group: up to two encodings (with more a lane has loads enough in
+// flight) and two rounds of the workgroups the device holds (8 a CU).  One encoding, 512 000 mesh
+// rows: 30.6 -> 23.7 us, 216 000: 14.0 -> 11.8, 200 000 rows of 40: 28.6 -> 23.5; two
+// encodings: 36.1 -> 33.6, 17.1 -> 15.6, 32.1 -> 31.0.  Four: 57.3 -> 54.4, but 125 000 rows 15.6
+// -> 16.1.  Fewer rows leave CUs idle (27 000, two encodings: 3.5 -> 3.7 us; 2000 rows of
+// 500, one: 8.5 -> 15.4).
+static bool csr_two_rows(int64_t n_rows, int n_enc)
+{
+    return n_enc <= 2 && cdiv(n_rows, 32) >= (int64_t)16 * device_cu_count();
 }
 
 // ---------------------------------------------------------------------------
@@ -1373,15 +1407,20 @@ extern "C" int fm_csr_spmv_c128(int64_t n_rows, int n_enc, const int64_t *indptr
     if (n_rows == 0) return FM_OK;
     FM_CHECK_ARG(indptr && indices && data && x && y, "NULL array");
     FM_CHECK_ARG(cdiv(n_rows * 16, 256) <= 0x7fffffff, "too many rows for one launch");
-    const unsigned grid = xcd_grid(cdiv(n_rows, 16));
-    auto launch = [&](auto vb) {
-        k_csr_spmv_c128<decltype(vb)::value><<<grid, 256, 0, as_stream(stream)>>>(
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    auto launch = [&](auto vb, auto rows) {
+        constexpr int kRows = decltype(rows)::value;
+        k_csr_spmv_c128<decltype(vb)::value, kRows><<<xcd_grid(cdiv(n_rows, 16 * kRows)), 256, 0, as_stream(stream)>>>(
             n_rows, n_enc, indptr, indices, data, reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y));
     };
-    if (n_enc == 1) launch(std::integral_constant<int, 1>{});
-    else if (n_enc == 2) launch(std::integral_constant<int, 2>{});
-    else if (n_enc == 3) launch(std::integral_constant<int, 3>{});
-    else launch(std::integral_constant<int, 4>{});
+    const bool two = csr_two_rows(n_rows, n_enc);
+    if (n_enc == 1 && two) launch(One{}, Two{});
+    else if (n_enc == 2 && two) launch(Two{}, Two{});
+    else if (n_enc == 1) launch(One{}, One{});
+    else if (n_enc == 2) launch(Two{}, One{});
+    else if (n_enc == 3) launch(std::integral_constant<int, 3>{}, One{});
+    else launch(std::integral_constant<int, 4>{}, One{});
     FM_LAUNCH_CHECK("k_csr_spmv_c128");
     return FM_OK;
 }
