@@ -11,7 +11,7 @@
 // of a spiral, the spokes of a radial set) fill the lanes together.  Nodes
 // pass through LDS in chunks: the threads stage, per (node, group of the
 // tile), b exp(-t/T2), the off-resonance phase and for moving nodes the
-// position (one loop over the modes for four groups at a time); the lanes then
+// position (one loop over the modes for up to four groups at a time); the lanes then
 // read one record for their two samples, whose phases start from the staged
 // one (no instruction more than the product k.x, and one sine and cosine less
 // to round than with a staged factor).
@@ -36,12 +36,12 @@
 // so that several waves share a SIMD.  Measured, whole calls (before: tiles of two
 // 256-sample slots, one group to a slot or 32, 64, 128-sample groups packed,
 // 3 waves per SIMD):
-//   spiral, 973 000 nodes, 2048 x 32, mixed: 15.07 -> 13.1 ms (the FP32 series
-//   for the staged factors, 0.9 ms of it less with the hardware sine and
-//   cosine, takes the error against 64 bits from 7.8e-8 to 4.2e-8);
-//   spiral, 120 011 nodes, 1024 x 32, FP64: 6.53 -> 3.23 ms;
+//   spiral, 973 000 nodes, 2048 x 32, mixed: 15.06 -> 13.2-13.5 ms (the staged factors by
+//   FP32 series and their product in FP64, 0.5-0.9 ms of it less with the hardware sine and
+//   cosine, take the error against 64 bits from 7.8e-8 to 3.6e-8);
+//   spiral, 120 011 nodes, 1024 x 32, FP64: 6.54 -> 3.23-3.28 ms;
 //   radial, 200 003 moving nodes, 256 x 96, 8 modes, 2 encodings, mixed: 5.70 ->
-//   2.67 ms;
+//   2.65 ms;
 //   spiral, 138 519 nodes, 1504 x 48, mixed (per-sample t before): 5.49 -> 1.9 ms.
 #include <algorithm>
 #include <type_traits>
